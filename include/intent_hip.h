@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define INTENT_HIP_ABI_VERSION 17
+#define INTENT_HIP_ABI_VERSION 18
 
 enum IntentHipStatus {
   INTENT_HIP_OK = 0,
@@ -134,6 +134,17 @@ int intent_hip_gemm_bf16(const void *a, const void *b, void *c, int64_t m, int64
  * Casts round to nearest even. A [m,k], B [k,n], C [m,n], row strides lda/ldb/ldc. */
 int intent_hip_gemm(int dtype, int activation, const void *a, const void *b, void *c, int64_t m,
                     int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, void *stream);
+
+/* intent_hip_gemm with a K split for products of few rows and columns, the same definitions (no
+ * counterpart call in the reference: its launch has no workspace; the split changes only the
+ * association of the f32 sums). Where one workgroup per output tile would leave most of the chip idle,
+ * several take a share of K each, write f32 sums to `workspace`, and a second kernel adds them in
+ * order. The workspace must hold intent_hip_gemm_workspace_bytes (0: nothing to split) and be
+ * 16-byte aligned; with a null or smaller workspace the launch is unsplit, as intent_hip_gemm. */
+int intent_hip_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, size_t *bytes);
+int intent_hip_gemm_ws(int dtype, int activation, const void *a, const void *b, void *c, int64_t m,
+                       int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, void *workspace,
+                       size_t workspace_bytes, void *stream);
 
 /* f32 GEMM with f32 accumulation (no TF32).
  * transpose_b = 0: gemm_f32   (gemm.py:15-27), C = A @ B,   B [k,n];

@@ -28,6 +28,8 @@
 //   * tiles are walked in groups of 2 tile rows, column by column, in dispatch order: the
 //     tiles resident at one time share A row panels and B column panels, across XCDs
 //     through the MALL and within each XCD through its L2.
+// Calls of up to 128 rows run gemm_skinny instead (f16 relu 32 x 14336 x 4096: 221 us in 256 x 256 tiles,
+// 27.9 there).
 // Shapes the fast path cannot take (K or N not a multiple of 8, unaligned rows) use a
 // simple LDS-tiled f32 FMA kernel.
 #include "common.hpp"
@@ -36,6 +38,7 @@ namespace intent_hip {
 namespace {
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // Operand element type: __bf16 (bf16_gemm) or _Float16 (gemm). Fragments of 8 elements feed
 // v_mfma_f32_32x32x16_{bf16,f16}; results are stored 4 at a time.
@@ -46,12 +49,18 @@ template <> struct Elem<__bf16> {
   static __device__ __forceinline__ f32x16_t mma(x8 a, x8 b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f32x4_t mma16(x8 a, x8 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
 };
 template <> struct Elem<_Float16> {
   typedef _Float16 x8 __attribute__((ext_vector_type(8)));
   typedef _Float16 x4 __attribute__((ext_vector_type(4)));
   static __device__ __forceinline__ f32x16_t mma(x8 a, x8 b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4_t mma16(x8 a, x8 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
 };
 
@@ -485,6 +494,174 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_mfma(const uint16_t *__restr
     gemm_tile<E, Epi, true>(A, B, ep, M, N, K, lda, ldb, m0, n0, lds);
 }
 
+// ---------------------------------------------------------------- few rows: waves stream B, no LDS tiles
+// With few rows the time is the time to read B, and 256-row tiles would leave most of the chip idle and multiply
+// padding. A workgroup owns MT * 16 rows and 64 columns (128 bytes, one cache line, of each row of B; a CU
+// holds a bounded number of lines in flight, so half lines halve its rate). Its waves take
+// the 64-deep units of K in turn, loading straight into registers, the next unit in flight while the
+// current one is multiplied. Lane (g = l / 16, c = l % 16) loads rows 8 g + j (j = 0..7) of a
+// 32-deep step, columns 4 c .. 4 c + 3. Pairing the words of rows 2 p and 2 p + 1 with v_perm_b32
+// gives, for each i < 4, the 8 consecutive k of column 4 c + i that the MFMA takes, so MFMA i covers the columns
+// 4 c + i and a lane accumulates 16 consecutive columns of one row. The waves' sums meet in LDS and
+// are added in wave order.
+// One CU reads about 19 GB/s of B at most, so a call with few column blocks also divides K over workgroups
+// (blockIdx.y): each then writes its f32 sums to `partials` and gemm_splits adds them in order.
+constexpr int kSkinnyCols = 64;
+constexpr int kSkinnyUnit = 64;           // k of one unit (two 32-deep steps)
+constexpr int kSkinnyWaves = 8;
+constexpr int kSkinnyRows = 128;          // most rows a call may have to run here
+
+// 4 columns of one row of B: non-temporal where one row block reads B (nothing reads it again in the call).
+template <bool kStream>
+__device__ __forceinline__ uint2 load_columns(const uint16_t *p) {
+  if constexpr (kStream) return __builtin_bit_cast(uint2, __builtin_nontemporal_load(reinterpret_cast<const uint64_t *>(p)));
+  return *reinterpret_cast<const uint2 *>(p);
+}
+
+template <typename E, typename Epi, int MT, bool kStream>
+__global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_skinny(const uint16_t *__restrict__ A,
+                                                                 const uint16_t *__restrict__ B, Epi ep, int M, int N,
+                                                                 int K, int64_t lda, int64_t ldb, int tiles_m,
+                                                                 float *__restrict__ partials) {
+  typedef typename Elem<E>::x8 x8;
+  constexpr int kRows = MT * 16, kPad = kSkinnyCols + 4, W = kSkinnyWaves;
+  __shared__ float4 sums[W * kRows * kPad / 4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  // The row blocks of one column block share its B through the L2 of one XCD: consecutive workgroups
+  // go to the 8 XCDs in turn.
+  const int slot = blockIdx.x >> 3;
+  const int m0 = (slot % tiles_m) * kRows, n0 = ((slot / tiles_m) * 8 + (blockIdx.x & 7)) * kSkinnyCols;
+  if (n0 >= N) return;   // the last group of 8 column blocks may be short (uniform)
+  // Columns past N and rows past M read valid ones instead; their products are not stored.
+  const int n = n0 + 4 * c < N ? n0 + 4 * c : 0;
+  const uint32_t b_lane = static_cast<uint32_t>(8 * g) * static_cast<uint32_t>(ldb) + n;
+  uint32_t a_lane[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+    a_lane[t] = static_cast<uint32_t>(min(m0 + 16 * t + c, M - 1)) * static_cast<uint32_t>(lda) + 8 * g;
+
+  f32x4_t acc[MT][4];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[t][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // One whole 32-deep step starting at k0.
+  auto load_step = [&](int k0, uint2 (&b)[8], uint4 (&a)[MT]) {
+    const uint16_t *rows = B + static_cast<int64_t>(k0) * ldb;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b[j] = load_columns<kStream>(rows + j * ldb + b_lane);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) a[t] = *reinterpret_cast<const uint4 *>(A + k0 + a_lane[t]);
+  };
+  auto multiply = [&](const uint2 (&b)[8], const uint4 (&a)[MT]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint4 bt;
+      uint32_t *w = reinterpret_cast<uint32_t *>(&bt);
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        w[p] = __builtin_amdgcn_perm(i < 2 ? b[2 * p + 1].x : b[2 * p + 1].y, i < 2 ? b[2 * p].x : b[2 * p].y,
+                                     (i & 1) ? 0x07060302u : 0x05040100u);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t][i] = Elem<E>::mma16(__builtin_bit_cast(x8, bt), __builtin_bit_cast(x8, a[t]), acc[t][i]);
+    }
+  };
+
+  const int units = K / kSkinnyUnit;
+  const int first = static_cast<int>(static_cast<int64_t>(units) * blockIdx.y / gridDim.y);
+  const int last = static_cast<int>(static_cast<int64_t>(units) * (blockIdx.y + 1) / gridDim.y);
+  uint2 b[2][2][8];
+  uint4 a[2][2][MT];
+  auto load_unit = [&](int unit, int buffer) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) load_step(unit * kSkinnyUnit + 32 * u, b[buffer][u], a[buffer][u]);
+  };
+  auto multiply_unit = [&](int buffer) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) multiply(b[buffer][u], a[buffer][u]);
+  };
+  int unit = first + wave;
+  if (unit < last) load_unit(unit, 0);
+  for (; unit + W < last; unit += 2 * W) {
+    load_unit(unit + W, 1);
+    multiply_unit(0);
+    if (unit + 2 * W < last) load_unit(unit + 2 * W, 0);
+    multiply_unit(1);
+  }
+  if (unit < last) multiply_unit(0);
+  // The last K % 64 (a multiple of 8), by the next wave in turn of the last split: groups of 8 k
+  // past K are zero in both operands.
+  if (K % kSkinnyUnit != 0 && blockIdx.y == gridDim.y - 1 && wave == (last - first) % W) {
+    for (int k0 = units * kSkinnyUnit; k0 < K; k0 += 32) {
+      const bool live = k0 + 8 * g < K;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        b[0][0][j] = make_uint2(0u, 0u);
+        if (live) b[0][0][j] = *reinterpret_cast<const uint2 *>(B + (static_cast<int64_t>(k0) + j) * ldb + b_lane);
+      }
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        a[0][0][t] = make_uint4(0u, 0u, 0u, 0u);
+        if (live) a[0][0][t] = *reinterpret_cast<const uint4 *>(A + k0 + a_lane[t]);
+      }
+      multiply(b[0][0], a[0][0]);
+    }
+  }
+
+  // acc[t][i][r] is row 16 t + c, column 16 g + 4 r + i of this wave's share of the sum.
+  float *own = reinterpret_cast<float *>(sums) + wave * kRows * kPad;
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<float4 *>(own + (16 * t + c) * kPad + 16 * g + 4 * r) =
+          make_float4(acc[t][0][r], acc[t][1][r], acc[t][2][r], acc[t][3][r]);
+  __syncthreads();
+  const float *all = reinterpret_cast<const float *>(sums);
+  for (int quad = threadIdx.x; quad < kRows * kSkinnyCols / 4; quad += W * 64) {
+    const int row = quad / (kSkinnyCols / 4), col = 4 * (quad % (kSkinnyCols / 4));
+    if (m0 + row >= M || n0 + col >= N) continue;
+    float4 total = *reinterpret_cast<const float4 *>(all + row * kPad + col);
+#pragma unroll
+    for (int w = 1; w < W; ++w) {
+      const float4 v = *reinterpret_cast<const float4 *>(all + (w * kRows + row) * kPad + col);
+      total.x += v.x;
+      total.y += v.y;
+      total.z += v.z;
+      total.w += v.w;
+    }
+    if (partials != nullptr)
+      *reinterpret_cast<float4 *>(partials + (static_cast<int64_t>(blockIdx.y) * M + m0 + row) * N + n0 + col) = total;
+    else
+      ep.quad(m0 + row, n0 + col, total.x, total.y, total.z, total.w);
+  }
+}
+
+// Adds the K splits of a product in order and stores the result: one thread per 4 columns.
+template <typename Epi>
+__global__ __launch_bounds__(256) void gemm_splits(const float *__restrict__ partials, Epi ep, int M, int N, int splits) {
+  const int quads = N / 4;
+  const int64_t quad = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (quad >= static_cast<int64_t>(M) * quads) return;
+  const int row = static_cast<int>(quad / quads), col = 4 * static_cast<int>(quad % quads);
+  const int64_t split = static_cast<int64_t>(M) * N;
+  const float *p = partials + static_cast<int64_t>(row) * N + col;
+  float4 total = *reinterpret_cast<const float4 *>(p);
+#pragma unroll 8
+  for (int s = 1; s < splits; ++s) {
+    const float4 v = *reinterpret_cast<const float4 *>(p + s * split);
+    total.x += v.x;
+    total.y += v.y;
+    total.z += v.z;
+    total.w += v.w;
+  }
+  ep.quad(row, col, total.x, total.y, total.z, total.w);
+}
+
 // ---------------------------------------------------------------- general-shape fallback
 // 64 x 64 output tile per 256 threads (4 x 4 per thread), K in steps of 16 through LDS,
 // f32 fused multiply-add in increasing k.
@@ -539,22 +716,72 @@ int quantized_gemm_resources(IntentHipKernelResources *out) {
                          kThreads, out);
 }
 
+namespace {
+
+template <typename E>
+int resources_of(int64_t m, const char *few, const char *tiles, IntentHipKernelResources *out) {
+  typedef CastStore<E, 0> Epi;
+  const void *kernel = m <= 16   ? reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 1, true>)
+                       : m <= 32 ? reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 2, true>)
+                       : m <= 64 ? reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 4, true>)
+                                 : reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 4, false>);
+  if (m <= kSkinnyRows) return describe_kernel(kernel, few, kSkinnyWaves * 64, out);
+  return describe_kernel(reinterpret_cast<const void *>(&gemm_mfma<E, Epi>), tiles, kThreads, out);
+}
+
+}  // namespace
+
 int gemm_resources(int dtype, int64_t m, int64_t n, IntentHipKernelResources *out) {
-  (void)m;
   (void)n;
-  if (dtype == INTENT_HIP_F16)
-    return describe_kernel(reinterpret_cast<const void *>(&gemm_mfma<_Float16, CastStore<_Float16, 0>>), "gemm_mfma<f16>",
-                           kThreads, out);
-  return describe_kernel(reinterpret_cast<const void *>(&gemm_mfma<__bf16, CastStore<__bf16, 0>>), "gemm_mfma<bf16>",
-                         kThreads, out);
+  return dtype == INTENT_HIP_F16 ? resources_of<_Float16>(m, "gemm_skinny<f16>", "gemm_mfma<f16>", out)
+                                 : resources_of<__bf16>(m, "gemm_skinny<bf16>", "gemm_mfma<bf16>", out);
 }
 
 namespace {
 
-// The MFMA kernel when `fast` (the operand shape and layout it takes), else the general one.
+// Workgroups along K of a few-row product: enough that every CU reads a share of B. The second
+// launch costs about 3 us, which the split returns from 2048 rows of B on (m 16, n 1024: k 1024 4.5 us
+// unsplit against 6.7, k 2048 7.9 against 7.5; n 2048, k 8192: 37.4 against 12.2; m 64, n = k = 4096:
+// 33.1 against 15.5).
+int skinny_splits(int64_t m, int64_t n, int64_t k) {
+  if (m < 1 || n < 1 || m > kSkinnyRows || k < 2048) return 1;
+  const int64_t blocks = (n + kSkinnyCols - 1) / kSkinnyCols * (m <= 64 ? 1 : 2);
+  const int64_t splits = 256 / blocks < k / 256 ? 256 / blocks : k / 256;
+  return splits < 2 ? 1 : static_cast<int>(splits);
+}
+
+template <typename E, typename Epi, int MT, bool kStream>
+void launch_skinny(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, int n, int k, int64_t lda, int64_t ldb,
+                   float *partials, int splits, hipStream_t s) {
+  const int tiles_m = (m + 16 * MT - 1) / (16 * MT), tiles_n = (n + kSkinnyCols - 1) / kSkinnyCols;
+  gemm_skinny<E, Epi, MT, kStream><<<dim3((tiles_n + 7) / 8 * 8 * tiles_m, splits), dim3(kSkinnyWaves * 64), 0, s>>>(
+      A, B, ep, m, n, k, lda, ldb, tiles_m, splits > 1 ? partials : nullptr);
+  if (splits > 1) {
+    const int64_t quads = static_cast<int64_t>(m) * n / 4;
+    gemm_splits<Epi><<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, ep, m, n, splits);
+  }
+}
+
+// Few rows, and strides that keep a lane's offset (24 rows of B, all rows of A) below 2^31 elements.
+bool skinny(int64_t m, int64_t lda, int64_t ldb) {
+  return m <= kSkinnyRows && lda < (int64_t{1} << 22) && ldb < (int64_t{1} << 25);
+}
+
+// The MFMA kernels when `fast` (the operand shape and layout they take), else the general one.
+// `partials`: null, or room for the f32 sums of skinny_splits(m, n, k) splits.
 template <typename E, typename Epi>
 int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t m, int64_t n, int64_t k, int64_t lda,
-                    int64_t ldb, bool fast, hipStream_t s) {
+                    int64_t ldb, bool fast, float *partials, hipStream_t s) {
+  if (k > 0 && fast && skinny(m, lda, ldb)) {
+    const int splits = partials != nullptr ? skinny_splits(m, n, k) : 1;
+    const int M = static_cast<int>(m), N = static_cast<int>(n), depth = static_cast<int>(k);
+    if (m <= 16) launch_skinny<E, Epi, 1, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
+    else if (m <= 32) launch_skinny<E, Epi, 2, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
+    else if (m <= 64) launch_skinny<E, Epi, 4, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
+    else launch_skinny<E, Epi, 4, false>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
+    if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_skinny");
+    return INTENT_HIP_OK;
+  }
   if (k > 0 && fast) {
     const int tiles_m = static_cast<int>((m + kBM - 1) / kBM), tiles_n = static_cast<int>((n + kBN - 1) / kBN);
     gemm_mfma<E, Epi><<<dim3(tiles_m * tiles_n), dim3(kThreads), 0, s>>>(
@@ -569,9 +796,15 @@ int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t
   return INTENT_HIP_OK;
 }
 
+// Bytes of the f32 partial sums of a product's K splits (0: one workgroup per output tile).
+size_t splits_bytes(int64_t m, int64_t n, int64_t k) {
+  const int splits = skinny_splits(m, n, k);
+  return splits > 1 ? static_cast<size_t>(splits) * m * n * sizeof(float) : 0;
+}
+
 template <typename E, int kAct>
 int launch_gemm(const void *a, const void *b, void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
-                int64_t ldc, void *stream) {
+                int64_t ldc, void *stream, void *workspace = nullptr, size_t workspace_bytes = 0) {
   if (m < 0 || n < 0 || k < 0) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "negative extent");
   if (m > INT32_MAX / 2 || n > INT32_MAX / 2 || k > INT32_MAX / 2)
     return fail(INTENT_HIP_ERR_UNSUPPORTED, "GEMM extents must stay below 2^30");
@@ -585,7 +818,9 @@ int launch_gemm(const void *a, const void *b, void *c, int64_t m, int64_t n, int
   const auto *A = static_cast<const uint16_t *>(a);
   const auto *B = static_cast<const uint16_t *>(b);
   const CastStore<E, kAct> ep{static_cast<uint16_t *>(c), ldc};
-  return launch_epilogue<E>(A, B, ep, m, n, k, lda, ldb, fast_path(a, b, c, n, k, lda, ldb, ldc), s);
+  const bool room = workspace != nullptr && aligned(workspace, 16) && workspace_bytes >= splits_bytes(m, n, k);
+  return launch_epilogue<E>(A, B, ep, m, n, k, lda, ldb, fast_path(a, b, c, n, k, lda, ldb, ldc),
+                            room ? static_cast<float *>(workspace) : nullptr, s);
 }
 
 }  // namespace
@@ -598,17 +833,29 @@ extern "C" int intent_hip_gemm_bf16(const void *a, const void *b, void *c, int64
   return launch_gemm<__bf16, 0>(a, b, c, m, n, k, lda, ldb, ldc, stream);
 }
 
-extern "C" int intent_hip_gemm(int dtype, int activation, const void *a, const void *b, void *c, int64_t m, int64_t n,
-                               int64_t k, int64_t lda, int64_t ldb, int64_t ldc, void *stream) {
+extern "C" int intent_hip_gemm_ws(int dtype, int activation, const void *a, const void *b, void *c, int64_t m,
+                                  int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, void *workspace,
+                                  size_t workspace_bytes, void *stream) {
   if (activation != 0 && activation != 1)
     return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "activation code %d (0 = none, 1 = relu)", activation);
-  if (dtype == INTENT_HIP_F16)
-    return activation ? launch_gemm<_Float16, 1>(a, b, c, m, n, k, lda, ldb, ldc, stream)
-                      : launch_gemm<_Float16, 0>(a, b, c, m, n, k, lda, ldb, ldc, stream);
-  if (dtype == INTENT_HIP_BF16)
-    return activation ? launch_gemm<__bf16, 1>(a, b, c, m, n, k, lda, ldb, ldc, stream)
-                      : launch_gemm<__bf16, 0>(a, b, c, m, n, k, lda, ldb, ldc, stream);
+  const auto launch = [&](auto run) {
+    return run(a, b, c, m, n, k, lda, ldb, ldc, stream, workspace, workspace_bytes);
+  };
+  if (dtype == INTENT_HIP_F16) return activation ? launch(launch_gemm<_Float16, 1>) : launch(launch_gemm<_Float16, 0>);
+  if (dtype == INTENT_HIP_BF16) return activation ? launch(launch_gemm<__bf16, 1>) : launch(launch_gemm<__bf16, 0>);
   return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "16-bit GEMM dtype code %d (1 = f16, 2 = bf16)", dtype);
+}
+
+extern "C" int intent_hip_gemm(int dtype, int activation, const void *a, const void *b, void *c, int64_t m, int64_t n,
+                               int64_t k, int64_t lda, int64_t ldb, int64_t ldc, void *stream) {
+  return intent_hip_gemm_ws(dtype, activation, a, b, c, m, n, k, lda, ldb, ldc, nullptr, 0, stream);
+}
+
+extern "C" int intent_hip_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, size_t *bytes) {
+  if (bytes == nullptr) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "null output");
+  if (m < 0 || n < 0 || k < 0) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "negative extent");
+  *bytes = splits_bytes(m, n, k);
+  return INTENT_HIP_OK;
 }
 
 extern "C" int intent_hip_quantized_gemm(const void *a, const void *b, const float *bias, const void *residual,
@@ -629,5 +876,5 @@ extern "C" int intent_hip_quantized_gemm(const void *a, const void *b, const flo
   const bool fast = k % 8 == 0 && n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned(a, 16) && aligned(b, 16) &&
                     ldr % 4 == 0 && aligned(residual, 8) && ldo % 4 == 0 && aligned(out, 4);
   return launch_epilogue<_Float16>(static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(b), ep, m, n, k, lda,
-                                   ldb, fast, as_stream(stream));
+                                   ldb, fast, nullptr, as_stream(stream));
 }

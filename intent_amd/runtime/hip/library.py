@@ -11,7 +11,7 @@ from pathlib import Path
 
 from ...diagnostics import CompilationStageError
 
-ABI_VERSION = 17
+ABI_VERSION = 18
 # INTENT_HIP_STATIC_SCRATCH_BYTES: the static scratch of intent_hip_csr_spmv_f32_static.
 STATIC_SCRATCH_BYTES = 32 << 20
 LIBRARY_NAME = "libintent_hip.so"
@@ -54,6 +54,8 @@ SIGNATURES = {
     "intent_hip_softmax_bwd": (_int, (_int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p)),
     "intent_hip_gemm_bf16": (_int, (_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p)),
     "intent_hip_gemm": (_int, (_int, _int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p)),
+    "intent_hip_gemm_workspace_bytes": (_int, (_i64, _i64, _i64, ctypes.POINTER(_sz))),
+    "intent_hip_gemm_ws": (_int, (_int, _int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p, _sz, _p)),
     "intent_hip_gemm_f32": (_int, (_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p)),
     "intent_hip_gemm_i8": (_int, (_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p)),
     "intent_hip_quantized_gemm": (_int, (_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p)),

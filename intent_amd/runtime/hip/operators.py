@@ -302,18 +302,39 @@ def _softmax_bwd(dtype_code):
 
 
 # ------------------------------------------------------------------------------ GEMM
-def _gemm_bf16(lib, bound, constexprs, device):
-    a, b, c = bound.arguments
+def _gemm_launch(lib, dtype_code, activation, a, b, c, entry, configuration, device):
+    """A 16-bit product. One of few rows and columns divides K over workgroups through a workspace of
+    f32 sums (none with workspace='static': one workgroup per output tile)."""
+    import ctypes
+
+    import torch
+
     keep, before, after = [a, b, c], [], []
     ak, bk, ck = _readable(a, keep, before), _readable(b, keep, before), _writable(c, keep, after)
     m, k = a.shape
     n = b.shape[1]
-    fn = lib.fn["gemm_bf16"]
-    args = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk),
-            _row_stride(ck))
-    return Launch("intent_hip_gemm_bf16", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
-                  tuple(after), (("m", m), ("n", n), ("k", k)),
-                  lambda: lib.kernel_resources(OP_GEMM_BF16, BF16, m, n))
+    operands = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk),
+                _row_stride(ck))
+    facts = (("m", m), ("n", n), ("k", k)) + configuration
+    op = OP_GEMM_BF16 if entry == "intent_hip_gemm_bf16" else OP_GEMM
+    resources = lambda: lib.kernel_resources(op, dtype_code, m, n)  # noqa: E731
+    size = ctypes.c_size_t(0)
+    lib.check(lib.fn["gemm_workspace_bytes"](m, n, k, ctypes.byref(size)), "provider_preparation")
+    if size.value and not _static_workspace():
+        workspace = torch.empty(size.value, dtype=torch.uint8, device=device)
+        keep.append(workspace)
+        fn = lib.fn["gemm_ws"]
+        args = (dtype_code, activation, *operands, workspace.data_ptr(), size.value)
+        return Launch("intent_hip_gemm_ws", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
+                      tuple(after), facts + (("workspace_bytes", size.value),), resources)
+    fn = lib.fn[entry[len("intent_hip_"):]]
+    args = operands if entry == "intent_hip_gemm_bf16" else (dtype_code, activation, *operands)
+    return Launch(entry, lambda stream: fn(*args, stream), tuple(keep), tuple(before), tuple(after), facts,
+                  resources)
+
+
+def _gemm_bf16(lib, bound, constexprs, device):
+    return _gemm_launch(lib, BF16, 0, *bound.arguments, "intent_hip_gemm_bf16", (), device)
 
 
 def _activation_code(value) -> int:
@@ -327,18 +348,9 @@ def _activation_code(value) -> int:
 
 def _gemm16(dtype_code):
     def plan(lib, bound, constexprs, device):
-        a, b, c = bound.arguments
         activation = _activation_code(constexprs.get("ACTIVATION", 0))
-        keep, before, after = [a, b, c], [], []
-        ak, bk, ck = _readable(a, keep, before), _readable(b, keep, before), _writable(c, keep, after)
-        m, k = a.shape
-        n = b.shape[1]
-        fn = lib.fn["gemm"]
-        args = (dtype_code, activation, ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak),
-                _row_stride(bk), _row_stride(ck))
-        return Launch("intent_hip_gemm", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
-                      tuple(after), (("m", m), ("n", n), ("k", k), ("activation", activation)),
-                      lambda: lib.kernel_resources(OP_GEMM, dtype_code, m, n))
+        return _gemm_launch(lib, dtype_code, activation, *bound.arguments, "intent_hip_gemm",
+                            (("activation", activation),), device)
     return plan
 
 

@@ -83,3 +83,31 @@ def test_gemm_config3_full(device):
     got = bf16_tensor_bits(c)[rows]
     assert_16bit(bf16_to_f32(got), bf16_to_f32(want))
     assert (np.abs(got.astype(np.int32) - want.astype(np.int32)) <= 2).mean() > 0.999
+
+
+# The few-row kernel: row blocks of 16, 32 and 64 and their edges, two row blocks (m > 64), column
+# counts below and past one 64-column workgroup, K below one 64-deep unit, past it by every multiple
+# of 8, and long enough that K is divided over workgroups (from 2048 rows on; 2056 leaves a tail).
+@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (15, 64, 24), (16, 72, 40), (17, 56, 64), (32, 520, 56), (33, 136, 72),
+                                   (64, 64, 120), (65, 200, 1000), (128, 72, 520), (1, 24, 2048), (31, 1000, 2056),
+                                   (100, 136, 4104), (128, 8, 2048), (3, 16384, 2048)])
+@pytest.mark.parametrize("workspace", ["prepare", "static"])
+def test_gemm_few_rows(device, m, n, k, workspace):
+    """Against the oracle, and exact on small integers whose sums f32 holds (an element read from the wrong place,
+    twice or not at all shows); rows of NaN in A and columns of NaN in B stay in their own row and
+    column of C, so no padding row, column or K group reaches a result."""
+    announce("gemm few rows", m, n, k, workspace)
+    kernel = intent.jit(bf16_gemm, backend="hip", backend_options={"workspace": workspace})
+    call = lambda a, b: bf16_tensor_bits(kernel.run(to_bf16_tensor(a, device), to_bf16_tensor(b, device)))  # noqa: E731
+    a, b = inputs.gemm_bf16(seed=m + n + k, m=m, n=n, k=k)
+    got, want = call(a, b), oracle.gemm_bf16(a, b)
+    assert_16bit(bf16_to_f32(got), bf16_to_f32(want))
+    assert (np.abs(got.astype(np.int32) - want.astype(np.int32)) <= 2).mean() > 0.999
+    rng = np.random.default_rng(m * n + k)
+    ints = [inputs._bf16_bits(rng.integers(-2, 3, shape).astype(np.float32)) for shape in ((m, k), (k, n))]
+    assert (call(*ints) == oracle.gemm_bf16(*ints)).all()
+    a[m - 1, k - 1] = b[0, n - 1] = 0x7FC0
+    nan = np.isnan(bf16_to_f32(call(a, b)))
+    expected = np.zeros((m, n), bool)
+    expected[m - 1, :] = expected[:, n - 1] = True
+    assert (nan == expected).all()
