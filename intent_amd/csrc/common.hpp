@@ -114,11 +114,8 @@ __device__ __forceinline__ f16_t from_f32<f16_t>(float v) {
 }
 template <>
 __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) {
-  // Round to nearest even on the bit pattern; NaN stays a (quiet) NaN.
-  uint32_t u = __float_as_uint(v);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return bf16_t{static_cast<uint16_t>((u >> 16) | 0x40u)};
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return bf16_t{static_cast<uint16_t>(u >> 16)};
+  // v_cvt_pk_bf16_f32: round to nearest even; NaN stays a (quiet) NaN.
+  return bf16_t{__builtin_bit_cast(uint16_t, round_to<__bf16>(v))};
 }
 
 }  // namespace intent_hip

@@ -17,9 +17,9 @@
 // before it computes the current one, so the reads of one row overlap the exponentials of the
 // previous (16384 x 4096 f16: 46.7 against 52 us, bit-identical; one wave per row and launch
 // leaves HBM idle while a whole round of waves computes).
-// Rows longer than the register-resident limit, or rows whose layout rules out 128-bit
-// access, use a scalar variant; rows longer than 64 * 64 scalar elements use a streaming
-// variant that re-reads the row (3 passes forward, 2 backward).
+// Longer rows, and rows whose layout rules out aligned 128-bit access, belong to a workgroup
+// (softmax_*_block), which holds them in registers too, up to 131072 16-bit or 65536 f32 elements (forward;
+// backward half of that); rows beyond are read again in each pass (softmax_*_stream).
 #include <math.h>
 
 #include <algorithm>
@@ -190,47 +190,6 @@ __global__ __launch_bounds__(kBlock) void softmax_fwd_wave(const T *x, T *y, int
   const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
   if (row >= rows) return;  // wave-uniform
   const T *xr = x + row * xs;
-  if constexpr (std::is_same<T, f16_t>::value && V == 8) {
-    // x stays in its raw f16 words until the exponentials replace it: 79 VGPRs instead of 90,
-    // six waves per SIMD instead of five (forward of the 16384 x 4096 step, bit-identical:
-    // 51.2 against 53.4 us). Loads are unconditional, as in the backward.
-    u32x4_t xw[CHUNKS];
-    float m = -INFINITY;
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const int col = (c * kWave + lane) * V;
-      const bool live = col < cols;
-      xw[c] = load_words(xr + (live ? col : 0));
-#pragma unroll
-      for (int i = 0; i < V; ++i) m = live ? fmaxf(m, widen<T>(xw[c], i)) : m;
-    }
-    m = wave_max(m);
-    float v[CHUNKS][V];
-    float s = 0.0f;
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const bool live = (c * kWave + lane) * V < cols;
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        v[c][i] = live ? shifted_exp<T>(widen<T>(xw[c], i), m) : 0.0f;
-        s += v[c][i];
-      }
-    }
-    s = wave_sum(s);
-    const float r = 1.0f / s;
-    T *yr = y + row * ys;
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const int col = (c * kWave + lane) * V;
-      if (col < cols) {
-        float o[V];
-#pragma unroll
-        for (int i = 0; i < V; ++i) o[i] = quotient(v[c][i], s, r);
-        store_row_chunk<T, V, false>(yr + col, o);
-      }
-    }
-    return;
-  }
   float v[CHUNKS][V];
   float m = -INFINITY;
 #pragma unroll
@@ -271,25 +230,227 @@ __global__ __launch_bounds__(kBlock) void softmax_fwd_wave(const T *x, T *y, int
   }
 }
 
-// ---------------------------------------------------------------- forward, streaming
+// ---------------------------------------------------------------- rows of a workgroup
+// A row as its 16-byte chunks: chunk q holds columns [q V - shift, q V - shift + V), where shift (0 when
+// the row starts at a 16-byte boundary) makes every chunk of x (of p) a 16-byte aligned address. Chunks
+// that reach past an end of the row are written one element at a time, and read so where they would leave
+// the operand; so is every chunk of another operand whose rows are aligned differently.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void softmax_fwd_stream(const T *x, T *y, int64_t rows, int cols,
-                                                             int64_t xs, int64_t ys) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const T *xr = x + row * xs;
-  float m = -INFINITY;
-  for (int c = lane; c < cols; c += kWave) m = fmaxf(m, to_f32(xr[c]));
-  m = wave_max(m);
-  float s = 0.0f;
-  for (int c = lane; c < cols; c += kWave) s += shifted_exp<T>(to_f32(xr[c]), m);
-  s = wave_sum(s);
-  const float r = 1.0f / s;
-  T *yr = y + row * ys;
-  for (int c = lane; c < cols; c += kWave) {
-    const float e = shifted_exp<T>(to_f32(xr[c]), m);
-    yr[c] = from_f32<T>(sizeof(T) == 4 ? e * r : quotient(e, s, r));
+constexpr int kChunk = 16 / sizeof(T);
+
+template <typename T>
+__device__ __forceinline__ int row_shift(const T *row) {
+  return static_cast<int>((reinterpret_cast<uintptr_t>(row) & 15) / sizeof(T));
+}
+
+template <typename T>
+__device__ __forceinline__ uint32_t element_bits(T v) {
+  if constexpr (sizeof(T) == 4) return __float_as_uint(v);
+  else return v.bits;
+}
+
+// Element i of a chunk, widened.
+template <typename T>
+__device__ __forceinline__ float element(const u32x4_t &w, int i) {
+  if constexpr (sizeof(T) == 4) {
+    const uint32_t word = w[i];
+    return __uint_as_float(word);
+  } else {
+    return widen<T>(w, i);
+  }
+}
+
+// Two 16-bit or one 32-bit -infinity: what the forward puts for elements outside the row (the maximum
+// and the sum are those of the row alone: exp(-inf - m) is 0, and where m is -inf the row's own sum is NaN).
+template <typename T>
+constexpr uint32_t kMinusInf = sizeof(T) == 4                   ? 0xff800000u
+                               : std::is_same<T, f16_t>::value ? 0xfc00fc00u
+                                                               : 0xff80ff80u;
+
+// The bytes from an operand's first element to its last: what a row's edge chunks may read (the neighbouring rows'
+// elements there, or the gap between rows, are replaced after the load).
+struct Span {
+  uintptr_t begin, end;
+};
+template <typename T>
+__device__ __forceinline__ Span span_of(const T *base, int64_t rows, int cols, int64_t stride) {
+  return {reinterpret_cast<uintptr_t>(base), reinterpret_cast<uintptr_t>(base + (rows - 1) * stride + cols)};
+}
+
+// The chunk at `start`, elements outside the row as in `outside`. kRagged false: chunks lie wholly
+// inside or wholly outside the row and are aligned.
+template <typename T, bool kRagged>
+__device__ __forceinline__ u32x4_t load_chunk(const T *row, int start, int cols, bool whole, uint32_t outside,
+                                              const Span &span) {
+  constexpr int V = kChunk<T>;
+  u32x4_t w;
+  if constexpr (!kRagged) {
+    const bool live = start < cols;
+    w = load_words(row + (live ? start : 0));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = live ? w[k] : outside;
+  } else {
+    w = u32x4_t{outside, outside, outside, outside};
+    const uintptr_t at = reinterpret_cast<uintptr_t>(row) + static_cast<int64_t>(start) * sizeof(T);
+    if (start >= cols) return w;
+    if (whole && at >= span.begin && at + 16 <= span.end) {
+      w = load_words(row + start);
+      if (start < 0 || start + V > cols) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const bool keep = start + i >= 0 && start + i < cols;
+          if constexpr (sizeof(T) == 4) w[i] = keep ? w[i] : outside;
+          else w[i / 2] = keep ? w[i / 2] : (i & 1) ? (w[i / 2] & 0xffffu) | (outside & 0xffff0000u)
+                                                    : (w[i / 2] & 0xffff0000u) | (outside & 0xffffu);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        if (start + i < 0 || start + i >= cols) continue;
+        const uint32_t bits = element_bits<T>(row[start + i]);
+        if constexpr (sizeof(T) == 4) w[i] = bits;
+        else w[i / 2] = (i & 1) ? (w[i / 2] & 0xffffu) | (bits << 16) : (w[i / 2] & 0xffff0000u) | bits;
+      }
+    }
+  }
+  return w;
+}
+
+// Keeps a chunk's raw words: without it the compiler keeps the widened elements of one pass for the
+// next, twice the registers (and spills at 1024 threads).
+__device__ __forceinline__ void keep_raw(u32x4_t &w) { asm("" : "+v"(w)); }
+
+template <typename T, bool kRagged, bool kStream>
+__device__ __forceinline__ void store_chunk(T *row, int start, int cols, bool whole, const float (&in)[kChunk<T>]) {
+  constexpr int V = kChunk<T>;
+  if (!kRagged ? start < cols : whole && start >= 0 && start + V <= cols) {
+    store_row_chunk<T, V, kStream>(row + start, in);
+  } else if (kRagged) {
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (start + i >= 0 && start + i < cols) row[start + i] = from_f32<T>(in[i]);
+  }
+}
+
+// Maximum / sum over a workgroup, in wave order. `parts` holds one value per wave; two calls in a row
+// take different arrays, so one barrier each is enough.
+template <int THREADS, bool kMax>
+__device__ __forceinline__ float block_reduce(float v, float *parts) {
+  v = kMax ? wave_max(v) : wave_sum(v);
+  if constexpr (THREADS > kWave) {
+    if ((threadIdx.x & (kWave - 1)) == 0) parts[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = parts[0];
+#pragma unroll
+    for (int w = 1; w < THREADS / kWave; ++w) v = kMax ? fmaxf(v, parts[w]) : v + parts[w];
+  }
+  return v;
+}
+
+// One workgroup per row (grid stride), the row in registers as raw words until its exponentials
+// replace them; from 16 chunks of 16-bit elements on, the exponentials are computed again for the output instead
+// (they would take the registers of half the waves). Bound by HBM: bf16 2048 x 32000 in 46 us,
+// 5.7 TB/s (548 us with a wave per row, 2-byte accesses and three passes over the row; 4096 x 9001 33
+// against 165; backward f16 1024 x 32000 34 against 403).
+// THREADS threads per row; rows of one wave go four to a workgroup (16384 x 129 f16: 12.9 us with
+// one each).
+template <int THREADS>
+constexpr int kBlockRows = THREADS == kWave ? 4 : 1;
+
+template <typename T, int THREADS, int CHUNKS, bool kRagged>
+__global__ __launch_bounds__(THREADS * kBlockRows<THREADS>) void softmax_fwd_block(const T *x, T *y, int64_t rows, int cols, int64_t xs,
+                                                             int64_t ys) {
+  constexpr int V = kChunk<T>;
+  constexpr bool kHold = CHUNKS * V <= 64;
+  constexpr int kRows = kBlockRows<THREADS>;
+  __shared__ float maxima[THREADS / kWave], sums[THREADS / kWave];
+  const int thread = kRows > 1 ? threadIdx.x % THREADS : threadIdx.x;
+  const Span span = span_of(x, rows, cols, xs);
+  for (int64_t row = static_cast<int64_t>(blockIdx.x) * kRows + threadIdx.x / THREADS; row < rows;
+       row += static_cast<int64_t>(gridDim.x) * kRows) {
+    const T *xr = x + row * xs;
+    T *yr = y + row * ys;
+    const int shift = kRagged ? row_shift(xr) : 0;
+    const bool whole = !kRagged || row_shift(yr) == shift;
+    const int at = thread * V - shift;
+    u32x4_t w[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) w[c] = load_chunk<T, kRagged>(xr, at + c * THREADS * V, cols, true, kMinusInf<T>, span);
+    float m = -INFINITY;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+      for (int i = 0; i < V; ++i) m = fmaxf(m, element<T>(w[c], i));
+    m = block_reduce<THREADS, true>(m, maxima);
+    float v[kHold ? CHUNKS : 1][V];
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      keep_raw(w[c]);
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        const float e = shifted_exp<T>(element<T>(w[c], i), m);
+        if constexpr (kHold) v[c][i] = e;
+        s += e;
+      }
+    }
+    s = block_reduce<THREADS, false>(s, sums);
+    const float r = 1.0f / s;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      if constexpr (!kHold) keep_raw(w[c]);
+      float o[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        const float e = kHold ? v[kHold ? c : 0][i] : shifted_exp<T>(element<T>(w[c], i), m);
+        o[i] = sizeof(T) == 4 ? e * r : quotient(e, s, r);
+      }
+      store_chunk<T, kRagged, false>(yr, at + c * THREADS * V, cols, whole, o);
+    }
+  }
+}
+
+// Rows that no workgroup's registers hold: the row is read once for each of the maximum, the sum and the output.
+constexpr int kStreamBlock = 1024;
+
+template <typename T>
+__global__ __launch_bounds__(kStreamBlock) void softmax_fwd_stream(const T *x, T *y, int64_t rows, int cols,
+                                                                   int64_t xs, int64_t ys) {
+  constexpr int V = kChunk<T>;
+  __shared__ float maxima[kStreamBlock / kWave], sums[kStreamBlock / kWave];
+  const Span span = span_of(x, rows, cols, xs);
+  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+    const T *xr = x + row * xs;
+    T *yr = y + row * ys;
+    const int shift = row_shift(xr);
+    const bool whole = row_shift(yr) == shift;
+    const int64_t first = static_cast<int64_t>(threadIdx.x) * V - shift;
+    float m = -INFINITY;
+    for (int64_t at = first; at < cols; at += kStreamBlock * V) {
+      const u32x4_t w = load_chunk<T, true>(xr, static_cast<int>(at), cols, true, kMinusInf<T>, span);
+#pragma unroll
+      for (int i = 0; i < V; ++i) m = fmaxf(m, element<T>(w, i));
+    }
+    m = block_reduce<kStreamBlock, true>(m, maxima);
+    float s = 0.0f;
+    for (int64_t at = first; at < cols; at += kStreamBlock * V) {
+      const u32x4_t w = load_chunk<T, true>(xr, static_cast<int>(at), cols, true, kMinusInf<T>, span);
+#pragma unroll
+      for (int i = 0; i < V; ++i) s += shifted_exp<T>(element<T>(w, i), m);
+    }
+    s = block_reduce<kStreamBlock, false>(s, sums);
+    const float r = 1.0f / s;
+    for (int64_t at = first; at < cols; at += kStreamBlock * V) {
+      const u32x4_t w = load_chunk<T, true>(xr, static_cast<int>(at), cols, true, kMinusInf<T>, span);
+      float o[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        const float e = shifted_exp<T>(element<T>(w, i), m);
+        o[i] = sizeof(T) == 4 ? e * r : quotient(e, s, r);
+      }
+      store_chunk<T, true, false>(yr, static_cast<int>(at), cols, whole, o);
+    }
   }
 }
 
@@ -366,44 +527,150 @@ __global__ __launch_bounds__(kBlock) void softmax_bwd_wave(const T *p, const T *
   }
 }
 
+// One workgroup per row (grid stride), p and dy in registers as raw words.
+template <typename T, int THREADS, int CHUNKS, bool kRagged>
+__global__ __launch_bounds__(THREADS * kBlockRows<THREADS>) void softmax_bwd_block(const T *p, const T *dy, T *dx, int64_t rows, int cols,
+                                                             int64_t ps, int64_t dys, int64_t dxs) {
+  constexpr int V = kChunk<T>;
+  constexpr int kRows = kBlockRows<THREADS>;
+  __shared__ float sums[2][THREADS / kWave];
+  const int thread = kRows > 1 ? threadIdx.x % THREADS : threadIdx.x;
+  const Span span_p = span_of(p, rows, cols, ps), span_g = span_of(dy, rows, cols, dys);
+  int turn = 0;
+  for (int64_t row = static_cast<int64_t>(blockIdx.x) * kRows + threadIdx.x / THREADS; row < rows;
+       row += static_cast<int64_t>(gridDim.x) * kRows, turn ^= 1) {
+    const T *pr = p + row * ps;
+    const T *gr = dy + row * dys;
+    T *dr = dx + row * dxs;
+    const int shift = kRagged ? row_shift(pr) : 0;
+    const bool whole_g = !kRagged || row_shift(gr) == shift, whole_d = !kRagged || row_shift(dr) == shift;
+    const int at = thread * V - shift;
+    u32x4_t pw[CHUNKS], gw[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      pw[c] = load_chunk<T, kRagged>(pr, at + c * THREADS * V, cols, true, 0, span_p);
+      gw[c] = load_chunk<T, kRagged>(gr, at + c * THREADS * V, cols, whole_g, 0, span_g);
+    }
+    float proj = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+      for (int i = 0; i < V; ++i) proj = fmaf(element<T>(pw[c], i), element<T>(gw[c], i), proj);
+    proj = block_reduce<THREADS, false>(proj, sums[turn]);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      keep_raw(pw[c]);
+      keep_raw(gw[c]);
+      float o[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) o[i] = element<T>(pw[c], i) * (element<T>(gw[c], i) - proj);
+      store_chunk<T, kRagged, true>(dr, at + c * THREADS * V, cols, whole_d, o);
+    }
+  }
+}
+
 template <typename T>
-__global__ __launch_bounds__(kBlock) void softmax_bwd_stream(const T *p, const T *dy, T *dx, int64_t rows,
-                                                             int cols, int64_t ps, int64_t dys,
-                                                             int64_t dxs) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const T *pr = p + row * ps;
-  const T *gr = dy + row * dys;
-  float proj = 0.0f;
-  for (int c = lane; c < cols; c += kWave) proj = fmaf(to_f32(pr[c]), to_f32(gr[c]), proj);
-  proj = wave_sum(proj);
-  T *dr = dx + row * dxs;
-  for (int c = lane; c < cols; c += kWave) {
-    const float pc = to_f32(pr[c]);
-    dr[c] = from_f32<T>(pc * (to_f32(gr[c]) - proj));
+__global__ __launch_bounds__(kStreamBlock) void softmax_bwd_stream(const T *p, const T *dy, T *dx, int64_t rows,
+                                                                   int cols, int64_t ps, int64_t dys, int64_t dxs) {
+  constexpr int V = kChunk<T>;
+  __shared__ float sums[2][kStreamBlock / kWave];
+  const Span span_p = span_of(p, rows, cols, ps), span_g = span_of(dy, rows, cols, dys);
+  int turn = 0;
+  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x, turn ^= 1) {
+    const T *pr = p + row * ps;
+    const T *gr = dy + row * dys;
+    T *dr = dx + row * dxs;
+    const int shift = row_shift(pr);
+    const bool whole_g = row_shift(gr) == shift, whole_d = row_shift(dr) == shift;
+    const int64_t first = static_cast<int64_t>(threadIdx.x) * V - shift;
+    float proj = 0.0f;
+    for (int64_t at = first; at < cols; at += kStreamBlock * V) {
+      const u32x4_t pw = load_chunk<T, true>(pr, static_cast<int>(at), cols, true, 0, span_p);
+      const u32x4_t gw = load_chunk<T, true>(gr, static_cast<int>(at), cols, whole_g, 0, span_g);
+#pragma unroll
+      for (int i = 0; i < V; ++i) proj = fmaf(element<T>(pw, i), element<T>(gw, i), proj);
+    }
+    proj = block_reduce<kStreamBlock, false>(proj, sums[turn]);
+    for (int64_t at = first; at < cols; at += kStreamBlock * V) {
+      const u32x4_t pw = load_chunk<T, true>(pr, static_cast<int>(at), cols, true, 0, span_p);
+      const u32x4_t gw = load_chunk<T, true>(gr, static_cast<int>(at), cols, whole_g, 0, span_g);
+      float o[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) o[i] = element<T>(pw, i) * (element<T>(gw, i) - proj);
+      store_chunk<T, true, true>(dr, static_cast<int>(at), cols, whole_d, o);
+    }
   }
 }
 
 // ---------------------------------------------------------------- variant selection
-// Register-resident limits: 16 vector chunks (f32: 4096 columns, 16-bit: 8192) or
-// 64 scalar chunks (4096 columns); anything longer streams.
 struct Variant {
   const void *kernel;
   const char *name;
-  int block = kBlock;         // threads per workgroup
-  bool persistent = false;    // grid of resident waves walking the rows (rows per wave: any)
+  int block = kBlock;                  // threads per workgroup
+  int rows_per_block = kRowsPerBlock;  // rows a workgroup takes at a time
+  bool persistent = false;             // grid of resident waves walking the rows (rows per wave: any)
 };
 
 template <typename T>
 Variant pick_fwd_pipe(int chunks) {
+  constexpr int kRows = kPipeBlock / kWave;
   switch (chunks) {
-    case 1: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 1>), "softmax_fwd_pipe", kPipeBlock, true};
-    case 2: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 2>), "softmax_fwd_pipe", kPipeBlock, true};
-    case 4: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 4>), "softmax_fwd_pipe", kPipeBlock, true};
-    default: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 8>), "softmax_fwd_pipe", kPipeBlock, true};
+    case 1: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 1>), "softmax_fwd_pipe", kPipeBlock, kRows, true};
+    case 2: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 2>), "softmax_fwd_pipe", kPipeBlock, kRows, true};
+    case 4: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 4>), "softmax_fwd_pipe", kPipeBlock, kRows, true};
+    default: return {reinterpret_cast<const void *>(&softmax_fwd_pipe<T, 8>), "softmax_fwd_pipe", kPipeBlock, kRows, true};
   }
 }
+
+// The workgroup of a row: the fewest threads that hold it with the registers of many waves left, from one
+// wave per 512 16-bit elements on. A ragged row can reach into one more chunk than its length fills.
+#define INTENT_BLOCK(THREADS, CHUNKS)                                                                               \
+  if (elements <= static_cast<int64_t>(THREADS) * CHUNKS * kChunk<T>)                                               \
+    return {reinterpret_cast<const void *>(&INTENT_ROW_KERNEL<T, THREADS, CHUNKS, kRagged>), INTENT_ROW_NAME,   \
+            THREADS * kBlockRows<THREADS>, kBlockRows<THREADS>};
+
+template <typename T, bool kRagged>
+Variant pick_fwd_block(int64_t cols) {
+  const int64_t elements = kRagged ? cols + kChunk<T> - 1 : cols;
+#define INTENT_ROW_KERNEL softmax_fwd_block
+#define INTENT_ROW_NAME "softmax_fwd_block"
+  if constexpr (kRagged) {
+    INTENT_BLOCK(64, 1)
+    INTENT_BLOCK(64, 2)
+    INTENT_BLOCK(64, 4)
+    INTENT_BLOCK(64, 8)
+  }
+  INTENT_BLOCK(256, 4)
+  INTENT_BLOCK(512, 4)
+  INTENT_BLOCK(512, 8)
+  INTENT_BLOCK(1024, 8)
+  if constexpr (!kRagged) return pick_fwd_block<T, true>(cols);   // its edge selects spill at 16 chunks
+  INTENT_BLOCK(1024, 16)
+#undef INTENT_ROW_KERNEL
+#undef INTENT_ROW_NAME
+  return {reinterpret_cast<const void *>(&softmax_fwd_stream<T>), "softmax_fwd_stream", kStreamBlock, 1};
+}
+
+template <typename T, bool kRagged>
+Variant pick_bwd_block(int64_t cols) {
+  const int64_t elements = kRagged ? cols + kChunk<T> - 1 : cols;
+#define INTENT_ROW_KERNEL softmax_bwd_block
+#define INTENT_ROW_NAME "softmax_bwd_block"
+  if constexpr (kRagged) {
+    INTENT_BLOCK(64, 1)
+    INTENT_BLOCK(64, 2)
+    INTENT_BLOCK(64, 4)
+    INTENT_BLOCK(64, 8)
+  }
+  INTENT_BLOCK(256, 4)
+  INTENT_BLOCK(512, 4)
+  INTENT_BLOCK(1024, 4)
+  INTENT_BLOCK(1024, 8)
+#undef INTENT_ROW_KERNEL
+#undef INTENT_ROW_NAME
+  return {reinterpret_cast<const void *>(&softmax_bwd_stream<T>), "softmax_bwd_stream", kStreamBlock, 1};
+}
+#undef INTENT_BLOCK
 
 template <typename T, int V>
 Variant pick_fwd(int chunks) {
@@ -411,16 +678,8 @@ Variant pick_fwd(int chunks) {
     case 1: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 1>), "softmax_fwd_wave"};
     case 2: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 2>), "softmax_fwd_wave"};
     case 4: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 4>), "softmax_fwd_wave"};
-    case 8: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 8>), "softmax_fwd_wave"};
-    case 16: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 16>), "softmax_fwd_wave"};
-    case 32:
-      if constexpr (V == 1) return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, 1, 32>), "softmax_fwd_wave"};
-      break;
-    case 64:
-      if constexpr (V == 1) return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, 1, 64>), "softmax_fwd_wave"};
-      break;
+    default: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 8>), "softmax_fwd_wave"};
   }
-  return {reinterpret_cast<const void *>(&softmax_fwd_stream<T>), "softmax_fwd_stream"};
 }
 
 template <typename T, int V>
@@ -429,16 +688,11 @@ Variant pick_bwd(int chunks) {
     case 1: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 1>), "softmax_bwd_wave"};
     case 2: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 2>), "softmax_bwd_wave"};
     case 4: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 4>), "softmax_bwd_wave"};
-    case 8: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 8>), "softmax_bwd_wave"};
-    case 16: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 16>), "softmax_bwd_wave"};
-    case 32:
-      if constexpr (V == 1) return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, 1, 32>), "softmax_bwd_wave"};
-      break;
-    case 64:
-      if constexpr (V == 1) return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, 1, 64>), "softmax_bwd_wave"};
-      break;
+    case 16:
+      if constexpr (V == 4) return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 16>), "softmax_bwd_wave"};
+      [[fallthrough]];
+    default: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 8>), "softmax_bwd_wave"};
   }
-  return {reinterpret_cast<const void *>(&softmax_bwd_stream<T>), "softmax_bwd_stream"};
 }
 
 int round_chunks(int64_t cols, int per_chunk) {
@@ -448,32 +702,34 @@ int round_chunks(int64_t cols, int per_chunk) {
   return chunks;
 }
 
+// Up to 8 chunks a lane a wave holds an aligned row; longer rows belong to a workgroup, and so do ragged
+// ones, except short ones, whose ends are most of them: those stay with one element per lane and chunk
+// (16384 rows: 65 columns f16 4.6 us against 7.4, 129 f16 6.3 against 7.8, 257 f32 9.4 against 10.5; from there
+// on the workgroup leads: 450 f16 9.1 against 11.8, 1001 f16 16.4 against 31.9).
+template <typename T>
+constexpr int64_t kShortRow = sizeof(T) == 4 ? 512 : 256;
+
 template <typename T>
 Variant select_fwd(const void *x, const void *y, int64_t cols, int64_t xs, int64_t ys) {
-  constexpr int kVec = 16 / sizeof(T);
+  constexpr int kVec = kChunk<T>;
   const bool vector = cols % kVec == 0 && xs % kVec == 0 && ys % kVec == 0 && aligned(x, 16) && aligned(y, 16);
-  if (vector) {
-    const int chunks = round_chunks(cols, kWave * kVec);
-    if constexpr (sizeof(T) == 2)
-      if (chunks <= 8) return pick_fwd_pipe<T>(chunks);
-    return chunks <= 16 ? pick_fwd<T, kVec>(chunks) : pick_fwd<T, kVec>(0);
-  }
-  const int chunks = round_chunks(cols, kWave);
-  return chunks <= 64 ? pick_fwd<T, 1>(chunks) : pick_fwd<T, 1>(0);
+  if (!vector) return cols <= kShortRow<T> ? pick_fwd<T, 1>(round_chunks(cols, kWave)) : pick_fwd_block<T, true>(cols);
+  const int chunks = round_chunks(cols, kWave * kVec);
+  if (chunks > 8) return pick_fwd_block<T, false>(cols);
+  if constexpr (sizeof(T) == 2) return pick_fwd_pipe<T>(chunks);
+  else return pick_fwd<T, kVec>(chunks);
 }
 
 template <typename T>
 Variant select_bwd(const void *p, const void *dy, const void *dx, int64_t cols, int64_t ps, int64_t dys,
                    int64_t dxs) {
-  constexpr int kVec = 16 / sizeof(T);
+  constexpr int kVec = kChunk<T>;
   const bool vector = cols % kVec == 0 && ps % kVec == 0 && dys % kVec == 0 && dxs % kVec == 0 &&
                       aligned(p, 16) && aligned(dy, 16) && aligned(dx, 16);
-  if (vector) {
-    const int chunks = round_chunks(cols, kWave * kVec);
-    return chunks <= 16 ? pick_bwd<T, kVec>(chunks) : pick_bwd<T, kVec>(0);
-  }
-  const int chunks = round_chunks(cols, kWave);
-  return chunks <= 64 ? pick_bwd<T, 1>(chunks) : pick_bwd<T, 1>(0);
+  if (!vector) return cols <= kShortRow<T> ? pick_bwd<T, 1>(round_chunks(cols, kWave)) : pick_bwd_block<T, true>(cols);
+  const int chunks = round_chunks(cols, kWave * kVec);
+  // f32 4096 x 4096: 29.5 us in a wave, 31.7 in a workgroup.
+  return chunks > (sizeof(T) == 4 ? 16 : 8) ? pick_bwd_block<T, false>(cols) : pick_bwd<T, kVec>(chunks);
 }
 
 // Input rows may overlap (any non-negative stride, e.g. a broadcast row); output
@@ -489,13 +745,18 @@ int check_extents(int64_t rows, int64_t cols, int64_t in0, int64_t in1, int64_t 
   return INTENT_HIP_OK;
 }
 
+// Workgroups of a launch over `rows`: at most as many as the device holds at once for a persistent
+// kernel, and at most 2^30 for the softmax_*_block and _stream kernels, which walk the rest with a grid stride.
+int64_t grid_blocks(const Variant &v, int64_t rows) {
+  const int64_t blocks = (rows + v.rows_per_block - 1) / v.rows_per_block;
+  if (v.persistent) return std::min<int64_t>(blocks, resident_blocks(v.kernel, v.block));
+  return v.rows_per_block == kRowsPerBlock ? blocks : std::min<int64_t>(blocks, int64_t{1} << 30);
+}
+
 template <typename T>
 int launch_fwd(const void *x, void *y, int64_t rows, int64_t cols, int64_t xs, int64_t ys, hipStream_t stream) {
   const Variant v = select_fwd<T>(x, y, cols, xs, ys);
-  const int rows_per_block = v.block / kWave;
-  int64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
-  if (v.persistent) blocks = std::min<int64_t>(blocks, resident_blocks(v.kernel, v.block));
-  const dim3 grid(static_cast<unsigned>(blocks));
+  const dim3 grid(static_cast<unsigned>(grid_blocks(v, rows)));
   int icols = static_cast<int>(cols);
   void *args[] = {const_cast<void **>(&x), &y, &rows, &icols, &xs, &ys};
   if (hipLaunchKernel(v.kernel, grid, dim3(v.block), args, 0, stream) != hipSuccess) return launch_status(v.name);
@@ -506,10 +767,10 @@ template <typename T>
 int launch_bwd(const void *p, const void *dy, void *dx, int64_t rows, int64_t cols, int64_t ps, int64_t dys,
                int64_t dxs, hipStream_t stream) {
   const Variant v = select_bwd<T>(p, dy, dx, cols, ps, dys, dxs);
-  const dim3 grid(static_cast<unsigned>((rows + kRowsPerBlock - 1) / kRowsPerBlock));
+  const dim3 grid(static_cast<unsigned>(grid_blocks(v, rows)));
   int icols = static_cast<int>(cols);
   void *args[] = {const_cast<void **>(&p), const_cast<void **>(&dy), &dx, &rows, &icols, &ps, &dys, &dxs};
-  if (hipLaunchKernel(v.kernel, grid, dim3(kBlock), args, 0, stream) != hipSuccess) return launch_status(v.name);
+  if (hipLaunchKernel(v.kernel, grid, dim3(v.block), args, 0, stream) != hipSuccess) return launch_status(v.name);
   return INTENT_HIP_OK;
 }
 
@@ -537,7 +798,7 @@ int softmax_bwd_resources(int dtype, int64_t rows, int64_t cols, IntentHipKernel
     case INTENT_HIP_BF16: v = select_bwd<bf16_t>(nullptr, nullptr, nullptr, cols, cols, cols, cols); break;
     default: return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "unknown dtype code %d", dtype);
   }
-  return describe_kernel(v.kernel, v.name, kBlock, out);
+  return describe_kernel(v.kernel, v.name, v.block, out);
 }
 
 }  // namespace intent_hip

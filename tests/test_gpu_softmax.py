@@ -12,6 +12,7 @@ from intent_amd.examples import inputs
 from intent_amd.examples.kernels.backward.softmax import softmax_backward, softmax_backward_f16
 from intent_amd.examples.kernels.normalization.softmax import (chunked_softmax_bf16, stable_softmax,
                                                                stable_softmax_f16)
+from intent_amd.runtime.hip import library as hiplib
 from tests.gpu_util import (announce, assert_16bit, assert_f32_rel, bf16_tensor_bits, bf16_to_f32,
                             f16_ulp_distance, to_bf16_tensor)
 
@@ -193,3 +194,61 @@ def test_softmax_config2_seed0_fwd_bwd(device):
     p64 = y.astype(np.float64)
     spread = 1e-5 * np.abs(p64) * np.sum(np.abs(p64 * dy.astype(np.float64)), axis=1, keepdims=True)
     assert np.all(np.abs(dx.astype(np.float64) - want) <= 2 ** -9 * np.abs(want.astype(np.float64)) + spread + 6e-8)
+
+
+# Rows of a workgroup: both sides of every step of threads and chunks (16-bit 8192, 16384, 32768, 65536, 131072
+# elements; f32 half of that), ragged ends, short ragged rows (up to 256 and 512 elements) and their
+# successors, rows longer than any workgroup's registers.
+@pytest.mark.parametrize("rows,cols", [(5, 255), (5, 257), (9, 505), (3, 513), (7, 1017), (3, 2049), (2, 4095), (2, 4104),
+                                       (3, 8185), (2, 8192), (2, 8200), (3, 16384), (2, 16392), (2, 32768), (2, 32776),
+                                       (1, 65533), (2, 65544), (1, 131065), (1, 131072), (2, 131080), (1, 140001)])
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_softmax_workgroup_rows(device, rows, cols, kind):
+    """Forward (and for f32 and f16 backward) against the oracle, with the output inside a buffer whose other elements must
+    not change, and the operands' rows at a stride and start that leave them ragged and differently aligned."""
+    announce("softmax workgroup rows", rows, cols, kind)
+    dtype = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[kind]
+    rng = np.random.default_rng(rows * cols)
+    fwd = {"f32": stable_softmax, "f16": stable_softmax_f16, "bf16": chunked_softmax_bf16}[kind]
+    x = rng.standard_normal((rows, cols), dtype=np.float32) * 3
+    dy = rng.standard_normal((rows, cols), dtype=np.float32)
+    as_f64 = lambda t: t.float().cpu().numpy().astype(np.float64)  # noqa: E731
+    for pad, offsets in ((0, (0, 0, 0)), (3, (1, 1, 1)), (5, (0, 2, 3))):
+        def view(data, offset):
+            base = torch.full((rows * (cols + pad) + 16,), 7.0, dtype=dtype, device=device)
+            v = base[offset:offset + rows * (cols + pad)].view(rows, cols + pad)[:, :cols]
+            if data is not None:
+                v.copy_(torch.from_numpy(data).to(device).to(dtype))
+            return base, v
+
+        def untouched(base, v):
+            v.fill_(7.0)
+            return bool((base == 7.0).all())
+
+        _, xv = view(x, offsets[0])
+        y_base, yv = view(None, offsets[1])
+        intent.jit(fwd, backend="hip")(xv, yv)
+        want = torch.softmax(xv.double(), dim=1)
+        if kind == "f32":
+            assert_f32_rel(as_f64(yv), want.cpu().numpy())
+        else:
+            assert_16bit(as_f64(yv), want.cpu().numpy(), rel=2.0 ** (-10 if kind == "f16" else -7), abs_=2.0 ** -24)
+        p = yv.clone()
+        assert untouched(y_base, yv)
+        if kind != "bf16":       # through the C ABI: the f32 definition's extents are fixed
+            _, pv = view(as_f64(p).astype(np.float32), offsets[0])
+            _, gv = view(dy, offsets[2])
+            d_base, dv = view(None, offsets[1])
+            lib, stride = hiplib.library(), cols + pad
+            lib.check(lib.fn["softmax_bwd"](hiplib.F32 if kind == "f32" else hiplib.F16, pv.data_ptr(), gv.data_ptr(),
+                                            dv.data_ptr(), rows, cols, stride, stride, stride,
+                                            torch.cuda.current_stream().cuda_stream))
+            p64, g64 = as_f64(pv), as_f64(gv)
+            proj = (p64 * g64).sum(1, keepdims=True)
+            # f32: the projection's sum in another order, at most 160 roundings deep (137 elements of a lane,
+            # then lanes and waves), and the roundings of the difference and the product; f16 adds its cast
+            bound = p64 * 2.0 ** -24 * (160 * np.abs(p64 * g64).sum(1, keepdims=True) + 4 * np.abs(g64 - proj))
+            if kind == "f16":
+                bound = bound + 2.0 ** -11 * np.abs(p64 * (g64 - proj)) + 2.0 ** -25
+            assert (np.abs(as_f64(dv) - p64 * (g64 - proj)) <= bound + 1e-40).all()
+            assert untouched(d_base, dv)
