@@ -153,6 +153,14 @@ int intent_hip_gemm_ws(int dtype, int activation, const void *a, const void *b, 
 int intent_hip_gemm_f32(const float *a, const float *b, float *c, int64_t m, int64_t n, int64_t k,
                         int64_t lda, int64_t ldb, int64_t ldc, int transpose_b, void *stream);
 
+/* intent_hip_gemm_f32 with a K split for products of few output tiles, as intent_hip_gemm_ws is to
+ * intent_hip_gemm. The workspace must hold intent_hip_gemm_f32_workspace_bytes (0: nothing to split) and be 16-byte
+ * aligned; with a null or smaller workspace one workgroup takes each output tile. */
+int intent_hip_gemm_f32_workspace_bytes(int64_t m, int64_t n, int64_t k, size_t *bytes);
+int intent_hip_gemm_f32_ws(const float *a, const float *b, float *c, int64_t m, int64_t n, int64_t k,
+                           int64_t lda, int64_t ldb, int64_t ldc, int transpose_b, void *workspace,
+                           size_t workspace_bytes, void *stream);
+
 /* f16 GEMM with f32 accumulation and a quantizing epilogue, int8 output:
  * quantized_gemm (python/intent/examples/kernels/contraction/gemm.py:95-121). Per element, each
  * step an f32 operation: v = maximum(acc + bias[n], 0) (NaN propagates), v += residual[i][n],

@@ -44,7 +44,26 @@ int attention_bwd_resources(int64_t which, int64_t rows, int64_t d, IntentHipKer
 int decode_resources(int64_t which, int64_t d, int64_t group, IntentHipKernelResources *out);
 int spmm_resources(int64_t features, IntentHipKernelResources *out);
 
+// f32 products of few output tiles (gemm_f32_few.hip); `workspace` may be null (one workgroup per tile).
+bool gemm_f32_few_applies(int64_t m, int64_t n);
+size_t gemm_f32_few_bytes(int64_t m, int64_t n, int64_t k);
+int gemm_f32_few_resources(int64_t m, IntentHipKernelResources *out);
+int launch_gemm_f32_few(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb,
+                        int64_t ldc, int transpose_b, void *workspace, size_t workspace_bytes, hipStream_t s);
+
 constexpr int kWave = 64;
+
+// Tile of this workgroup, or -1 for none, when each XCD shall take one run of consecutive tiles (neighbouring tiles
+// share an operand through its L2): workgroups go to the 8 XCDs in turn, so the launch has
+// xcd_blocks(tiles) of them in x, and any number in y and z. The runs differ by one tile at most.
+inline unsigned xcd_blocks(int64_t tiles) { return static_cast<unsigned>((tiles + 7) / 8 * 8); }
+__device__ __forceinline__ int xcd_tile(int tiles) {
+  const int xcd = blockIdx.x & 7;
+  const int first = static_cast<int>(static_cast<int64_t>(tiles) * xcd / 8);
+  const int last = static_cast<int>(static_cast<int64_t>(tiles) * (xcd + 1) / 8);
+  const int tile = first + static_cast<int>(blockIdx.x >> 3);
+  return tile < last ? tile : -1;
+}
 
 // ---------------------------------------------------------------- wave-wide reductions
 // Cross-lane moves use DPP within each 16-lane row (quad permutes, half-row and

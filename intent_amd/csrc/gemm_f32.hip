@@ -18,8 +18,9 @@
 //     halves, 8 rows apart, use different banks); W (linear_f32) is stored like A;
 //   * the MFMA computes the transposed tile (B fragment first), so each lane holds 4
 //     consecutive output columns of one row per register quad and stores them as one float4.
-// Rows need 16-byte alignment and row strides that are multiples of 4 for the vector loads;
-// other layouts take the same kernel with scalar loads.
+// Products of up to 192 such tiles, or of up to 64 rows, run gemm_f32_few.hip instead, and so do layouts that are
+// not 16-byte aligned or whose strides are not multiples of 4 (2048 x 4095 x 4095: 816 us here with scalar loads,
+// 620 - 660 there).
 #include "common.hpp"
 
 namespace intent_hip {
@@ -35,7 +36,7 @@ constexpr int kStageA = kBM * kRowA;
 constexpr int kStageB = (kBN * kRowA > kBK * kRowB) ? kBN * kRowA : kBK * kRowB;
 constexpr int kStage = kStageA + kStageB;
 
-template <bool kTransB, bool kVec>
+template <bool kTransB>
 __global__ __launch_bounds__(kThreads) void gemm_f32_mfma(const float *__restrict__ A, const float *__restrict__ B,
                                                           float *__restrict__ C, int M, int N, int K, int64_t lda,
                                                           int64_t ldb, int64_t ldc) {
@@ -54,18 +55,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma(const float *__restric
     for (int i = 0; i < 2; ++i) {
       const int c = tid + kThreads * i;
       const int row = row0 + (c >> 2), kq = k0 + 4 * (c & 3);
-      if (kVec) {
-        const bool ok = row < rows_total && kq < K;
-        r[i] = ok ? *reinterpret_cast<const float4 *>(base + static_cast<int64_t>(row) * ld + kq)
-                  : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        const float *p = base + static_cast<int64_t>(row) * ld;
-        const bool okr = row < rows_total;
-        r[i].x = okr && kq < K ? p[kq] : 0.f;
-        r[i].y = okr && kq + 1 < K ? p[kq + 1] : 0.f;
-        r[i].z = okr && kq + 2 < K ? p[kq + 2] : 0.f;
-        r[i].w = okr && kq + 3 < K ? p[kq + 3] : 0.f;
-      }
+      const bool ok = row < rows_total && kq < K;
+      r[i] = ok ? *reinterpret_cast<const float4 *>(base + static_cast<int64_t>(row) * ld + kq)
+                : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   };
   auto load_b_natural = [&](int k0) {
@@ -73,18 +65,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma(const float *__restric
     for (int i = 0; i < 2; ++i) {
       const int c = tid + kThreads * i;
       const int k = k0 + (c >> 5), nq = n0 + 4 * (c & 31);
-      if (kVec) {
-        const bool ok = k < K && nq < N;
-        rb[i] = ok ? *reinterpret_cast<const float4 *>(B + static_cast<int64_t>(k) * ldb + nq)
-                   : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        const float *p = B + static_cast<int64_t>(k) * ldb;
-        const bool okk = k < K;
-        rb[i].x = okk && nq < N ? p[nq] : 0.f;
-        rb[i].y = okk && nq + 1 < N ? p[nq + 1] : 0.f;
-        rb[i].z = okk && nq + 2 < N ? p[nq + 2] : 0.f;
-        rb[i].w = okk && nq + 3 < N ? p[nq + 3] : 0.f;
-      }
+      const bool ok = k < K && nq < N;
+      rb[i] = ok ? *reinterpret_cast<const float4 *>(B + static_cast<int64_t>(k) * ldb + nq)
+                 : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   };
   auto load = [&](int k0) {
@@ -171,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma(const float *__restric
       for (int g = 0; g < 4; ++g) {
         const int n = n0 + wn * 64 + nt * 32 + 8 * g + 4 * half;
         const f32x16_t &v = acc[mt][nt];
-        if (kVec && n + 3 < N) {
+        if (n + 3 < N) {
           *reinterpret_cast<float4 *>(crow + n) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
         } else {
 #pragma unroll
@@ -185,9 +168,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma(const float *__restric
 }  // namespace
 
 int gemm_f32_resources(int64_t m, int64_t n, IntentHipKernelResources *out) {
-  (void)m;
-  (void)n;
-  return describe_kernel(reinterpret_cast<const void *>(&gemm_f32_mfma<false, true>), "gemm_f32_mfma", kThreads, out);
+  if (gemm_f32_few_applies(m, n)) return gemm_f32_few_resources(m, out);
+  return describe_kernel(reinterpret_cast<const void *>(&gemm_f32_mfma<false>), "gemm_f32_mfma", kThreads, out);
 }
 
 }  // namespace intent_hip
@@ -196,6 +178,19 @@ using namespace intent_hip;
 
 extern "C" int intent_hip_gemm_f32(const float *a, const float *b, float *c, int64_t m, int64_t n, int64_t k,
                                    int64_t lda, int64_t ldb, int64_t ldc, int transpose_b, void *stream) {
+  return intent_hip_gemm_f32_ws(a, b, c, m, n, k, lda, ldb, ldc, transpose_b, nullptr, 0, stream);
+}
+
+extern "C" int intent_hip_gemm_f32_workspace_bytes(int64_t m, int64_t n, int64_t k, size_t *bytes) {
+  if (bytes == nullptr) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "null output");
+  if (m < 0 || n < 0 || k < 0) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "negative extent");
+  *bytes = gemm_f32_few_bytes(m, n, k);
+  return INTENT_HIP_OK;
+}
+
+extern "C" int intent_hip_gemm_f32_ws(const float *a, const float *b, float *c, int64_t m, int64_t n, int64_t k,
+                                      int64_t lda, int64_t ldb, int64_t ldc, int transpose_b, void *workspace,
+                                      size_t workspace_bytes, void *stream) {
   if (m < 0 || n < 0 || k < 0) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "negative extent");
   if (transpose_b != 0 && transpose_b != 1)
     return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "transpose_b must be 0 or 1 (got %d)", transpose_b);
@@ -213,13 +208,10 @@ extern "C" int intent_hip_gemm_f32(const float *a, const float *b, float *c, int
   const dim3 grid(static_cast<unsigned>((n + kBN - 1) / kBN), static_cast<unsigned>((m + kBM - 1) / kBM));
   const hipStream_t s = as_stream(stream);
   const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
-  if (transpose_b) {
-    if (vec) gemm_f32_mfma<true, true><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);
-    else gemm_f32_mfma<true, false><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);
-  } else {
-    if (vec) gemm_f32_mfma<false, true><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);
-    else gemm_f32_mfma<false, false><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);
-  }
+  if (!vec || gemm_f32_few_applies(m, n))
+    return launch_gemm_f32_few(a, b, c, M, N, K, lda, ldb, ldc, transpose_b, workspace, workspace_bytes, s);
+  if (transpose_b) gemm_f32_mfma<true><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);
+  else gemm_f32_mfma<false><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);
   if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_f32_mfma");
   return INTENT_HIP_OK;
 }

@@ -57,6 +57,8 @@ SIGNATURES = {
     "intent_hip_gemm_workspace_bytes": (_int, (_i64, _i64, _i64, ctypes.POINTER(_sz))),
     "intent_hip_gemm_ws": (_int, (_int, _int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p, _sz, _p)),
     "intent_hip_gemm_f32": (_int, (_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p)),
+    "intent_hip_gemm_f32_workspace_bytes": (_int, (_i64, _i64, _i64, ctypes.POINTER(_sz))),
+    "intent_hip_gemm_f32_ws": (_int, (_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _int, _p, _sz, _p)),
     "intent_hip_gemm_i8": (_int, (_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p)),
     "intent_hip_quantized_gemm": (_int, (_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p)),
     "intent_hip_attention_fwd_f16": (_int, (_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64,

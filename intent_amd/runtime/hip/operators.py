@@ -302,35 +302,40 @@ def _softmax_bwd(dtype_code):
 
 
 # ------------------------------------------------------------------------------ GEMM
-def _gemm_launch(lib, dtype_code, activation, a, b, c, entry, configuration, device):
-    """A 16-bit product. One of few rows and columns divides K over workgroups through a workspace of
-    f32 sums (none with workspace='static': one workgroup per output tile)."""
+def _split_sums(lib, name, m, n, k, device, keep):
+    """(address, bytes) of a workspace for the f32 sums of a product whose K is divided over workgroups; ()
+    where nothing is split (enough output tiles, or workspace='static')."""
     import ctypes
 
     import torch
 
+    size = ctypes.c_size_t(0)
+    lib.check(lib.fn[name + "_workspace_bytes"](m, n, k, ctypes.byref(size)), "provider_preparation")
+    if not size.value or _static_workspace():
+        return ()
+    workspace = torch.empty(size.value, dtype=torch.uint8, device=device)
+    keep.append(workspace)
+    return workspace.data_ptr(), size.value
+
+
+def _gemm_launch(lib, dtype_code, activation, a, b, c, entry, configuration, device):
     keep, before, after = [a, b, c], [], []
     ak, bk, ck = _readable(a, keep, before), _readable(b, keep, before), _writable(c, keep, after)
     m, k = a.shape
     n = b.shape[1]
-    operands = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk),
-                _row_stride(ck))
+    args = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk), _row_stride(ck))
     facts = (("m", m), ("n", n), ("k", k)) + configuration
     op = OP_GEMM_BF16 if entry == "intent_hip_gemm_bf16" else OP_GEMM
-    resources = lambda: lib.kernel_resources(op, dtype_code, m, n)  # noqa: E731
-    size = ctypes.c_size_t(0)
-    lib.check(lib.fn["gemm_workspace_bytes"](m, n, k, ctypes.byref(size)), "provider_preparation")
-    if size.value and not _static_workspace():
-        workspace = torch.empty(size.value, dtype=torch.uint8, device=device)
-        keep.append(workspace)
-        fn = lib.fn["gemm_ws"]
-        args = (dtype_code, activation, *operands, workspace.data_ptr(), size.value)
-        return Launch("intent_hip_gemm_ws", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
-                      tuple(after), facts + (("workspace_bytes", size.value),), resources)
-    fn = lib.fn[entry[len("intent_hip_"):]]
-    args = operands if entry == "intent_hip_gemm_bf16" else (dtype_code, activation, *operands)
+    extra = _split_sums(lib, "gemm", m, n, k, device, keep)
+    if extra:
+        fn, entry, args, facts = (lib.fn["gemm_ws"], "intent_hip_gemm_ws", (dtype_code, activation, *args, *extra),
+                                  facts + (("workspace_bytes", extra[1]),))
+    elif entry == "intent_hip_gemm_bf16":
+        fn = lib.fn["gemm_bf16"]
+    else:
+        fn, args = lib.fn["gemm"], (dtype_code, activation, *args)
     return Launch(entry, lambda stream: fn(*args, stream), tuple(keep), tuple(before), tuple(after), facts,
-                  resources)
+                  lambda: lib.kernel_resources(op, dtype_code, m, n))
 
 
 def _gemm_bf16(lib, bound, constexprs, device):
@@ -361,11 +366,14 @@ def _gemm_f32(transpose_b: bool):
         ak, bk, ck = _readable(a, keep, before), _readable(b, keep, before), _writable(c, keep, after)
         m, k = a.shape
         n = b.shape[0] if transpose_b else b.shape[1]
-        fn = lib.fn["gemm_f32"]
         args = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk),
                 _row_stride(ck), int(transpose_b))
-        return Launch("intent_hip_gemm_f32", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
-                      tuple(after), (("m", m), ("n", n), ("k", k), ("transpose_b", transpose_b)),
+        facts = (("m", m), ("n", n), ("k", k), ("transpose_b", transpose_b))
+        fn, entry, extra = lib.fn["gemm_f32"], "intent_hip_gemm_f32", _split_sums(lib, "gemm_f32", m, n, k, device, keep)
+        if extra:
+            fn, entry, args, facts = (lib.fn["gemm_f32_ws"], "intent_hip_gemm_f32_ws", (*args, *extra),
+                                      facts + (("workspace_bytes", extra[1]),))
+        return Launch(entry, lambda stream: fn(*args, stream), tuple(keep), tuple(before), tuple(after), facts,
                       lambda: lib.kernel_resources(OP_GEMM_F32, F32, m, n))
     return plan
 

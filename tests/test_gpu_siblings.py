@@ -161,6 +161,35 @@ def run_attention(device, defn, q, k, v, scale, group, causal, bf16):
     return bf16_tensor_bits(out) if bf16 else out.cpu().numpy()
 
 
+# Few output tiles: 16-, 32- and 64-row blocks and their edges, column counts around one 64-column block and
+# off every 4 (partial 16-byte groups), K below one 32-deep unit, off it by 1 to 31, and divided over workgroups
+# (from 512 on), one and several row blocks, rows of every 4-byte alignment.
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (15, 63, 31), (16, 64, 32), (17, 65, 33), (32, 61, 47), (33, 130, 100),
+                                   (64, 70, 511), (65, 7, 513), (100, 67, 1031), (3, 1000, 2050), (300, 129, 777),
+                                   (1, 30000, 40)])
+@pytest.mark.parametrize("workspace", ["prepare", "static"])
+def test_gemm_f32_few_tiles(device, m, n, k, workspace):
+    """Against 64-bit products within the error of K f32 roundings, exact on small integers, and with NaN in the last
+    row of A and the first column of B confined to their own row and column of the result."""
+    announce("gemm f32 few tiles", m, n, k, workspace)
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    ints = rng.integers(-8, 9, (m, k)).astype(np.float32), rng.integers(-8, 9, (k, n)).astype(np.float32)
+    options = dict(backend="hip", backend_options={"workspace": workspace})
+    natural, weight = intent.jit(gemm_f32, **options), intent.jit(linear_f32, **options)
+    for run in (lambda x, y: natural.run(t(x, device), t(y, device)),
+                lambda x, y: weight.run(t(x, device), t(np.ascontiguousarray(y.T), device))):
+        got = run(a, b).cpu().numpy()
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        assert (np.abs(got - want) <= k * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b)) + 1e-30).all()
+        assert (run(*ints).cpu().numpy() == ints[0].astype(np.float64) @ ints[1].astype(np.float64)).all()
+        x, y = a.copy(), b.copy()
+        x[m - 1, k - 1] = y[k - 1, 0] = np.nan
+        expected = np.zeros((m, n), bool)
+        expected[m - 1, :] = expected[:, 0] = True
+        assert (np.isnan(run(x, y).cpu().numpy()) == expected).all()
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_attention_family_golden(device, golden, causal):
     announce("attention family golden", causal)
