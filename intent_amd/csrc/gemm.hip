@@ -4,34 +4,26 @@
 // accumulator = matmul(a, b, acc_dtype=f32); c = cast(accumulator, bf16) (round to
 // nearest even). A [M,K], B [K,N], C [M,N], row-major with row strides lda/ldb/ldc.
 //
-// Design (fast path):
-//   * workgroup tile 256 x 256, 8 waves in 2 x 4, each wave 128 x 64 = 4 x 2 tiles of
+// Design: three MFMA kernels, chosen by the shape (launch_epilogue).
+//   * 256 x 256 tiles (gemm_mfma) for many tiles: 8 waves in 2 x 4, each wave 128 x 64 = 4 x 2 tiles of
 //     v_mfma_f32_32x32x16_bf16 (128 accumulator registers per lane, so two waves share
-//     each SIMD);
-//   * interior tiles with K % 32 == 0 (gemm_tile_dma) stream A and B into LDS with
-//     global_load_lds (five 32 KB stages) and read B fragments with transposing LDS reads;
-//     the two waves of a SIMD alternate between their MFMA cluster and their LDS reads
-//     (ping-pong), so the matrix pipe is fed while the other wave waits on LDS;
-//   * other tiles (gemm_tile) use K step 64 and two register-staged LDS stages
-//     (2 x 64 KB): the next K step's global loads are in flight while the current one is
-//     consumed;
-//   * MFMA operands need 8 consecutive k per lane. A rows are k-contiguous already;
-//     in gemm_tile B is [K,N], so each thread of waves 4-7 loads an 8 (k) x 8 (n) block,
-//     transposes it in registers and stores n-rows of 8 k into LDS ("Bt", k-contiguous);
-//     waves 0-3 copy A;
-//   * gemm_tile's LDS tiles are rows of 8 16-byte chunks; chunk c of row r is stored at
-//     c ^ ((r & 7) ^ ((r >> 3) & 1)), so the 16-byte fragment reads of 16 consecutive
-//     rows (one LDS cycle) hit distinct banks;
+//     each SIMD); A and B stream into LDS with global_load_lds (five 32 KB stages) and B fragments are read
+//     with transposing LDS reads; the two waves of a SIMD alternate between their MFMA cluster and their
+//     LDS reads (ping-pong), so the matrix pipe is fed while the other wave waits on LDS;
+//   * 128 x 128 and 64 x 64 tiles (gemm_small) where 256 x 256 tiles would leave CUs idle, and for
+//     operands that the DMA does not take (odd extents, strides or addresses);
+//   * up to 128 rows (gemm_skinny): waves stream B into registers (f16 relu 32 x 14336 x 4096: 221 us in
+//     256 x 256 tiles, 28 there).
+// Tiles that reach past M or N read valid rows and columns in their place and do not store them; past
+// K (a multiple of 8 where the DMA runs) they read zeros.
 //   * the MFMA is issued as D = Bt_frag x A_frag, i.e. the transposed product, so each
 //     lane ends with 4 consecutive output columns of one output row per register
 //     quad and writes them as one 8-byte store;
-//   * tiles are walked in groups of 2 tile rows, column by column, in dispatch order: the
+//   * 256 x 256 tiles are walked in groups of 2 tile rows, column by column, in dispatch order: the
 //     tiles resident at one time share A row panels and B column panels, across XCDs
 //     through the MALL and within each XCD through its L2.
-// Calls of up to 128 rows run gemm_skinny instead (f16 relu 32 x 14336 x 4096: 221 us in 256 x 256 tiles,
-// 27.9 there).
-// Shapes the fast path cannot take (K or N not a multiple of 8, unaligned rows) use a
-// simple LDS-tiled f32 FMA kernel.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace intent_hip {
@@ -82,27 +74,14 @@ __device__ __forceinline__ typename Elem<E>::x4 pack4(float a, float b, float c,
   return r;
 }
 
-constexpr int kBM = 256, kBN = 256, kBK = 64;
+constexpr int kBM = 256, kBN = 256;
 constexpr int kThreads = 512;
-constexpr int kChunksA = kBM * kBK / 8;          // 16-byte chunks of one A stage
-constexpr int kStageChunks = (kBM + kBN) * kBK / 8;
 constexpr int kGroupM = 2;
-
-__device__ __forceinline__ int swizzle(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 template <typename E>
 __device__ __forceinline__ float element_to_f32(uint16_t bits) { return static_cast<float>(__builtin_bit_cast(E, bits)); }
 template <typename E>
 __device__ __forceinline__ uint16_t f32_to_element(float v) { return __builtin_bit_cast(uint16_t, static_cast<E>(v)); }
-
-__device__ __forceinline__ uint32_t word(const uint4 &v, int i) {
-  return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
-}
-
-// Component-wise select (a whole-struct select is lowered through scratch memory).
-__device__ __forceinline__ uint4 select(bool keep, uint4 v) {
-  return make_uint4(keep ? v.x : 0u, keep ? v.y : 0u, keep ? v.z : 0u, keep ? v.w : 0u);
-}
 
 // Epilogues: quad(i, n, a, b, c, d) receives the f32 accumulators of output row i, columns n .. n+3
 // (n a multiple of 4); one(i, n, a) a single element (the general-shape kernel).
@@ -173,148 +152,7 @@ __device__ __forceinline__ void tile_of_block(int block, int tiles_m, int tiles_
   tn = in_group / rows_in_group;
 }
 
-template <typename E, typename Epi, bool kEdge>
-__device__ __forceinline__ void gemm_tile(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                                          const Epi &ep, int M, int N, int K, int64_t lda, int64_t ldb, int m0,
-                                          int n0, uint4 *lds) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 2, wn = wave & 3;   // wave tile: rows wm*128..+128, cols wn*64..+64
-
-  // Loader roles (wave-uniform). Waves 0-3 copy the A tile: rows a_row + 32 i, 16-byte
-  // chunk a_chunk (8 k). Waves 4-7 copy the B tile: k rows b_kg * 8 + j, n chunk b_nc
-  // (8 n), transposed in registers into Bt rows b_nc * 8 + m (8 k each).
-  const bool loads_a = wave < 4;
-  const int lt = tid & 255;
-  const int a_chunk = lt & 7, a_row = lt >> 3;
-  const int b_kg = lt & 7, b_nc = lt >> 3;
-  uint4 r[8];
-
-  auto load = [&](int k0) {
-    if (loads_a) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int row = m0 + a_row + 32 * i;
-        const int col = k0 + a_chunk * 8;
-        if (!kEdge) {
-          r[i] = *reinterpret_cast<const uint4 *>(A + static_cast<int64_t>(row) * lda + col);
-        } else {
-          const bool ok = row < M && col < K;
-          const uint16_t *p = A + static_cast<int64_t>(ok ? row : 0) * lda + (ok ? col : 0);
-          r[i] = select(ok, *reinterpret_cast<const uint4 *>(p));
-        }
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int krow = k0 + b_kg * 8 + j;
-        const int col = n0 + b_nc * 8;
-        if (!kEdge) {
-          r[j] = *reinterpret_cast<const uint4 *>(B + static_cast<int64_t>(krow) * ldb + col);
-        } else {
-          const bool ok = krow < K && col < N;
-          const uint16_t *p = B + static_cast<int64_t>(ok ? krow : 0) * ldb + (ok ? col : 0);
-          r[j] = select(ok, *reinterpret_cast<const uint4 *>(p));
-        }
-      }
-    }
-  };
-
-  auto store = [&](int stage) {
-    uint4 *sa = lds + stage * kStageChunks;
-    uint4 *sb = sa + kChunksA;
-    if (loads_a) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int row = a_row + 32 * i;
-        sa[row * 8 + (a_chunk ^ swizzle(row))] = r[i];
-      }
-    } else {
-      // r[j] word p holds (n = 2p, n = 2p + 1) at k = j: gather the 8 k of each n.
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        uint32_t even[4], odd[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t k_lo = word(r[2 * q], p), k_hi = word(r[2 * q + 1], p);
-          even[q] = (k_lo & 0xffffu) | (k_hi << 16);
-          odd[q] = (k_lo >> 16) | (k_hi & 0xffff0000u);
-        }
-        const int n_even = b_nc * 8 + 2 * p, n_odd = n_even + 1;
-        sb[n_even * 8 + (b_kg ^ swizzle(n_even))] = make_uint4(even[0], even[1], even[2], even[3]);
-        sb[n_odd * 8 + (b_kg ^ swizzle(n_odd))] = make_uint4(odd[0], odd[1], odd[2], odd[3]);
-      }
-    }
-  };
-
-  f32x16_t acc[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  // Fragment rows of this lane: the swizzle depends only on the lane (rows differ by 32s).
-  const int frag_row = lane & 31;
-  const int frag_swz = swizzle(frag_row);
-  const int frag_half = lane >> 5;
-
-  auto compute = [&](int stage) {
-    const uint4 *sa = lds + stage * kStageChunks;
-    const uint4 *sb = sa + kChunksA;
-#pragma unroll
-    for (int kk = 0; kk < kBK / 16; ++kk) {
-      const int chunk = (kk * 2 + frag_half) ^ frag_swz;
-      typedef typename Elem<E>::x8 x8;
-      x8 af[4], bf[2];
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        af[t] = __builtin_bit_cast(x8, sa[(wm * 128 + t * 32 + frag_row) * 8 + chunk]);
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-        bf[t] = __builtin_bit_cast(x8, sb[(wn * 64 + t * 32 + frag_row) * 8 + chunk]);
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-          acc[mt][nt] = Elem<E>::mma(bf[nt], af[mt], acc[mt][nt]);
-    }
-  };
-
-  const int k_tiles = (K + kBK - 1) / kBK;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int kt = 0; kt < k_tiles; ++kt) {
-    const bool more = kt + 1 < k_tiles;
-    if (more) load((kt + 1) * kBK);
-    compute(kt & 1);
-    if (more) store((kt + 1) & 1);
-    __syncthreads();
-  }
-
-  // Epilogue: acc[mt][nt][4g + e] is C[i][n] with i = the A fragment's row (lane & 31) and
-  // n = 8g + 4 * (lane >> 5) + e within the 32-column tile; 4 consecutive n -> one 8-byte store.
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int i = m0 + wm * 128 + mt * 32 + frag_row;
-    if (kEdge && i >= M) continue;
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn * 64 + nt * 32 + 8 * g + 4 * frag_half;
-        if (kEdge && n >= N) continue;
-        const f32x16_t &v = acc[mt][nt];
-        ep.quad(i, n, v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------- interior tiles: LDS-DMA pipeline
+// ---------------------------------------------------------------- 256 x 256 tiles: LDS-DMA pipeline
 // K step 32, five LDS stages of 32 KB (160 KB): up to three later tiles are in flight
 // (global_load_lds_dwordx4 writes them straight into LDS, no registers) while tile kt is multiplied. A stage holds A [256 m][32 k]
 // (rows of 4 16-byte chunks, chunk c of row r at c ^ ((r >> 2) & 3), which spreads the fragment
@@ -349,10 +187,15 @@ __device__ __forceinline__ void dma_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <typename E, typename Epi>
+// What the DMA reads for chunks past K.
+__device__ const uint4 kZeroChunk = {0u, 0u, 0u, 0u};
+
+// Rows past M and columns past N read valid ones instead, and their products are not stored; kTail: K is not a
+// multiple of 32, and the last tile's chunks past K are zeros (K is a multiple of 8).
+template <typename E, typename Epi, bool kTail>
 __device__ __forceinline__ void gemm_tile_dma(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                                              const Epi &ep, int K, int64_t lda, int64_t ldb, int m0, int n0,
-                                              uint4 *lds) {
+                                              const Epi &ep, int M, int N, int K, int64_t lda, int64_t ldb, int m0,
+                                              int n0, uint4 *lds) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -362,23 +205,31 @@ __device__ __forceinline__ void gemm_tile_dma(const uint16_t *__restrict__ A, co
   // fetches is the one its LDS slot (base + 16 * lane) must hold under the swizzle.
   const uint16_t *a_src[2];
   const uint16_t *b_src[2];
+  int a_k[2], b_row[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int pa = (wave * 2 + i) * 64 + lane;      // A chunk slot: row pa / 4, physical chunk pa % 4
     const int ra = pa >> 2, ca = (pa & 3) ^ ((ra >> 2) & 3);
-    a_src[i] = A + static_cast<int64_t>(m0 + ra) * lda + ca * 8;
+    a_src[i] = A + static_cast<int64_t>(min(m0 + ra, M - 1)) * lda + ca * 8;
+    a_k[i] = ca * 8;
     const int pb = (wave * 2 + i) * 64 + lane;      // B chunk slot: row pb / 32, physical chunk pb % 32
     const int kb = pb >> 5, cb = (pb & 31) ^ (4 * (kb & 3));
-    b_src[i] = B + static_cast<int64_t>(kb) * ldb + n0 + cb * 8;
+    b_src[i] = B + static_cast<int64_t>(kb) * ldb + (n0 + cb * 8 < N ? n0 + cb * 8 : 0);
+    b_row[i] = kb;
   }
   auto issue = [&](int kt) {
     uint4 *stage = lds + (kt % kDmaStages) * kDmaStageChunks;
     const int k0 = kt * kDmaBK;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      __builtin_amdgcn_global_load_lds(a_src[i] + k0, (lds_void_t *)(stage + (wave * 2 + i) * 64), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(b_src[i] + static_cast<int64_t>(k0) * ldb,
-                                       (lds_void_t *)(stage + kDmaChunksA + (wave * 2 + i) * 64), 16, 0, 0);
+      const uint16_t *a = a_src[i] + k0, *b = b_src[i] + static_cast<int64_t>(k0) * ldb;
+      if (kTail && k0 + kDmaBK > K) {
+        const uint16_t *zero = reinterpret_cast<const uint16_t *>(&kZeroChunk);
+        if (k0 + a_k[i] >= K) a = zero;
+        if (k0 + b_row[i] >= K) b = zero;
+      }
+      __builtin_amdgcn_global_load_lds(a, (lds_void_t *)(stage + (wave * 2 + i) * 64), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(b, (lds_void_t *)(stage + kDmaChunksA + (wave * 2 + i) * 64), 16, 0, 0);
     }
   };
 
@@ -409,7 +260,7 @@ __device__ __forceinline__ void gemm_tile_dma(const uint16_t *__restrict__ A, co
   // t + S - 1 overwrites stage (t - 1) % S, whose reads every wave completed (lgkmcnt 0) before an
   // earlier barrier.
   const bool lag = wave >= 4;
-  const int k_tiles = K / kDmaBK;
+  const int k_tiles = kTail ? (K + kDmaBK - 1) / kDmaBK : K / kDmaBK;
 #pragma unroll
   for (int kt = 0; kt < kDmaStages - 1; ++kt)
     if (kt < k_tiles) issue(kt);
@@ -462,36 +313,36 @@ __device__ __forceinline__ void gemm_tile_dma(const uint16_t *__restrict__ A, co
   }
   if (!lag) dma_barrier();
 
+  // The tests cost 5 us of 49 at 4096 x 4096 x 1024 where they are not needed.
+  const auto store = [&](auto inside) {
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int i = m0 + wm * 128 + mt * 32 + frag_row;
+    for (int mt = 0; mt < 4; ++mt) {
+      const int i = m0 + wm * 128 + mt * 32 + frag_row;
+      if (!inside && i >= M) continue;
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+      for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn * 64 + nt * 32 + 8 * g + 4 * half;
-        const f32x16_t &v = acc[mt][nt];
-        ep.quad(i, n, v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
-      }
-  }
+        for (int g = 0; g < 4; ++g) {
+          const int n = n0 + wn * 64 + nt * 32 + 8 * g + 4 * half;
+          if (!inside && n >= N) continue;
+          const f32x16_t &v = acc[mt][nt];
+          ep.quad(i, n, v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+        }
+    }
+  };
+  if (m0 + kBM <= M && n0 + kBN <= N) store(std::true_type{});
+  else store(std::false_type{});
 }
 
-template <typename E, typename Epi>
+template <typename E, typename Epi, bool kTail>
 __global__ __launch_bounds__(kThreads, 1) void gemm_mfma(const uint16_t *__restrict__ A,
                                                               const uint16_t *__restrict__ B, Epi ep, int M,
                                                               int N, int K, int64_t lda, int64_t ldb, int tiles_m,
                                                               int tiles_n) {
-  __shared__ uint4 lds[2 * kStageChunks > kDmaStages * kDmaStageChunks ? 2 * kStageChunks : kDmaStages * kDmaStageChunks];
+  __shared__ uint4 lds[kDmaStages * kDmaStageChunks];
   int tm, tn;
   tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * kBM, n0 = tn * kBN;
-  const bool interior = m0 + kBM <= M && n0 + kBN <= N;
-  if (interior && (K % kDmaBK) == 0)
-    gemm_tile_dma<E, Epi>(A, B, ep, K, lda, ldb, m0, n0, lds);
-  else if (interior && (K % kBK) == 0)
-    gemm_tile<E, Epi, false>(A, B, ep, M, N, K, lda, ldb, m0, n0, lds);
-  else
-    gemm_tile<E, Epi, true>(A, B, ep, M, N, K, lda, ldb, m0, n0, lds);
+  gemm_tile_dma<E, Epi, kTail>(A, B, ep, M, N, K, lda, ldb, tm * kBM, tn * kBN, lds);
 }
 
 // ---------------------------------------------------------------- few rows: waves stream B, no LDS tiles
@@ -641,67 +492,259 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_skinny(const uint16_t 
   }
 }
 
-// Adds the K splits of a product in order and stores the result: one thread per 4 columns.
-template <typename Epi>
+// Adds the K splits of a product in order and stores the result: one thread per 4 columns (rows of `partials` are
+// padded to a multiple of 4). kQuads: 4 columns may be stored together.
+template <typename Epi, bool kQuads>
 __global__ __launch_bounds__(256) void gemm_splits(const float *__restrict__ partials, Epi ep, int M, int N, int splits) {
-  const int quads = N / 4;
-  const int64_t quad = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (quad >= static_cast<int64_t>(M) * quads) return;
+  const int quads = (N + 3) / 4;
+  const int64_t quad = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, all = static_cast<int64_t>(M) * quads;
+  if (quad >= all) return;
   const int row = static_cast<int>(quad / quads), col = 4 * static_cast<int>(quad % quads);
-  const int64_t split = static_cast<int64_t>(M) * N;
-  const float *p = partials + static_cast<int64_t>(row) * N + col;
-  float4 total = *reinterpret_cast<const float4 *>(p);
+  const f32x4_t *p = reinterpret_cast<const f32x4_t *>(partials) + quad;
+  f32x4_t total = p[0];
 #pragma unroll 8
-  for (int s = 1; s < splits; ++s) {
-    const float4 v = *reinterpret_cast<const float4 *>(p + s * split);
-    total.x += v.x;
-    total.y += v.y;
-    total.z += v.z;
-    total.w += v.w;
-  }
-  ep.quad(row, col, total.x, total.y, total.z, total.w);
-}
-
-// ---------------------------------------------------------------- general-shape fallback
-// 64 x 64 output tile per 256 threads (4 x 4 per thread), K in steps of 16 through LDS,
-// f32 fused multiply-add in increasing k.
-constexpr int kFT = 64, kFK = 16;
-
-template <typename E, typename Epi>
-__global__ __launch_bounds__(256) void gemm_simple(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
-                                                        Epi ep, int M, int N, int K, int64_t lda, int64_t ldb) {
-  __shared__ float sa[kFK][kFT + 1];
-  __shared__ float sb[kFK][kFT + 1];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * kFT, n0 = blockIdx.x * kFT;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += kFK) {
-    for (int e = threadIdx.x; e < kFT * kFK; e += 256) {
-      const int r = e / kFK, kc = e % kFK;
-      const int gm = m0 + r, gk = k0 + kc;
-      sa[kc][r] = (gm < M && gk < K) ? element_to_f32<E>(A[static_cast<int64_t>(gm) * lda + gk]) : 0.0f;
-      const int kr = e / kFT, nc = e % kFT;
-      const int gk2 = k0 + kr, gn = n0 + nc;
-      sb[kr][nc] = (gk2 < K && gn < N) ? element_to_f32<E>(B[static_cast<int64_t>(gk2) * ldb + gn]) : 0.0f;
-    }
-    __syncthreads();
+  for (int s = 1; s < splits; ++s) total += p[s * all];
+  if (kQuads) {
+    ep.quad(row, col, total[0], total[1], total[2], total[3]);
+  } else {
 #pragma unroll
-    for (int kc = 0; kc < kFK; ++kc)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(sa[kc][ty * 4 + i], sb[kc][tx * 4 + j], acc[i][j]);
-    __syncthreads();
-  }
-  for (int i = 0; i < 4; ++i) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= M) continue;
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn < N) ep.one(gm, gn, acc[i][j]);
-    }
+    for (int e = 0; e < 4; ++e)
+      if (col + e < N) ep.one(row, col + e, total[e]);
   }
 }
+
+// ---------------------------------------------------------------- small tiles
+// Workgroups of four waves (2 x 2, each a BM / 2 x BN / 2 quarter in 32 x 32 MFMA tiles) for products of too few
+// 256 x 256 tiles. One barrier per K step; S stages of LDS, written by DMA, the next S - 1 steps in flight. A CU
+// gets its operands at 20 to 50 GB/s when they come from HBM or the MALL, so such products are bound by the
+// bytes of the busiest CU and the latency of its K steps, and the tiles are chosen to reach every CU.
+// The layouts are those of the 256 x 256 kernel, for any BM, BN and BK. kDma false, for operands that are
+// not 16-byte aligned or whose extents or strides are not multiples of 8: the same tiles through registers (two
+// steps ahead), with 16-byte loads at 2-byte boundaries, single elements only where a chunk reaches past K
+// or N, and single-element stores (bf16 2048 x 2049 x 2047: 97 us; 1222 in f32 FMAs).
+template <int BM, int BN, int BK, int S>
+struct SmallTile {
+  static constexpr int kRowChunks = BK / 8;                       // 16-byte chunks of an A row
+  static constexpr int kChunksA = BM * kRowChunks, kChunksB = BK * BN / 8;
+  static constexpr int kStage = kChunksA + kChunksB;              // chunks of one stage
+  static constexpr int kLoadsA = kChunksA / 256, kLoadsB = kChunksB / 256;   // per thread and stage
+  // Chunk c of A row r is stored at c ^ swz_a(r): 16 consecutive rows' fragment reads hit every bank once.
+  static __device__ __forceinline__ int swz_a(int r) {
+    if constexpr (BK == 64) return (r & 7) ^ ((r >> 3) & 1);
+    return (r >> 2) & 3;
+  }
+  // Chunk c of B row k is stored at c ^ swz_b(k): the transposing reads of 4 consecutive rows hit every bank once.
+  static __device__ __forceinline__ int swz_b(int k) {
+    if constexpr (BN == 64) return 4 * ((k >> 1) & 1);
+    return 4 * (k & 3);
+  }
+};
+
+// 8 elements at p, `count` of them (0..8) present, at any 2-byte boundary; zeros for the others.
+__device__ __forceinline__ uint4 load_8(const uint16_t *p, int count) {
+  struct __attribute__((packed, aligned(2))) Chunk { uint32_t w[4]; };
+  if (count >= 8) {
+    const Chunk c = *reinterpret_cast<const Chunk *>(p);
+    return make_uint4(c.w[0], c.w[1], c.w[2], c.w[3]);
+  }
+  uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int i = 0; i < 7; ++i)
+    if (i < count) w[i / 2] |= static_cast<uint32_t>(p[i]) << (16 * (i & 1));
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma>
+__global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, Epi ep,
+                                                  int M, int N, int K, int64_t lda, int64_t ldb, int tiles_m,
+                                                  int tiles_n, float *__restrict__ partials) {
+  typedef SmallTile<BM, BN, BK, S> T;
+  typedef typename Elem<E>::x8 x8;
+  constexpr int MT = BM / 64, NT = BN / 64, KT = BK / 16;
+  __shared__ uint4 lds[S * T::kStage];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int tile = xcd_tile(tiles_m * tiles_n);   // the row blocks of one column block are neighbours
+  if (tile < 0) return;
+  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+
+  // Slot p = tid + 256 i of a stage's A holds chunk (p % kRowChunks) ^ swz of row p / kRowChunks; of its B,
+  // chunk (p % (BN / 8)) ^ swz of row p / (BN / 8). Rows past M and columns past N read valid
+  // ones instead; their products are not stored.
+  const uint16_t *a_src[T::kLoadsA], *b_src[T::kLoadsB];
+  int a_k[T::kLoadsA], b_k[T::kLoadsB], b_n[T::kLoadsB];
+#pragma unroll
+  for (int i = 0; i < T::kLoadsA; ++i) {
+    const int p = tid + 256 * i, r = p / T::kRowChunks;
+    a_k[i] = ((p % T::kRowChunks) ^ T::swz_a(r)) * 8;
+    a_src[i] = A + static_cast<int64_t>(min(m0 + r, M - 1)) * lda + a_k[i];
+  }
+#pragma unroll
+  for (int i = 0; i < T::kLoadsB; ++i) {
+    const int p = tid + 256 * i, n = ((p % (BN / 8)) ^ T::swz_b(p / (BN / 8))) * 8;
+    b_k[i] = p / (BN / 8);
+    b_n[i] = n0 + n < N ? n0 + n : 0;
+    b_src[i] = B + static_cast<int64_t>(b_k[i]) * ldb + b_n[i];
+  }
+
+  f32x16_t acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+  const int frag = lane & 31, half = lane >> 5;
+  const int g16 = lane >> 4, i16 = lane & 15;
+  const int t_k = 8 * (g16 >> 1) + (i16 >> 2), t_n = 16 * (g16 & 1) + 4 * (i16 & 3);
+  x8 af[KT][MT], bf[KT][NT];
+  auto read_tile = [&](int stage) {
+    const uint4 *sa = lds + stage * T::kStage;
+    const uint16_t *sb = reinterpret_cast<const uint16_t *>(sa + T::kChunksA);
+#pragma unroll
+    for (int kk = 0; kk < KT; ++kk) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int r = wm * (BM / 2) + t * 32 + frag;
+        af[kk][t] = __builtin_bit_cast(x8, sa[r * T::kRowChunks + ((kk * 2 + half) ^ T::swz_a(r))]);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        i16x4_t parts[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = kk * 16 + t_k + 4 * h, n = wn * (BN / 2) + t * 32 + t_n;
+          parts[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_i16x4_t *)(sb + k * BN + ((n >> 3) ^ T::swz_b(k)) * 8 + (n & 7)));
+        }
+        bf[kk][t] = __builtin_bit_cast(x8, parts);
+      }
+    }
+  };
+  auto multiply = [&]() {
+#pragma unroll
+    for (int kk = 0; kk < KT; ++kk)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = Elem<E>::mma(bf[kk][nt], af[kk][mt], acc[mt][nt]);
+  };
+
+  const int all_tiles = (K + BK - 1) / BK;
+  const int first = static_cast<int>(static_cast<int64_t>(all_tiles) * blockIdx.y / gridDim.y);
+  const int k_tiles = static_cast<int>(static_cast<int64_t>(all_tiles) * (blockIdx.y + 1) / gridDim.y) - first;
+  if constexpr (kDma) {
+    constexpr int kLoads = T::kLoadsA + T::kLoadsB;
+    const uint16_t *zero = reinterpret_cast<const uint16_t *>(&kZeroChunk);
+    auto issue = [&](int kt) {
+      uint4 *stage = lds + (kt % S) * T::kStage;
+      const int k0 = (first + kt) * BK;
+      const bool tail = k0 + BK > K;   // uniform
+#pragma unroll
+      for (int i = 0; i < T::kLoadsA; ++i) {
+        const uint16_t *src = a_src[i] + k0;
+        if (tail && k0 + a_k[i] >= K) src = zero;
+        __builtin_amdgcn_global_load_lds(src, (lds_void_t *)(stage + wave * 64 + 256 * i), 16, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < T::kLoadsB; ++i) {
+        const uint16_t *src = b_src[i] + static_cast<int64_t>(k0) * ldb;
+        if (tail && k0 + b_k[i] >= K) src = zero;
+        __builtin_amdgcn_global_load_lds(src, (lds_void_t *)(stage + T::kChunksA + wave * 64 + 256 * i), 16, 0, 0);
+      }
+    };
+#pragma unroll
+    for (int kt = 0; kt < S - 1; ++kt)
+      if (kt < k_tiles) issue(kt);
+    for (int kt = 0; kt < k_tiles; ++kt) {
+      // This wave's loads of tile kt complete; up to S - 2 later tiles stay in flight.
+      const int later = min(k_tiles - 1 - kt, S - 2);
+      if (S > 4 && later >= 3) INTENT_WAIT_VMCNT(3 * kLoads);
+      else if (S > 3 && later == 2) INTENT_WAIT_VMCNT(2 * kLoads);
+      else if (later == 1) INTENT_WAIT_VMCNT(kLoads);
+      else INTENT_WAIT_VMCNT(0);
+      dma_barrier();
+      read_tile(kt % S);
+      // Overwrites the stage of tile kt - 1, which every wave read before the barrier.
+      if (kt + S - 1 < k_tiles) issue(kt + S - 1);
+      multiply();
+      INTENT_WAIT_LGKMCNT0();
+    }
+  } else {
+    // Two register sets: the loads of tile kt + 2 are in flight while tile kt is multiplied.
+    uint4 ra[2][T::kLoadsA], rb[2][T::kLoadsB];
+    auto load = [&](int kt, uint4 (&qa)[T::kLoadsA], uint4 (&qb)[T::kLoadsB]) {
+      const int k0 = (first + kt) * BK;
+#pragma unroll
+      for (int i = 0; i < T::kLoadsA; ++i) qa[i] = load_8(a_src[i] + k0, K - (k0 + a_k[i]));
+#pragma unroll
+      for (int i = 0; i < T::kLoadsB; ++i)
+        qb[i] = load_8(b_src[i] + static_cast<int64_t>(k0) * ldb, k0 + b_k[i] < K ? N - b_n[i] : 0);
+    };
+    auto store = [&](int stage, const uint4 (&qa)[T::kLoadsA], const uint4 (&qb)[T::kLoadsB]) {
+#pragma unroll
+      for (int i = 0; i < T::kLoadsA; ++i) lds[stage * T::kStage + tid + 256 * i] = qa[i];
+#pragma unroll
+      for (int i = 0; i < T::kLoadsB; ++i) lds[stage * T::kStage + T::kChunksA + tid + 256 * i] = qb[i];
+    };
+    if (k_tiles > 0) load(0, ra[0], rb[0]);
+    if (k_tiles > 1) load(1, ra[1], rb[1]);
+    if (k_tiles > 0) store(0, ra[0], rb[0]);
+    __syncthreads();
+    for (int kt = 0; kt < k_tiles; kt += 2) {
+      if (kt + 2 < k_tiles) load(kt + 2, ra[0], rb[0]);
+      read_tile(0);
+      multiply();
+      if (kt + 1 >= k_tiles) break;
+      store(1, ra[1], rb[1]);
+      __syncthreads();
+      if (kt + 3 < k_tiles) load(kt + 3, ra[1], rb[1]);
+      read_tile(1);
+      multiply();
+      if (kt + 2 < k_tiles) store(0, ra[0], rb[0]);
+      __syncthreads();
+    }
+  }
+
+  // acc[mt][nt][4 g + e] is row wm BM / 2 + 32 mt + frag, column wn BN / 2 + 32 nt + 8 g + 4 half + e.
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int i = m0 + wm * (BM / 2) + mt * 32 + frag;
+    if (i >= M) continue;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int n = n0 + wn * (BN / 2) + nt * 32 + 8 * g + 4 * half;
+        const f32x16_t &v = acc[mt][nt];
+        if (partials != nullptr) {
+          const int64_t width = (N + 3) & ~3;
+          if (n < N)
+            *reinterpret_cast<float4 *>(partials + (static_cast<int64_t>(blockIdx.y) * M + i) * width + n) =
+                make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+        } else if (kDma) {
+          if (n < N) ep.quad(i, n, v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) ep.one(i, n + e, v[4 * g + e]);
+        }
+      }
+  }
+}
+
+// ---------------------------------------------------------------- launches
+// The tile size follows from how many tiles the chip's 256 CUs hold at once, bf16 measured on both sides of each line:
+//   * up to 128 tiles of 128 x 128: 64 x 64 ones, K divided over workgroups where these are few too (1000^3
+//     10.5 us against 15.5 in 128 x 128, 512 x 512 x 4096 14 against 45);
+//   * up to 256: 128 x 128 with four stages, one a CU (1021 x 2304 x 768 13.4 us against 15.3 in 64 x 64 and 48
+//     in 256 x 256; 2048^3 32 against 46 and 54);
+//   * up to 512: the same with two stages, two a CU (2639 x 2880 x 6912 125 us against 173 with four stages
+//     and 155 in 256 x 256; 8192 x 1024 x 4096 90 against 103 in 256 x 256);
+//   * more: 256 x 256 (4096 x 4096 x 1024 44 us against 61, 8000 x 2048 x 520 32 against 41).
+constexpr int64_t kChip = 256;
 
 bool fast_path(const void *a, const void *b, const void *c, int64_t n, int64_t k, int64_t lda, int64_t ldb,
                int64_t ldc) {
@@ -712,29 +755,38 @@ bool fast_path(const void *a, const void *b, const void *c, int64_t n, int64_t k
 }  // namespace
 
 int quantized_gemm_resources(IntentHipKernelResources *out) {
-  return describe_kernel(reinterpret_cast<const void *>(&gemm_mfma<_Float16, QuantizeStore>), "gemm_mfma<f16,quantize>",
+  return describe_kernel(reinterpret_cast<const void *>(&gemm_mfma<_Float16, QuantizeStore, false>), "gemm_mfma<f16,quantize>",
                          kThreads, out);
 }
 
 namespace {
 
 template <typename E>
-int resources_of(int64_t m, const char *few, const char *tiles, IntentHipKernelResources *out) {
+int resources_of(int64_t m, int64_t n, IntentHipKernelResources *out) {   // aligned operands
   typedef CastStore<E, 0> Epi;
-  const void *kernel = m <= 16   ? reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 1, true>)
-                       : m <= 32 ? reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 2, true>)
-                       : m <= 64 ? reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 4, true>)
-                                 : reinterpret_cast<const void *>(&gemm_skinny<E, Epi, 4, false>);
-  if (m <= kSkinnyRows) return describe_kernel(kernel, few, kSkinnyWaves * 64, out);
-  return describe_kernel(reinterpret_cast<const void *>(&gemm_mfma<E, Epi>), tiles, kThreads, out);
+  const auto describe = [&](auto kernel, const char *f16, const char *bf16, int threads) {
+    return describe_kernel(reinterpret_cast<const void *>(kernel), std::is_same<E, _Float16>::value ? f16 : bf16, threads,
+                           out);
+  };
+  const int64_t tiles = (m + 127) / 128 * ((n + 127) / 128);
+  if (m <= kSkinnyRows) {
+    const auto kernel = m <= 16   ? &gemm_skinny<E, Epi, 1, true>
+                        : m <= 32 ? &gemm_skinny<E, Epi, 2, true>
+                        : m <= 64 ? &gemm_skinny<E, Epi, 4, true>
+                                  : &gemm_skinny<E, Epi, 4, false>;
+    return describe(kernel, "gemm_skinny<f16>", "gemm_skinny<bf16>", kSkinnyWaves * 64);
+  }
+  if (tiles > 2 * kChip) return describe(&gemm_mfma<E, Epi, false>, "gemm_mfma<f16>", "gemm_mfma<bf16>", kThreads);
+  const auto kernel = tiles <= kChip / 2 ? &gemm_small<E, Epi, 64, 64, 64, 4, true>
+                      : tiles <= kChip   ? &gemm_small<E, Epi, 128, 128, 64, 4, true>
+                                         : &gemm_small<E, Epi, 128, 128, 64, 2, true>;
+  return describe(kernel, "gemm_small<f16>", "gemm_small<bf16>", 256);
 }
 
 }  // namespace
 
 int gemm_resources(int dtype, int64_t m, int64_t n, IntentHipKernelResources *out) {
-  (void)n;
-  return dtype == INTENT_HIP_F16 ? resources_of<_Float16>(m, "gemm_skinny<f16>", "gemm_mfma<f16>", out)
-                                 : resources_of<__bf16>(m, "gemm_skinny<bf16>", "gemm_mfma<bf16>", out);
+  return dtype == INTENT_HIP_F16 ? resources_of<_Float16>(m, n, out) : resources_of<__bf16>(m, n, out);
 }
 
 namespace {
@@ -750,16 +802,37 @@ int skinny_splits(int64_t m, int64_t n, int64_t k) {
   return splits < 2 ? 1 : static_cast<int>(splits);
 }
 
+// The same for 64 x 64 tiles.
+int small_splits(int64_t m, int64_t n, int64_t k) {
+  if (m < 1 || n < 1 || k < 1024) return 1;
+  const int64_t tiles = (m + 63) / 64 * ((n + 63) / 64);
+  const int64_t splits = 256 / tiles < k / 256 ? 256 / tiles : k / 256;
+  return splits < 2 ? 1 : static_cast<int>(splits);
+}
+
+template <typename E, typename Epi, bool kQuads>
+void launch_splits(const float *partials, const Epi &ep, int m, int n, int splits, hipStream_t s) {
+  const int64_t quads = static_cast<int64_t>(m) * ((n + 3) / 4);
+  gemm_splits<Epi, kQuads><<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, ep, m, n, splits);
+}
+
+template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma>
+void launch_small(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, int n, int k, int64_t lda, int64_t ldb,
+                  float *partials, int splits, hipStream_t s) {
+  const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
+  gemm_small<E, Epi, BM, BN, BK, S, kDma>
+      <<<dim3(xcd_blocks(static_cast<int64_t>(tiles_m) * tiles_n), splits), dim3(256), 0, s>>>(
+          A, B, ep, m, n, k, lda, ldb, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
+  if (splits > 1) launch_splits<E, Epi, kDma>(partials, ep, m, n, splits, s);
+}
+
 template <typename E, typename Epi, int MT, bool kStream>
 void launch_skinny(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, int n, int k, int64_t lda, int64_t ldb,
                    float *partials, int splits, hipStream_t s) {
   const int tiles_m = (m + 16 * MT - 1) / (16 * MT), tiles_n = (n + kSkinnyCols - 1) / kSkinnyCols;
   gemm_skinny<E, Epi, MT, kStream><<<dim3(xcd_blocks(tiles_m * tiles_n), splits), dim3(kSkinnyWaves * 64), 0, s>>>(
       A, B, ep, m, n, k, lda, ldb, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
-  if (splits > 1) {
-    const int64_t quads = static_cast<int64_t>(m) * n / 4;
-    gemm_splits<Epi><<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, ep, m, n, splits);
-  }
+  if (splits > 1) launch_splits<E, Epi, true>(partials, ep, m, n, splits, s);
 }
 
 // Few rows, and strides that keep a lane's offset (24 rows of B, all rows of A) below 2^31 elements.
@@ -767,14 +840,14 @@ bool skinny(int64_t m, int64_t lda, int64_t ldb) {
   return m <= kSkinnyRows && lda < (int64_t{1} << 22) && ldb < (int64_t{1} << 25);
 }
 
-// The MFMA kernels when `fast` (the operand shape and layout they take), else the general one.
-// `partials`: null, or room for the f32 sums of skinny_splits(m, n, k) splits.
+// `fast`: the operand layout that the DMA takes (fast_path); every other one runs in 64 x 64 tiles through registers.
+// `partials`: null, or room for splits_bytes(m, n, k).
 template <typename E, typename Epi>
 int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t m, int64_t n, int64_t k, int64_t lda,
                     int64_t ldb, bool fast, float *partials, hipStream_t s) {
+  const int M = static_cast<int>(m), N = static_cast<int>(n), depth = static_cast<int>(k);
   if (k > 0 && fast && skinny(m, lda, ldb)) {
     const int splits = partials != nullptr ? skinny_splits(m, n, k) : 1;
-    const int M = static_cast<int>(m), N = static_cast<int>(n), depth = static_cast<int>(k);
     if (m <= 16) launch_skinny<E, Epi, 1, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
     else if (m <= 32) launch_skinny<E, Epi, 2, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
     else if (m <= 64) launch_skinny<E, Epi, 4, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
@@ -782,24 +855,29 @@ int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t
     if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_skinny");
     return INTENT_HIP_OK;
   }
-  if (k > 0 && fast) {
-    const int tiles_m = static_cast<int>((m + kBM - 1) / kBM), tiles_n = static_cast<int>((n + kBN - 1) / kBN);
-    gemm_mfma<E, Epi><<<dim3(tiles_m * tiles_n), dim3(kThreads), 0, s>>>(
-        A, B, ep, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), lda, ldb, tiles_m, tiles_n);
-    if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_mfma");
-    return INTENT_HIP_OK;
+  const int splits = partials != nullptr ? small_splits(m, n, k) : 1;
+  const auto tiles = [&](int64_t edge) { return (m + edge - 1) / edge * ((n + edge - 1) / edge); };
+  if (!fast || k == 0) {
+    launch_small<E, Epi, 64, 64, 64, 2, false>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
+  } else if (tiles(128) <= kChip / 2) {
+    launch_small<E, Epi, 64, 64, 64, 4, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
+  } else if (tiles(128) <= kChip) {
+    launch_small<E, Epi, 128, 128, 64, 4, true>(A, B, ep, M, N, depth, lda, ldb, nullptr, 1, s);
+  } else if (tiles(128) <= 2 * kChip) {
+    launch_small<E, Epi, 128, 128, 64, 2, true>(A, B, ep, M, N, depth, lda, ldb, nullptr, 1, s);
+  } else {
+    const int tiles_m = (M + kBM - 1) / kBM, tiles_n = (N + kBN - 1) / kBN;
+    const auto kernel = depth % kDmaBK == 0 ? &gemm_mfma<E, Epi, false> : &gemm_mfma<E, Epi, true>;
+    kernel<<<dim3(tiles_m * tiles_n), dim3(kThreads), 0, s>>>(A, B, ep, M, N, depth, lda, ldb, tiles_m, tiles_n);
   }
-  const dim3 grid(static_cast<unsigned>((n + kFT - 1) / kFT), static_cast<unsigned>((m + kFT - 1) / kFT));
-  gemm_simple<E, Epi><<<grid, dim3(256), 0, s>>>(A, B, ep, static_cast<int>(m), static_cast<int>(n),
-                                                 static_cast<int>(k), lda, ldb);
-  if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_simple");
+  if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm");
   return INTENT_HIP_OK;
 }
 
 // Bytes of the f32 partial sums of a product's K splits (0: one workgroup per output tile).
 size_t splits_bytes(int64_t m, int64_t n, int64_t k) {
-  const int splits = skinny_splits(m, n, k);
-  return splits > 1 ? static_cast<size_t>(splits) * m * n * sizeof(float) : 0;
+  const int few = skinny_splits(m, n, k), small = small_splits(m, n, k), splits = few > small ? few : small;
+  return splits > 1 ? static_cast<size_t>(splits) * m * ((n + 3) / 4 * 4) * sizeof(float) : 0;
 }
 
 template <typename E, int kAct>

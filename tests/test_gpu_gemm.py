@@ -85,18 +85,11 @@ def test_gemm_config3_full(device):
     assert (np.abs(got.astype(np.int32) - want.astype(np.int32)) <= 2).mean() > 0.999
 
 
-# The few-row kernel: row blocks of 16, 32 and 64 and their edges, two row blocks (m > 64), column
-# counts below and past one 64-column workgroup, K below one 64-deep unit, past it by every multiple
-# of 8, and long enough that K is divided over workgroups (from 2048 rows on; 2056 leaves a tail).
-@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (15, 64, 24), (16, 72, 40), (17, 56, 64), (32, 520, 56), (33, 136, 72),
-                                   (64, 64, 120), (65, 200, 1000), (128, 72, 520), (1, 24, 2048), (31, 1000, 2056),
-                                   (100, 136, 4104), (128, 8, 2048), (3, 16384, 2048)])
-@pytest.mark.parametrize("workspace", ["prepare", "static"])
-def test_gemm_few_rows(device, m, n, k, workspace):
+def check_product(device, m, n, k, workspace):
     """Against the oracle, and exact on small integers whose sums f32 holds (an element read from the wrong place,
     twice or not at all shows); rows of NaN in A and columns of NaN in B stay in their own row and
     column of C, so no padding row, column or K group reaches a result."""
-    announce("gemm few rows", m, n, k, workspace)
+    announce("gemm", m, n, k, workspace)
     kernel = intent.jit(bf16_gemm, backend="hip", backend_options={"workspace": workspace})
     call = lambda a, b: bf16_tensor_bits(kernel.run(to_bf16_tensor(a, device), to_bf16_tensor(b, device)))  # noqa: E731
     a, b = inputs.gemm_bf16(seed=m + n + k, m=m, n=n, k=k)
@@ -111,3 +104,54 @@ def test_gemm_few_rows(device, m, n, k, workspace):
     expected = np.zeros((m, n), bool)
     expected[m - 1, :] = expected[:, n - 1] = True
     assert (nan == expected).all()
+
+
+# 64 x 64 and 128 x 128 tiles (up to 128, 256 and 512 of the latter) and 256 x 256 ones, each with its last row and column
+# of tiles partly filled, K below one step, off it by every multiple of 8, and divided over workgroups;
+# then operands the DMA does not take: odd extents, one below and above a tile, every K remainder class.
+@pytest.mark.parametrize("m,n,k", [(129, 8, 8), (200, 72, 56), (192, 64, 64), (130, 1000, 136), (300, 264, 1032),
+                                   (257, 136, 2056), (1500, 1400, 72), (1409, 1416, 192), (2300, 2200, 40),
+                                   (2310, 2304, 128), (3000, 3080, 8), (2900, 3088, 104), (2900, 3072, 192),
+                                   (1, 1, 1), (63, 65, 7), (65, 63, 9), (130, 129, 63), (64, 200, 65), (129, 77, 1027),
+                                   (200, 131, 2049), (33, 8, 17)])
+@pytest.mark.parametrize("workspace", ["prepare", "static"])
+def test_gemm_tiles(device, m, n, k, workspace):
+    """As test_gemm_few_rows; the last element of each operand and of the result lies at its buffer's end."""
+    check_product(device, m, n, k, workspace)
+
+
+@pytest.mark.parametrize("lda,ldb,ldc,offset", [(8, 0, 0, 0), (3, 0, 0, 0), (0, 5, 0, 0), (0, 0, 1, 0), (0, 0, 4, 0),
+                                                (0, 0, 0, 1), (8, 8, 4, 8), (1, 2, 3, 3)])
+@pytest.mark.parametrize("m,n,k", [(40, 64, 72), (200, 136, 72), (1500, 1400, 64)])
+def test_gemm_strides_and_offsets(device, m, n, k, lda, ldb, ldc, offset):
+    """Row strides `lda`, `ldb`, `ldc` elements past the row, and operands `offset` elements into their buffers: whichever
+    kernel takes a layout, the result is that of the contiguous operands up to the order of the f32 sums,
+    and the result's buffer is unchanged outside it."""
+    announce("gemm layouts", m, n, k, lda, ldb, ldc, offset)
+    rng = np.random.default_rng(m + n + k)
+    ints = [rng.integers(-2, 3, shape).astype(np.float32) for shape in ((m, k), (k, n))]
+
+    def place(data, rows, cols, pad):
+        base = torch.full((rows * (cols + pad) + offset,), 9.0, dtype=torch.bfloat16, device=device)
+        view = base[offset:].view(rows, cols + pad)[:, :cols]
+        if data is not None:
+            view.copy_(torch.from_numpy(data).to(device))
+        return base, view
+
+    (_, a), (_, b), (base, c) = place(ints[0], m, k, lda), place(ints[1], k, n, ldb), place(None, m, n, ldc)
+    intent.jit(bf16_gemm, backend="hip")(a, b, c)
+    want = torch.from_numpy(ints[0] @ ints[1]).to(device).to(torch.bfloat16)     # exact in f32
+    assert torch.equal(c, want)
+    c.fill_(9.0)
+    assert bool((base == 9.0).all())
+
+
+# The few-row kernel: row blocks of 16, 32 and 64 and their edges, two row blocks (m > 64), column
+# counts below and past one 64-column workgroup, K below one 64-deep unit, past it by every multiple
+# of 8, and long enough that K is divided over workgroups (from 2048 rows on; 2056 leaves a tail).
+@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (15, 64, 24), (16, 72, 40), (17, 56, 64), (32, 520, 56), (33, 136, 72),
+                                   (64, 64, 120), (65, 200, 1000), (128, 72, 520), (1, 24, 2048), (31, 1000, 2056),
+                                   (100, 136, 4104), (128, 8, 2048), (3, 16384, 2048)])
+@pytest.mark.parametrize("workspace", ["prepare", "static"])
+def test_gemm_few_rows(device, m, n, k, workspace):
+    check_product(device, m, n, k, workspace)
