@@ -447,18 +447,19 @@ __global__ __launch_bounds__(kThreads) void attention_bwd_dq_reduce(const float 
 }
 
 // ---------------------------------------------------------------- dK / dV
-// kSplit: the workgroup takes one query head of the group and one of `qsplits` consecutive
-// ranges of its query tiles (grid x head_group x qsplits) and writes its unscaled f32 dK and dV
-// sums to `partial` (head_group * qsplits parts of dK, then as many of dV, each
+// kSplit: the workgroup takes one of `head_parts` parts of the group's query heads and one of `qsplits`
+// consecutive ranges of their query tiles (grid x head_parts x qsplits) and writes its unscaled f32 dK and dV
+// sums to `partial` (head_parts * qsplits parts of dK, then as many of dV, each
 // [D / 8][batch * kv_heads * sk][8] as in dQ), which attention_bwd_dkdv_reduce folds. Used when too
-// few workgroups would run.
+// few workgroups would run, or uneven ones (DkdvPlan).
 // kPart: dK and dV together, or one of them (DkdvPart); kW: waves of 32 keys per workgroup.
 template <int D, bool kSplit, int kPart, int kW>
 __device__ __forceinline__ void attention_bwd_dkdv_body(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ G, const float *__restrict__ LSE, const float *__restrict__ DELTA,
     uint16_t *__restrict__ DK, uint16_t *__restrict__ DV, float *__restrict__ partial, int kv_heads,
-    int head_group, int sq, int sk, BwdGeometry g, float scale, int causal, int k_blocks, int qsplits, uint4 *lds) {
+    int head_group, int sq, int sk, BwdGeometry g, float scale, int causal, int k_blocks, int head_parts, int qsplits,
+    uint4 *lds) {
   constexpr int kChunks = kTile * D / 8;          // 16-byte chunks of one Q (or dO) tile
   constexpr int kDma = kChunks / (kW * 64);
   constexpr int kKRows = kW * 32;
@@ -472,8 +473,8 @@ __device__ __forceinline__ void attention_bwd_dkdv_body(
   const int bhs = static_cast<int>(blockIdx.x) % bh_count;
   const int qs = kSplit ? bhs % qsplits : 0;                 // the query-tile range (split mode)
   const int rest = kSplit ? bhs / qsplits : bhs;
-  const int split = kSplit ? rest % head_group : 0;          // the query head of the group (split mode)
-  const int bh = kSplit ? rest / head_group : rest;
+  const int split = kSplit ? rest % head_parts : 0;          // the part of the group's query heads (split mode)
+  const int bh = kSplit ? rest / head_parts : rest;
   const int b = bh / kv_heads, kh = bh % kv_heads;
 
   const int wk0 = kb * kKRows + wave * 32;
@@ -502,9 +503,10 @@ __device__ __forceinline__ void attention_bwd_dkdv_body(
   const int span = q_tiles - first_all;
   const int first = first_all + (kSplit ? qs * span / qsplits : 0);
   const int per_head = kSplit ? first_all + (qs + 1) * span / qsplits - first : span;
-  const int tiles = (kSplit ? 1 : head_group) * per_head;
+  const int heads = kSplit ? head_group / head_parts : head_group;   // query heads of this workgroup
+  const int tiles = heads * per_head;
 
-  auto tile_head = [&](int t) { return kh * head_group + (kSplit ? split : t / per_head); };
+  auto tile_head = [&](int t) { return kh * head_group + (kSplit ? split * heads : 0) + t / per_head; };
   auto tile_q0 = [&](int t) { return (first + t % per_head) * kTile; };
   auto issue = [&](int t) {
     uint4 *stage = lds + (t % kStages) * kStage;
@@ -645,9 +647,9 @@ __device__ __forceinline__ void attention_bwd_dkdv_body(
 
   if (!k_ok) return;
   if constexpr (kSplit) {
-    const int64_t rows = static_cast<int64_t>(gridDim.x / (k_blocks * head_group * qsplits)) * sk;   // batch * kv_heads * sk
+    const int64_t rows = static_cast<int64_t>(gridDim.x / (k_blocks * head_parts * qsplits)) * sk;   // batch * kv_heads * sk
     const int64_t row = (static_cast<int64_t>(b) * kv_heads + kh) * sk + lane_k;
-    const int parts = head_group * qsplits, part = split * qsplits + qs;
+    const int parts = head_parts * qsplits, part = split * qsplits + qs;
     float *pk = partial + part * rows * D + row * 8 + 4 * half;
     float *pv = partial + (parts + part) * rows * D + row * 8 + 4 * half;
 #pragma unroll
@@ -686,11 +688,11 @@ __global__ __launch_bounds__(kW * 64, 1) void attention_bwd_dkdv(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ G, const float *__restrict__ LSE, const float *__restrict__ DELTA,
     uint16_t *__restrict__ DK, uint16_t *__restrict__ DV, float *__restrict__ partial, int kv_heads,
-    int head_group, int sq, int sk, BwdGeometry g, float scale, int causal, int k_blocks, int qsplits) {
+    int head_group, int sq, int sk, BwdGeometry g, float scale, int causal, int k_blocks, int head_parts, int qsplits) {
   constexpr int kStage = 2 * (kTile * D / 8) + 2 * (kTile / 4);
   __shared__ uint4 lds[kStages * kStage];
   attention_bwd_dkdv_body<D, kSplit, kPart, kW>(Q, K, V, G, LSE, DELTA, DK, DV, partial, kv_heads, head_group, sq, sk, g,
-                                     scale, causal, k_blocks, qsplits, lds);
+                                     scale, causal, k_blocks, head_parts, qsplits, lds);
 }
 
 // dK = f16(scale * sum of the `parts` partial dK), dV = f16(sum of the partial dV); four columns
@@ -862,24 +864,48 @@ int64_t dq_workspace(int splits, int64_t batch, int64_t q_heads, int64_t sq, int
   return splits > 1 ? splits * batch * q_heads * sq * d * static_cast<int64_t>(sizeof(float)) : 0;
 }
 
-// dK/dV: split by query head of the group and by query-tile range; returns the number of ranges
-// per head (0 = no split).
-int dkdv_qsplits(int64_t batch, int64_t q_heads, int64_t head_group, int64_t sq, int64_t sk) {
-  if (batch <= 0 || q_heads <= 0 || sq <= 0 || sk <= 0) return 0;
-  const int64_t blocks = batch * (q_heads / head_group) * ((sk + kRows - 1) / kRows);
-  if (blocks >= kSplitBelow) return 0;
+// dK/dV: how one call divides the query heads of a group and their query tiles over workgroups (parts() = 0: not at all).
+// Fewer than kSplitBelow workgroups: by query head, and by up to kMaxSplits query ranges. From there to twice as many
+// (4-wave kernel, or the 8-wave ones on wide grids) every CU has a workgroup, but with a causal mask
+// the first key block's walk is twice the average one's and sets the time: two parts, so that the
+// 2 x kSplitBelow or more workgroups, heaviest first, even out. The fold moves 32 D bytes per key, which walks of
+// at least kEvenPairs queries (over the group's heads) return: dK/dV with the fold, causal, D128, B2 HQ32 HK8 S2048
+// 434 -> 279 us, B1 HQ32 HK16 S2048 219 -> 149; but B2 HQ32 HK32 S1024 120 -> 146, B1 HQ32 HK32 S1500 97 -> 130. Without
+// the mask the walks are even (B2 HQ32 HK8 S2048 424 -> 450), and the launch leaves them whole.
+constexpr int64_t kEvenPairs = 4096;
+
+struct DkdvPlan {
+  int head_parts = 0, qsplits = 0;
+  bool wide = false;       // 8-wave kernels, dK and dV apart
+  bool optional = false;   // runs unsplit without a mask, or with a workspace too small for it
+  int parts() const { return head_parts * qsplits; }
+};
+
+DkdvPlan dkdv_plan(int64_t batch, int64_t q_heads, int64_t head_group, int64_t sq, int64_t sk) {
+  DkdvPlan plan;
+  if (batch <= 0 || q_heads <= 0 || sq <= 0 || sk <= 0) return plan;
+  const int64_t groups = batch * (q_heads / head_group);
+  plan.wide = groups * sk >= kWideRows;
+  const int64_t rows = plan.wide ? 2 * kRows : kRows, blocks = groups * ((sk + rows - 1) / rows);
+  const int64_t query_tiles = (sq + kTile - 1) / kTile;
+  if (blocks >= kSplitBelow) {
+    if (blocks >= 2 * kSplitBelow || head_group * sq < kEvenPairs) return plan;
+    plan.optional = true;
+    plan.head_parts = head_group % 2 == 0 ? 2 : 1;
+    plan.qsplits = 2 / plan.head_parts;
+    return plan;
+  }
   int64_t qsplits = (kSplitTarget + blocks * head_group - 1) / (blocks * head_group);
   qsplits = qsplits < kMaxSplits ? qsplits : kMaxSplits;
-  const int64_t query_tiles = (sq + kTile - 1) / kTile;
   qsplits = qsplits < query_tiles ? qsplits : query_tiles;
-  if (head_group == 1 && qsplits <= 1) return 0;
-  return static_cast<int>(qsplits < 1 ? 1 : qsplits);
+  if (head_group == 1 && qsplits <= 1) return plan;
+  plan.head_parts = static_cast<int>(head_group);
+  plan.qsplits = static_cast<int>(qsplits < 1 ? 1 : qsplits);
+  return plan;
 }
 
-int64_t dkdv_workspace(int qsplits, int64_t batch, int64_t q_heads, int64_t head_group, int64_t sk, int64_t d) {
-  return qsplits > 0 ? 2 * head_group * qsplits * batch * (q_heads / head_group) * sk * d *
-                           static_cast<int64_t>(sizeof(float))
-                     : 0;
+int64_t dkdv_workspace(const DkdvPlan &plan, int64_t batch, int64_t kv_heads, int64_t sk, int64_t d) {
+  return 2 * plan.parts() * batch * kv_heads * sk * d * static_cast<int64_t>(sizeof(float));
 }
 
 // attention_bwd_dq<D, kW> over every (batch, query head), block of 32 kW queries and key range;
@@ -906,51 +932,51 @@ int launch_dq(const uint16_t *Q, const uint16_t *K, const uint16_t *V, const uin
 }
 
 // attention_bwd_dkdv<D, kSplit, kPart, kW> over every (batch, key head) and block of 32 kW keys
-// (times head_group when split).
+// (times the parts of the plan when split).
 template <int D, bool kSplit, int kPart, int kW>
 int launch_dkdv(const uint16_t *Q, const uint16_t *K, const uint16_t *V, const uint16_t *G, const float *lse,
                 const float *delta, uint16_t *DK, uint16_t *DV, float *partial, int64_t batch, int64_t kv_heads,
                 int64_t head_group, int64_t sq, int64_t sk, const BwdGeometry &g, float scale, int causal,
-                int qsplits, hipStream_t s) {
+                int head_parts, int qsplits, hipStream_t s) {
   const int k_blocks = static_cast<int>((sk + kW * 32 - 1) / (kW * 32));
-  const int64_t blocks = batch * kv_heads * k_blocks * (kSplit ? head_group * qsplits : 1);
+  const int64_t blocks = batch * kv_heads * k_blocks * (kSplit ? head_parts * qsplits : 1);
   if (blocks > INT32_MAX) return fail(INTENT_HIP_ERR_UNSUPPORTED, "too many workgroups");
   attention_bwd_dkdv<D, kSplit, kPart, kW><<<dim3(static_cast<unsigned>(blocks)), dim3(kW * 64), 0, s>>>(
       Q, K, V, G, lse, delta, DK, DV, partial, static_cast<int>(kv_heads), static_cast<int>(head_group),
-      static_cast<int>(sq), static_cast<int>(sk), g, scale, causal, k_blocks, qsplits);
+      static_cast<int>(sq), static_cast<int>(sk), g, scale, causal, k_blocks, head_parts, qsplits);
   if (hipPeekAtLastError() != hipSuccess)
     return launch_status(kPart == kOnlyDk ? "attention_bwd_dk" : kPart == kOnlyDv ? "attention_bwd_dv" : "attention_bwd_dkdv");
   return INTENT_HIP_OK;
 }
 
-// dK and dV of one call: split by query head and query-tile range with a workspace (qsplits > 0;
-// then folded), as two 8-wave kernels on wide grids, or as one 4-wave kernel.
+// dK and dV of one call: divided as `plan` says (with a workspace; then folded), as two 8-wave
+// kernels on wide grids, or as one 4-wave kernel.
 template <int D>
 int run_dkdv(const uint16_t *Q, const uint16_t *K, const uint16_t *V, const uint16_t *G, const float *lse,
-             const float *delta, uint16_t *DK, uint16_t *DV, float *partial, int qsplits, int64_t batch,
+             const float *delta, uint16_t *DK, uint16_t *DV, float *partial, const DkdvPlan &plan, int64_t batch,
              int64_t kv_heads, int64_t head_group, int64_t sq, int64_t sk, const BwdGeometry &g, float scale,
              int causal, hipStream_t s) {
-  if (qsplits > 0) {
-    if (int rc = launch_dkdv<D, true, kBoth, 4>(Q, K, V, G, lse, delta, DK, DV, partial, batch, kv_heads, head_group,
-                                                sq, sk, g, scale, causal, qsplits, s))
-      return rc;
-    const int64_t rows = batch * kv_heads * sk;
-    const dim3 rgrid(static_cast<unsigned>((rows * (D / 4) + kThreads - 1) / kThreads));
-    attention_bwd_dkdv_reduce<D><<<rgrid, dim3(kThreads), 0, s>>>(partial, DK, DV, static_cast<int>(kv_heads),
-                                                                  static_cast<int>(head_group * qsplits),
-                                                                  static_cast<int>(sk), rows, g, scale);
-    if (hipPeekAtLastError() != hipSuccess) return launch_status("attention_bwd_dkdv_reduce");
-    return INTENT_HIP_OK;
+  const auto launch = [&](auto run, int head_parts, int qsplits) {
+    return run(Q, K, V, G, lse, delta, DK, DV, partial, batch, kv_heads, head_group, sq, sk, g, scale, causal, head_parts,
+               qsplits, s);
+  };
+  if (plan.parts() == 0) {
+    if (!plan.wide) return launch(launch_dkdv<D, false, kBoth, 4>, 1, 1);
+    if (int rc = launch(launch_dkdv<D, false, kOnlyDk, 8>, 1, 1)) return rc;
+    return launch(launch_dkdv<D, false, kOnlyDv, 8>, 1, 1);
   }
-  if (batch * kv_heads * sk >= kWideRows) {
-    if (int rc = launch_dkdv<D, false, kOnlyDk, 8>(Q, K, V, G, lse, delta, DK, DV, nullptr, batch, kv_heads,
-                                                   head_group, sq, sk, g, scale, causal, 1, s))
-      return rc;
-    return launch_dkdv<D, false, kOnlyDv, 8>(Q, K, V, G, lse, delta, DK, DV, nullptr, batch, kv_heads, head_group, sq,
-                                             sk, g, scale, causal, 1, s);
+  if (plan.wide) {
+    if (int rc = launch(launch_dkdv<D, true, kOnlyDk, 8>, plan.head_parts, plan.qsplits)) return rc;
+    if (int rc = launch(launch_dkdv<D, true, kOnlyDv, 8>, plan.head_parts, plan.qsplits)) return rc;
+  } else {
+    if (int rc = launch(launch_dkdv<D, true, kBoth, 4>, plan.head_parts, plan.qsplits)) return rc;
   }
-  return launch_dkdv<D, false, kBoth, 4>(Q, K, V, G, lse, delta, DK, DV, nullptr, batch, kv_heads, head_group, sq, sk,
-                                         g, scale, causal, 1, s);
+  const int64_t rows = batch * kv_heads * sk;
+  const dim3 rgrid(static_cast<unsigned>((rows * (D / 4) + kThreads - 1) / kThreads));
+  attention_bwd_dkdv_reduce<D><<<rgrid, dim3(kThreads), 0, s>>>(partial, DK, DV, static_cast<int>(kv_heads), plan.parts(),
+                                                                static_cast<int>(sk), rows, g, scale);
+  if (hipPeekAtLastError() != hipSuccess) return launch_status("attention_bwd_dkdv_reduce");
+  return INTENT_HIP_OK;
 }
 
 }  // namespace
@@ -1017,7 +1043,7 @@ extern "C" int intent_hip_attention_bwd_dkdv_workspace_bytes(int64_t batch, int6
   if (bytes == nullptr) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "null output");
   if (const int rc = check_common(batch, q_heads, head_group, sq, sk, d)) return rc;
   *bytes = static_cast<size_t>(
-      dkdv_workspace(dkdv_qsplits(batch, q_heads, head_group, sq, sk), batch, q_heads, head_group, sk, d));
+      dkdv_workspace(dkdv_plan(batch, q_heads, head_group, sq, sk), batch, q_heads / head_group, sk, d));
   return INTENT_HIP_OK;
 }
 
@@ -1040,12 +1066,13 @@ extern "C" int intent_hip_attention_bwd_dkdv_ws(const void *q, const void *k, co
   BwdGeometry g{};
   load_geometry(g, strides, true);
   const int64_t kv_heads = q_heads / head_group;
-  int qsplits = dkdv_qsplits(batch, q_heads, head_group, sq, sk);
-  const int64_t need = dkdv_workspace(qsplits, batch, q_heads, head_group, sk, d);
-  if (need > 0 && workspace != nullptr && (workspace_bytes < static_cast<size_t>(need) || !aligned(workspace, 16)))
+  DkdvPlan plan = dkdv_plan(batch, q_heads, head_group, sq, sk);
+  const int64_t need = dkdv_workspace(plan, batch, kv_heads, sk, d);
+  const bool small = workspace == nullptr || workspace_bytes < static_cast<size_t>(need) || !aligned(workspace, 16);
+  if (need > 0 && workspace != nullptr && small && !plan.optional)
     return fail(INTENT_HIP_ERR_WORKSPACE, "dK/dV needs %lld 16-byte aligned workspace bytes, got %zu",
                 static_cast<long long>(need), workspace_bytes);
-  if (workspace == nullptr) qsplits = 0;
+  if (small || (plan.optional && !causal)) plan.head_parts = plan.qsplits = 0;
   const auto *Q = static_cast<const uint16_t *>(q);
   const auto *K = static_cast<const uint16_t *>(k);
   const auto *V = static_cast<const uint16_t *>(v);
@@ -1056,9 +1083,9 @@ extern "C" int intent_hip_attention_bwd_dkdv_ws(const void *q, const void *k, co
   const hipStream_t s = as_stream(stream);
   const int c = causal ? 1 : 0;
   if (d == 64)
-    return run_dkdv<64>(Q, K, V, G, lse, delta, DK, DV, P, qsplits, batch, kv_heads, head_group, sq, sk, g, scale,
+    return run_dkdv<64>(Q, K, V, G, lse, delta, DK, DV, P, plan, batch, kv_heads, head_group, sq, sk, g, scale,
                         c, s);
-  return run_dkdv<128>(Q, K, V, G, lse, delta, DK, DV, P, qsplits, batch, kv_heads, head_group, sq, sk, g, scale, c,
+  return run_dkdv<128>(Q, K, V, G, lse, delta, DK, DV, P, plan, batch, kv_heads, head_group, sq, sk, g, scale, c,
                        s);
 }
 

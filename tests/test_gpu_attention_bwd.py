@@ -173,6 +173,47 @@ def test_dkdv_split_matches_unsplit_through_the_c_abi(device, shape):
     assert small.value == 0                                     # large grids never split
 
 
+# 256 to 511 workgroups and at least 4096 queries per key head: two parts by head or, with an odd group, by query range;
+# the 4-wave kernel and (from 65536 key rows) the 8-wave ones, ragged keys and queries.
+@pytest.mark.parametrize("shape", [(64, 16, 2, 520, 256, 64), (43, 6, 2, 1400, 300, 128), (128, 4, 2, 2050, 256, 64),
+                                   (128, 2, 2, 4100, 256, 128)])
+def test_dkdv_two_parts_match_one(device, shape):
+    """With the workspace the query names, against the launch without one (which the tests above check against the oracle):
+    equal up to the association of the f32 sums, so within 2 f16 ulp plus 1e-3 of the largest magnitude.
+    Without a mask the two are the same launch; a workspace too small for the parts is left unused."""
+    import ctypes
+
+    from intent_amd.runtime.hip.library import library
+
+    batch, hq, hk, sq, sk, d = shape
+    announce("dK/dV in two parts", shape)
+    g = torch.Generator(device=device).manual_seed(sum(shape))
+    normal = lambda *dims: torch.randn(dims, generator=g, device=device)  # noqa: E731
+    q, do = normal(batch, hq, sq, d).half(), normal(batch, hq, sq, d).half()
+    k, v = normal(batch, hk, sk, d).half(), normal(batch, hk, sk, d).half()
+    lse, delta = normal(batch, hq, sq) * 0.5 + float(np.log(sk)), normal(batch, hq, sq)
+    lib = library()
+    size = ctypes.c_size_t(0)
+    assert lib.fn["attention_bwd_dkdv_workspace_bytes"](batch, hq, hq // hk, sq, sk, d, ctypes.byref(size)) == 0
+    assert size.value == 2 * 2 * batch * hk * sk * d * 4
+    workspace = torch.empty(size.value, dtype=torch.uint8, device=device)
+
+    def run(causal, bytes_):
+        dk, dv = torch.full_like(k, 7.0), torch.full_like(v, 7.0)
+        strides = (ctypes.c_int64 * 30)(*(x for a in (q, k, v, do, lse, delta, dk, dv) for x in a.stride()))
+        lib.check(lib.fn["attention_bwd_dkdv_ws"](
+            *(a.data_ptr() for a in (q, k, v, do, lse, delta, dk, dv)), batch, hq, hq // hk, sq, sk, d, strides,
+            float(np.float32(d ** -0.5)), causal, workspace.data_ptr() if bytes_ else None, bytes_,
+            torch.cuda.current_stream().cuda_stream))
+        return dk, dv
+
+    for parts, whole in zip(run(1, size.value), run(1, 0)):
+        parts, whole = parts.double(), whole.double()
+        assert bool(((parts - whole).abs() <= 2 * 2.0 ** -10 * whole.abs() + 1e-3 * whole.abs().max()).all())
+    for causal, bytes_ in ((0, size.value), (1, 256)):
+        assert all(torch.equal(a, b) for a, b in zip(run(causal, bytes_), run(causal, 0)))
+
+
 # Calls with at least 256 x 256 rows (batch x heads x sequence) take the 8-wave kernels: dQ with
 # 256-query workgroups, dK/dV as two kernels (dK, then dV) with 256-key workgroups. These shapes
 # reach that bound with short sequences so the oracle stays fast; 260 and 300 leave ragged blocks.
