@@ -24,7 +24,7 @@ from dataclasses import dataclass
 from inspect import Parameter, Signature
 from typing import Protocol, runtime_checkable
 
-from ..language.dtypes import DType, DTypeCategory
+from ..language.dtypes import DTYPES, DType, DTypeCategory
 from ..runtime.interface import ScalarParameter, ViewParameter
 
 _FLOAT8_NAMES = {"f8e4m3fn": "float8_e4m3fn", "f8e5m2": "float8_e5m2"}
@@ -55,13 +55,21 @@ def _torch_name(element: DType) -> str:
     return _FLOAT8_NAMES.get(element.name, f"float{element.bits}")
 
 
+_TORCH_DTYPES: dict = {}   # name of a language element type -> its torch dtype
+
+
 def torch_dtype(element: DType):
     """The torch dtype of an Intent element type (I.f32 -> torch.float32, I.index -> torch.int64)."""
+    known = DTYPES.get(element.name) is element
+    if known and element.name in _TORCH_DTYPES:
+        return _TORCH_DTYPES[element.name]
     import torch
 
     result = getattr(torch, _torch_name(element), None)
     if not isinstance(result, torch.dtype):
         raise TypeError(f"{element!r} has no torch element type")
+    if known:
+        _TORCH_DTYPES[element.name] = result
     return result
 
 

@@ -105,7 +105,7 @@ class JITKernel:
 
     def _artifact(self, arguments: tuple, outputs):
         local = self._provider.local
-        device = select_device(self.backend, arguments + tuple(outputs or ()), self.device)
+        device = select_device(self.backend, arguments + tuple(outputs or ()), self.device, local)
         key = local.execution_key(device)
         with self._lock:
             if self._closed:

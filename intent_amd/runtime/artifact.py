@@ -76,7 +76,7 @@ class CompiledArtifact:
 
         Keep the arguments alive while using the prepared call; prepare again when
         their shape/stride metadata change."""
-        if not isinstance(self.runtime, PreparedRuntime):
+        if not hasattr(self.runtime, "prepare_call"):   # PreparedRuntime; isinstance of a Protocol costs 5 us
             raise NotImplementedError("this runtime does not expose prepared calls")
         return self.runtime.prepare_call(arguments, outputs=outputs)
 

@@ -143,6 +143,25 @@ def tuning_policy(rows):
         _TUNING.reset(token)
 
 
+class plan_policies:
+    """workspace_policy, numerics_policy and tuning_policy at once, for the plan of one call."""
+
+    __slots__ = ("_values", "_tokens")
+
+    def __init__(self, workspace: str, numerics: str, rows):
+        self._values = (workspace, numerics, rows)
+
+    def __enter__(self):
+        workspace, numerics, rows = self._values
+        self._tokens = (_WORKSPACE.set(workspace), _NUMERICS.set(numerics), _TUNING.set(rows))
+
+    def __exit__(self, *_):
+        workspace, numerics, rows = self._tokens
+        _TUNING.reset(rows)
+        _NUMERICS.reset(numerics)
+        _WORKSPACE.reset(workspace)
+
+
 def _split_choice(family: str, split_bytes: int) -> tuple[int, tuple]:
     """The first eligible row of `family` (columns: split) and every row's assessment. split = 1
     needs a grid small enough to split (split_bytes > 0: the workspace it takes) and a workspace

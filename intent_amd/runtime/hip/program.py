@@ -9,16 +9,17 @@ current stream, asynchronously; `result()` does not synchronize.
 """
 from __future__ import annotations
 
+import functools
 import threading
 
 from ...diagnostics import CompilationStageError
 from ..artifact import CompiledArtifact
 from ..diagnostics import ConfigurationAssessment, NativeObservation, NativeResource
 from ..interface import PublicInterface, ViewParameter
-from ..invocation import bind_arguments
+from ..invocation import Binding, bind_arguments
 from ..torch_views import allocate_output, observe_view
 from .library import library
-from .operators import OperatorSpec, numerics_policy, tuning_policy, workspace_policy
+from .operators import OperatorSpec, plan_policies
 from .tuning import FAMILY_OF, SPLIT, TuningConfiguration
 
 
@@ -43,6 +44,7 @@ def _constexpr_parameters(definition) -> tuple[tuple[str, object], ...]:
     return tuple(out)
 
 
+@functools.lru_cache(maxsize=1)
 def _raw_stream_getter():
     """Fast accessor of the current HIP stream handle of a device (an int)."""
     import torch
@@ -132,6 +134,12 @@ class HipProgram:
         self.library = library()
         self._derived = {symbols[name]: (symbols[source], offset) for name, source, offset in spec.derived
                          if name in symbols and source in symbols}
+        self._binding = Binding(interface, self._derived)
+        # Pairs of views of which one or both are written, as positions in the parameter list.
+        views = [p for p in interface.parameters if isinstance(p, ViewParameter)]
+        self._written_pairs = tuple((left.position, right.position, left.writable and right.writable)
+                                    for i, left in enumerate(views) for right in views[i + 1:]
+                                    if left.writable or right.writable)
         self._last_launch = None
         self._lock = threading.Lock()
         self._closed = False
@@ -148,23 +156,21 @@ class HipProgram:
             self.interface, tuple(arguments), outputs,
             observe_view=lambda p, v: observe_view(p, v, device=device, abstract=abstract),
             allocate_output=lambda p, shape: allocate_output(p, shape, device=device, abstract=abstract),
-            abstract=abstract, derived=self._derived)
+            abstract=abstract, binding=self._binding)
 
     def _check_writable_overlap(self, bound) -> None:
         """Writable views may not overlap another view, except an exact in-place alias that the
         kernel supports (same address and strides; each element is read before it is written)."""
-        views = [(p, f) for p, f in zip(self.interface.parameters, bound.views) if isinstance(p, ViewParameter)]
-        for i, (left, lf) in enumerate(views):
-            for right, rf in views[i + 1:]:
-                if not (left.writable or right.writable):
-                    continue
-                if not (lf.begin < lf.end and rf.begin < rf.end and lf.begin < rf.end and rf.begin < lf.end):
-                    continue
-                exact = (lf.pointer == rf.pointer and lf.shape == rf.shape and lf.strides == rf.strides)
-                if exact and self.spec.inplace_safe and not (left.writable and right.writable):
-                    continue
-                raise ValueError(f"{left.name} and {right.name} overlap; the hip kernel for "
-                                 f"{self.spec.name} requires writable views that do not alias other views")
+        for i, j, both in self._written_pairs:
+            lf, rf = bound.views[i], bound.views[j]
+            if not (lf.begin < lf.end and rf.begin < rf.end and lf.begin < rf.end and rf.begin < lf.end):
+                continue
+            exact = (lf.pointer == rf.pointer and lf.shape == rf.shape and lf.strides == rf.strides)
+            if exact and self.spec.inplace_safe and not both:
+                continue
+            left, right = self.interface.parameters[i], self.interface.parameters[j]
+            raise ValueError(f"{left.name} and {right.name} overlap; the hip kernel for "
+                             f"{self.spec.name} requires writable views that do not alias other views")
 
     def prepare_call(self, arguments: tuple, *, outputs: tuple | None = None) -> HipPreparedCall:
         if self._closed:
@@ -173,7 +179,7 @@ class HipProgram:
             raise TypeError("outputs must be a tuple in declared Out order")
         bound = self._bind(arguments, outputs)
         self._check_writable_overlap(bound)
-        with workspace_policy(self.workspace), numerics_policy(self.numerics), tuning_policy(self.tuning_rows):
+        with plan_policies(self.workspace, self.numerics, self.tuning_rows):
             launch = self.spec.plan(self.library, bound, self.constexprs, self.device)
         return HipPreparedCall(self, bound, launch)
 
@@ -205,7 +211,7 @@ class HipProgram:
             self.interface, tuple(arguments), None,
             observe_view=lambda p, v: observe_view(p, v, device=device, abstract=True),
             allocate_output=lambda p, shape: allocate_output(p, shape, device=device, abstract=True),
-            abstract=True, derived=self._derived)
+            abstract=True, binding=self._binding)
         del torch
         return bound.result()
 

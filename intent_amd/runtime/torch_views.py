@@ -23,8 +23,12 @@ def byte_span(pointer: int, shape: tuple, strides: tuple, itemsize: int) -> tupl
     """[begin, end) of the bytes a strided view's elements occupy (empty views: an empty range)."""
     if 0 in shape:
         return pointer, pointer
-    below = sum((extent - 1) * stride for extent, stride in zip(shape, strides) if stride < 0)
-    above = sum((extent - 1) * stride for extent, stride in zip(shape, strides) if stride > 0)
+    below = above = 0
+    for extent, stride in zip(shape, strides):
+        if stride > 0:
+            above += (extent - 1) * stride
+        else:
+            below += (extent - 1) * stride
     return pointer + below * itemsize, pointer + (above + 1) * itemsize
 
 
@@ -47,14 +51,15 @@ def observe_view(parameter: ViewParameter, value, *, device, abstract: bool = Fa
     shape, strides = tuple(value.shape), tuple(value.stride())
     if abstract:
         return ViewFacts(shape, strides, None, None, None, None, value.dtype, None, None, None)
+    pointer = value.data_ptr()
     storage = value.untyped_storage()
     base, size = storage.data_ptr(), storage.nbytes()
     # A zero-byte storage has no meaningful address (several may report the same or a null
     # pointer), so each is identified by its own storage object, never by the pointer: two
     # distinct empty buffers are two allocations (reference runtime/torch_views.py:53).
     identity = (value.device, base) if size else (value.device, "empty", storage._cdata)
-    begin, end = byte_span(value.data_ptr(), shape, strides, value.element_size())
-    return ViewFacts(shape, strides, value.data_ptr(), base, base + size, value.storage_offset(), value.dtype,
+    begin, end = byte_span(pointer, shape, strides, value.element_size())
+    return ViewFacts(shape, strides, pointer, base, base + size, value.storage_offset(), value.dtype,
                      begin, end, identity)
 
 

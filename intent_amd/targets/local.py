@@ -52,9 +52,17 @@ def _merge(explicit: LocalDevice | None, placed: LocalDevice | None) -> LocalDev
     return explicit
 
 
-def select_device(backend: str, arguments: tuple, explicit=None) -> LocalDevice:
-    execution = provider(backend).local
-    placed = {_parse(getattr(value, "device", "cpu"), execution) for value in arguments if hasattr(value, "shape")}
+def select_device(backend: str, arguments: tuple, explicit=None, execution=None) -> LocalDevice:
+    """`execution`: the backend's LocalExecution, from a caller that holds its provider."""
+    if execution is None:
+        execution = provider(backend).local
+    placed, previous = set(), None
+    for value in arguments:
+        if hasattr(value, "shape"):
+            device = getattr(value, "device", "cpu")
+            if previous is None or device != previous:
+                placed.add(_parse(device, execution))
+                previous = device
     if len(placed) > 1:
         raise ValueError(f"the tensor arguments are on several devices: {', '.join(sorted(map(str, placed)))}")
     chosen = _merge(None if explicit is None else _parse(explicit, execution), next(iter(placed), None))
