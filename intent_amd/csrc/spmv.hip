@@ -230,7 +230,7 @@ __device__ __forceinline__ void block_prefix(const Plan &plan, int block, int mi
 __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, const int32_t *__restrict__ col,
                                            const float *__restrict__ val, const float *__restrict__ x,
                                            float *__restrict__ y, int32_t rows, int32_t cols, int64_t nnz, Plan plan,
-                                           int block) {
+                                           int block, bool fold) {
   __shared__ int s_wave[2][4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t base = static_cast<int64_t>(block) * kBlockRows;
@@ -244,7 +244,7 @@ __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, cons
     length[k] = r < rows ? e - b : -1;
   }
   // Lane rows: all column and value loads, then all gathers, then the ordered folds.
-  {
+  if (fold) {   // a constant
     int32_t c[kRowsPerThread][kLaneRow];
     float v[kRowsPerThread][kLaneRow], xs[kRowsPerThread][kLaneRow];
 #pragma unroll
@@ -311,6 +311,7 @@ __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, cons
     first[1] += s_wave[1][0] + s_wave[1][1] + s_wave[1][2] + s_wave[1][3];
     __syncthreads();
   }
+  if (!fold) return;
   // Rows of 5..127 nonzeros: group g (16 lanes) takes the g-th pending row of the wave.
   const int g = lane >> 4, l16 = lane & 15;
 #pragma unroll
@@ -342,6 +343,52 @@ __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, cons
       for (int q = 0; q < 4 && pending != 0; ++q) pending &= pending - 1;   // four rows consumed
     }
   }
+}
+
+// Short rows of a small matrix: one 16-lane group per row, 16 rows per workgroup. rows_block folds 1024 rows per
+// workgroup, which leaves most of the chip idle below some 10^5 rows, each wave walking up to 256 rows in steps
+// of four, a chain of loads each (19413 rows of up to 78: 29.7 us, 16.3 this way; 262100 of up to 100: 53.6,
+// 38.0; from 2^18 rows on the larger workgroups lead, their loads being enough to fill the chip). Up to 4 nonzeros: the group's
+// first lanes take one product each, added in order by all of them; 5 to 127 as in rows_block.
+constexpr int kSmallGroups = 256 / kGroup;
+constexpr int64_t kSmallRows = int64_t{1} << 18;
+__device__ __forceinline__ void rows_small(const int32_t *__restrict__ off, const int32_t *__restrict__ col,
+                                           const float *__restrict__ val, const float *__restrict__ x,
+                                           float *__restrict__ y, int32_t rows, int32_t cols, int64_t nnz, int block) {
+  const int l16 = threadIdx.x & (kGroup - 1);
+  const int64_t r = static_cast<int64_t>(block) * kSmallGroups + threadIdx.x / kGroup;
+  int32_t b = 0, e = 0;
+  if (r < rows) row_span(off, r, nnz, b, e);
+  const int length = r < rows ? e - b : kGroupRow;   // a group past the end stores nothing, like a long row's
+  constexpr int kPer = kGroupRow / kGroup;
+  int32_t c[kPer];
+  float v[kPer], xs[kPer];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int32_t p = b + l16 + kGroup * q;
+    const bool ok = length < kGroupRow && p < e;
+    c[q] = ok ? col[p] : 0;
+    v[q] = ok ? val[p] : 0.0f;
+  }
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) xs[q] = length < kGroupRow && b + l16 + kGroup * q < e ? x[clamp_col(c[q], cols)] : 0.0f;
+  float acc = 0.0f;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q)
+    if (b + l16 + kGroup * q < e) acc = fmaf(v[q], xs[q], acc);
+  acc = group16_sum(acc);
+  float ordered = 0.0f;
+  {
+    // Each product is rounded before its add (hipcc would otherwise fuse the two).
+#pragma clang fp contract(off)
+    const float product = v[0] * xs[0];
+#pragma unroll
+    for (int j = 0; j < kLaneRow; ++j) {
+      const float term = __shfl(product, j, kGroup);
+      if (j < length) ordered = ordered + term;
+    }
+  }
+  if (l16 == 0 && length < kGroupRow) y[r] = length <= kLaneRow ? ordered : acc;
 }
 
 // Cuts of one row by a group of G lanes (gl: lane in the group, gbase: its first lane). Cut k
@@ -418,11 +465,13 @@ __device__ __forceinline__ void cut_row(const int32_t *__restrict__ col, int32_t
 // classified again (as spmv_count did) and ranked in row order, which gives each its list position
 // from the block's list offset (block_prefix), the position spmv_rows writes the row id at. Medium
 // rows go eight at a time, one 8-lane group per row (9 cuts: the starts of windows 0..8); large
-// rows one at a time, the whole wave (slices + 1 cuts). `list` is the wave's LDS scratch for the block's rows.
+// rows one at a time, the whole wave (slices + 1 cuts). Wave `share` of a block's `shares` takes every
+// shares-th of these steps. `list` is the wave's LDS scratch for the block's rows.
 constexpr int kMidGroup = 8;
 __device__ __forceinline__ void cut_block(const int32_t *__restrict__ off, const int32_t *__restrict__ col,
                                           int32_t rows, int32_t cols, int64_t nnz, const Plan &plan, int block,
-                                          int lane, int32_t *list, int first_mid, int first_big) {
+                                          int lane, int32_t *list, int first_mid, int first_big, int share,
+                                          int shares) {
   const int64_t base = static_cast<int64_t>(block) * kBlockRows;
   // Medium rows at list[0 ..), large rows at list[kBlockRows - 1] downwards, in row order. The
   // offsets are read 256 rows (4 per lane) at a time, all loads of a batch issued together (rows
@@ -455,7 +504,7 @@ __device__ __forceinline__ void cut_block(const int32_t *__restrict__ off, const
 
   const int64_t window = (static_cast<int64_t>(cols) + kWindows - 1) / kWindows;
   const int g = lane / kMidGroup;
-  for (int q = 0; q < n_mid; q += 64 / kMidGroup) {   // wave-uniform
+  for (int q = share * (64 / kMidGroup); q < n_mid; q += shares * (64 / kMidGroup)) {   // wave-uniform
     const int i = q + g;
     const int at = first_mid + i;
     const bool ok = i < n_mid && at < plan.cap_mid;
@@ -465,7 +514,7 @@ __device__ __forceinline__ void cut_block(const int32_t *__restrict__ off, const
                        lane % kMidGroup, g * kMidGroup, plan.mid_cuts + static_cast<int64_t>(ok ? at : 0) * (kWindows + 1));
   }
   const int big_cuts = plan.slices + 1;
-  for (int i = 0; i < n_big; ++i) {   // wave-uniform
+  for (int i = share; i < n_big; i += shares) {   // wave-uniform
     const int at = first_big + i;
     if (at >= plan.cap_big) break;
     int32_t b, e;
@@ -477,27 +526,34 @@ __device__ __forceinline__ void cut_block(const int32_t *__restrict__ off, const
 
 // Short rows, row lists and cuts in one launch. The first cut_groups workgroups compute the cuts
 // (one wave per 1024-row block), the rest fold the short rows and write the lists (one workgroup
-// per block). The cuts are chains of dependent probes, the short rows are bound by the fabric's
+// per block; small matrices fold in the workgroups of rows_small). The cuts are chains of dependent probes, the short rows are bound by the fabric's
 // random line fetches; in one grid the cut chains run beside the short rows instead of after them
 // (config 5: 165 us for both, against 140 + 52 us as two launches).
+template <bool kSmall>   // up to kSmallRows rows: small_groups > 0, several cutting waves per block
 __global__ __launch_bounds__(256) void spmv_rows(const int32_t *__restrict__ off, const int32_t *__restrict__ col,
                                                     const float *__restrict__ val, const float *__restrict__ x,
                                                     float *__restrict__ y, int32_t rows, int32_t cols, int64_t nnz,
-                                                    Plan plan, int cut_groups) {
+                                                    Plan plan, int cut_groups, int shares, int small_groups) {
+  const int cut_shares = kSmall ? shares : 1;
   __shared__ int32_t s_list[4][kBlockRows];
   if (static_cast<int>(blockIdx.x) < cut_groups) {   // workgroup-uniform
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int block = static_cast<int>(blockIdx.x) * 4 + wave;   // the four blocks of one superblock
+    // One wave per block (the four blocks of one superblock), or four of a block's cut_shares (4 or more) waves.
+    const int at = static_cast<int>(blockIdx.x) * 4 + wave;
+    const int block = at / cut_shares;
     __shared__ int s_pre[2][4];
     int mid_super, big_super, first_mid, first_big;
-    superblock_prefix(plan, static_cast<int>(blockIdx.x), mid_super, big_super, s_pre);
+    superblock_prefix(plan, static_cast<int>(blockIdx.x) * 4 / cut_shares / kSuperBlocks, mid_super, big_super, s_pre);
     if (block < plan.blocks) {   // wave-uniform; the last group may hold fewer than four blocks
       block_prefix(plan, block, mid_super, big_super, first_mid, first_big);
-      cut_block(off, col, rows, cols, nnz, plan, block, lane, s_list[wave], first_mid, first_big);
+      cut_block(off, col, rows, cols, nnz, plan, block, lane, s_list[wave], first_mid, first_big,
+                at % cut_shares, cut_shares);
     }
     return;
   }
-  rows_block(off, col, val, x, y, rows, cols, nnz, plan, static_cast<int>(blockIdx.x) - cut_groups);
+  const int block = static_cast<int>(blockIdx.x) - cut_groups;
+  if (kSmall && block < small_groups) rows_small(off, col, val, x, y, rows, cols, nnz, block);
+  else rows_block(off, col, val, x, y, rows, cols, nnz, plan, block - (kSmall ? small_groups : 0), !kSmall);
 }
 
 // Pieces of listed rows. Wave w of a workgroup takes the pieces of list rows i = k + K t for
@@ -803,25 +859,37 @@ extern "C" int intent_hip_csr_spmv_f32(const int32_t *row_offsets, const int32_t
   const Plan plan = carve(workspace, rows, cols, nnz);
   const hipStream_t s = as_stream(stream);
   const int32_t r32 = static_cast<int32_t>(rows), c32 = static_cast<int32_t>(cols > 0 ? cols : 1);
-  spmv_count<<<dim3(static_cast<unsigned>(plan.supers)), dim3(256 * kSuperBlocks), 0, s>>>(row_offsets, r32, nnz,
-                                                                                          plan);
-  // No row can be medium or large: no cut workgroups.
-  const int cut_groups = plan.cap_mid == 0 && plan.cap_big == 0 ? 0 : (plan.blocks + 3) / 4;
-  spmv_rows<<<dim3(static_cast<unsigned>(plan.blocks + cut_groups)), dim3(256), 0, s>>>(
-      row_offsets, column_indices, values, x, y, r32, c32, nnz, plan, cut_groups);
+  // No row can be medium or large: no cut workgroups. No length lies between the classes: no medium rows.
+  const bool listed = plan.cap_mid > 0 || plan.cap_big > 0, medium = plan.cap_mid > 0 && plan.big > kGroupRow;
+  // Waves per block that cut its listed rows: one walks them all beside the short rows of a large matrix (4.2M rows 337
+  // us, 352 with four waves); with few blocks that walk is what the launch waits for (27674 rows 54.7 us, 22.2
+  // with 16; 100000 rows 80.7, 27.4; 250000 rows 83.6, 50.4 with four and 56.8 with 16).
+  static_assert(kSmallRows == 256 * kBlockRows, "large matrices cut with one wave per block");
+  const int cut_shares = plan.blocks <= 128 ? 16 : plan.blocks <= 256 ? 4 : 1;
+  const int cut_groups = listed ? (plan.blocks * cut_shares + 3) / 4 : 0;
+  const int small_groups = rows <= kSmallRows ? static_cast<int>((rows + kSmallGroups - 1) / kSmallGroups) : 0;
+  const int list_blocks = small_groups > 0 && !listed ? 0 : plan.blocks;
+  if (list_blocks > 0)
+    spmv_count<<<dim3(static_cast<unsigned>(plan.supers)), dim3(256 * kSuperBlocks), 0, s>>>(row_offsets, r32, nnz, plan);
+  const auto rows_kernel = small_groups > 0 ? &spmv_rows<true> : &spmv_rows<false>;
+  rows_kernel<<<dim3(static_cast<unsigned>(list_blocks + cut_groups + small_groups)), dim3(256), 0, s>>>(
+      row_offsets, column_indices, values, x, y, r32, c32, nnz, plan, cut_groups, cut_shares, small_groups);
   if (hipPeekAtLastError() != hipSuccess) return launch_status("spmv_rows");
-  if (plan.cap_mid == 0 && plan.cap_big == 0) return INTENT_HIP_OK;   // no row can be medium or large
-  if (plan.cap_mid > 0)
-    spmv_windows<<<dim3(kWindows * kWindowTiles), dim3(kSliceThreads), 0, s>>>(
+  if (!listed) return INTENT_HIP_OK;
+  if (medium) {   // at least 16 rows for the waves of a workgroup
+    const int tiles = static_cast<int>(std::min<int64_t>(kWindowTiles, (plan.cap_mid + kSliceWaves - 1) / kSliceWaves));
+    spmv_windows<<<dim3(kWindows * tiles), dim3(kSliceThreads), 0, s>>>(
         column_indices, values, x, c32, plan.mid_cuts, kWindows + 1, plan.mid_parts, kWindows, plan.counters + 0,
         plan.cap_mid);
+  }
   if (plan.cap_big > 0) {
-    const int K = static_cast<int>((kSliceTiles + plan.slices - 1) / plan.slices);
+    const int K = static_cast<int>(std::min<int64_t>((kSliceTiles + plan.slices - 1) / plan.slices,
+                                                     (plan.cap_big + kSliceWaves - 1) / kSliceWaves));
     spmv_slices<<<dim3(static_cast<unsigned>(plan.slices) * static_cast<unsigned>(K)), dim3(kSliceThreads), 0,
                   s>>>(column_indices, values, x, c32, plan.big_cuts, plan.slices + 1, plan.big_parts,
                        plan.slices, plan.counters + 1, plan.cap_big);
   }
-  const int mid_groups = static_cast<int>(std::min<int64_t>((plan.cap_mid + 255) / 256, 128)) + 1;
+  const int mid_groups = medium ? static_cast<int>(std::min<int64_t>((plan.cap_mid + 255) / 256, 128)) + 1 : 0;
   const int big_groups = static_cast<int>(std::min<int64_t>((plan.cap_big + 3) / 4, 512)) + 1;
   spmv_combine<<<dim3(static_cast<unsigned>(mid_groups + big_groups)), dim3(256), 0, s>>>(y, plan, mid_groups);
   if (hipPeekAtLastError() != hipSuccess) return launch_status("spmv_combine");

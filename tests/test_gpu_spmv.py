@@ -265,3 +265,56 @@ def test_static_workspace_option(device):
     with pytest.raises(intent.CompilationStageError) as error:
         static.prepare(*huge)
     assert error.value.stage == "provider_preparation"
+
+
+def test_small_matrices_fold_as_large_ones_do(device):
+    """Matrices of up to 2^18 rows fold their short rows in 16-lane groups, larger ones in 1024-row blocks: the same
+    products in the same order, so appending a row to a matrix of 2^18 leaves every other result bit-identical.
+    Lengths cover 0 to 4 (the ordered fold), 5 to 127, 128 to 300 (listed rows), NaN and inf among the
+    values of short rows."""
+    announce("spmv small / large fold")
+    rows, cols = 1 << 18, 5000
+    rng = np.random.default_rng(9)
+    lengths = rng.integers(0, 7, rows)
+    lengths[rng.integers(0, rows, 6000)] = rng.integers(5, 128, 6000)
+    lengths[rng.integers(0, rows, 200)] = rng.integers(128, 301, 200)
+    lengths[-1] = 127
+    offsets, columns = inputs.csr_matrix(rng, lengths, cols)
+    values = inputs.uniform(rng, int(offsets[-1]), -1, 1)
+    values[rng.integers(0, values.size, 50)] = np.inf
+    values[rng.integers(0, values.size, 50)] = np.nan
+    vec = inputs.uniform(rng, cols, -1, 1)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    kernel = intent.jit(csr_spmv, backend="hip")
+    small = kernel.run(t(offsets), t(columns), t(values), t(vec)).cpu().numpy()
+    more = np.concatenate([offsets, offsets[-1:]])
+    large = kernel.run(t(more.astype(np.int32)), t(columns), t(values), t(vec)).cpu().numpy()
+    assert large[-1] == 0.0
+    assert (small.view(np.uint32) == large[:-1].view(np.uint32)).all()
+    ordered = oracle.csr_spmv(offsets, columns, values, vec)
+    short = lengths <= 4
+    assert np.array_equal(small[short], ordered[short], equal_nan=True)
+
+
+@pytest.mark.parametrize("rows,cols", [(3000, 30000), (3000, 1200000), (131072, 40000), (131073, 1200000),
+                                       (200000, 1200000), (262145, 1200000)])
+def test_listed_rows_of_small_matrices(device, rows, cols):
+    """Medium and large rows, many to a 1024-row block, with 16, 4 and 1 waves cutting a block's rows and with and without
+    a class of medium rows (none up to 4 slices of x): within the bound of a float64 sum, and exact with
+    small integers."""
+    announce("spmv listed rows", rows, cols)
+    rng = np.random.default_rng(rows + cols)
+    lengths = np.zeros(rows, np.int64)
+    crowd = np.concatenate([np.arange(0, 700), np.arange(rows - 40, rows), rng.integers(0, rows, 300)])
+    lengths[crowd] = rng.integers(100, 1500, crowd.size)
+    offsets, columns = inputs.csr_matrix(rng, lengths, cols)
+    for values, vec in ((inputs.uniform(rng, int(offsets[-1]), -1, 1), inputs.uniform(rng, cols, -1, 1)),
+                        (rng.integers(-3, 4, int(offsets[-1])).astype(np.float32),
+                         rng.integers(-3, 4, cols).astype(np.float32))):
+        products = values.astype(np.float64) * vec[columns]
+        row_of = np.repeat(np.arange(rows), lengths)
+        want = np.bincount(row_of, products, rows)
+        bound = 1e-5 * np.bincount(row_of, np.abs(products), rows)
+        got = run(device, offsets, columns, values, vec)
+        assert (np.abs(got - want) <= bound).all()
+    assert (got == want).all()
