@@ -39,8 +39,10 @@ namespace {
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
-constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
+constexpr int kWaves = 4;             // waves of a workgroup of the partials kernel
+// Waves of a workgroup where few paged jobs leave the chip idle and each walks many chunks (head groups beyond 4 hold
+// more registers and LDS per wave).
+constexpr int many_waves(int group) { return group <= 4 ? 16 : 8; }
 constexpr int kChunk = 64;            // tokens per wave step
 constexpr int kMaxGroup = 16;          // query heads per key head
 constexpr float kLog2e = 1.4426950408889634f;
@@ -110,8 +112,8 @@ __device__ __forceinline__ float lane_xor(float v, int m) {
 
 // kG bounds the query heads per key head (the group runs 1..kG; register arrays are sized by kG
 // and every loop over them is unrolled with a uniform guard, so nothing is indexed dynamically).
-template <typename E, int D, int kG, int kSrc, int kOut>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kG <= 4 ? 4 : 2))) void decode_partials(
+template <typename E, int D, int kG, int kSrc, int kOut, int W>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(kG <= 4 ? 4 : 2))) void decode_partials(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ KC, const uint16_t *__restrict__ VC, int kv_heads,
     int group, int splits, DecodeSource src, DecodeTarget dst, DecodeGeometry g, float scale) {
   typedef E e8_t __attribute__((ext_vector_type(8)));
@@ -120,15 +122,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kG <= 
   constexpr int kSlots = kChunk / kTokensPerLoad;   // loads per lane for a whole chunk
   constexpr int kBatch = kG >= 16 ? kSlots / 4 : kSlots / 2;
   __shared__ __attribute__((aligned(16))) uint16_t q_s[kG * D];
-  __shared__ float p_s[kWaves][kG][kChunk];
-  __shared__ int64_t row_s[kWaves][kChunk];   // per token: physical row offset (elements) in the caches
-  __shared__ float m_s[kWaves][kG], den_s[kWaves][kG];
-  __shared__ float acc_s[kWaves][kG][D];
-  __shared__ int valid_s[kWaves];
+  __shared__ float p_s[W][kG][kChunk];
+  __shared__ int64_t row_s[W][kChunk];   // per token: physical row offset (elements) in the caches
+  __shared__ float m_s[W][kG], den_s[W][kG];
+  __shared__ float acc_s[W][kG][D];
+  __shared__ int valid_s[W];
   // Groups of up to four query heads score with coalesced K loads (kLanesPerToken lanes per token
   // row, 16 bytes each) and fold the lanes' partial dot products by a reduce-scatter in registers.
   constexpr bool kCoalesced = kG <= 4;
-  __shared__ int64_t key_s[kWaves][kCoalesced ? kChunk : 1];   // per token: K row offset, -1 if inactive
+  __shared__ int64_t key_s[W][kCoalesced ? kChunk : 1];   // per token: K row offset, -1 if inactive
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kG <= 
   }
   const float c1 = scale * kLog2e;
 
-  for (int i = tid; i < group * D; i += kThreads) {
+  for (int i = tid; i < group * D; i += W * 64) {
     const int gq = i / D, c = i % D;
     q_s[i] = Q[b * g.q[0] + (kh * group + gq) * g.q[1] + c];
   }
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kG <= 
       qr[gq] = gq < group ? *reinterpret_cast<const uint4 *>(q_s + gq * D + dim0) : make_uint4(0, 0, 0, 0);
   }
 
-  for (int c0 = wave * kChunk; c0 < tokens; c0 += kWaves * kChunk) {
+  for (int c0 = wave * kChunk; c0 < tokens; c0 += W * kChunk) {
     // Addresses: lane t <-> token c0 + t (its K row offset, and its V row offset for P @ V).
     const int flat = c0 + lane;
     bool active = false;
@@ -385,17 +387,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kG <= 
     }
   }
   __syncthreads();
-  for (int i = tid; i < group * D; i += kThreads) {
+  for (int i = tid; i < group * D; i += W * 64) {
     const int gq = i / D, c = i % D;
     float top = -INFINITY;
     bool any = false;
-    for (int w = 0; w < kWaves; ++w)
+    for (int w = 0; w < W; ++w)
       if (valid_s[w]) {
         any = true;
         top = fmaxf(top, m_s[w][gq]);
       }
     float total = 0.0f, value = 0.0f;
-    for (int w = 0; w < kWaves; ++w)
+    for (int w = 0; w < W; ++w)
       if (valid_s[w]) {
         const float f = __builtin_amdgcn_exp2f(m_s[w][gq] - top);
         total = fmaf(f, den_s[w][gq], total);
@@ -507,10 +509,15 @@ __global__ __launch_bounds__(64) void decode_merge(const float *__restrict__ sta
 }  // namespace
 
 template <typename E, int D, int kSrc, int kOut>
-const void *partials_kernel(int64_t group) {
-  if (group <= 4) return reinterpret_cast<const void *>(&decode_partials<E, D, 4, kSrc, kOut>);
-  if (group <= 8) return reinterpret_cast<const void *>(&decode_partials<E, D, 8, kSrc, kOut>);
-  return reinterpret_cast<const void *>(&decode_partials<E, D, 16, kSrc, kOut>);
+const void *partials_kernel(int64_t group, bool many) {
+  if constexpr (kSrc == kPaged) {
+    if (many && group <= 4) return reinterpret_cast<const void *>(&decode_partials<E, D, 4, kSrc, kOut, many_waves(4)>);
+    if (many && group <= 8) return reinterpret_cast<const void *>(&decode_partials<E, D, 8, kSrc, kOut, many_waves(8)>);
+    if (many) return reinterpret_cast<const void *>(&decode_partials<E, D, 16, kSrc, kOut, many_waves(16)>);
+  }
+  if (group <= 4) return reinterpret_cast<const void *>(&decode_partials<E, D, 4, kSrc, kOut, kWaves>);
+  if (group <= 8) return reinterpret_cast<const void *>(&decode_partials<E, D, 8, kSrc, kOut, kWaves>);
+  return reinterpret_cast<const void *>(&decode_partials<E, D, 16, kSrc, kOut, kWaves>);
 }
 
 // The instantiation serving one definition: paged (f16 partials in f32), dense bf16 partials
@@ -518,7 +525,7 @@ const void *partials_kernel(int64_t group) {
 // (varlen_gqa_decode_with_sink_logits), the last two into split states.
 enum DecodeVariant { kVariantPaged = 0, kVariantGroupedBf16 = 1, kVariantContinuous = 2, kVariantPackedSink = 3 };
 
-const void *variant_kernel(int variant, int64_t d, int64_t group, char *name, size_t size) {
+const void *variant_kernel(int variant, int64_t d, int64_t group, bool many, char *name, size_t size) {
   static const char *const names[] = {"paged_decode_partials", "decode_partials<bf16,dense>",
                                       "decode_partials<f16,dense,state>", "decode_partials<f16,packed,state>"};
   const int g = group <= 4 ? 4 : group <= 8 ? 8 : 16;
@@ -526,17 +533,17 @@ const void *variant_kernel(int variant, int64_t d, int64_t group, char *name, si
   const bool wide = d == 128;
   switch (variant) {
     case kVariantGroupedBf16:
-      return wide ? partials_kernel<__bf16, 128, kDense, kOutElem>(group)
-                  : partials_kernel<__bf16, 64, kDense, kOutElem>(group);
+      return wide ? partials_kernel<__bf16, 128, kDense, kOutElem>(group, many)
+                  : partials_kernel<__bf16, 64, kDense, kOutElem>(group, many);
     case kVariantContinuous:
-      return wide ? partials_kernel<_Float16, 128, kDense, kOutState>(group)
-                  : partials_kernel<_Float16, 64, kDense, kOutState>(group);
+      return wide ? partials_kernel<_Float16, 128, kDense, kOutState>(group, many)
+                  : partials_kernel<_Float16, 64, kDense, kOutState>(group, many);
     case kVariantPackedSink:
-      return wide ? partials_kernel<_Float16, 128, kPacked, kOutState>(group)
-                  : partials_kernel<_Float16, 64, kPacked, kOutState>(group);
+      return wide ? partials_kernel<_Float16, 128, kPacked, kOutState>(group, many)
+                  : partials_kernel<_Float16, 64, kPacked, kOutState>(group, many);
     default:
-      return wide ? partials_kernel<_Float16, 128, kPaged, kOutF32>(group)
-                  : partials_kernel<_Float16, 64, kPaged, kOutF32>(group);
+      return wide ? partials_kernel<_Float16, 128, kPaged, kOutF32>(group, many)
+                  : partials_kernel<_Float16, 64, kPaged, kOutF32>(group, many);
   }
 }
 
@@ -553,8 +560,8 @@ int decode_resources(int64_t which, int64_t d, int64_t group, IntentHipKernelRes
   if (d != 64 && d != 128) return fail(INTENT_HIP_ERR_UNSUPPORTED, "decode kernels take D = 64 or 128");
   char name[64];
   const int variant = which == 0 ? kVariantPaged : static_cast<int>(which) - 1;
-  const void *kernel = variant_kernel(variant, d, group, name, sizeof name);
-  return describe_kernel(kernel, name, kThreads, out);
+  const void *kernel = variant_kernel(variant, d, group, false, name, sizeof name);
+  return describe_kernel(kernel, name, kWaves * 64, out);
 }
 
 // Splits of a dense or packed decode: enough (batch, key head, split) workgroups to fill the chip
@@ -582,15 +589,16 @@ StateLayout state_layout(int64_t rows_heads, int64_t splits, int64_t dv) {
 
 int launch_partials(int variant, int64_t d, const uint16_t *Q, const uint16_t *K, const uint16_t *V, int64_t kv_heads,
                     int64_t group, int64_t splits, int64_t blocks, const DecodeSource &src, const DecodeTarget &dst,
-                    const DecodeGeometry &g, float scale, void *stream) {
+                    const DecodeGeometry &g, float scale, void *stream, bool many = false) {
   char name[64];
-  const void *kernel = variant_kernel(variant, d, group, name, sizeof name);
+  const void *kernel = variant_kernel(variant, d, group, many, name, sizeof name);
+  const int waves = many ? many_waves(static_cast<int>(group)) : kWaves;
   int kv = static_cast<int>(kv_heads), grp = static_cast<int>(group), spl = static_cast<int>(splits);
   DecodeSource s = src;
   DecodeTarget t = dst;
   DecodeGeometry geometry = g;
   void *args[] = {&Q, &K, &V, &kv, &grp, &spl, &s, &t, &geometry, &scale};
-  const hipError_t rc = hipLaunchKernel(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), args, 0,
+  const hipError_t rc = hipLaunchKernel(kernel, dim3(static_cast<unsigned>(blocks)), dim3(waves * 64), args, 0,
                                         as_stream(stream));
   if (rc != hipSuccess) return launch_status(name);
   return INTENT_HIP_OK;
@@ -659,7 +667,10 @@ extern "C" int intent_hip_paged_decode_partials(const void *q, const void *key_c
   DecodeTarget dst{};
   dst.lse = partial_lse;
   dst.out = partial_output;
-  return launch_partials(kVariantPaged, d, Q, K, V, kv_heads, head_group, splits, blocks, src, dst, g, scale, stream);
+  // Up to one workgroup per CU, and more than one chunk per wave of a job on average: more waves share the job's chunks
+  // (B8 HQ32 HK8 D128, 8191 tokens in 4 splits 103 -> 54 us; B4 HQ8 HK2 D64, 3783 tokens unsplit 120 -> 45).
+  const bool many = blocks <= 256 && positions * ps > kWaves * kChunk * batch * splits;
+  return launch_partials(kVariantPaged, d, Q, K, V, kv_heads, head_group, splits, blocks, src, dst, g, scale, stream, many);
 }
 
 extern "C" int intent_hip_splitk_reduce_f32_to_f16(const float *partial, const float *lse, void *out, int64_t batch,

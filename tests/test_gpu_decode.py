@@ -91,6 +91,16 @@ CASES = {
                              lengths=(513, 64, 1), splits=3, shuffle=True),
     "group4_d128_one_split": dict(kind="uniform", batch=1, query_heads=8, kv_heads=2, dim=128, page_size=64,
                                   lengths=(4097,), splits=1, shuffle=True),
+    # few jobs of many chunks each (16 and 8 waves per job): whole and partial chunks for every wave, fewer chunks
+    # than waves, one job with no live token
+    "many_waves_group4": dict(kind="uniform", batch=2, query_heads=8, kv_heads=2, dim=128, page_size=64,
+                              lengths=(2100, 1), splits=1, shuffle=True),
+    "many_waves_group3_d64": dict(kind="uniform", batch=3, query_heads=6, kv_heads=2, dim=64, page_size=16,
+                                  lengths=(1030, 300, 513), splits=2, shuffle=True),
+    "many_waves_group8": dict(kind="uniform", batch=2, query_heads=16, kv_heads=2, dim=128, page_size=64,
+                              lengths=(1500, 577), splits=2, shuffle=True, layout="exact"),
+    "many_waves_group16_d128": dict(kind="uniform", batch=1, query_heads=32, kv_heads=2, dim=128, page_size=32,
+                                    lengths=(999,), splits=1, shuffle=True),
     "ragged_empty": dict(kind="ragged", batch=3, query_heads=6, kv_heads=2, dim=64, ps=16,
                          lengths=(0, 37, 300), splits=4, pages_per_sequence=20, page_size=16),
     "logical_page_larger": dict(kind="ragged", batch=2, query_heads=4, kv_heads=1, dim=128, ps=16,
