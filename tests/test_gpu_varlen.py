@@ -130,3 +130,21 @@ def test_varlen_other_head_dims(device):
     scale = float(np.float32(48 ** -0.5))
     o = run_gqa(device, q, k, v, lengths, scale, 2)
     assert_16bit(o, oracle.attention_varlen_fwd(q, k, v, offsets(lengths), scale, True, head_group=2))
+
+
+# 64 sequences are the most that one wave lists with the longest walks first; the heads of 16 and 24 run one eighth per
+# XCD, those of 6 in order; empty sequences first, last and between.
+@pytest.mark.parametrize("sequences", [1, 2, 63, 64, 65])
+@pytest.mark.parametrize("heads,group", [(16, 4), (24, 1), (6, 3)])
+def test_varlen_item_order(device, sequences, heads, group):
+    announce("varlen item order", sequences, heads, group)
+    g = np.random.default_rng(sequences * heads + group)
+    lengths = [int(n) for n in g.integers(0, 60, sequences)]
+    lengths[sequences // 2] = 600
+    if sequences > 2:
+        lengths[0], lengths[-1], lengths[1] = 0, 0, 257
+    total = sum(lengths)
+    q = inputs.normal(g, (total, heads, 64), "f16")
+    k, v = (inputs.normal(g, (total, heads // group, 64), "f16") for _ in range(2))
+    o = run_gqa(device, q, k, v, lengths, 0.125, group)
+    assert_16bit(o, oracle.attention_varlen_fwd(q, k, v, offsets(lengths), 0.125, True, head_group=group))
