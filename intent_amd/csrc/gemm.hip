@@ -514,7 +514,7 @@ __global__ __launch_bounds__(256) void gemm_splits(const float *__restrict__ par
 }
 
 // ---------------------------------------------------------------- small tiles
-// Workgroups of four waves (2 x 2, each a BM / 2 x BN / 2 quarter in 32 x 32 MFMA tiles) for products of too few
+// Workgroups of 2 x WN waves (each BM / 2 x BN / WN in 32 x 32 MFMA tiles) for products of too few
 // 256 x 256 tiles. One barrier per K step; S stages of LDS, written by DMA, the next S - 1 steps in flight. A CU
 // gets its operands at 20 to 50 GB/s when they come from HBM or the MALL, so such products are bound by the
 // bytes of the busiest CU and the latency of its K steps, and the tiles are chosen to reach every CU.
@@ -522,12 +522,13 @@ __global__ __launch_bounds__(256) void gemm_splits(const float *__restrict__ par
 // not 16-byte aligned or whose extents or strides are not multiples of 8: the same tiles through registers (two
 // steps ahead), with 16-byte loads at 2-byte boundaries, single elements only where a chunk reaches past K
 // or N, and single-element stores (bf16 2048 x 2049 x 2047: 97 us; 1222 in f32 FMAs).
-template <int BM, int BN, int BK, int S>
+template <int BM, int BN, int BK, int S, int WN>
 struct SmallTile {
+  static constexpr int kThreads = 128 * WN;                       // 2 x WN waves
   static constexpr int kRowChunks = BK / 8;                       // 16-byte chunks of an A row
   static constexpr int kChunksA = BM * kRowChunks, kChunksB = BK * BN / 8;
   static constexpr int kStage = kChunksA + kChunksB;              // chunks of one stage
-  static constexpr int kLoadsA = kChunksA / 256, kLoadsB = kChunksB / 256;   // per thread and stage
+  static constexpr int kLoadsA = kChunksA / kThreads, kLoadsB = kChunksB / kThreads;   // per thread and stage
   // Chunk c of A row r is stored at c ^ swz_a(r): 16 consecutive rows' fragment reads hit every bank once.
   static __device__ __forceinline__ int swz_a(int r) {
     if constexpr (BK == 64) return (r & 7) ^ ((r >> 3) & 1);
@@ -554,17 +555,17 @@ __device__ __forceinline__ uint4 load_8(const uint16_t *p, int count) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma>
-__global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, Epi ep,
+template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma, int WN>
+__global__ __launch_bounds__(128 * WN) void gemm_small(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, Epi ep,
                                                   int M, int N, int K, int64_t lda, int64_t ldb, int tiles_m,
                                                   int tiles_n, float *__restrict__ partials) {
-  typedef SmallTile<BM, BN, BK, S> T;
+  typedef SmallTile<BM, BN, BK, S, WN> T;
   typedef typename Elem<E>::x8 x8;
-  constexpr int MT = BM / 64, NT = BN / 64, KT = BK / 16;
+  constexpr int MT = BM / 64, NT = BN / (32 * WN), KT = BK / 16, TH = T::kThreads;
   __shared__ uint4 lds[S * T::kStage];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WN, wn = wave % WN;
   const int tile = xcd_tile(tiles_m * tiles_n);   // the row blocks of one column block are neighbours
   if (tile < 0) return;
   const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
@@ -576,13 +577,13 @@ __global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A
   int a_k[T::kLoadsA], b_k[T::kLoadsB], b_n[T::kLoadsB];
 #pragma unroll
   for (int i = 0; i < T::kLoadsA; ++i) {
-    const int p = tid + 256 * i, r = p / T::kRowChunks;
+    const int p = tid + TH * i, r = p / T::kRowChunks;
     a_k[i] = ((p % T::kRowChunks) ^ T::swz_a(r)) * 8;
     a_src[i] = A + static_cast<int64_t>(min(m0 + r, M - 1)) * lda + a_k[i];
   }
 #pragma unroll
   for (int i = 0; i < T::kLoadsB; ++i) {
-    const int p = tid + 256 * i, n = ((p % (BN / 8)) ^ T::swz_b(p / (BN / 8))) * 8;
+    const int p = tid + TH * i, n = ((p % (BN / 8)) ^ T::swz_b(p / (BN / 8))) * 8;
     b_k[i] = p / (BN / 8);
     b_n[i] = n0 + n < N ? n0 + n : 0;
     b_src[i] = B + static_cast<int64_t>(b_k[i]) * ldb + b_n[i];
@@ -615,7 +616,7 @@ __global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A
         i16x4_t parts[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const int k = kk * 16 + t_k + 4 * h, n = wn * (BN / 2) + t * 32 + t_n;
+          const int k = kk * 16 + t_k + 4 * h, n = wn * (BN / WN) + t * 32 + t_n;
           parts[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
               (lds_i16x4_t *)(sb + k * BN + ((n >> 3) ^ T::swz_b(k)) * 8 + (n & 7)));
         }
@@ -646,13 +647,13 @@ __global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A
       for (int i = 0; i < T::kLoadsA; ++i) {
         const uint16_t *src = a_src[i] + k0;
         if (tail && k0 + a_k[i] >= K) src = zero;
-        __builtin_amdgcn_global_load_lds(src, (lds_void_t *)(stage + wave * 64 + 256 * i), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(src, (lds_void_t *)(stage + wave * 64 + TH * i), 16, 0, 0);
       }
 #pragma unroll
       for (int i = 0; i < T::kLoadsB; ++i) {
         const uint16_t *src = b_src[i] + static_cast<int64_t>(k0) * ldb;
         if (tail && k0 + b_k[i] >= K) src = zero;
-        __builtin_amdgcn_global_load_lds(src, (lds_void_t *)(stage + T::kChunksA + wave * 64 + 256 * i), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(src, (lds_void_t *)(stage + T::kChunksA + wave * 64 + TH * i), 16, 0, 0);
       }
     };
 #pragma unroll
@@ -685,9 +686,9 @@ __global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A
     };
     auto store = [&](int stage, const uint4 (&qa)[T::kLoadsA], const uint4 (&qb)[T::kLoadsB]) {
 #pragma unroll
-      for (int i = 0; i < T::kLoadsA; ++i) lds[stage * T::kStage + tid + 256 * i] = qa[i];
+      for (int i = 0; i < T::kLoadsA; ++i) lds[stage * T::kStage + tid + TH * i] = qa[i];
 #pragma unroll
-      for (int i = 0; i < T::kLoadsB; ++i) lds[stage * T::kStage + T::kChunksA + tid + 256 * i] = qb[i];
+      for (int i = 0; i < T::kLoadsB; ++i) lds[stage * T::kStage + T::kChunksA + tid + TH * i] = qb[i];
     };
     if (k_tiles > 0) load(0, ra[0], rb[0]);
     if (k_tiles > 1) load(1, ra[1], rb[1]);
@@ -717,7 +718,7 @@ __global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn * (BN / 2) + nt * 32 + 8 * g + 4 * half;
+        const int n = n0 + wn * (BN / WN) + nt * 32 + 8 * g + 4 * half;
         const f32x16_t &v = acc[mt][nt];
         if (partials != nullptr) {
           const int64_t width = (N + 3) & ~3;
@@ -739,8 +740,8 @@ __global__ __launch_bounds__(256) void gemm_small(const uint16_t *__restrict__ A
 // The tile size follows from how many tiles the chip's 256 CUs hold at once, bf16 measured on both sides of each line:
 //   * up to 128 tiles of 128 x 128: 64 x 64 ones, K divided over workgroups where these are few too (1000^3
 //     10.5 us against 15.5 in 128 x 128, 512 x 512 x 4096 14 against 45);
-//   * up to 256: 128 x 128 with four stages, one a CU (1021 x 2304 x 768 13.4 us against 15.3 in 64 x 64 and 48
-//     in 256 x 256; 2048^3 32 against 46 and 54);
+//   * up to 256: 128 x 128 with four stages and eight waves, one a CU (1021 x 2304 x 768 12.1 us against 13.3 with
+//     four waves, 15.3 in 64 x 64 and 48 in 256 x 256; 2048^3 30.7 against 32.3, 46 and 54);
 //   * up to 512: the same with two stages, two a CU (2639 x 2880 x 6912 125 us against 173 with four stages
 //     and 155 in 256 x 256; 8192 x 1024 x 4096 90 against 103 in 256 x 256);
 //   * more: 256 x 256 (4096 x 4096 x 1024 44 us against 61, 8000 x 2048 x 520 32 against 41).
@@ -777,10 +778,10 @@ int resources_of(int64_t m, int64_t n, IntentHipKernelResources *out) {   // ali
     return describe(kernel, "gemm_skinny<f16>", "gemm_skinny<bf16>", kSkinnyWaves * 64);
   }
   if (tiles > 2 * kChip) return describe(&gemm_mfma<E, Epi, false>, "gemm_mfma<f16>", "gemm_mfma<bf16>", kThreads);
-  const auto kernel = tiles <= kChip / 2 ? &gemm_small<E, Epi, 64, 64, 64, 4, true>
-                      : tiles <= kChip   ? &gemm_small<E, Epi, 128, 128, 64, 4, true>
-                                         : &gemm_small<E, Epi, 128, 128, 64, 2, true>;
-  return describe(kernel, "gemm_small<f16>", "gemm_small<bf16>", 256);
+  const auto kernel = tiles <= kChip / 2 ? &gemm_small<E, Epi, 64, 64, 64, 4, true, 2>
+                      : tiles <= kChip   ? &gemm_small<E, Epi, 128, 128, 64, 4, true, 4>
+                                         : &gemm_small<E, Epi, 128, 128, 64, 2, true, 2>;
+  return describe(kernel, "gemm_small<f16>", "gemm_small<bf16>", tiles > kChip / 2 && tiles <= kChip ? 512 : 256);
 }
 
 }  // namespace
@@ -816,12 +817,12 @@ void launch_splits(const float *partials, const Epi &ep, int m, int n, int split
   gemm_splits<Epi, kQuads><<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, ep, m, n, splits);
 }
 
-template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma>
+template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma, int WN = 2>
 void launch_small(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, int n, int k, int64_t lda, int64_t ldb,
                   float *partials, int splits, hipStream_t s) {
   const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
-  gemm_small<E, Epi, BM, BN, BK, S, kDma>
-      <<<dim3(xcd_blocks(static_cast<int64_t>(tiles_m) * tiles_n), splits), dim3(256), 0, s>>>(
+  gemm_small<E, Epi, BM, BN, BK, S, kDma, WN>
+      <<<dim3(xcd_blocks(static_cast<int64_t>(tiles_m) * tiles_n), splits), dim3(128 * WN), 0, s>>>(
           A, B, ep, m, n, k, lda, ldb, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
   if (splits > 1) launch_splits<E, Epi, kDma>(partials, ep, m, n, splits, s);
 }
@@ -862,7 +863,7 @@ int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t
   } else if (tiles(128) <= kChip / 2) {
     launch_small<E, Epi, 64, 64, 64, 4, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
   } else if (tiles(128) <= kChip) {
-    launch_small<E, Epi, 128, 128, 64, 4, true>(A, B, ep, M, N, depth, lda, ldb, nullptr, 1, s);
+    launch_small<E, Epi, 128, 128, 64, 4, true, 4>(A, B, ep, M, N, depth, lda, ldb, nullptr, 1, s);
   } else if (tiles(128) <= 2 * kChip) {
     launch_small<E, Epi, 128, 128, 64, 2, true>(A, B, ep, M, N, depth, lda, ldb, nullptr, 1, s);
   } else {
