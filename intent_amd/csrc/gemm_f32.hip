@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma(const float *__restric
 }  // namespace
 
 int gemm_f32_resources(int64_t m, int64_t n, IntentHipKernelResources *out) {
-  if (gemm_f32_few_applies(m, n)) return gemm_f32_few_resources(m, out);
+  if (gemm_f32_few_applies(m, n)) return gemm_f32_few_resources(m, n, out);
   return describe_kernel(reinterpret_cast<const void *>(&gemm_f32_mfma<false>), "gemm_f32_mfma", kThreads, out);
 }
 

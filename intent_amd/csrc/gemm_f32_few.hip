@@ -19,7 +19,7 @@ namespace {
 //     per row; column tile t is then the columns 4 r + t;
 //   * 16-byte loads need only 4-byte alignment, so every row stride takes this path; groups of 4 that
 //     reach past K, or past N for natural B, are loaded one element at a time, zeros past K.
-// Measured: linear_f32 256 x 1000 x 2048 158 -> 18.4 us (matrix-rate floor 7; the rest is the first loads, the LDS
+// Measured: linear_f32 256 x 1000 x 2048 158 -> 17.5 us (matrix-rate floor 7; the rest is the first loads, the LDS
 // sum and the second launch), 1 x 4096 x 4096 310 -> 20, 2048 x 1024 x 4096 316 -> 157 (110 TFLOP/s).
 constexpr int kFewCols = 64, kFewUnit = 32, kFewWaves = 4;
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -172,14 +172,27 @@ __global__ __launch_bounds__(256) void gemm_f32_splits(const float *__restrict__
   store_4(C + static_cast<int64_t>(m) * ldc + n, total, N - n);
 }
 
-int few_rows(int64_t m) { return m <= 16 ? 16 : m <= 32 ? 32 : 64; }
-int64_t few_tiles(int64_t m, int64_t n) { return (m + few_rows(m) - 1) / few_rows(m) * ((n + kFewCols - 1) / kFewCols); }
+// Rows of a tile. 64 load two thirds of the operand bytes per product that 32 do, but with at most 128 such tiles
+// twice as many of 32 rows still run in one pass and leave fewer K parts to add: measured (32 against 64 rows)
+// 512^3 9.6 / 11.6 us, 1067 x 312 x 1560 20.7 / 33.5, 128 x 4096 x 1024 17.0 / 20.5, 256 x 1000 x 2048 19.2 / 20.0.
+// Past that a second pass costs more (640 x 832 x 1000, 130 tiles: 30.5 / 22.9; 1024^3 33.4 / 25.3), and in a long
+// K the bytes do (48 x 8192 x 2048 29.6 / 29.3, 128 x 4096 x 4096 52.7 / 49.0).
+constexpr int64_t kFewTallTiles = 128, kFewTallDepth = 2048;
+int few_rows(int64_t m, int64_t n, int64_t k) {
+  if (m <= 16) return 16;
+  const bool pair = (m + 63) / 64 * ((n + kFewCols - 1) / kFewCols) <= kFewTallTiles && k <= kFewTallDepth;
+  return m <= 32 || pair ? 32 : 64;
+}
+int64_t few_tiles(int64_t m, int64_t n, int64_t k) {
+  const int64_t rows = few_rows(m, n, k);
+  return (m + rows - 1) / rows * ((n + kFewCols - 1) / kFewCols);
+}
 
 // Workgroups along K: about one workgroup per CU, at least 128 k each, and only where the second
-// launch returns more than its 3 us (512^3: 11.2 us against 13.2 unsplit; 256 x 1000 x 2048: 20 against 42).
+// launch returns more than its 3 us (512^3: 9.6 us against 13.2 unsplit; 256 x 1000 x 2048: 19 against 42).
 int few_splits(int64_t m, int64_t n, int64_t k) {
   if (m < 1 || n < 1 || k < 512) return 1;
-  const int64_t tiles = few_tiles(m, n);
+  const int64_t tiles = few_tiles(m, n, k);
   const int64_t splits = 256 / tiles < k / 128 ? 256 / tiles : k / 128;
   return splits < 2 ? 1 : static_cast<int>(splits);
 }
@@ -199,7 +212,7 @@ void launch_few(const float *a, const float *b, float *c, int M, int N, int K, i
 template <bool kTransB>
 void launch_few_rows(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb,
                      int64_t ldc, float *partials, int splits, hipStream_t s) {
-  switch (few_rows(M)) {
+  switch (few_rows(M, N, K)) {
     case 16: return launch_few<kTransB, 1>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
     case 32: return launch_few<kTransB, 2>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
     default: return launch_few<kTransB, 4>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
@@ -217,10 +230,11 @@ size_t gemm_f32_few_bytes(int64_t m, int64_t n, int64_t k) {
   return splits > 1 ? static_cast<size_t>(splits) * m * ((n + 3) / 4 * 4) * sizeof(float) : 0;
 }
 
-int gemm_f32_few_resources(int64_t m, IntentHipKernelResources *out) {
-  const void *kernel = few_rows(m) == 16   ? reinterpret_cast<const void *>(&gemm_f32_few<false, 1>)
-                       : few_rows(m) == 32 ? reinterpret_cast<const void *>(&gemm_f32_few<false, 2>)
-                                           : reinterpret_cast<const void *>(&gemm_f32_few<false, 4>);
+int gemm_f32_few_resources(int64_t m, int64_t n, IntentHipKernelResources *out) {
+  const int rows = few_rows(m, n, kFewTallDepth);   // the query has no depth: a short one's
+  const void *kernel = rows == 16   ? reinterpret_cast<const void *>(&gemm_f32_few<false, 1>)
+                       : rows == 32 ? reinterpret_cast<const void *>(&gemm_f32_few<false, 2>)
+                                    : reinterpret_cast<const void *>(&gemm_f32_few<false, 4>);
   return describe_kernel(kernel, "gemm_f32_few", kFewWaves * 64, out);
 }
 

@@ -161,12 +161,14 @@ def run_attention(device, defn, q, k, v, scale, group, causal, bf16):
     return bf16_tensor_bits(out) if bf16 else out.cpu().numpy()
 
 
-# Few output tiles: 16-, 32- and 64-row blocks and their edges, column counts around one 64-column block and
+# Few output tiles: 16-, 32- and 64-row blocks and their edges (64 rows from 129
+# such tiles or K = 2049 on: the last four sizes), column counts around one 64-column block and
 # off every 4 (partial 16-byte groups), K below one 32-deep unit, off it by 1 to 31, and divided over workgroups
 # (from 512 on), one and several row blocks, rows of every 4-byte alignment.
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (15, 63, 31), (16, 64, 32), (17, 65, 33), (32, 61, 47), (33, 130, 100),
                                    (64, 70, 511), (65, 7, 513), (100, 67, 1031), (3, 1000, 2050), (300, 129, 777),
-                                   (1, 30000, 40)])
+                                   (1, 30000, 40), (705, 741, 129), (520, 960, 600), (513, 897, 40),
+                                   (65, 70, 2053)])
 @pytest.mark.parametrize("workspace", ["prepare", "static"])
 def test_gemm_f32_few_tiles(device, m, n, k, workspace):
     """Against 64-bit products within the error of K f32 roundings, exact on small integers, and with NaN in the last
