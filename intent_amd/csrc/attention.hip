@@ -172,7 +172,8 @@ __device__ __forceinline__ void lane_halves(float v, float &lo, float &hi) {
 
 // Index i of `count` dealt to the 8 XCDs in runs: workgroup x goes to XCD x % 8, so with `count` a multiple of 8
 // each XCD gets count / 8 consecutive indices, and query heads that share a key head share its L2 (B4 HQ32 HK8 S4096
-// D128 bf16 causal 671 -> 635 us, B4 HQ16 HK4 S1932 164 -> 156; equal heads are indifferent).
+// D128 bf16 causal 671 -> 635 us, B4 HQ16 HK4 S1932 164 -> 156). Heads of their own keys share nothing and keep
+// the plain order (B4 H32 S4096 f16 causal 662.6 us, 665.0 in runs).
 __device__ __forceinline__ int xcd_run(int i, int count) { return count % 8 == 0 ? (i % 8) * (count / 8) + i / 8 : i; }
 
 template <typename E, int D, int DV, int kMode>
@@ -214,7 +215,8 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd(const uint16_t *__r
   int64_t row0 = 0;           // first row of the sequence (packed sequences)
   if constexpr (kVarlen) {
     const int item = static_cast<int>(blockIdx.x) / heads;   // the heads of an item are neighbours
-    h = xcd_run(static_cast<int>(blockIdx.x) % heads, heads);
+    h = static_cast<int>(blockIdx.x) % heads;
+    if (head_group > 1) h = xcd_run(h, heads);
     if (item >= *r.count) return;                            // the grid covers the item capacity
     const int2 work = r.items[item];
     const int start = min(max(r.cu[work.x], 0), r.total);
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd(const uint16_t *__r
     part = split.grouped ? x / items : x % split.count;
     const int bh_count = items / q_blocks;
     qb = q_blocks - 1 - item / bh_count;   // heaviest blocks first
-    const int bh = xcd_run(item % bh_count, bh_count);
+    const int nth = item % bh_count, bh = head_group > 1 ? xcd_run(nth, bh_count) : nth;
     b = bh / heads;
     h = bh % heads;
     sq = sq_all;

@@ -132,10 +132,10 @@ def test_varlen_other_head_dims(device):
     assert_16bit(o, oracle.attention_varlen_fwd(q, k, v, offsets(lengths), scale, True, head_group=2))
 
 
-# 64 sequences are the most that one wave lists with the longest walks first; the heads of 16 and 24 run one eighth per
-# XCD, those of 6 in order; empty sequences first, last and between.
+# 64 sequences are the most that one wave lists with the longest walks first; the heads of 16 and 24 that share keys run
+# one eighth per XCD, those of 6 and of their own keys in order; empty sequences first, last and between.
 @pytest.mark.parametrize("sequences", [1, 2, 63, 64, 65])
-@pytest.mark.parametrize("heads,group", [(16, 4), (24, 1), (6, 3)])
+@pytest.mark.parametrize("heads,group", [(16, 4), (24, 3), (24, 1), (6, 3)])
 def test_varlen_item_order(device, sequences, heads, group):
     announce("varlen item order", sequences, heads, group)
     g = np.random.default_rng(sequences * heads + group)
