@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define INTENT_HIP_ABI_VERSION 18
+#define INTENT_HIP_ABI_VERSION 19
 
 enum IntentHipStatus {
   INTENT_HIP_OK = 0,
@@ -313,18 +313,26 @@ int intent_hip_attention_bwd_dkdv(const void *q, const void *k, const void *v, c
                                   int64_t sk, int64_t d, const int64_t strides[30], float scale,
                                   int causal, void *stream);
 
-/* The same with a caller-owned device workspace. When the grid above would hold fewer than 256
- * workgroups (batch * kv_heads * ceil(sk / 128)), each query head of the group, and each of up to
- * 8 ranges of its query tiles (qsplits, enough for about 512 workgroups), gets its own workgroups, which write unscaled f32
- * partial sums to the workspace ([2][head_group * qsplits][batch][kv_heads][sk][d]: dK, then dV);
- * a second kernel folds them in (head, range) order, scales dK and casts. With head_group == 1
- * the split is taken only when qsplits > 1. intent_hip_attention_bwd_dkdv_workspace_bytes gives
- * the size (0 when the split is not taken; the workspace may then be NULL, and a NULL workspace
- * always selects the unsplit kernel). The workspace must be 16-byte aligned. No counterpart in
+/* The same with a caller-owned device workspace, through which workgroups share the walk of a key block: each writes unscaled
+ * f32 partial sums ([2][parts][d / 8][batch * kv_heads * sk][8]: dK, then dV), and a second kernel folds
+ * them in part order, scales dK and casts. The grid is batch * kv_heads * ceil(sk / 128) workgroups, or
+ * ceil(sk / 256) from 65536 key rows (batch * kv_heads * sk) on.
+ *   - Fewer than 256 workgroups: each query head of the group, and each of up to 8 ranges of its query tiles (enough for
+ *     about 512 workgroups), is a part. With head_group == 1 only when there is more than one range.
+ *   - 256 to 511 workgroups, causal, and at least 4096 queries per key head (head_group * sq): two parts, halves of the
+ *     group's query heads, or of the query tiles when head_group is odd.
+ *   - Otherwise the walk is whole.
+ * intent_hip_attention_bwd_dkdv_masked_workspace_bytes gives the size for a causal (1) or unmasked (0) call, 0 when the
+ * walk is whole; intent_hip_attention_bwd_dkdv_workspace_bytes the size that either of them takes, the causal one's.
+ * A NULL workspace always selects the whole walk. The workspace must be 16-byte aligned. One that is too small or not
+ * aligned is an error with fewer than 256 workgroups, and with more it is left unused. No counterpart in
  * the reference: the reference's single kernel launch (backward/attention.py:87-137) has no
  * workspace. */
 int intent_hip_attention_bwd_dkdv_workspace_bytes(int64_t batch, int64_t q_heads, int64_t head_group,
                                                   int64_t sq, int64_t sk, int64_t d, size_t *bytes);
+int intent_hip_attention_bwd_dkdv_masked_workspace_bytes(int64_t batch, int64_t q_heads, int64_t head_group,
+                                                         int64_t sq, int64_t sk, int64_t d, int causal,
+                                                         size_t *bytes);
 int intent_hip_attention_bwd_dkdv_ws(const void *q, const void *k, const void *v, const void *dout,
                                      const float *lse, const float *delta, void *dk, void *dv,
                                      int64_t batch, int64_t q_heads, int64_t head_group, int64_t sq,

@@ -871,17 +871,17 @@ int64_t dq_workspace(int splits, int64_t batch, int64_t q_heads, int64_t sq, int
 // 2 x kSplitBelow or more workgroups, heaviest first, even out. The fold moves 32 D bytes per key, which walks of
 // at least kEvenPairs queries (over the group's heads) return: dK/dV with the fold, causal, D128, B2 HQ32 HK8 S2048
 // 434 -> 279 us, B1 HQ32 HK16 S2048 219 -> 149; but B2 HQ32 HK32 S1024 120 -> 146, B1 HQ32 HK32 S1500 97 -> 130. Without
-// the mask the walks are even (B2 HQ32 HK8 S2048 424 -> 450), and the launch leaves them whole.
+// the mask the walks are even (B2 HQ32 HK8 S2048 424 -> 450), and they stay whole.
 constexpr int64_t kEvenPairs = 4096;
 
 struct DkdvPlan {
   int head_parts = 0, qsplits = 0;
   bool wide = false;       // 8-wave kernels, dK and dV apart
-  bool optional = false;   // runs unsplit without a mask, or with a workspace too small for it
+  bool optional = false;   // runs unsplit with a workspace too small for it
   int parts() const { return head_parts * qsplits; }
 };
 
-DkdvPlan dkdv_plan(int64_t batch, int64_t q_heads, int64_t head_group, int64_t sq, int64_t sk) {
+DkdvPlan dkdv_plan(int64_t batch, int64_t q_heads, int64_t head_group, int64_t sq, int64_t sk, bool causal) {
   DkdvPlan plan;
   if (batch <= 0 || q_heads <= 0 || sq <= 0 || sk <= 0) return plan;
   const int64_t groups = batch * (q_heads / head_group);
@@ -889,7 +889,7 @@ DkdvPlan dkdv_plan(int64_t batch, int64_t q_heads, int64_t head_group, int64_t s
   const int64_t rows = plan.wide ? 2 * kRows : kRows, blocks = groups * ((sk + rows - 1) / rows);
   const int64_t query_tiles = (sq + kTile - 1) / kTile;
   if (blocks >= kSplitBelow) {
-    if (blocks >= 2 * kSplitBelow || head_group * sq < kEvenPairs) return plan;
+    if (!causal || blocks >= 2 * kSplitBelow || head_group * sq < kEvenPairs) return plan;
     plan.optional = true;
     plan.head_parts = head_group % 2 == 0 ? 2 : 1;
     plan.qsplits = 2 / plan.head_parts;
@@ -1040,10 +1040,16 @@ extern "C" int intent_hip_attention_bwd_dq(const void *q, const void *k, const v
 
 extern "C" int intent_hip_attention_bwd_dkdv_workspace_bytes(int64_t batch, int64_t q_heads, int64_t head_group,
                                                              int64_t sq, int64_t sk, int64_t d, size_t *bytes) {
+  return intent_hip_attention_bwd_dkdv_masked_workspace_bytes(batch, q_heads, head_group, sq, sk, d, 1, bytes);
+}
+
+extern "C" int intent_hip_attention_bwd_dkdv_masked_workspace_bytes(int64_t batch, int64_t q_heads, int64_t head_group,
+                                                                    int64_t sq, int64_t sk, int64_t d, int causal,
+                                                                    size_t *bytes) {
   if (bytes == nullptr) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "null output");
   if (const int rc = check_common(batch, q_heads, head_group, sq, sk, d)) return rc;
   *bytes = static_cast<size_t>(
-      dkdv_workspace(dkdv_plan(batch, q_heads, head_group, sq, sk), batch, q_heads / head_group, sk, d));
+      dkdv_workspace(dkdv_plan(batch, q_heads, head_group, sq, sk, causal != 0), batch, q_heads / head_group, sk, d));
   return INTENT_HIP_OK;
 }
 
@@ -1066,13 +1072,13 @@ extern "C" int intent_hip_attention_bwd_dkdv_ws(const void *q, const void *k, co
   BwdGeometry g{};
   load_geometry(g, strides, true);
   const int64_t kv_heads = q_heads / head_group;
-  DkdvPlan plan = dkdv_plan(batch, q_heads, head_group, sq, sk);
+  DkdvPlan plan = dkdv_plan(batch, q_heads, head_group, sq, sk, causal != 0);
   const int64_t need = dkdv_workspace(plan, batch, kv_heads, sk, d);
   const bool small = workspace == nullptr || workspace_bytes < static_cast<size_t>(need) || !aligned(workspace, 16);
   if (need > 0 && workspace != nullptr && small && !plan.optional)
     return fail(INTENT_HIP_ERR_WORKSPACE, "dK/dV needs %lld 16-byte aligned workspace bytes, got %zu",
                 static_cast<long long>(need), workspace_bytes);
-  if (small || (plan.optional && !causal)) plan.head_parts = plan.qsplits = 0;
+  if (small) plan.head_parts = plan.qsplits = 0;
   const auto *Q = static_cast<const uint16_t *>(q);
   const auto *K = static_cast<const uint16_t *>(k);
   const auto *V = static_cast<const uint16_t *>(v);

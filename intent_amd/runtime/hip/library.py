@@ -11,7 +11,7 @@ from pathlib import Path
 
 from ...diagnostics import CompilationStageError
 
-ABI_VERSION = 18
+ABI_VERSION = 19
 # INTENT_HIP_STATIC_SCRATCH_BYTES: the static scratch of intent_hip_csr_spmv_f32_static.
 STATIC_SCRATCH_BYTES = 32 << 20
 LIBRARY_NAME = "libintent_hip.so"
@@ -95,6 +95,8 @@ SIGNATURES = {
                                              _i64, ctypes.POINTER(_i64), _f32, _p, _sz, _p)),
     "intent_hip_attention_bwd_dkdv_workspace_bytes": (_int, (_i64, _i64, _i64, _i64, _i64, _i64,
                                                               ctypes.POINTER(_sz))),
+    "intent_hip_attention_bwd_dkdv_masked_workspace_bytes": (_int, (_i64, _i64, _i64, _i64, _i64, _i64, _int,
+                                                                     ctypes.POINTER(_sz))),
     "intent_hip_attention_bwd_dq_workspace_bytes": (_int, (_i64, _i64, _i64, _i64, _i64, _i64,
                                                             ctypes.POINTER(_sz))),
     "intent_hip_attention_bwd_dq_ws": (_int, (_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64,

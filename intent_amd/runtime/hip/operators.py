@@ -675,8 +675,12 @@ def _attention_bwd(kind):
 
         # (tuning family hip.attention_backward: split = 0 runs the unsplit kernels)
         size = ctypes.c_size_t(0)
-        lib.check(lib.fn[f"attention_bwd_{kind}_workspace_bytes"](batch, q_heads, group, sq, sk, d,
-                                                                 ctypes.byref(size)), "provider_preparation")
+        extents = (batch, q_heads, group, sq, sk, d)
+        if kind == "dq":
+            status = lib.fn["attention_bwd_dq_workspace_bytes"](*extents, ctypes.byref(size))
+        else:
+            status = lib.fn["attention_bwd_dkdv_masked_workspace_bytes"](*extents, int(causal), ctypes.byref(size))
+        lib.check(status, "provider_preparation")
         split, candidates = _split_choice("hip.attention_backward", size.value)
         workspace = torch.empty(size.value, dtype=torch.uint8, device=device) if split else None
         if workspace is not None:

@@ -214,6 +214,25 @@ def test_dkdv_two_parts_match_one(device, shape):
         assert all(torch.equal(a, b) for a, b in zip(run(causal, bytes_), run(causal, 0)))
 
 
+@pytest.mark.parametrize("causal", [True, False])
+def test_dkdv_without_a_mask_takes_no_workspace(device, causal):
+    """256 to 511 workgroups run in two parts under a causal mask only: an unmasked call is prepared without the parts' sums
+    and says so, and its split row is not one to choose."""
+    from intent_amd.examples.kernels.backward.attention import attention_backward_dkdv
+
+    batch, hq, hk, sq, sk, d = 64, 16, 2, 520, 256, 64
+    announce("dK/dV workspace and mask", causal)
+    q, k = (torch.zeros(batch, h, n, d, dtype=torch.float16, device=device) for h, n in ((hq, sq), (hk, sk)))
+    rows = torch.zeros(batch, hq, sq, device=device)
+    kernel = intent.jit(attention_backward_dkdv, backend="hip", constexprs={"HEAD_GROUP": hq // hk, "CAUSAL": causal})
+    call = kernel.prepare(q, k, k.clone(), q.clone(), rows, rows.clone(), 0.125)
+    chosen, *others = call.inspect_configurations()
+    facts = dict(chosen.configuration)
+    assert facts["split"] == int(causal)
+    assert facts["workspace_bytes"] == (2 * 2 * batch * hk * sk * d * 4 if causal else 0)
+    assert [a.eligible for a in others] == [causal]
+
+
 # Calls with at least 256 x 256 rows (batch x heads x sequence) take the 8-wave kernels: dQ with
 # 256-query workgroups, dK/dV as two kernels (dK, then dV) with 256-key workgroups. These shapes
 # reach that bound with short sequences so the oracle stays fast; 260 and 300 leave ragged blocks.

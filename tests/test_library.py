@@ -54,6 +54,27 @@ def test_argument_validation_without_gpu():
     assert lib.fn["csr_spmv_f32"](1, 1, 1, 1, 1, 2**31 - 5, 10, 10, 1, 1 << 30, None) == 2
 
 
+def test_dkdv_workspace_follows_the_mask():
+    """256 to 511 workgroups have two parts under a causal mask and none without; smaller grids split, and larger ones do not,
+    whatever the mask. The query without a mask gives what either takes."""
+    lib = hiplib.library()
+
+    def size(extents, *causal):
+        out = ctypes.c_size_t(7)
+        query = lib.fn["attention_bwd_dkdv_masked_workspace_bytes" if causal else "attention_bwd_dkdv_workspace_bytes"]
+        assert query(*extents, *causal, ctypes.byref(out)) == 0
+        return out.value
+
+    for extents in ((2, 32, 4, 2048, 2048, 128), (64, 16, 8, 520, 256, 64), (128, 2, 1, 4100, 256, 128)):
+        batch, heads, group, _, sk, d = extents
+        assert size(extents, 1) == size(extents) == 2 * 2 * batch * (heads // group) * sk * d * 4
+        assert size(extents, 0) == 0
+    for extents in ((2, 8, 4, 1024, 1024, 64), (4, 32, 4, 4096, 4096, 128), (2, 32, 1, 1024, 1024, 128)):
+        assert size(extents, 1) == size(extents, 0) == size(extents)
+    assert size((2, 8, 4, 1024, 1024, 64)) > 0 and size((4, 32, 4, 4096, 4096, 128)) == 0
+    assert lib.fn["attention_bwd_dkdv_masked_workspace_bytes"](1, 1, 1, 1, 1, 64, 0, None) == 1
+
+
 def test_attention_bias_validation_without_gpu():
     """The key-bias entry refuses a non-unit key stride, a negative stride and a null bias before
     any HIP call; empty work is a successful no-op."""
