@@ -53,15 +53,23 @@ int launch_gemm_f32_few(const float *a, const float *b, float *c, int M, int N, 
 
 constexpr int kWave = 64;
 
-// Tile of this workgroup, or -1 for none, when each XCD shall take one run of consecutive tiles (neighbouring tiles
-// share an operand through its L2): workgroups go to the 8 XCDs in turn, so the launch has
-// xcd_blocks(tiles) of them in x, and any number in y and z. The runs differ by one tile at most.
-inline unsigned xcd_blocks(int64_t tiles) { return static_cast<unsigned>((tiles + 7) / 8 * 8); }
-__device__ __forceinline__ int xcd_tile(int tiles) {
-  const int xcd = blockIdx.x & 7;
+// A launch has fewer than 2^32 threads along each axis. Grids of one workgroup per tile go on along z past kGridX
+// workgroups in x (a multiple of 8, below the limit for workgroups of up to 512 threads).
+constexpr int64_t kGridX = int64_t{1} << 22;
+inline dim3 tile_grid(int64_t tiles, int splits) {
+  const int64_t blocks = (tiles + 7) / 8 * 8, z = (blocks + kGridX - 1) / kGridX;
+  return dim3(static_cast<unsigned>(z > 1 ? kGridX : blocks), static_cast<unsigned>(splits), static_cast<unsigned>(z));
+}
+__device__ __forceinline__ int grid_block() { return static_cast<int>(blockIdx.x + blockIdx.z * static_cast<unsigned>(kGridX)); }
+
+// Tile of workgroup `block` of a tile_grid (grid_block(), or blockIdx.x where there are few tiles), or -1 for none, when
+// each XCD shall take one run of consecutive tiles (neighbouring tiles share an operand through its L2): workgroups go
+// to the 8 XCDs in turn. The runs differ by one tile at most.
+__device__ __forceinline__ int xcd_tile(int block, int tiles) {
+  const int xcd = block & 7;
   const int first = static_cast<int>(static_cast<int64_t>(tiles) * xcd / 8);
   const int last = static_cast<int>(static_cast<int64_t>(tiles) * (xcd + 1) / 8);
-  const int tile = first + static_cast<int>(blockIdx.x >> 3);
+  const int tile = first + (block >> 3);
   return tile < last ? tile : -1;
 }
 

@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_skinny(const uint16_t 
   const int c = lane & 15, g = lane >> 4;
   // The row blocks of one column block are neighbours, so they share its B through the L2 of one XCD. With
   // one row block the XCDs take the column blocks in turn (28.9 against 27.9 us at 32 x 14336 x 4096).
-  const int tile = kStream ? static_cast<int>(blockIdx.x) : xcd_tile(tiles_m * tiles_n);
+  const int tile = kStream ? grid_block() : xcd_tile(grid_block(), tiles_m * tiles_n);
   if (tile < 0 || tile >= tiles_m * tiles_n) return;
   const int m0 = (tile % tiles_m) * kRows, n0 = (tile / tiles_m) * kSkinnyCols;
   // Columns past N and rows past M read valid ones instead; their products are not stored.
@@ -566,7 +566,9 @@ __global__ __launch_bounds__(128 * WN) void gemm_small(const uint16_t *__restric
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
-  const int tile = xcd_tile(tiles_m * tiles_n);   // the row blocks of one column block are neighbours
+  // The row blocks of one column block are neighbours. The DMA kernels run few tiles, along x (grid_block() there:
+  // 1021 x 2304 x 768 12.1 -> 12.9 us).
+  const int tile = xcd_tile(kDma ? static_cast<int>(blockIdx.x) : grid_block(), tiles_m * tiles_n);
   if (tile < 0) return;
   const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
 
@@ -822,7 +824,7 @@ void launch_small(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, in
                   float *partials, int splits, hipStream_t s) {
   const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
   gemm_small<E, Epi, BM, BN, BK, S, kDma, WN>
-      <<<dim3(xcd_blocks(static_cast<int64_t>(tiles_m) * tiles_n), splits), dim3(128 * WN), 0, s>>>(
+      <<<tile_grid(static_cast<int64_t>(tiles_m) * tiles_n, splits), dim3(128 * WN), 0, s>>>(
           A, B, ep, m, n, k, lda, ldb, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
   if (splits > 1) launch_splits<E, Epi, kDma>(partials, ep, m, n, splits, s);
 }
@@ -831,7 +833,7 @@ template <typename E, typename Epi, int MT, bool kStream>
 void launch_skinny(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, int n, int k, int64_t lda, int64_t ldb,
                    float *partials, int splits, hipStream_t s) {
   const int tiles_m = (m + 16 * MT - 1) / (16 * MT), tiles_n = (n + kSkinnyCols - 1) / kSkinnyCols;
-  gemm_skinny<E, Epi, MT, kStream><<<dim3(xcd_blocks(tiles_m * tiles_n), splits), dim3(kSkinnyWaves * 64), 0, s>>>(
+  gemm_skinny<E, Epi, MT, kStream><<<tile_grid(static_cast<int64_t>(tiles_m) * tiles_n, splits), dim3(kSkinnyWaves * 64), 0, s>>>(
       A, B, ep, m, n, k, lda, ldb, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
   if (splits > 1) launch_splits<E, Epi, true>(partials, ep, m, n, splits, s);
 }

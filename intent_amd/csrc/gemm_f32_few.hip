@@ -57,7 +57,7 @@ __global__ __launch_bounds__(kFewWaves * 64) void gemm_f32_few(const float *__re
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   // The row blocks of one column block are neighbours on one XCD; with one row block the XCDs take turns.
-  const int tile = tiles_m == 1 ? static_cast<int>(blockIdx.x) : xcd_tile(tiles_m * tiles_n);
+  const int tile = tiles_m == 1 ? grid_block() : xcd_tile(grid_block(), tiles_m * tiles_n);
   if (tile < 0 || tile >= tiles_m * tiles_n) return;
   const int m0 = (tile % tiles_m) * kRows, n0 = (tile / tiles_m) * kFewCols;
 
@@ -201,7 +201,7 @@ template <bool kTransB, int MT>
 void launch_few(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
                 float *partials, int splits, hipStream_t s) {
   const int tiles_m = (M + 16 * MT - 1) / (16 * MT), tiles_n = (N + kFewCols - 1) / kFewCols;
-  gemm_f32_few<kTransB, MT><<<dim3(xcd_blocks(tiles_m * tiles_n), splits), dim3(kFewWaves * 64), 0, s>>>(
+  gemm_f32_few<kTransB, MT><<<tile_grid(static_cast<int64_t>(tiles_m) * tiles_n, splits), dim3(kFewWaves * 64), 0, s>>>(
       a, b, c, M, N, K, lda, ldb, ldc, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
   if (splits > 1) {
     const int64_t quads = static_cast<int64_t>(M) * ((N + 3) / 4);

@@ -746,11 +746,12 @@ int check_extents(int64_t rows, int64_t cols, int64_t in0, int64_t in1, int64_t 
 }
 
 // Workgroups of a launch over `rows`: at most as many as the device holds at once for a persistent
-// kernel, and at most 2^30 for the softmax_*_block and _stream kernels, which walk the rest with a grid stride.
+// kernel, and for the softmax_*_block and _stream kernels as many as a launch may have (fewer than 2^32 threads in
+// all), which walk the rest with a grid stride.
 int64_t grid_blocks(const Variant &v, int64_t rows) {
   const int64_t blocks = (rows + v.rows_per_block - 1) / v.rows_per_block;
   if (v.persistent) return std::min<int64_t>(blocks, resident_blocks(v.kernel, v.block));
-  return v.rows_per_block == kRowsPerBlock ? blocks : std::min<int64_t>(blocks, int64_t{1} << 30);
+  return v.rows_per_block == kRowsPerBlock ? blocks : std::min<int64_t>(blocks, UINT32_MAX / v.block);
 }
 
 template <typename T>

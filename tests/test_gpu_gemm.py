@@ -155,3 +155,19 @@ def test_gemm_strides_and_offsets(device, m, n, k, lda, ldb, ldc, offset):
 @pytest.mark.parametrize("workspace", ["prepare", "static"])
 def test_gemm_few_rows(device, m, n, k, workspace):
     check_product(device, m, n, k, workspace)
+
+
+# One row against more columns, and one column against more rows, than workgroups of one tile each fit one axis of a launch
+# (2^32 threads): the few-row kernel, and 64 x 64 tiles through registers.
+@pytest.mark.parametrize("m,n,k", [(1, (1 << 29) + 72, 8), ((1 << 30) - 1, 1, 1)])
+def test_gemm_longest_extents(device, m, n, k):
+    announce("gemm longest extents", m, n, k)
+    g = torch.Generator(device=device).manual_seed(11)
+    small = lambda *shape: torch.randint(-3, 4, shape, generator=g, device=device, dtype=torch.int8)  # noqa: E731
+    a, b = small(m, k), small(k, n)
+    c = intent.jit(bf16_gemm, backend="hip").run(a.bfloat16(), b.bfloat16())
+    step = 1 << 26
+    for at in range(0, max(m, n), step):        # small integers: exact
+        rows, columns = (a[at:at + step], b) if m > n else (a, b[:, at:at + step])
+        want = sum(rows[:, i:i + 1] * columns[i:i + 1] for i in range(k))
+        assert torch.equal(c[at:at + step] if m > n else c[:, at:at + step], want.bfloat16())

@@ -192,6 +192,15 @@ def test_gemm_f32_few_tiles(device, m, n, k, workspace):
         assert (np.isnan(run(x, y).cpu().numpy()) == expected).all()
 
 
+def test_gemm_f32_longest_extents(device):
+    """More row blocks than workgroups fit one axis of a launch (2^32 threads)."""
+    m = (1 << 30) - 1
+    announce("gemm f32 longest extents", m)
+    a = torch.arange(m, device=device, dtype=torch.int32).remainder_(1021).float()[:, None]
+    c = intent.jit(gemm_f32, backend="hip").run(a, torch.full((1, 1), -2.0, device=device))
+    assert torch.equal(c, a.mul_(-2))
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_attention_family_golden(device, golden, causal):
     announce("attention family golden", causal)

@@ -252,3 +252,22 @@ def test_softmax_workgroup_rows(device, rows, cols, kind):
                 bound = bound + 2.0 ** -11 * np.abs(p64 * (g64 - proj)) + 2.0 ** -25
             assert (np.abs(as_f64(dv) - p64 * (g64 - proj)) <= bound + 1e-40).all()
             assert untouched(d_base, dv)
+
+
+def test_softmax_more_rows_than_a_launch_has_workgroups(device):
+    """Rows of one workgroup each, more of them than a launch may have (2^32 threads), all reading one row of x."""
+    rows, cols = (1 << 24) + 5, 4097
+    announce("softmax most rows", rows, cols)
+    if torch.cuda.mem_get_info(device)[0] < 160e9:
+        pytest.skip("the result takes 137 GB of device memory")
+    x = torch.randn(cols, generator=torch.Generator(device=device).manual_seed(3), device=device).bfloat16()
+    y = torch.empty((rows, cols), dtype=torch.bfloat16, device=device)
+    lib = hiplib.library()
+    lib.check(lib.fn["softmax_fwd"](hiplib.BF16, x.data_ptr(), y.data_ptr(), rows, cols, 0, cols,
+                                    torch.cuda.current_stream().cuda_stream))
+    want = torch.softmax(x.double(), dim=0)
+    assert_16bit(y[0].double().cpu().numpy(), want.cpu().numpy(), rel=2.0 ** -7, abs_=2.0 ** -24)
+    for at in range(0, rows, 1 << 20):
+        assert bool((y[at:at + (1 << 20)] == y[0]).all())
+    del y
+    torch.cuda.empty_cache()
