@@ -278,9 +278,10 @@ __device__ __forceinline__ Span span_of(const T *base, int64_t rows, int cols, i
 }
 
 // The chunk at `start`, elements outside the row as in `outside`. kRagged false: chunks lie wholly
-// inside or wholly outside the row and are aligned.
-template <typename T, bool kRagged>
-__device__ __forceinline__ u32x4_t load_chunk(const T *row, int start, int cols, bool whole, uint32_t outside,
+// inside or wholly outside the row and are aligned. Index: int, or int64_t where a row may end within a
+// chunk of 2^31 (start + V).
+template <typename T, bool kRagged, typename Index>
+__device__ __forceinline__ u32x4_t load_chunk(const T *row, Index start, int cols, bool whole, uint32_t outside,
                                               const Span &span) {
   constexpr int V = kChunk<T>;
   u32x4_t w;
@@ -321,8 +322,8 @@ __device__ __forceinline__ u32x4_t load_chunk(const T *row, int start, int cols,
 // next, twice the registers (and spills at 1024 threads).
 __device__ __forceinline__ void keep_raw(u32x4_t &w) { asm("" : "+v"(w)); }
 
-template <typename T, bool kRagged, bool kStream>
-__device__ __forceinline__ void store_chunk(T *row, int start, int cols, bool whole, const float (&in)[kChunk<T>]) {
+template <typename T, bool kRagged, bool kStream, typename Index>
+__device__ __forceinline__ void store_chunk(T *row, Index start, int cols, bool whole, const float (&in)[kChunk<T>]) {
   constexpr int V = kChunk<T>;
   if (!kRagged ? start < cols : whole && start >= 0 && start + V <= cols) {
     store_row_chunk<T, V, kStream>(row + start, in);
@@ -428,28 +429,28 @@ __global__ __launch_bounds__(kStreamBlock) void softmax_fwd_stream(const T *x, T
     const int64_t first = static_cast<int64_t>(threadIdx.x) * V - shift;
     float m = -INFINITY;
     for (int64_t at = first; at < cols; at += kStreamBlock * V) {
-      const u32x4_t w = load_chunk<T, true>(xr, static_cast<int>(at), cols, true, kMinusInf<T>, span);
+      const u32x4_t w = load_chunk<T, true>(xr, at, cols, true, kMinusInf<T>, span);
 #pragma unroll
       for (int i = 0; i < V; ++i) m = fmaxf(m, element<T>(w, i));
     }
     m = block_reduce<kStreamBlock, true>(m, maxima);
     float s = 0.0f;
     for (int64_t at = first; at < cols; at += kStreamBlock * V) {
-      const u32x4_t w = load_chunk<T, true>(xr, static_cast<int>(at), cols, true, kMinusInf<T>, span);
+      const u32x4_t w = load_chunk<T, true>(xr, at, cols, true, kMinusInf<T>, span);
 #pragma unroll
       for (int i = 0; i < V; ++i) s += shifted_exp<T>(element<T>(w, i), m);
     }
     s = block_reduce<kStreamBlock, false>(s, sums);
     const float r = 1.0f / s;
     for (int64_t at = first; at < cols; at += kStreamBlock * V) {
-      const u32x4_t w = load_chunk<T, true>(xr, static_cast<int>(at), cols, true, kMinusInf<T>, span);
+      const u32x4_t w = load_chunk<T, true>(xr, at, cols, true, kMinusInf<T>, span);
       float o[V];
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         const float e = shifted_exp<T>(element<T>(w, i), m);
         o[i] = sizeof(T) == 4 ? e * r : quotient(e, s, r);
       }
-      store_chunk<T, true, false>(yr, static_cast<int>(at), cols, whole, o);
+      store_chunk<T, true, false>(yr, at, cols, whole, o);
     }
   }
 }
@@ -585,19 +586,19 @@ __global__ __launch_bounds__(kStreamBlock) void softmax_bwd_stream(const T *p, c
     const int64_t first = static_cast<int64_t>(threadIdx.x) * V - shift;
     float proj = 0.0f;
     for (int64_t at = first; at < cols; at += kStreamBlock * V) {
-      const u32x4_t pw = load_chunk<T, true>(pr, static_cast<int>(at), cols, true, 0, span_p);
-      const u32x4_t gw = load_chunk<T, true>(gr, static_cast<int>(at), cols, whole_g, 0, span_g);
+      const u32x4_t pw = load_chunk<T, true>(pr, at, cols, true, 0, span_p);
+      const u32x4_t gw = load_chunk<T, true>(gr, at, cols, whole_g, 0, span_g);
 #pragma unroll
       for (int i = 0; i < V; ++i) proj = fmaf(element<T>(pw, i), element<T>(gw, i), proj);
     }
     proj = block_reduce<kStreamBlock, false>(proj, sums[turn]);
     for (int64_t at = first; at < cols; at += kStreamBlock * V) {
-      const u32x4_t pw = load_chunk<T, true>(pr, static_cast<int>(at), cols, true, 0, span_p);
-      const u32x4_t gw = load_chunk<T, true>(gr, static_cast<int>(at), cols, whole_g, 0, span_g);
+      const u32x4_t pw = load_chunk<T, true>(pr, at, cols, true, 0, span_p);
+      const u32x4_t gw = load_chunk<T, true>(gr, at, cols, whole_g, 0, span_g);
       float o[V];
 #pragma unroll
       for (int i = 0; i < V; ++i) o[i] = element<T>(pw, i) * (element<T>(gw, i) - proj);
-      store_chunk<T, true, true>(dr, static_cast<int>(at), cols, whole_d, o);
+      store_chunk<T, true, true>(dr, at, cols, whole_d, o);
     }
   }
 }

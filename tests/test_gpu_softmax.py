@@ -254,6 +254,37 @@ def test_softmax_workgroup_rows(device, rows, cols, kind):
             assert untouched(d_base, dv)
 
 
+def test_softmax_longest_row(device):
+    """2^31 - 1 columns, the most an entry takes: the last 16-byte chunk reaches past 2^31 elements, and what follows the row
+    in the result's buffer stays as it was."""
+    cols, tail = 2 ** 31 - 1, 24
+    announce("softmax longest row", cols)
+    lib, stream = hiplib.library(), torch.cuda.current_stream().cuda_stream
+    step = torch.arange(tail, device=device, dtype=torch.float32)
+    x, buffer = torch.zeros(cols, dtype=torch.bfloat16, device=device), torch.full((cols + 9,), 7.0, dtype=torch.bfloat16,
+                                                                                   device=device)
+    # The maximum is 0, so that almost every exponential is 1 and a thread's 2^21 terms add up without rounding (a sum of
+    # 2^21 other f32 terms may be off by 2^21 x 2^-24).
+    x[-tail:] = -step / 8
+    lib.check(lib.fn["softmax_fwd"](hiplib.BF16, x.data_ptr(), buffer.data_ptr(), 1, cols, cols, cols, stream))
+    total = cols - tail + float(torch.exp(-step.double() / 8).sum())
+    assert bool((buffer[cols:] == 7.0).all())
+    assert_16bit(buffer[cols - tail:cols].double().cpu().numpy(), torch.exp(-step.double() / 8).cpu().numpy() / total,
+                 rel=2.0 ** -7, abs_=0)
+    first = buffer[:1].clone()
+    assert abs(float(first) * total - 1) <= 2.0 ** -8 and bool((buffer[:cols - tail] == first).all())
+    del x, buffer
+
+    p = torch.zeros(cols, dtype=torch.float16, device=device)
+    dy, dx = torch.ones_like(p), torch.full((cols + 9,), 7.0, dtype=torch.float16, device=device)
+    p[-tail:], dy[-tail:] = 1 / 32, step.half()
+    lib.check(lib.fn["softmax_bwd"](hiplib.F16, p.data_ptr(), dy.data_ptr(), dx.data_ptr(), 1, cols, cols, cols, cols, stream))
+    assert bool((dx[cols:] == 7.0).all()) and bool((dx[:cols - tail] == 0).all())
+    assert torch.equal(dx[cols - tail:cols], ((step - step.sum() / 32) / 32).half())      # exact in f32
+    del p, dy, dx
+    torch.cuda.empty_cache()
+
+
 def test_softmax_more_rows_than_a_launch_has_workgroups(device):
     """Rows of one workgroup each, more of them than a launch may have (2^32 threads), all reading one row of x."""
     rows, cols = (1 << 24) + 5, 4097
