@@ -50,6 +50,7 @@ from dataclasses import dataclass, field
 from typing import Callable
 
 from ...diagnostics import CompilationStageError
+from ..torch_views import raw_stream_getter
 from .library import (BF16, F16, F32, STATIC_SCRATCH_BYTES, OP_ATTENTION_BWD_DELTA, OP_ATTENTION_BWD_DKDV, OP_ATTENTION_BWD_DQ,
                       OP_ATTENTION_FWD, OP_ATTENTION_FWD_F16, OP_ATTENTION_BIAS, OP_ATTENTION_VARLEN, OP_MLA_PREFILL, OP_CSR_SPMV_F32, OP_GEMM, OP_GEMM_BF16, OP_GEMM_F32, OP_GEMM_I8, OP_QUANTIZED_GEMM,
                       OP_CSR_SPMM_F32, OP_CONTINUOUS_DECODE, OP_GROUPED_DECODE_PARTIALS, OP_PAGED_DECODE_PARTIALS, OP_VARLEN_DECODE, OP_SOFTMAX_BWD, OP_SOFTMAX_FWD, OP_SPLITK_REDUCE)
@@ -232,6 +233,25 @@ def _refuse_staging(tensor, vector: int) -> None:
                          f"kernel needs {need}, got strides {tuple(tensor.stride())}")
 
 
+def _workspace_run(fn, args, size, device, keep):
+    """The launch fn(*args, workspace, size, stream) with a workspace allocated here. That one is ordered with the stream it
+    was allocated on and may be freed with the call, so a launch on another stream, or into a graph (never on stream 0),
+    takes one that belongs to that stream or graph."""
+    import torch
+
+    home = raw_stream_getter()(device.index)
+    kept = torch.empty(size, dtype=torch.uint8, device=device)
+    keep.append(kept)
+    address, capturing = kept.data_ptr(), torch.cuda.is_current_stream_capturing
+
+    def run(stream):
+        if stream == home and (stream == 0 or not capturing()):
+            return fn(*args, address, size, stream)
+        workspace = torch.empty(size, dtype=torch.uint8, device=device)
+        return fn(*args, workspace.data_ptr(), size, stream)
+    return run
+
+
 # ------------------------------------------------------------------------------ attention head dimensions
 # The attention kernels are built for key and value head dimensions of 64 and 128. Any other width up
 # to 128 (the reference declares D and DV symbolic, streaming/attention.py:428-553) runs on the next of
@@ -321,20 +341,14 @@ def _softmax_bwd(dtype_code):
 
 
 # ------------------------------------------------------------------------------ GEMM
-def _split_sums(lib, name, m, n, k, device, keep):
-    """(address, bytes) of a workspace for the f32 sums of a product whose K is divided over workgroups; ()
-    where nothing is split (enough output tiles, or workspace='static')."""
+def _split_bytes(lib, name, m, n, k) -> int:
+    """Bytes of the f32 sums of a product whose K is divided over workgroups; 0 where nothing is split (enough output
+    tiles, or workspace='static')."""
     import ctypes
-
-    import torch
 
     size = ctypes.c_size_t(0)
     lib.check(lib.fn[name + "_workspace_bytes"](m, n, k, ctypes.byref(size)), "provider_preparation")
-    if not size.value or _static_workspace():
-        return ()
-    workspace = torch.empty(size.value, dtype=torch.uint8, device=device)
-    keep.append(workspace)
-    return workspace.data_ptr(), size.value
+    return 0 if _static_workspace() else size.value
 
 
 def _gemm_launch(lib, dtype_code, activation, a, b, c, entry, configuration, device):
@@ -345,15 +359,17 @@ def _gemm_launch(lib, dtype_code, activation, a, b, c, entry, configuration, dev
     args = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk), _row_stride(ck))
     facts = (("m", m), ("n", n), ("k", k)) + configuration
     op = OP_GEMM_BF16 if entry == "intent_hip_gemm_bf16" else OP_GEMM
-    extra = _split_sums(lib, "gemm", m, n, k, device, keep)
-    if extra:
-        fn, entry, args, facts = (lib.fn["gemm_ws"], "intent_hip_gemm_ws", (dtype_code, activation, *args, *extra),
-                                  facts + (("workspace_bytes", extra[1]),))
-    elif entry == "intent_hip_gemm_bf16":
-        fn = lib.fn["gemm_bf16"]
+    size = _split_bytes(lib, "gemm", m, n, k)
+    if size:
+        entry, facts = "intent_hip_gemm_ws", facts + (("workspace_bytes", size),)
+        run = _workspace_run(lib.fn["gemm_ws"], (dtype_code, activation, *args), size, device, keep)
     else:
-        fn, args = lib.fn["gemm"], (dtype_code, activation, *args)
-    return Launch(entry, lambda stream: fn(*args, stream), tuple(keep), tuple(before), tuple(after), facts,
+        if entry == "intent_hip_gemm_bf16":
+            fn = lib.fn["gemm_bf16"]
+        else:
+            fn, args = lib.fn["gemm"], (dtype_code, activation, *args)
+        run = lambda stream: fn(*args, stream)  # noqa: E731
+    return Launch(entry, run, tuple(keep), tuple(before), tuple(after), facts,
                   lambda: lib.kernel_resources(op, dtype_code, m, n))
 
 
@@ -388,11 +404,13 @@ def _gemm_f32(transpose_b: bool):
         args = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk),
                 _row_stride(ck), int(transpose_b))
         facts = (("m", m), ("n", n), ("k", k), ("transpose_b", transpose_b))
-        fn, entry, extra = lib.fn["gemm_f32"], "intent_hip_gemm_f32", _split_sums(lib, "gemm_f32", m, n, k, device, keep)
-        if extra:
-            fn, entry, args, facts = (lib.fn["gemm_f32_ws"], "intent_hip_gemm_f32_ws", (*args, *extra),
-                                      facts + (("workspace_bytes", extra[1]),))
-        return Launch(entry, lambda stream: fn(*args, stream), tuple(keep), tuple(before), tuple(after), facts,
+        fn, entry = lib.fn["gemm_f32"], "intent_hip_gemm_f32"
+        run = lambda stream: fn(*args, stream)  # noqa: E731
+        size = _split_bytes(lib, "gemm_f32", m, n, k)
+        if size:
+            entry, facts = "intent_hip_gemm_f32_ws", facts + (("workspace_bytes", size),)
+            run = _workspace_run(lib.fn["gemm_f32_ws"], args, size, device, keep)
+        return Launch(entry, run, tuple(keep), tuple(before), tuple(after), facts,
                       lambda: lib.kernel_resources(OP_GEMM_F32, F32, m, n))
     return plan
 
@@ -671,8 +689,6 @@ def _attention_bwd(kind):
         # workspace, allocated here once per prepared call.
         import ctypes
 
-        import torch
-
         # (tuning family hip.attention_backward: split = 0 runs the unsplit kernels)
         size = ctypes.c_size_t(0)
         extents = (batch, q_heads, group, sq, sk, d)
@@ -682,19 +698,17 @@ def _attention_bwd(kind):
             status = lib.fn["attention_bwd_dkdv_masked_workspace_bytes"](*extents, int(causal), ctypes.byref(size))
         lib.check(status, "provider_preparation")
         split, candidates = _split_choice("hip.attention_backward", size.value)
-        workspace = torch.empty(size.value, dtype=torch.uint8, device=device) if split else None
-        if workspace is not None:
-            keep.append(workspace)
         fn = lib.fn[f"attention_bwd_{kind}_ws"]
-        args = (*args, workspace.data_ptr() if workspace is not None else None,
-                size.value if workspace is not None else 0)
-        configuration += (("split", split), ("workspace_bytes", size.value if workspace is not None else 0))
+        if split:
+            run = _workspace_run(fn, args, size.value, device, keep)
+        else:
+            run = lambda stream: fn(*args, None, 0, stream)  # noqa: E731
+        configuration += (("split", split), ("workspace_bytes", size.value if split else 0))
         op = OP_ATTENTION_BWD_DQ if kind == "dq" else OP_ATTENTION_BWD_DKDV
         # The kernel variant depends on the rows of the call: batch x query heads x queries for dQ,
         # batch x key heads x keys for dK/dV.
         rows = batch * q_heads * sq if kind == "dq" else batch * (q_heads // group) * sk
-        return Launch(f"intent_hip_attention_bwd_{kind}", lambda stream: fn(*args, stream), tuple(keep),
-                      tuple(before), tuple(after), configuration,
+        return Launch(f"intent_hip_attention_bwd_{kind}", run, tuple(keep), tuple(before), tuple(after), configuration,
                       lambda: lib.kernel_resources(op, F16, rows, d), candidates)
     return plan
 

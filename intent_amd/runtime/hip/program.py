@@ -9,7 +9,6 @@ current stream, asynchronously; `result()` does not synchronize.
 """
 from __future__ import annotations
 
-import functools
 import threading
 
 from ...diagnostics import CompilationStageError
@@ -17,7 +16,7 @@ from ..artifact import CompiledArtifact
 from ..diagnostics import ConfigurationAssessment, NativeObservation, NativeResource
 from ..interface import PublicInterface, ViewParameter
 from ..invocation import Binding, bind_arguments
-from ..torch_views import allocate_output, observe_view
+from ..torch_views import allocate_output, observe_view, raw_stream_getter
 from .library import library
 from .operators import OperatorSpec, plan_policies
 from .tuning import FAMILY_OF, SPLIT, TuningConfiguration
@@ -44,17 +43,6 @@ def _constexpr_parameters(definition) -> tuple[tuple[str, object], ...]:
     return tuple(out)
 
 
-@functools.lru_cache(maxsize=1)
-def _raw_stream_getter():
-    """Fast accessor of the current HIP stream handle of a device (an int)."""
-    import torch
-
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is not None:
-        return raw
-    return lambda index: torch.cuda.current_stream(index).cuda_stream
-
-
 class HipPreparedCall:
     """Bound arguments, allocated outputs/workspace and the native call that uses them."""
 
@@ -66,7 +54,7 @@ class HipPreparedCall:
         self._run = launch.run
         self._before, self._after = launch.before, launch.after
         self._current_device = torch.cuda.current_device
-        self._stream = _raw_stream_getter()
+        self._stream = raw_stream_getter()
         self._launched = False
 
     def compile(self) -> None:

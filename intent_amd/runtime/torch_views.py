@@ -15,6 +15,8 @@ records shape, strides and dtype only.
 """
 from __future__ import annotations
 
+import functools
+
 from ..integrations.torch import torch_dtype
 from .interface import ViewParameter
 from .invocation import ViewFacts
@@ -69,3 +71,14 @@ def allocate_output(parameter: ViewParameter, shape: tuple, *, device, abstract:
 
     value = torch.empty(shape, dtype=torch_dtype(parameter.dtype), device=device)
     return value, observe_view(parameter, value, device=device, abstract=abstract)
+
+
+@functools.lru_cache(maxsize=1)
+def raw_stream_getter():
+    """Fast accessor of the current HIP stream handle of a device (an int)."""
+    import torch
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None:
+        return raw
+    return lambda index: torch.cuda.current_stream(index).cuda_stream

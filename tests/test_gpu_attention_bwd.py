@@ -233,6 +233,50 @@ def test_dkdv_without_a_mask_takes_no_workspace(device, causal):
     assert [a.eligible for a in others] == [causal]
 
 
+@pytest.mark.parametrize("shape", [(1, 4, 2, 300, 300, 64), (64, 16, 2, 520, 256, 64)])
+def test_dkdv_workspace_on_another_stream_and_in_a_graph(device, shape):
+    """A prepared call launched on another stream and captured in a graph, then dropped before that stream comes to it: the
+    memory it gives back is other tensors' by then and stays theirs, and the gradients are those of a plain launch."""
+    from intent_amd.examples.kernels.backward.attention import attention_backward_dkdv
+
+    batch, hq, hk, sq, sk, d = shape
+    announce("dK/dV workspace, other stream and graph", shape)
+    g = torch.Generator(device=device).manual_seed(sum(shape))
+    normal = lambda *dims: torch.randn(dims, generator=g, device=device)  # noqa: E731
+    q, do = normal(batch, hq, sq, d).half(), normal(batch, hq, sq, d).half()
+    k, v = normal(batch, hk, sk, d).half(), normal(batch, hk, sk, d).half()
+    lse, delta = normal(batch, hq, sq) * 0.5 + float(np.log(sk)), normal(batch, hq, sq)
+    kernel = intent.jit(attention_backward_dkdv, backend="hip", constexprs={"HEAD_GROUP": hq // hk, "CAUSAL": True})
+    args = (q, k, v, do, lse, delta, d ** -0.5)
+    want = kernel.run(*args)
+    eager, captured = ((torch.zeros_like(k), torch.zeros_like(v)) for _ in range(2))
+    calls = [kernel.prepare(*args, outputs=pair) for pair in (eager, captured)]
+    size = dict(calls[0].inspect_configurations()[0].configuration)["workspace_bytes"]
+    assert size > 0
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            calls[1].launch()
+    busy = normal(4096, 4096)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            busy = busy @ busy * 1e-3
+        calls[0].launch()
+    del calls
+    others = [torch.full((size,), 77, dtype=torch.uint8, device=device) for _ in range(3)]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for t in captured:
+            t.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for pair in (eager, captured) for a, b in zip(pair, want))
+        assert all(bool((o == 77).all()) for o in others)
+
+
 # Calls with at least 256 x 256 rows (batch x heads x sequence) take the 8-wave kernels: dQ with
 # 256-query workgroups, dK/dV as two kernels (dK, then dV) with 256-key workgroups. These shapes
 # reach that bound with short sequences so the oracle stays fast; 260 and 300 leave ragged blocks.

@@ -10,7 +10,7 @@ import torch
 import intent_amd as intent
 import oracle
 from intent_amd.examples import inputs
-from intent_amd.examples.kernels.contraction.gemm import bf16_gemm
+from intent_amd.examples.kernels.contraction.gemm import bf16_gemm, gemm_f32
 from tests.gpu_util import announce, assert_16bit, bf16_tensor_bits, bf16_to_f32, to_bf16_tensor
 
 pytestmark = pytest.mark.gpu
@@ -155,6 +155,68 @@ def test_gemm_strides_and_offsets(device, m, n, k, lda, ldb, ldc, offset):
 @pytest.mark.parametrize("workspace", ["prepare", "static"])
 def test_gemm_few_rows(device, m, n, k, workspace):
     check_product(device, m, n, k, workspace)
+
+
+def split_product(device, kind):
+    """A prepared product whose K is divided over workgroups, its result's buffer, the exact result, and its workspace's bytes."""
+    g = torch.Generator(device=device).manual_seed(5)
+    a, b = (torch.randint(-3, 4, shape, generator=g, device=device).float() for shape in ((16, 4096), (4096, 640)))
+    want, c = a @ b, torch.zeros(16, 640, device=device)          # exact: whole sums below 2^24
+    if kind == "bf16":
+        a, b, c, want = a.bfloat16(), b.bfloat16(), c.bfloat16(), want.bfloat16()
+    kernel = intent.jit(bf16_gemm if kind == "bf16" else gemm_f32, backend="hip")
+    call = kernel.prepare(a, b, outputs=(c,))
+    size = dict(call.inspect_configurations()[0].configuration)["workspace_bytes"]
+    assert size > 0
+    return call, (a, b), c, want, size
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f32"])
+def test_split_gemm_on_another_stream(device, kind):
+    """A prepared call launched on another stream and dropped before that stream comes to it: the memory it gives back is
+    another tensor's by then and stays that tensor's."""
+    announce("split gemm, other stream", kind)
+    call, operands, c, want, size = split_product(device, kind)
+    busy = torch.randn(4096, 4096, device=device)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            busy = busy @ busy * 1e-3
+        call.launch()
+        call.launch()
+    del call
+    others = [torch.full((size,), 77, dtype=torch.uint8, device=device) for _ in range(3)]
+    torch.cuda.synchronize()
+    assert torch.equal(c, want) and all(bool((o == 77).all()) for o in others)
+
+
+@pytest.mark.parametrize("own_stream", [False, True])
+@pytest.mark.parametrize("kind", ["bf16", "f32"])
+def test_split_gemm_graph_outlives_its_call(device, kind, own_stream):
+    """A graph that captured a prepared call, whether the call was prepared on the capturing stream or not, is replayed after
+    the call was dropped and its memory given away."""
+    announce("split gemm, graph", kind, own_stream)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream if own_stream else torch.cuda.current_stream()):
+        call, (a, b), c, want, size = split_product(device, kind)
+        call.launch()
+    torch.cuda.synchronize()
+    assert torch.equal(c, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            call.launch()
+        del call
+        others = [torch.full((size,), 77, dtype=torch.uint8, device=device) for _ in range(3)]
+    others += [torch.full((size,), 77, dtype=torch.uint8, device=device) for _ in range(3)]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        c.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want) and all(bool((o == 77).all()) for o in others)
 
 
 # One row against more columns, and one column against more rows, than workgroups of one tile each fit one axis of a launch
