@@ -126,8 +126,10 @@ extern "C" int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int6
   switch (op) {
     case INTENT_HIP_OP_SOFTMAX_FWD: return softmax_fwd_resources(dtype, rows, cols, out);
     case INTENT_HIP_OP_SOFTMAX_BWD: return softmax_bwd_resources(dtype, rows, cols, out);
-    case INTENT_HIP_OP_GEMM_BF16: return gemm_resources(INTENT_HIP_BF16, rows, cols, out);
-    case INTENT_HIP_OP_GEMM: return gemm_resources(dtype, rows, cols, out);
+    // 16-bit products: aligned operands of a K that whole steps divide.
+    case INTENT_HIP_OP_GEMM_BF16: dtype = INTENT_HIP_BF16; [[fallthrough]];
+    case INTENT_HIP_OP_GEMM:
+      return gemm_resources(dtype, 0, nullptr, nullptr, nullptr, rows, (cols + 7) / 8 * 8, 64, 64, 64, 64, out);
     case INTENT_HIP_OP_GEMM_F32: return gemm_f32_resources(rows, cols, out);
     // cols = d, or d | dv << 16 when dv differs from d.
     case INTENT_HIP_OP_ATTENTION_FWD_F16:
@@ -153,10 +155,33 @@ extern "C" int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int6
       return attention_resources(INTENT_HIP_F16, rows, cols & 0xFFFF, cols >> 16, 3, out);
     case INTENT_HIP_OP_CSR_SPMM_F32: return spmm_resources(cols, out);
     case INTENT_HIP_OP_GEMM_I8: return gemm_i8_resources(rows, cols, out);
-    case INTENT_HIP_OP_QUANTIZED_GEMM: return quantized_gemm_resources(out);
+    case INTENT_HIP_OP_QUANTIZED_GEMM:
+      return quantized_gemm_resources(nullptr, nullptr, nullptr, nullptr, rows, (cols + 7) / 8 * 8, 64, 64, 64, 64, 64, out);
     case INTENT_HIP_OP_ATTENTION_BIAS:
       return attention_resources(INTENT_HIP_F16, rows, cols & 0xFFFF, (cols >> 16) ? (cols >> 16) : (cols & 0xFFFF), 2,
                                  out);
   }
   return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "unknown operator code %d", op);
+}
+
+extern "C" int intent_hip_call_resources(int op, int dtype, const int64_t *facts, int count,
+                                         IntentHipKernelResources *out) {
+  if (facts == nullptr) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "null facts");
+  const int64_t *f = facts;
+  const auto address = [f](int i) { return reinterpret_cast<const void *>(static_cast<uintptr_t>(f[i])); };
+  const auto takes = [&](int n) {
+    return count == n ? INTENT_HIP_OK : fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "operator %d takes %d facts, got %d", op, n, count);
+  };
+  switch (op) {
+    case INTENT_HIP_OP_GEMM_BF16: dtype = INTENT_HIP_BF16; [[fallthrough]];
+    case INTENT_HIP_OP_GEMM:
+      if (const int rc = takes(10)) return rc;
+      return gemm_resources(dtype, static_cast<int>(f[9]), address(0), address(1), address(2), f[3], f[4], f[5], f[6], f[7],
+                            f[8], out);
+    case INTENT_HIP_OP_QUANTIZED_GEMM:
+      if (const int rc = takes(11)) return rc;
+      return quantized_gemm_resources(address(0), address(1), address(2), address(3), f[4], f[5], f[6], f[7], f[8], f[9],
+                                      f[10], out);
+  }
+  return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "operator code %d has no facts of a call", op);
 }

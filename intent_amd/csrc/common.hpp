@@ -31,13 +31,16 @@ int device_cus();
 int describe_kernel(const void *kernel, const char *name, int block_threads,
                     IntentHipKernelResources *out);
 
-// Kernel selection facts exported by each operator file for intent_hip_kernel_resources().
+// Kernel selection facts exported by each operator file for intent_hip_kernel_resources() and
+// intent_hip_call_resources().
 int softmax_fwd_resources(int dtype, int64_t rows, int64_t cols, IntentHipKernelResources *out);
 int softmax_bwd_resources(int dtype, int64_t rows, int64_t cols, IntentHipKernelResources *out);
-int gemm_resources(int dtype, int64_t m, int64_t n, IntentHipKernelResources *out);
+int gemm_resources(int dtype, int activation, const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k,
+                   int64_t lda, int64_t ldb, int64_t ldc, IntentHipKernelResources *out);
 int gemm_f32_resources(int64_t m, int64_t n, IntentHipKernelResources *out);
 int gemm_i8_resources(int64_t m, int64_t n, IntentHipKernelResources *out);
-int quantized_gemm_resources(IntentHipKernelResources *out);
+int quantized_gemm_resources(const void *a, const void *b, const void *residual, const void *out, int64_t m, int64_t n,
+                             int64_t k, int64_t lda, int64_t ldb, int64_t ldr, int64_t ldo, IntentHipKernelResources *to);
 int attention_resources(int dtype, int64_t sq, int64_t d, int64_t dv, int mode, IntentHipKernelResources *out);
 int spmv_resources(int64_t rows, int64_t nnz, IntentHipKernelResources *out);
 int attention_bwd_resources(int64_t which, int64_t rows, int64_t d, IntentHipKernelResources *out);

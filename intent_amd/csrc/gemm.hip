@@ -22,6 +22,8 @@
 //   * 256 x 256 tiles are walked in groups of 2 tile rows, column by column, in dispatch order: the
 //     tiles resident at one time share A row panels and B column panels, across XCDs
 //     through the MALL and within each XCD through its L2.
+#include <stdio.h>
+
 #include <type_traits>
 
 #include "common.hpp"
@@ -757,39 +759,82 @@ bool fast_path(const void *a, const void *b, const void *c, int64_t n, int64_t k
 
 }  // namespace
 
-int quantized_gemm_resources(IntentHipKernelResources *out) {
-  return describe_kernel(reinterpret_cast<const void *>(&gemm_mfma<_Float16, QuantizeStore, false>), "gemm_mfma<f16,quantize>",
-                         kThreads, out);
-}
-
 namespace {
 
-template <typename E>
-int resources_of(int64_t m, int64_t n, IntentHipKernelResources *out) {   // aligned operands
-  typedef CastStore<E, 0> Epi;
-  const auto describe = [&](auto kernel, const char *f16, const char *bf16, int threads) {
-    return describe_kernel(reinterpret_cast<const void *>(kernel), std::is_same<E, _Float16>::value ? f16 : bf16, threads,
-                           out);
-  };
+// Few rows, and strides that keep a lane's offset (24 rows of B, all rows of A) below 2^31 elements.
+bool skinny(int64_t m, int64_t lda, int64_t ldb) {
+  return m <= kSkinnyRows && lda < (int64_t{1} << 22) && ldb < (int64_t{1} << 25);
+}
+
+// The kernel of a product, its threads and its tile.
+enum Family { kSkinnyFamily, kSmallFamily, kLargeFamily };
+constexpr const char *kFamilyNames[] = {"gemm_skinny", "gemm_small", "gemm_mfma"};
+struct Choice {
+  const void *kernel;
+  Family family;
+  int threads, rows, cols;
+};
+
+template <typename E, typename Epi, int MT, bool kStream>
+Choice skinny_choice() {
+  return {reinterpret_cast<const void *>(&gemm_skinny<E, Epi, MT, kStream>), kSkinnyFamily, kSkinnyWaves * 64, 16 * MT,
+          kSkinnyCols};
+}
+template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma, int WN = 2>
+Choice small_choice() {
+  return {reinterpret_cast<const void *>(&gemm_small<E, Epi, BM, BN, BK, S, kDma, WN>), kSmallFamily, 128 * WN, BM, BN};
+}
+
+// `fast`: the operand layout that the DMA takes (fast_path); every other one runs in 64 x 64 tiles through registers.
+template <typename E, typename Epi>
+Choice choose(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool fast) {
+  if (!fast || k == 0) return small_choice<E, Epi, 64, 64, 64, 2, false>();
+  if (skinny(m, lda, ldb))
+    return m <= 16   ? skinny_choice<E, Epi, 1, true>()
+           : m <= 32 ? skinny_choice<E, Epi, 2, true>()
+           : m <= 64 ? skinny_choice<E, Epi, 4, true>()
+                     : skinny_choice<E, Epi, 4, false>();
   const int64_t tiles = (m + 127) / 128 * ((n + 127) / 128);
-  if (m <= kSkinnyRows) {
-    const auto kernel = m <= 16   ? &gemm_skinny<E, Epi, 1, true>
-                        : m <= 32 ? &gemm_skinny<E, Epi, 2, true>
-                        : m <= 64 ? &gemm_skinny<E, Epi, 4, true>
-                                  : &gemm_skinny<E, Epi, 4, false>;
-    return describe(kernel, "gemm_skinny<f16>", "gemm_skinny<bf16>", kSkinnyWaves * 64);
-  }
-  if (tiles > 2 * kChip) return describe(&gemm_mfma<E, Epi, false>, "gemm_mfma<f16>", "gemm_mfma<bf16>", kThreads);
-  const auto kernel = tiles <= kChip / 2 ? &gemm_small<E, Epi, 64, 64, 64, 4, true, 2>
-                      : tiles <= kChip   ? &gemm_small<E, Epi, 128, 128, 64, 4, true, 4>
-                                         : &gemm_small<E, Epi, 128, 128, 64, 2, true, 2>;
-  return describe(kernel, "gemm_small<f16>", "gemm_small<bf16>", tiles > kChip / 2 && tiles <= kChip ? 512 : 256);
+  if (tiles <= kChip / 2) return small_choice<E, Epi, 64, 64, 64, 4, true>();
+  if (tiles <= kChip) return small_choice<E, Epi, 128, 128, 64, 4, true, 4>();
+  if (tiles <= 2 * kChip) return small_choice<E, Epi, 128, 128, 64, 2, true>();
+  const void *kernel = k % kDmaBK == 0 ? reinterpret_cast<const void *>(&gemm_mfma<E, Epi, false>)
+                                       : reinterpret_cast<const void *>(&gemm_mfma<E, Epi, true>);
+  return {kernel, kLargeFamily, kThreads, kBM, kBN};
+}
+
+template <typename E, typename Epi>
+int describe(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool fast, const char *elements,
+             IntentHipKernelResources *out) {
+  const Choice choice = choose<E, Epi>(m, n, k, lda, ldb, fast);
+  char name[64];
+  snprintf(name, sizeof name, "%s<%s>", kFamilyNames[choice.family], elements);
+  return describe_kernel(choice.kernel, name, choice.threads, out);
+}
+
+// The MFMA kernels' quantizing epilogue reads 4 residuals as 8 bytes and stores 4 outputs as 4 bytes.
+bool quantize_fast_path(const void *a, const void *b, const void *residual, const void *out, int64_t n, int64_t k, int64_t lda,
+                        int64_t ldb, int64_t ldr, int64_t ldo) {
+  return k % 8 == 0 && n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned(a, 16) && aligned(b, 16) &&
+         ldr % 4 == 0 && aligned(residual, 8) && ldo % 4 == 0 && aligned(out, 4);
 }
 
 }  // namespace
 
-int gemm_resources(int dtype, int64_t m, int64_t n, IntentHipKernelResources *out) {
-  return dtype == INTENT_HIP_F16 ? resources_of<_Float16>(m, n, out) : resources_of<__bf16>(m, n, out);
+int quantized_gemm_resources(const void *a, const void *b, const void *residual, const void *out, int64_t m, int64_t n,
+                             int64_t k, int64_t lda, int64_t ldb, int64_t ldr, int64_t ldo, IntentHipKernelResources *to) {
+  return describe<_Float16, QuantizeStore>(m, n, k, lda, ldb, quantize_fast_path(a, b, residual, out, n, k, lda, ldb, ldr, ldo),
+                                           "f16,quantize", to);
+}
+
+int gemm_resources(int dtype, int activation, const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k,
+                   int64_t lda, int64_t ldb, int64_t ldc, IntentHipKernelResources *out) {
+  const bool fast = fast_path(a, b, c, n, k, lda, ldb, ldc);
+  if (dtype == INTENT_HIP_F16)
+    return activation ? describe<_Float16, CastStore<_Float16, 1>>(m, n, k, lda, ldb, fast, "f16", out)
+                      : describe<_Float16, CastStore<_Float16, 0>>(m, n, k, lda, ldb, fast, "f16", out);
+  return activation ? describe<__bf16, CastStore<__bf16, 1>>(m, n, k, lda, ldb, fast, "bf16", out)
+                    : describe<__bf16, CastStore<__bf16, 0>>(m, n, k, lda, ldb, fast, "bf16", out);
 }
 
 namespace {
@@ -819,61 +864,28 @@ void launch_splits(const float *partials, const Epi &ep, int m, int n, int split
   gemm_splits<Epi, kQuads><<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, ep, m, n, splits);
 }
 
-template <typename E, typename Epi, int BM, int BN, int BK, int S, bool kDma, int WN = 2>
-void launch_small(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, int n, int k, int64_t lda, int64_t ldb,
-                  float *partials, int splits, hipStream_t s) {
-  const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
-  gemm_small<E, Epi, BM, BN, BK, S, kDma, WN>
-      <<<tile_grid(static_cast<int64_t>(tiles_m) * tiles_n, splits), dim3(128 * WN), 0, s>>>(
-          A, B, ep, m, n, k, lda, ldb, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
-  if (splits > 1) launch_splits<E, Epi, kDma>(partials, ep, m, n, splits, s);
-}
-
-template <typename E, typename Epi, int MT, bool kStream>
-void launch_skinny(const uint16_t *A, const uint16_t *B, const Epi &ep, int m, int n, int k, int64_t lda, int64_t ldb,
-                   float *partials, int splits, hipStream_t s) {
-  const int tiles_m = (m + 16 * MT - 1) / (16 * MT), tiles_n = (n + kSkinnyCols - 1) / kSkinnyCols;
-  gemm_skinny<E, Epi, MT, kStream><<<tile_grid(static_cast<int64_t>(tiles_m) * tiles_n, splits), dim3(kSkinnyWaves * 64), 0, s>>>(
-      A, B, ep, m, n, k, lda, ldb, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
-  if (splits > 1) launch_splits<E, Epi, true>(partials, ep, m, n, splits, s);
-}
-
-// Few rows, and strides that keep a lane's offset (24 rows of B, all rows of A) below 2^31 elements.
-bool skinny(int64_t m, int64_t lda, int64_t ldb) {
-  return m <= kSkinnyRows && lda < (int64_t{1} << 22) && ldb < (int64_t{1} << 25);
-}
-
-// `fast`: the operand layout that the DMA takes (fast_path); every other one runs in 64 x 64 tiles through registers.
 // `partials`: null, or room for splits_bytes(m, n, k).
 template <typename E, typename Epi>
 int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t m, int64_t n, int64_t k, int64_t lda,
                     int64_t ldb, bool fast, float *partials, hipStream_t s) {
-  const int M = static_cast<int>(m), N = static_cast<int>(n), depth = static_cast<int>(k);
-  if (k > 0 && fast && skinny(m, lda, ldb)) {
-    const int splits = partials != nullptr ? skinny_splits(m, n, k) : 1;
-    if (m <= 16) launch_skinny<E, Epi, 1, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
-    else if (m <= 32) launch_skinny<E, Epi, 2, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
-    else if (m <= 64) launch_skinny<E, Epi, 4, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
-    else launch_skinny<E, Epi, 4, false>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
-    if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_skinny");
-    return INTENT_HIP_OK;
+  const Choice choice = choose<E, Epi>(m, n, k, lda, ldb, fast);
+  int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
+  int tiles_m = (M + choice.rows - 1) / choice.rows, tiles_n = (N + choice.cols - 1) / choice.cols;
+  int splits = 1;
+  if (partials != nullptr && choice.family == kSkinnyFamily) splits = skinny_splits(m, n, k);
+  if (partials != nullptr && choice.family == kSmallFamily && choice.rows == 64) splits = small_splits(m, n, k);
+  if (splits == 1) partials = nullptr;
+  const int64_t tiles = static_cast<int64_t>(tiles_m) * tiles_n;
+  const dim3 grid = choice.family == kLargeFamily ? dim3(static_cast<unsigned>(tiles)) : tile_grid(tiles, splits);
+  Epi epilogue = ep;
+  void *args[] = {&A, &B, &epilogue, &M, &N, &K, &lda, &ldb, &tiles_m, &tiles_n, &partials};
+  if (hipLaunchKernel(choice.kernel, grid, dim3(choice.threads), args, 0, s) != hipSuccess)
+    return launch_status(kFamilyNames[choice.family]);
+  if (splits > 1) {
+    if (fast) launch_splits<E, Epi, true>(partials, ep, M, N, splits, s);
+    else launch_splits<E, Epi, false>(partials, ep, M, N, splits, s);
+    if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_splits");
   }
-  const int splits = partials != nullptr ? small_splits(m, n, k) : 1;
-  const auto tiles = [&](int64_t edge) { return (m + edge - 1) / edge * ((n + edge - 1) / edge); };
-  if (!fast || k == 0) {
-    launch_small<E, Epi, 64, 64, 64, 2, false>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
-  } else if (tiles(128) <= kChip / 2) {
-    launch_small<E, Epi, 64, 64, 64, 4, true>(A, B, ep, M, N, depth, lda, ldb, partials, splits, s);
-  } else if (tiles(128) <= kChip) {
-    launch_small<E, Epi, 128, 128, 64, 4, true, 4>(A, B, ep, M, N, depth, lda, ldb, nullptr, 1, s);
-  } else if (tiles(128) <= 2 * kChip) {
-    launch_small<E, Epi, 128, 128, 64, 2, true>(A, B, ep, M, N, depth, lda, ldb, nullptr, 1, s);
-  } else {
-    const int tiles_m = (M + kBM - 1) / kBM, tiles_n = (N + kBN - 1) / kBN;
-    const auto kernel = depth % kDmaBK == 0 ? &gemm_mfma<E, Epi, false> : &gemm_mfma<E, Epi, true>;
-    kernel<<<dim3(tiles_m * tiles_n), dim3(kThreads), 0, s>>>(A, B, ep, M, N, depth, lda, ldb, tiles_m, tiles_n);
-  }
-  if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm");
   return INTENT_HIP_OK;
 }
 
@@ -953,9 +965,7 @@ extern "C" int intent_hip_quantized_gemm(const void *a, const void *b, const flo
     return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "row stride smaller than the row length");
   const QuantizeStore ep{bias, static_cast<const uint16_t *>(residual), ldr, output_scale, static_cast<int8_t *>(out),
                          ldo};
-  // The MFMA kernel's epilogue reads 4 residuals as 8 bytes and stores 4 outputs as 4 bytes.
-  const bool fast = k % 8 == 0 && n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned(a, 16) && aligned(b, 16) &&
-                    ldr % 4 == 0 && aligned(residual, 8) && ldo % 4 == 0 && aligned(out, 4);
-  return launch_epilogue<_Float16>(static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(b), ep, m, n, k, lda,
-                                   ldb, fast, nullptr, as_stream(stream));
+  return launch_epilogue<_Float16>(static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(b), ep, m, n, k, lda, ldb,
+                                   quantize_fast_path(a, b, residual, out, n, k, lda, ldb, ldr, ldo), nullptr,
+                                   as_stream(stream));
 }

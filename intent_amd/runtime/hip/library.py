@@ -11,7 +11,7 @@ from pathlib import Path
 
 from ...diagnostics import CompilationStageError
 
-ABI_VERSION = 19
+ABI_VERSION = 20
 # INTENT_HIP_STATIC_SCRATCH_BYTES: the static scratch of intent_hip_csr_spmv_f32_static.
 STATIC_SCRATCH_BYTES = 32 << 20
 LIBRARY_NAME = "libintent_hip.so"
@@ -50,6 +50,7 @@ SIGNATURES = {
     "intent_hip_device_count": (_int, (ctypes.POINTER(_int),)),
     "intent_hip_device_info": (_int, (_int, ctypes.POINTER(DeviceInfo))),
     "intent_hip_kernel_resources": (_int, (_int, _int, _i64, _i64, ctypes.POINTER(KernelResources))),
+    "intent_hip_call_resources": (_int, (_int, _int, ctypes.POINTER(_i64), _int, ctypes.POINTER(KernelResources))),
     "intent_hip_softmax_fwd": (_int, (_int, _p, _p, _i64, _i64, _i64, _i64, _p)),
     "intent_hip_softmax_bwd": (_int, (_int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p)),
     "intent_hip_gemm_bf16": (_int, (_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p)),
@@ -157,8 +158,17 @@ class HipLibrary:
                 "l2_bytes": info.l2_bytes}
 
     def kernel_resources(self, op: int, dtype: int, rows: int, cols: int) -> dict | None:
+        return self._resources(lambda out: self.fn["kernel_resources"](op, dtype, rows, cols, out))
+
+    def call_resources(self, op: int, dtype: int, *facts: int) -> dict | None:
+        """Facts of the kernel that one call launches, from the arguments include/intent_hip.h names for `op`."""
+        values = (_i64 * len(facts))(*facts)
+        return self._resources(lambda out: self.fn["call_resources"](op, dtype, values, len(facts), out))
+
+    @staticmethod
+    def _resources(query) -> dict | None:
         out = KernelResources()
-        if self.fn["kernel_resources"](op, dtype, rows, cols, ctypes.byref(out)) != 0:
+        if query(ctypes.byref(out)) != 0:
             return None
         return {"kernel": out.kernel.decode(), "vgprs": out.vgprs, "lds_bytes": out.lds_bytes,
                 "scratch_bytes": out.scratch_bytes, "block_threads": out.block_threads}

@@ -52,7 +52,7 @@ from typing import Callable
 from ...diagnostics import CompilationStageError
 from ..torch_views import raw_stream_getter
 from .library import (BF16, F16, F32, STATIC_SCRATCH_BYTES, OP_ATTENTION_BWD_DELTA, OP_ATTENTION_BWD_DKDV, OP_ATTENTION_BWD_DQ,
-                      OP_ATTENTION_FWD, OP_ATTENTION_FWD_F16, OP_ATTENTION_BIAS, OP_ATTENTION_VARLEN, OP_MLA_PREFILL, OP_CSR_SPMV_F32, OP_GEMM, OP_GEMM_BF16, OP_GEMM_F32, OP_GEMM_I8, OP_QUANTIZED_GEMM,
+                      OP_ATTENTION_FWD, OP_ATTENTION_FWD_F16, OP_ATTENTION_BIAS, OP_ATTENTION_VARLEN, OP_MLA_PREFILL, OP_CSR_SPMV_F32, OP_GEMM, OP_GEMM_F32, OP_GEMM_I8, OP_QUANTIZED_GEMM,
                       OP_CSR_SPMM_F32, OP_CONTINUOUS_DECODE, OP_GROUPED_DECODE_PARTIALS, OP_PAGED_DECODE_PARTIALS, OP_VARLEN_DECODE, OP_SOFTMAX_BWD, OP_SOFTMAX_FWD, OP_SPLITK_REDUCE)
 
 
@@ -356,9 +356,9 @@ def _gemm_launch(lib, dtype_code, activation, a, b, c, entry, configuration, dev
     ak, bk, ck = _readable(a, keep, before), _readable(b, keep, before), _writable(c, keep, after)
     m, k = a.shape
     n = b.shape[1]
-    args = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk), _row_stride(ck))
+    args = product = (ak.data_ptr(), bk.data_ptr(), ck.data_ptr(), m, n, k, _row_stride(ak), _row_stride(bk), _row_stride(ck))
     facts = (("m", m), ("n", n), ("k", k)) + configuration
-    op = OP_GEMM_BF16 if entry == "intent_hip_gemm_bf16" else OP_GEMM
+    resources = lambda: lib.call_resources(OP_GEMM, dtype_code, *product, activation)  # noqa: E731
     size = _split_bytes(lib, "gemm", m, n, k)
     if size:
         entry, facts = "intent_hip_gemm_ws", facts + (("workspace_bytes", size),)
@@ -369,8 +369,7 @@ def _gemm_launch(lib, dtype_code, activation, a, b, c, entry, configuration, dev
         else:
             fn, args = lib.fn["gemm"], (dtype_code, activation, *args)
         run = lambda stream: fn(*args, stream)  # noqa: E731
-    return Launch(entry, run, tuple(keep), tuple(before), tuple(after), facts,
-                  lambda: lib.kernel_resources(op, dtype_code, m, n))
+    return Launch(entry, run, tuple(keep), tuple(before), tuple(after), facts, resources)
 
 
 def _gemm_bf16(lib, bound, constexprs, device):
@@ -441,7 +440,8 @@ def _quantized_gemm(lib, bound, constexprs, device):
     args = (ak.data_ptr(), bk.data_ptr(), biask.data_ptr(), rk.data_ptr(), sk.data_ptr(), ok.data_ptr(), m, n, k,
             _row_stride(ak), _row_stride(bk), _row_stride(rk), _row_stride(ok))
     return Launch("intent_hip_quantized_gemm", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
-                  tuple(after), (("m", m), ("n", n), ("k", k)), lambda: lib.kernel_resources(OP_QUANTIZED_GEMM, 0, m, n))
+                  tuple(after), (("m", m), ("n", n), ("k", k)),
+                  lambda: lib.call_resources(OP_QUANTIZED_GEMM, F16, args[0], args[1], args[3], *args[5:]))
 
 
 # ------------------------------------------------------------------------------ attention

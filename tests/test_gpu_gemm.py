@@ -10,7 +10,7 @@ import torch
 import intent_amd as intent
 import oracle
 from intent_amd.examples import inputs
-from intent_amd.examples.kernels.contraction.gemm import bf16_gemm, gemm_f32
+from intent_amd.examples.kernels.contraction.gemm import Activation, bf16_gemm, gemm, gemm_f32, quantized_gemm
 from tests.gpu_util import announce, assert_16bit, bf16_tensor_bits, bf16_to_f32, to_bf16_tensor
 
 pytestmark = pytest.mark.gpu
@@ -155,6 +155,34 @@ def test_gemm_strides_and_offsets(device, m, n, k, lda, ldb, ldc, offset):
 @pytest.mark.parametrize("workspace", ["prepare", "static"])
 def test_gemm_few_rows(device, m, n, k, workspace):
     check_product(device, m, n, k, workspace)
+
+
+# (m, n, k): the kernel, its threads and its LDS, on both sides of each line of the dispatch.
+KERNELS = {(16, 72, 64): ("gemm_skinny", 512, 8 * 16 * 68 * 4), (17, 72, 64): ("gemm_skinny", 512, 8 * 32 * 68 * 4),
+           (128, 72, 64): ("gemm_skinny", 512, 8 * 64 * 68 * 4), (129, 72, 64): ("gemm_small", 256, 4 * 16384),
+           (129, 72, 65): ("gemm_small", 256, 2 * 16384), (1, 1, 1): ("gemm_small", 256, 2 * 16384),
+           (1024, 2048, 64): ("gemm_small", 256, 4 * 16384), (1025, 2048, 64): ("gemm_small", 512, 4 * 32768),
+           (2048, 2048, 64): ("gemm_small", 512, 4 * 32768), (2049, 2048, 64): ("gemm_small", 256, 2 * 32768),
+           (4096, 2048, 8): ("gemm_small", 256, 2 * 32768), (4097, 2048, 8): ("gemm_mfma", 512, 5 * 32768),
+           (4097, 2048, 64): ("gemm_mfma", 512, 5 * 32768), (4097, 2049, 64): ("gemm_small", 256, 2 * 16384)}
+
+
+@pytest.mark.parametrize("m,n,k", KERNELS)
+@pytest.mark.parametrize("kind", ["bf16", "f16", "quantize"])
+def test_gemm_observes_the_kernel_that_ran(device, m, n, k, kind):
+    announce("gemm observation", m, n, k, kind)
+    dtype = torch.bfloat16 if kind == "bf16" else torch.float16
+    args = [torch.zeros(shape, dtype=dtype, device=device) for shape in ((m, k), (k, n))]
+    if kind == "quantize":
+        args += [torch.zeros(n, device=device), torch.zeros(m, n, dtype=dtype, device=device), torch.ones(n, device=device)]
+    kernel = intent.jit({"bf16": bf16_gemm, "f16": gemm, "quantize": quantized_gemm}[kind], backend="hip",
+                        **({"constexprs": {"ACTIVATION": Activation.RELU}} if kind == "f16" else {}))
+    call = kernel.prepare(*args)
+    call.launch()
+    facts = {r.name: r.value for r in call.observation.resources}
+    name, threads, lds = KERNELS[m, n, k]
+    assert call.observation.kernel == name + {"bf16": "<bf16>", "f16": "<f16>", "quantize": "<f16,quantize>"}[kind]
+    assert facts["block_threads"] == threads and facts["lds_bytes"] == lds
 
 
 def split_product(device, kind):
