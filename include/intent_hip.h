@@ -101,14 +101,15 @@ int intent_hip_device_count(int *count);
 int intent_hip_device_info(int device, struct IntentHipDeviceInfo *out);
 
 /* Facts of the kernel a call with these extents would launch (observation,
- * python/intent/runtime/diagnostics.py:23-145; python/intent/runtime/triton/cuda.py:46-57). The 16-bit products
- * (rows = m, cols = n) are described for aligned operands and a K that is a multiple of 64. */
+ * python/intent/runtime/diagnostics.py:23-145; python/intent/runtime/triton/cuda.py:46-57). The products
+ * (rows = m, cols = n) are described for aligned operands and a K of 64, in f32 for transpose_b 0. */
 int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
                                 struct IntentHipKernelResources *out);
 
 /* The same for one call, from `count` of its own arguments, where the kernel depends on more than two extents (an address
  * matters by its alignment alone and is not read):
  *   GEMM_BF16, GEMM   a, b, c, m, n, k, lda, ldb, ldc, activation
+ *   GEMM_F32          a, b, c, m, n, k, lda, ldb, ldc, transpose_b
  *   QUANTIZED_GEMM    a, b, residual, out, m, n, k, lda, ldb, ldr, ldo */
 int intent_hip_call_resources(int op, int dtype, const int64_t *facts, int count, struct IntentHipKernelResources *out);
 

@@ -130,7 +130,8 @@ extern "C" int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int6
     case INTENT_HIP_OP_GEMM_BF16: dtype = INTENT_HIP_BF16; [[fallthrough]];
     case INTENT_HIP_OP_GEMM:
       return gemm_resources(dtype, 0, nullptr, nullptr, nullptr, rows, (cols + 7) / 8 * 8, 64, 64, 64, 64, out);
-    case INTENT_HIP_OP_GEMM_F32: return gemm_f32_resources(rows, cols, out);
+    case INTENT_HIP_OP_GEMM_F32:   // aligned operands of a short K, natural B
+      return gemm_f32_resources(nullptr, nullptr, nullptr, rows, (cols + 3) / 4 * 4, 64, 64, 64, 64, 0, out);
     // cols = d, or d | dv << 16 when dv differs from d.
     case INTENT_HIP_OP_ATTENTION_FWD_F16:
       return attention_resources(INTENT_HIP_F16, rows, cols & 0xFFFF, (cols >> 16) ? (cols >> 16) : (cols & 0xFFFF),
@@ -178,6 +179,10 @@ extern "C" int intent_hip_call_resources(int op, int dtype, const int64_t *facts
       if (const int rc = takes(10)) return rc;
       return gemm_resources(dtype, static_cast<int>(f[9]), address(0), address(1), address(2), f[3], f[4], f[5], f[6], f[7],
                             f[8], out);
+    case INTENT_HIP_OP_GEMM_F32:
+      if (const int rc = takes(10)) return rc;
+      return gemm_f32_resources(address(0), address(1), address(2), f[3], f[4], f[5], f[6], f[7], f[8],
+                                static_cast<int>(f[9]), out);
     case INTENT_HIP_OP_QUANTIZED_GEMM:
       if (const int rc = takes(11)) return rc;
       return quantized_gemm_resources(address(0), address(1), address(2), address(3), f[4], f[5], f[6], f[7], f[8], f[9],

@@ -37,7 +37,8 @@ int softmax_fwd_resources(int dtype, int64_t rows, int64_t cols, IntentHipKernel
 int softmax_bwd_resources(int dtype, int64_t rows, int64_t cols, IntentHipKernelResources *out);
 int gemm_resources(int dtype, int activation, const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k,
                    int64_t lda, int64_t ldb, int64_t ldc, IntentHipKernelResources *out);
-int gemm_f32_resources(int64_t m, int64_t n, IntentHipKernelResources *out);
+int gemm_f32_resources(const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                       int64_t ldc, int transpose_b, IntentHipKernelResources *out);
 int gemm_i8_resources(int64_t m, int64_t n, IntentHipKernelResources *out);
 int quantized_gemm_resources(const void *a, const void *b, const void *residual, const void *out, int64_t m, int64_t n,
                              int64_t k, int64_t lda, int64_t ldb, int64_t ldr, int64_t ldo, IntentHipKernelResources *to);
@@ -50,7 +51,7 @@ int spmm_resources(int64_t features, IntentHipKernelResources *out);
 // f32 products of few output tiles (gemm_f32_few.hip); `workspace` may be null (one workgroup per tile).
 bool gemm_f32_few_applies(int64_t m, int64_t n);
 size_t gemm_f32_few_bytes(int64_t m, int64_t n, int64_t k);
-int gemm_f32_few_resources(int64_t m, int64_t n, IntentHipKernelResources *out);
+int gemm_f32_few_resources(int64_t m, int64_t n, int64_t k, int transpose_b, IntentHipKernelResources *out);
 int launch_gemm_f32_few(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb,
                         int64_t ldc, int transpose_b, void *workspace, size_t workspace_bytes, hipStream_t s);
 

@@ -167,9 +167,24 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_mfma(const float *__restric
 
 }  // namespace
 
-int gemm_f32_resources(int64_t m, int64_t n, IntentHipKernelResources *out) {
-  if (gemm_f32_few_applies(m, n)) return gemm_f32_few_resources(m, n, out);
-  return describe_kernel(reinterpret_cast<const void *>(&gemm_f32_mfma<false>), "gemm_f32_mfma", kThreads, out);
+namespace {
+
+// The 128 x 128 kernel, or (false) that of gemm_f32_few.hip.
+bool large(const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+           int64_t ldc, int transpose_b) {
+  const bool vec = k % 4 == 0 && (transpose_b || n % 4 == 0) && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
+                   aligned(a, 16) && aligned(b, 16) && aligned(c, 16);
+  return vec && !gemm_f32_few_applies(m, n);
+}
+
+}  // namespace
+
+int gemm_f32_resources(const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                       int64_t ldc, int transpose_b, IntentHipKernelResources *out) {
+  if (!large(a, b, c, m, n, k, lda, ldb, ldc, transpose_b)) return gemm_f32_few_resources(m, n, k, transpose_b, out);
+  return describe_kernel(transpose_b ? reinterpret_cast<const void *>(&gemm_f32_mfma<true>)
+                                     : reinterpret_cast<const void *>(&gemm_f32_mfma<false>),
+                         "gemm_f32_mfma", kThreads, out);
 }
 
 }  // namespace intent_hip
@@ -203,12 +218,10 @@ extern "C" int intent_hip_gemm_f32_ws(const float *a, const float *b, float *c, 
   const int64_t b_rows = transpose_b ? n : k;
   if (lda < (m > 1 ? k : 0) || ldb < (b_rows > 1 ? b_row : 0) || ldc < (m > 1 ? n : 0))
     return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "row stride smaller than the row length");
-  const bool vec = k % 4 == 0 && (transpose_b || n % 4 == 0) && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
-                   aligned(a, 16) && aligned(b, 16) && aligned(c, 16);
   const dim3 grid(static_cast<unsigned>((n + kBN - 1) / kBN), static_cast<unsigned>((m + kBM - 1) / kBM));
   const hipStream_t s = as_stream(stream);
   const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
-  if (!vec || gemm_f32_few_applies(m, n))
+  if (!large(a, b, c, m, n, k, lda, ldb, ldc, transpose_b))
     return launch_gemm_f32_few(a, b, c, M, N, K, lda, ldb, ldc, transpose_b, workspace, workspace_bytes, s);
   if (transpose_b) gemm_f32_mfma<true><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);
   else gemm_f32_mfma<false><<<grid, dim3(kThreads), 0, s>>>(a, b, c, M, N, K, lda, ldb, ldc);

@@ -197,27 +197,13 @@ int few_splits(int64_t m, int64_t n, int64_t k) {
   return splits < 2 ? 1 : static_cast<int>(splits);
 }
 
-template <bool kTransB, int MT>
-void launch_few(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-                float *partials, int splits, hipStream_t s) {
-  const int tiles_m = (M + 16 * MT - 1) / (16 * MT), tiles_n = (N + kFewCols - 1) / kFewCols;
-  gemm_f32_few<kTransB, MT><<<tile_grid(static_cast<int64_t>(tiles_m) * tiles_n, splits), dim3(kFewWaves * 64), 0, s>>>(
-      a, b, c, M, N, K, lda, ldb, ldc, tiles_m, tiles_n, splits > 1 ? partials : nullptr);
-  if (splits > 1) {
-    const int64_t quads = static_cast<int64_t>(M) * ((N + 3) / 4);
-    gemm_f32_splits<<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, c, M, N, ldc, splits);
-  }
-}
-
 template <bool kTransB>
-void launch_few_rows(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb,
-                     int64_t ldc, float *partials, int splits, hipStream_t s) {
-  switch (few_rows(M, N, K)) {
-    case 16: return launch_few<kTransB, 1>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
-    case 32: return launch_few<kTransB, 2>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
-    default: return launch_few<kTransB, 4>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
-  }
+const void *few_kernel(int rows) {
+  return rows == 16   ? reinterpret_cast<const void *>(&gemm_f32_few<kTransB, 1>)
+         : rows == 32 ? reinterpret_cast<const void *>(&gemm_f32_few<kTransB, 2>)
+                      : reinterpret_cast<const void *>(&gemm_f32_few<kTransB, 4>);
 }
+const void *few_kernel(int rows, int transpose_b) { return transpose_b ? few_kernel<true>(rows) : few_kernel<false>(rows); }
 
 }  // namespace
 
@@ -230,22 +216,25 @@ size_t gemm_f32_few_bytes(int64_t m, int64_t n, int64_t k) {
   return splits > 1 ? static_cast<size_t>(splits) * m * ((n + 3) / 4 * 4) * sizeof(float) : 0;
 }
 
-int gemm_f32_few_resources(int64_t m, int64_t n, IntentHipKernelResources *out) {
-  const int rows = few_rows(m, n, kFewTallDepth);   // the query has no depth: a short one's
-  const void *kernel = rows == 16   ? reinterpret_cast<const void *>(&gemm_f32_few<false, 1>)
-                       : rows == 32 ? reinterpret_cast<const void *>(&gemm_f32_few<false, 2>)
-                                    : reinterpret_cast<const void *>(&gemm_f32_few<false, 4>);
-  return describe_kernel(kernel, "gemm_f32_few", kFewWaves * 64, out);
+int gemm_f32_few_resources(int64_t m, int64_t n, int64_t k, int transpose_b, IntentHipKernelResources *out) {
+  return describe_kernel(few_kernel(few_rows(m, n, k), transpose_b), "gemm_f32_few", kFewWaves * 64, out);
 }
 
 int launch_gemm_f32_few(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb,
                         int64_t ldc, int transpose_b, void *workspace, size_t workspace_bytes, hipStream_t s) {
   const bool room = workspace != nullptr && aligned(workspace, 16) && workspace_bytes >= gemm_f32_few_bytes(M, N, K);
-  const int splits = room ? few_splits(M, N, K) : 1;
-  float *partials = static_cast<float *>(workspace);
-  if (transpose_b) launch_few_rows<true>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
-  else launch_few_rows<false>(a, b, c, M, N, K, lda, ldb, ldc, partials, splits, s);
-  if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_f32_few");
+  const int splits = room ? few_splits(M, N, K) : 1, rows = few_rows(M, N, K);
+  float *partials = splits > 1 ? static_cast<float *>(workspace) : nullptr;
+  int tiles_m = (M + rows - 1) / rows, tiles_n = (N + kFewCols - 1) / kFewCols;
+  void *args[] = {&a, &b, &c, &M, &N, &K, &lda, &ldb, &ldc, &tiles_m, &tiles_n, &partials};
+  if (hipLaunchKernel(few_kernel(rows, transpose_b), tile_grid(static_cast<int64_t>(tiles_m) * tiles_n, splits),
+                      dim3(kFewWaves * 64), args, 0, s) != hipSuccess)
+    return launch_status("gemm_f32_few");
+  if (splits > 1) {
+    const int64_t quads = static_cast<int64_t>(M) * ((N + 3) / 4);
+    gemm_f32_splits<<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, c, M, N, ldc, splits);
+    if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_f32_splits");
+  }
   return INTENT_HIP_OK;
 }
 

@@ -410,7 +410,7 @@ def _gemm_f32(transpose_b: bool):
             entry, facts = "intent_hip_gemm_f32_ws", facts + (("workspace_bytes", size),)
             run = _workspace_run(lib.fn["gemm_f32_ws"], args, size, device, keep)
         return Launch(entry, run, tuple(keep), tuple(before), tuple(after), facts,
-                      lambda: lib.kernel_resources(OP_GEMM_F32, F32, m, n))
+                      lambda: lib.call_resources(OP_GEMM_F32, F32, *args))
     return plan
 
 

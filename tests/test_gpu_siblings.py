@@ -192,6 +192,27 @@ def test_gemm_f32_few_tiles(device, m, n, k, workspace):
         assert (np.isnan(run(x, y).cpu().numpy()) == expected).all()
 
 
+# (m, n, k): the kernel and its LDS (a padded f32 tile of each of four waves, or two stages), on both sides of each line of
+# the dispatch.
+F32_KERNELS = {(16, 64, 64): ("gemm_f32_few", 4 * 16 * 68 * 4), (17, 64, 64): ("gemm_f32_few", 4 * 32 * 68 * 4),
+               (33, 64, 2048): ("gemm_f32_few", 4 * 32 * 68 * 4), (33, 64, 2049): ("gemm_f32_few", 4 * 64 * 68 * 4),
+               (129, 8256, 64): ("gemm_f32_few", 4 * 64 * 68 * 4), (1536, 2048, 64): ("gemm_f32_few", 4 * 64 * 68 * 4),
+               (1540, 2048, 64): ("gemm_f32_mfma", None), (1540, 2048, 65): ("gemm_f32_few", 4 * 64 * 68 * 4)}
+
+
+@pytest.mark.parametrize("m,n,k", F32_KERNELS)
+@pytest.mark.parametrize("definition", [gemm_f32, linear_f32])
+def test_gemm_f32_observes_the_kernel_that_ran(device, m, n, k, definition):
+    announce("gemm f32 observation", m, n, k)
+    b = torch.zeros((k, n) if definition is gemm_f32 else (n, k), device=device)
+    call = intent.jit(definition, backend="hip").prepare(torch.zeros(m, k, device=device), b)
+    call.launch()
+    facts = {r.name: r.value for r in call.observation.resources}
+    name, lds = F32_KERNELS[m, n, k]
+    assert call.observation.kernel == name and facts["block_threads"] == 256
+    assert facts["lds_bytes"] == lds or (lds is None and facts["lds_bytes"] not in (4 * r * 68 * 4 for r in (16, 32, 64)))
+
+
 def test_gemm_f32_longest_extents(device):
     """More row blocks than workgroups fit one axis of a launch (2^32 threads)."""
     m = (1 << 30) - 1
