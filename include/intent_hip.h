@@ -102,7 +102,8 @@ int intent_hip_device_info(int device, struct IntentHipDeviceInfo *out);
 
 /* Facts of the kernel a call with these extents would launch (observation,
  * python/intent/runtime/diagnostics.py:23-145; python/intent/runtime/triton/cuda.py:46-57). The products
- * (rows = m, cols = n) are described for aligned operands and a K of 64, in f32 for transpose_b 0. */
+ * (rows = m, cols = n) are described for aligned operands and a K of 64, in f32 for transpose_b 0; the paged decode for more than
+ * 256 workgroups. */
 int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
                                 struct IntentHipKernelResources *out);
 
@@ -110,7 +111,8 @@ int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
  * matters by its alignment alone and is not read):
  *   GEMM_BF16, GEMM   a, b, c, m, n, k, lda, ldb, ldc, activation
  *   GEMM_F32          a, b, c, m, n, k, lda, ldb, ldc, transpose_b
- *   QUANTIZED_GEMM    a, b, residual, out, m, n, k, lda, ldb, ldr, ldo */
+ *   QUANTIZED_GEMM    a, b, residual, out, m, n, k, lda, ldb, ldr, ldo
+ *   PAGED_DECODE_PARTIALS  batch, kv_heads, head_group, d, positions, ps, splits */
 int intent_hip_call_resources(int op, int dtype, const int64_t *facts, int count, struct IntentHipKernelResources *out);
 
 /* Row softmax forward, y[r,:] = softmax(x[r,:]).

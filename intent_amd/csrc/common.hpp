@@ -46,6 +46,8 @@ int attention_resources(int dtype, int64_t sq, int64_t d, int64_t dv, int mode, 
 int spmv_resources(int64_t rows, int64_t nnz, IntentHipKernelResources *out);
 int attention_bwd_resources(int64_t which, int64_t rows, int64_t d, IntentHipKernelResources *out);
 int decode_resources(int64_t which, int64_t d, int64_t group, IntentHipKernelResources *out);
+int paged_decode_resources(int64_t batch, int64_t kv_heads, int64_t group, int64_t d, int64_t positions, int64_t ps,
+                           int64_t splits, IntentHipKernelResources *out);
 int spmm_resources(int64_t features, IntentHipKernelResources *out);
 
 // f32 products of few output tiles (gemm_f32_few.hip); `workspace` may be null (one workgroup per tile).

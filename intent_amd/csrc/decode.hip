@@ -547,6 +547,14 @@ const void *variant_kernel(int variant, int64_t d, int64_t group, bool many, cha
   }
 }
 
+// Paged jobs that more waves share: up to one workgroup per CU, and more than one chunk per wave of a job on average
+// (B8 HQ32 HK8 D128, 8191 tokens in 4 splits 103 -> 54 us; B4 HQ8 HK2 D64, 3783 tokens unsplit 120 -> 45).
+bool paged_many(int64_t batch, int64_t kv_heads, int64_t positions, int64_t ps, int64_t splits) {
+  return batch * splits * kv_heads <= 256 && positions * ps > kWaves * kChunk * batch * splits;
+}
+
+int partials_threads(int64_t group, bool many) { return (many ? many_waves(static_cast<int>(group)) : kWaves) * 64; }
+
 // which: 0 paged partials, 1 split-K merge, 2 grouped bf16 partials, 3 continuous partials,
 // 4 packed (sink) partials, 5 decode_merge.
 int decode_resources(int64_t which, int64_t d, int64_t group, IntentHipKernelResources *out) {
@@ -561,7 +569,16 @@ int decode_resources(int64_t which, int64_t d, int64_t group, IntentHipKernelRes
   char name[64];
   const int variant = which == 0 ? kVariantPaged : static_cast<int>(which) - 1;
   const void *kernel = variant_kernel(variant, d, group, false, name, sizeof name);
-  return describe_kernel(kernel, name, kWaves * 64, out);
+  return describe_kernel(kernel, name, partials_threads(group, false), out);
+}
+
+int paged_decode_resources(int64_t batch, int64_t kv_heads, int64_t group, int64_t d, int64_t positions, int64_t ps,
+                           int64_t splits, IntentHipKernelResources *out) {
+  if (d != 64 && d != 128) return fail(INTENT_HIP_ERR_UNSUPPORTED, "decode kernels take D = 64 or 128");
+  char name[64];
+  const bool many = paged_many(batch, kv_heads, positions, ps, splits);
+  const void *kernel = variant_kernel(kVariantPaged, d, group, many, name, sizeof name);
+  return describe_kernel(kernel, name, partials_threads(group, many), out);
 }
 
 // Splits of a dense or packed decode: enough (batch, key head, split) workgroups to fill the chip
@@ -592,13 +609,12 @@ int launch_partials(int variant, int64_t d, const uint16_t *Q, const uint16_t *K
                     const DecodeGeometry &g, float scale, void *stream, bool many = false) {
   char name[64];
   const void *kernel = variant_kernel(variant, d, group, many, name, sizeof name);
-  const int waves = many ? many_waves(static_cast<int>(group)) : kWaves;
   int kv = static_cast<int>(kv_heads), grp = static_cast<int>(group), spl = static_cast<int>(splits);
   DecodeSource s = src;
   DecodeTarget t = dst;
   DecodeGeometry geometry = g;
   void *args[] = {&Q, &K, &V, &kv, &grp, &spl, &s, &t, &geometry, &scale};
-  const hipError_t rc = hipLaunchKernel(kernel, dim3(static_cast<unsigned>(blocks)), dim3(waves * 64), args, 0,
+  const hipError_t rc = hipLaunchKernel(kernel, dim3(static_cast<unsigned>(blocks)), dim3(partials_threads(group, many)), args, 0,
                                         as_stream(stream));
   if (rc != hipSuccess) return launch_status(name);
   return INTENT_HIP_OK;
@@ -667,10 +683,8 @@ extern "C" int intent_hip_paged_decode_partials(const void *q, const void *key_c
   DecodeTarget dst{};
   dst.lse = partial_lse;
   dst.out = partial_output;
-  // Up to one workgroup per CU, and more than one chunk per wave of a job on average: more waves share the job's chunks
-  // (B8 HQ32 HK8 D128, 8191 tokens in 4 splits 103 -> 54 us; B4 HQ8 HK2 D64, 3783 tokens unsplit 120 -> 45).
-  const bool many = blocks <= 256 && positions * ps > kWaves * kChunk * batch * splits;
-  return launch_partials(kVariantPaged, d, Q, K, V, kv_heads, head_group, splits, blocks, src, dst, g, scale, stream, many);
+  return launch_partials(kVariantPaged, d, Q, K, V, kv_heads, head_group, splits, blocks, src, dst, g, scale, stream,
+                         paged_many(batch, kv_heads, positions, ps, splits));
 }
 
 extern "C" int intent_hip_splitk_reduce_f32_to_f16(const float *partial, const float *lse, void *out, int64_t batch,

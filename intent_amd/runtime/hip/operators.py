@@ -755,7 +755,8 @@ def _paged_decode_partials(lib, bound, constexprs, device):
                   tuple(after),
                   (("batch", batch), ("q_heads", q_heads), ("kv_heads", kv_heads), ("head_group", group),
                    ("d", d), ("pages", pages), ("ps", ps), ("page_size", page_size), ("splits", splits)),
-                  lambda: lib.kernel_resources(OP_PAGED_DECODE_PARTIALS, F16, group, d))
+                  lambda: lib.call_resources(OP_PAGED_DECODE_PARTIALS, F16, batch, kv_heads, group, d,
+                                             page_indices.shape[0], ps, splits))
 
 
 def _grouped_decode_partials(lib, bound, constexprs, device):

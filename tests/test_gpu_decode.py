@@ -133,6 +133,28 @@ def test_paged_decode_partials_match_oracle(device, name):
     check_partials(lse.cpu().numpy(), out.cpu().numpy(), want_lse, want_out)
 
 
+@pytest.mark.parametrize("group,many_threads", [(4, 1024), (8, 512), (16, 512)])
+def test_paged_decode_observes_the_kernel_that_ran(device, group, many_threads):
+    """Up to 256 jobs of more than 256 tokens on average have more waves each than others, and the observation says so."""
+    announce("paged decode observation", group)
+    kernel = jit(paged_gqa_decode_partials, constexprs={"PAGE_SIZE": 64, "HEAD_GROUP": group, "SPLITS": 2})
+
+    def observed(batch, pages):
+        arrays = inputs.paged_decode(seed=group, batch=batch, query_heads=2 * group, kv_heads=2, dim=64, page_size=64,
+                                     lengths=(64 * pages,) * batch, splits=2, shuffle=True)
+        call = kernel.prepare(*(t(a, device) for a in arrays), 0.125)
+        call.launch()
+        facts = {r.name: r.value for r in call.observation.resources}
+        assert call.observation.kernel == f"paged_decode_partials<64,{group}>"
+        return facts["block_threads"], facts["lds_bytes"]
+
+    few, lds = observed(2, 8)                      # 256 tokens per job
+    many, many_lds = observed(2, 9)
+    assert (few, many) == (256, many_threads) and lds < many_lds
+    assert observed(64, 9) == (many, many_lds)     # 256 workgroups
+    assert observed(65, 9) == (few, lds)
+
+
 @pytest.mark.parametrize("shape", [(8, 32, 16, 128), (2, 3, 1, 64), (1, 5, 7, 200), (3, 2, 40, 96)])
 def test_splitk_reduce_matches_oracle(device, shape):
     announce("splitk reduce", shape)
