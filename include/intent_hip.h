@@ -103,7 +103,7 @@ int intent_hip_device_info(int device, struct IntentHipDeviceInfo *out);
 /* Facts of the kernel a call with these extents would launch (observation,
  * python/intent/runtime/diagnostics.py:23-145; python/intent/runtime/triton/cuda.py:46-57). The products
  * (rows = m, cols = n) are described for aligned operands and a K of 64, in f32 for transpose_b 0; the paged decode for more than
- * 256 workgroups. */
+ * 256 workgroups; dK/dV for the whole walk. */
 int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
                                 struct IntentHipKernelResources *out);
 
@@ -112,6 +112,8 @@ int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
  *   GEMM_BF16, GEMM   a, b, c, m, n, k, lda, ldb, ldc, activation
  *   GEMM_F32          a, b, c, m, n, k, lda, ldb, ldc, transpose_b
  *   QUANTIZED_GEMM    a, b, residual, out, m, n, k, lda, ldb, ldr, ldo
+ *   ATTENTION_BWD_DKDV     batch, q_heads, head_group, sq, sk, d, causal, whether it has a workspace of the size it names
+ *                          (of the kernels of one call the first, not the fold)
  *   PAGED_DECODE_PARTIALS  batch, kv_heads, head_group, d, positions, ps, splits */
 int intent_hip_call_resources(int op, int dtype, const int64_t *facts, int count, struct IntentHipKernelResources *out);
 

@@ -187,6 +187,9 @@ extern "C" int intent_hip_call_resources(int op, int dtype, const int64_t *facts
       if (const int rc = takes(11)) return rc;
       return quantized_gemm_resources(address(0), address(1), address(2), address(3), f[4], f[5], f[6], f[7], f[8], f[9],
                                       f[10], out);
+    case INTENT_HIP_OP_ATTENTION_BWD_DKDV:
+      if (const int rc = takes(8)) return rc;
+      return attention_bwd_dkdv_resources(f[0], f[1], f[2], f[3], f[4], f[5], f[6] != 0, f[7] != 0, out);
     case INTENT_HIP_OP_PAGED_DECODE_PARTIALS:
       if (const int rc = takes(7)) return rc;
       return paged_decode_resources(f[0], f[1], f[2], f[3], f[4], f[5], f[6], out);

@@ -32,6 +32,8 @@
 //     dK and dV together.
 //   * Rows past the end of a tensor read its last row (finite data that the mask excludes).
 //     Causal work is skipped per wave where no pair of a tile is valid.
+#include <stdio.h>
+
 #include "common.hpp"
 
 namespace intent_hip {
@@ -728,9 +730,25 @@ __global__ __launch_bounds__(kThreads) void attention_bwd_dkdv_reduce(const floa
 
 namespace intent_hip {
 
+namespace {
+
+// dK/dV in parts or whole; the wide form launches dK and dV apart, and dK is described.
+template <int D>
+int dkdv_resources(bool wide, bool parts, IntentHipKernelResources *out) {
+  const void *kernel = wide ? parts ? reinterpret_cast<const void *>(&attention_bwd_dkdv<D, true, kOnlyDk, 8>)
+                                    : reinterpret_cast<const void *>(&attention_bwd_dkdv<D, false, kOnlyDk, 8>)
+                       : parts ? reinterpret_cast<const void *>(&attention_bwd_dkdv<D, true, kBoth, 4>)
+                               : reinterpret_cast<const void *>(&attention_bwd_dkdv<D, false, kBoth, 4>);
+  char name[64];
+  snprintf(name, sizeof name, "%s<%d,%d%s>", wide ? "attention_bwd_dk" : "attention_bwd_dkdv", D, wide ? 8 : 4,
+           parts ? ",parts" : "");
+  return describe_kernel(kernel, name, wide ? 512 : kThreads, out);
+}
+
+}  // namespace
+
 // rows: batch x heads x sequence of the call (query heads and queries for dQ, key heads and keys
-// for dK/dV); it selects the variant as the launch does. Wide dK/dV launches two kernels; the
-// first (dK) is described.
+// for dK/dV); it selects the variant as the launch does, of dK/dV the whole walk.
 int attention_bwd_resources(int64_t which, int64_t rows, int64_t d, IntentHipKernelResources *out) {
   const bool d64 = d == 64, wide = rows >= kWideRows;
   const auto describe = [out](const void *kernel, const char *name, int threads) {
@@ -748,16 +766,7 @@ int attention_bwd_resources(int64_t which, int64_t rows, int64_t d, IntentHipKer
       return d64 ? describe(reinterpret_cast<const void *>(&attention_bwd_dq<64, 4>), "attention_bwd_dq<64,4>", kThreads)
                  : describe(reinterpret_cast<const void *>(&attention_bwd_dq<128, 4>), "attention_bwd_dq<128,4>",
                             kThreads);
-    default:
-      if (wide)
-        return d64 ? describe(reinterpret_cast<const void *>(&attention_bwd_dkdv<64, false, kOnlyDk, 8>),
-                              "attention_bwd_dk<64,8>", 512)
-                   : describe(reinterpret_cast<const void *>(&attention_bwd_dkdv<128, false, kOnlyDk, 8>),
-                              "attention_bwd_dk<128,8>", 512);
-      return d64 ? describe(reinterpret_cast<const void *>(&attention_bwd_dkdv<64, false, kBoth, 4>),
-                            "attention_bwd_dkdv<64,4>", kThreads)
-                 : describe(reinterpret_cast<const void *>(&attention_bwd_dkdv<128, false, kBoth, 4>),
-                            "attention_bwd_dkdv<128,4>", kThreads);
+    default: return d64 ? dkdv_resources<64>(wide, false, out) : dkdv_resources<128>(wide, false, out);
   }
 }
 
@@ -907,6 +916,22 @@ DkdvPlan dkdv_plan(int64_t batch, int64_t q_heads, int64_t head_group, int64_t s
 int64_t dkdv_workspace(const DkdvPlan &plan, int64_t batch, int64_t kv_heads, int64_t sk, int64_t d) {
   return 2 * plan.parts() * batch * kv_heads * sk * d * static_cast<int64_t>(sizeof(float));
 }
+
+}  // namespace
+
+namespace intent_hip {
+
+int attention_bwd_dkdv_resources(int64_t batch, int64_t q_heads, int64_t head_group, int64_t sq, int64_t sk, int64_t d,
+                                 bool causal, bool workspace, IntentHipKernelResources *out) {
+  if (head_group < 1) return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "HEAD_GROUP must be positive");
+  const DkdvPlan plan = dkdv_plan(batch, q_heads, head_group, sq, sk, causal);
+  const bool parts = workspace && plan.parts() > 0;
+  return d == 64 ? dkdv_resources<64>(plan.wide, parts, out) : dkdv_resources<128>(plan.wide, parts, out);
+}
+
+}  // namespace intent_hip
+
+namespace {
 
 // attention_bwd_dq<D, kW> over every (batch, query head), block of 32 kW queries and key range;
 // with splits > 1 the partial sums in `partial` are then folded by attention_bwd_dq_reduce.

@@ -45,6 +45,8 @@ int quantized_gemm_resources(const void *a, const void *b, const void *residual,
 int attention_resources(int dtype, int64_t sq, int64_t d, int64_t dv, int mode, IntentHipKernelResources *out);
 int spmv_resources(int64_t rows, int64_t nnz, IntentHipKernelResources *out);
 int attention_bwd_resources(int64_t which, int64_t rows, int64_t d, IntentHipKernelResources *out);
+int attention_bwd_dkdv_resources(int64_t batch, int64_t q_heads, int64_t head_group, int64_t sq, int64_t sk, int64_t d,
+                                 bool causal, bool workspace, IntentHipKernelResources *out);
 int decode_resources(int64_t which, int64_t d, int64_t group, IntentHipKernelResources *out);
 int paged_decode_resources(int64_t batch, int64_t kv_heads, int64_t group, int64_t d, int64_t positions, int64_t ps,
                            int64_t splits, IntentHipKernelResources *out);

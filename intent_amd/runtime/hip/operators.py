@@ -704,12 +704,12 @@ def _attention_bwd(kind):
         else:
             run = lambda stream: fn(*args, None, 0, stream)  # noqa: E731
         configuration += (("split", split), ("workspace_bytes", size.value if split else 0))
-        op = OP_ATTENTION_BWD_DQ if kind == "dq" else OP_ATTENTION_BWD_DKDV
-        # The kernel variant depends on the rows of the call: batch x query heads x queries for dQ,
-        # batch x key heads x keys for dK/dV.
-        rows = batch * q_heads * sq if kind == "dq" else batch * (q_heads // group) * sk
+        if kind == "dq":   # the kernel variant depends on the rows of the call
+            resources = lambda: lib.kernel_resources(OP_ATTENTION_BWD_DQ, F16, batch * q_heads * sq, d)  # noqa: E731
+        else:
+            resources = lambda: lib.call_resources(OP_ATTENTION_BWD_DKDV, F16, *extents, int(causal), split)  # noqa: E731
         return Launch(f"intent_hip_attention_bwd_{kind}", run, tuple(keep), tuple(before), tuple(after), configuration,
-                      lambda: lib.kernel_resources(op, F16, rows, d), candidates)
+                      resources, candidates)
     return plan
 
 

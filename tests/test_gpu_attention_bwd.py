@@ -233,6 +233,28 @@ def test_dkdv_without_a_mask_takes_no_workspace(device, causal):
     assert [a.eligible for a in others] == [causal]
 
 
+@pytest.mark.parametrize("shape,causal,workspace,kernel", [
+    ((1, 4, 2, 300, 300, 64), False, "prepare", "attention_bwd_dkdv<64,4,parts>"),
+    ((1, 4, 2, 300, 300, 64), True, "static", "attention_bwd_dkdv<64,4>"),
+    ((64, 16, 2, 520, 256, 64), True, "prepare", "attention_bwd_dkdv<64,4,parts>"),
+    ((64, 16, 2, 520, 256, 64), False, "prepare", "attention_bwd_dkdv<64,4>"),
+    ((64, 16, 2, 504, 256, 64), True, "prepare", "attention_bwd_dkdv<64,4>"),
+    ((128, 4, 2, 2050, 256, 128), True, "prepare", "attention_bwd_dk<128,8,parts>"),
+    ((128, 4, 2, 2050, 256, 128), False, "prepare", "attention_bwd_dk<128,8>")])
+def test_dkdv_observes_the_kernel_that_ran(device, shape, causal, workspace, kernel):
+    from intent_amd.examples.kernels.backward.attention import attention_backward_dkdv
+
+    batch, hq, hk, sq, sk, d = shape
+    announce("dK/dV observation", shape, causal, workspace)
+    q, k = (torch.zeros(batch, h, n, d, dtype=torch.float16, device=device) for h, n in ((hq, sq), (hk, sk)))
+    rows = torch.zeros(batch, hq, sq, device=device)
+    call = intent.jit(attention_backward_dkdv, backend="hip", constexprs={"HEAD_GROUP": hq // hk, "CAUSAL": causal},
+                      backend_options={"workspace": workspace}).prepare(q, k, k.clone(), q.clone(), rows, rows.clone(), 0.125)
+    call.launch()
+    assert call.observation.kernel == kernel
+    assert {r.name: r.value for r in call.observation.resources}["block_threads"] == (512 if "8" in kernel.split(",")[1] else 256)
+
+
 @pytest.mark.parametrize("shape", [(1, 4, 2, 300, 300, 64), (64, 16, 2, 520, 256, 64)])
 def test_dkdv_workspace_on_another_stream_and_in_a_graph(device, shape):
     """A prepared call launched on another stream and captured in a graph, then dropped before that stream comes to it: the
