@@ -101,7 +101,8 @@ int intent_hip_device_count(int *count);
 int intent_hip_device_info(int device, struct IntentHipDeviceInfo *out);
 
 /* Facts of the kernel a call with these extents would launch (observation,
- * python/intent/runtime/diagnostics.py:23-145; python/intent/runtime/triton/cuda.py:46-57). The products
+ * python/intent/runtime/diagnostics.py:23-145; python/intent/runtime/triton/cuda.py:46-57). Softmax is
+ * described for aligned contiguous rows. The products
  * (rows = m, cols = n) are described for aligned operands and a K of 64, in f32 for transpose_b 0; the paged decode for more than
  * 256 workgroups; dK/dV for the whole walk. */
 int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
@@ -109,6 +110,8 @@ int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
 
 /* The same for one call, from `count` of its own arguments, where the kernel depends on more than two extents (an address
  * matters by its alignment alone and is not read):
+ *   SOFTMAX_FWD       x, y, rows, cols, x_row_stride, y_row_stride
+ *   SOFTMAX_BWD       p, dy, dx, rows, cols, p_row_stride, dy_row_stride, dx_row_stride
  *   GEMM_BF16, GEMM   a, b, c, m, n, k, lda, ldb, ldc, activation
  *   GEMM_F32          a, b, c, m, n, k, lda, ldb, ldc, transpose_b
  *   QUANTIZED_GEMM    a, b, residual, out, m, n, k, lda, ldb, ldr, ldo

@@ -778,26 +778,25 @@ int launch_bwd(const void *p, const void *dy, void *dx, int64_t rows, int64_t co
 
 }  // namespace
 
-int softmax_fwd_resources(int dtype, int64_t rows, int64_t cols, IntentHipKernelResources *out) {
-  (void)rows;
-  // Resources of the 16-byte-aligned, contiguous variant for this row length.
+int softmax_fwd_resources(int dtype, const void *x, const void *y, int64_t cols, int64_t xs, int64_t ys,
+                          IntentHipKernelResources *out) {
   Variant v;
   switch (dtype) {
-    case INTENT_HIP_F32: v = select_fwd<float>(nullptr, nullptr, cols, cols, cols); break;
-    case INTENT_HIP_F16: v = select_fwd<f16_t>(nullptr, nullptr, cols, cols, cols); break;
-    case INTENT_HIP_BF16: v = select_fwd<bf16_t>(nullptr, nullptr, cols, cols, cols); break;
+    case INTENT_HIP_F32: v = select_fwd<float>(x, y, cols, xs, ys); break;
+    case INTENT_HIP_F16: v = select_fwd<f16_t>(x, y, cols, xs, ys); break;
+    case INTENT_HIP_BF16: v = select_fwd<bf16_t>(x, y, cols, xs, ys); break;
     default: return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "unknown dtype code %d", dtype);
   }
   return describe_kernel(v.kernel, v.name, v.block, out);
 }
 
-int softmax_bwd_resources(int dtype, int64_t rows, int64_t cols, IntentHipKernelResources *out) {
-  (void)rows;
+int softmax_bwd_resources(int dtype, const void *p, const void *dy, const void *dx, int64_t cols, int64_t ps, int64_t dys,
+                          int64_t dxs, IntentHipKernelResources *out) {
   Variant v;
   switch (dtype) {
-    case INTENT_HIP_F32: v = select_bwd<float>(nullptr, nullptr, nullptr, cols, cols, cols, cols); break;
-    case INTENT_HIP_F16: v = select_bwd<f16_t>(nullptr, nullptr, nullptr, cols, cols, cols, cols); break;
-    case INTENT_HIP_BF16: v = select_bwd<bf16_t>(nullptr, nullptr, nullptr, cols, cols, cols, cols); break;
+    case INTENT_HIP_F32: v = select_bwd<float>(p, dy, dx, cols, ps, dys, dxs); break;
+    case INTENT_HIP_F16: v = select_bwd<f16_t>(p, dy, dx, cols, ps, dys, dxs); break;
+    case INTENT_HIP_BF16: v = select_bwd<bf16_t>(p, dy, dx, cols, ps, dys, dxs); break;
     default: return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "unknown dtype code %d", dtype);
   }
   return describe_kernel(v.kernel, v.name, v.block, out);

@@ -321,7 +321,7 @@ def _softmax_fwd(dtype_code):
         args = (dtype_code, xk.data_ptr(), yk.data_ptr(), rows, cols, _row_stride(xk), _row_stride(yk))
         return Launch("intent_hip_softmax_fwd", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
                       tuple(after), (("rows", rows), ("cols", cols)),
-                      lambda: lib.kernel_resources(OP_SOFTMAX_FWD, dtype_code, rows, cols))
+                      lambda: lib.call_resources(OP_SOFTMAX_FWD, *args))
     return plan
 
 
@@ -336,7 +336,7 @@ def _softmax_bwd(dtype_code):
                 _row_stride(gk), _row_stride(dk))
         return Launch("intent_hip_softmax_bwd", lambda stream: fn(*args, stream), tuple(keep), tuple(before),
                       tuple(after), (("rows", rows), ("cols", cols)),
-                      lambda: lib.kernel_resources(OP_SOFTMAX_BWD, dtype_code, rows, cols))
+                      lambda: lib.call_resources(OP_SOFTMAX_BWD, *args))
     return plan
 
 

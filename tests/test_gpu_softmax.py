@@ -254,6 +254,23 @@ def test_softmax_workgroup_rows(device, rows, cols, kind):
             assert untouched(d_base, dv)
 
 
+@pytest.mark.parametrize("cols,pad,fwd,bwd", [
+    (1024, 0, ("softmax_fwd_pipe", 256), ("softmax_bwd_wave", 128)), (1024, 3, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)),
+    (255, 0, ("softmax_fwd_wave", 128), ("softmax_bwd_wave", 128)), (257, 0, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)),
+    (4104, 0, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)), (40000, 1, ("softmax_fwd_block", 1024), ("softmax_bwd_block", 1024)),
+    (140000, 0, ("softmax_fwd_stream", 1024), ("softmax_bwd_stream", 1024))])
+def test_softmax_observes_the_kernel_that_ran(device, cols, pad, fwd, bwd):
+    """Rows at a stride that leaves them unaligned are described as the kernel that takes them."""
+    announce("softmax observation", cols, pad)
+    view = lambda: torch.zeros(3, cols + pad, dtype=torch.float16, device=device)[:, :cols]  # noqa: E731
+    x, y, d = view(), view(), view()
+    for kernel, args, out, want in ((stable_softmax_f16, (x,), y, fwd), (softmax_backward_f16, (x, y), d, bwd)):
+        call = intent.jit(kernel, backend="hip").prepare(*args, outputs=(out,))
+        call.launch()
+        facts = {r.name: r.value for r in call.observation.resources}
+        assert (call.observation.kernel, facts["block_threads"]) == want
+
+
 def test_softmax_longest_row(device):
     """2^31 - 1 columns, the most an entry takes: the last 16-byte chunk reaches past 2^31 elements, and what follows the row
     in the result's buffer stays as it was."""
