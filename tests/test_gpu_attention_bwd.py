@@ -453,6 +453,45 @@ def test_excluded_pairs_with_nonfinite_operands_match_oracle(device, shape, caus
         close(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("shape", [(64, 16, 2, 520, 256, 64), (43, 6, 2, 1400, 300, 128),     # 4-wave: heads, query ranges
+                                   (128, 4, 2, 2050, 256, 64), (128, 2, 2, 4100, 256, 128)])  # 8-wave dK and dV
+def test_two_parts_with_nonfinite_operands_match_oracle(device, shape):
+    """dK and dV in two parts with NaN and infinities in rows that the mask excludes for some pairs, and in the last tile, which
+    ends past the queries: the batch elements that hold them against the oracle, and every element
+    non-finite in the same places as the whole walk's."""
+    from intent_amd.examples.kernels.backward.attention import attention_backward_dkdv
+
+    batch, hq, hk, sq, sk, d = shape
+    announce("dK/dV in two parts, non-finite rows", shape)
+    rng = np.random.default_rng(sum(shape))
+    q, do = inputs.normal(rng, (batch, hq, sq, d), "f16"), inputs.normal(rng, (batch, hq, sq, d), "f16")
+    k, v = inputs.normal(rng, (batch, hk, sk, d), "f16"), inputs.normal(rng, (batch, hk, sk, d), "f16")
+    lse = (rng.standard_normal((batch, hq, sq)) * 0.5 + np.log(sk)).astype(np.float32)
+    delta = rng.standard_normal((batch, hq, sq)).astype(np.float32)
+    plant_nonfinite(q, k, v, do, seed=sum(shape))
+    q[0, hq // 2, 129, 3], do[0, 1, sq - 1, 5], q[batch - 1, hq - 1, sq - 2, 1] = np.nan, np.inf, -np.inf
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    scale = float(np.float32(1 / np.sqrt(d)))
+    args = (*map(t, (q, k, v, do, lse, delta)), scale)
+
+    def run(workspace):
+        kernel = intent.jit(attention_backward_dkdv, backend="hip", constexprs={"HEAD_GROUP": hq // hk, "CAUSAL": True},
+                            backend_options={"workspace": workspace})
+        call = kernel.prepare(*args)
+        assert dict(call.inspect_configurations()[0].configuration)["split"] == int(workspace == "prepare")
+        call.launch()
+        return [g.cpu().numpy() for g in call.result()]
+
+    parts, whole = run("prepare"), run("static")
+    for got, other in zip(parts, whole):
+        assert (np.isfinite(got) == np.isfinite(other)).all() and np.isfinite(got).mean() > 0.9
+    for b in (0, batch - 1):
+        at = slice(b, b + 1)
+        want = oracle.attention_bwd_dkdv(q[at], k[at], v[at], do[at], lse[at], delta[at], scale, True, head_group=hq // hk)
+        for got, expected in zip(parts, want):
+            close(got[at], expected.astype(np.float64))
+
+
 def test_benchmarked_shape_matches_autograd_and_oracle(device):
     """The benchmarked shape, B4 HQ32 HK8 S4096 D128 causal: all of dQ, dK, dV against float32
     autograd of grouped-head attention on the GPU (o and lse from the same float32 forward), and

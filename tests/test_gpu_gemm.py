@@ -157,6 +157,32 @@ def test_gemm_few_rows(device, m, n, k, workspace):
     check_product(device, m, n, k, workspace)
 
 
+# f16 on every kernel (few rows, 64 x 64 tiles, both with K divided; 128 x 128 with four and two stages; 256 x 256; through
+# registers, with K divided too), the activation applied after the whole sum.
+@pytest.mark.parametrize("m,n,k", [(32, 1000, 2056), (100, 72, 4104), (257, 136, 2056), (1500, 1400, 72), (2300, 2200, 40),
+                                   (3000, 3080, 40), (200, 131, 2049)])
+@pytest.mark.parametrize("activation", [Activation.NONE, Activation.RELU])
+def test_gemm_f16_kernels_and_activation(device, m, n, k, activation):
+    """Against the oracle and exact on small integers, half of whose sums are negative; NaN in the last row of A and the last column
+    of B passes the activation and stays in its own row and column."""
+    announce("gemm f16 kernels", m, n, k, activation.name)
+    kernel = intent.jit(gemm, backend="hip", constexprs={"ACTIVATION": activation})
+    call = lambda x, y: kernel.run(torch.from_numpy(x).to(device), torch.from_numpy(y).to(device)).cpu().numpy()  # noqa: E731
+    rng = np.random.default_rng(m + n + k)
+    relu = activation == Activation.RELU
+    a, b = inputs.normal(rng, (m, k), "f16"), inputs.normal(rng, (k, n), "f16")
+    got, want = call(a, b), oracle.gemm16(a, b, relu=relu)
+    assert_16bit(got, want)
+    assert (np.abs(got.view(np.int16).astype(np.int32) - want.view(np.int16).astype(np.int32))[np.abs(want) > 1e-2] <= 2).mean() > 0.999
+    ints = [rng.integers(-2, 3, shape).astype(np.float16) for shape in ((m, k), (k, n))]
+    got = call(*ints)
+    assert np.array_equal(got, oracle.gemm16(*ints, relu=relu)) and (got < 0).any() == (not relu)
+    a[m - 1, k - 1] = b[0, n - 1] = np.nan
+    expected = np.zeros((m, n), bool)
+    expected[m - 1, :] = expected[:, n - 1] = True
+    assert (np.isnan(call(a, b)) == expected).all()
+
+
 # (m, n, k): the kernel, its threads and its LDS, on both sides of each line of the dispatch.
 KERNELS = {(16, 72, 64): ("gemm_skinny", 512, 8 * 16 * 68 * 4), (17, 72, 64): ("gemm_skinny", 512, 8 * 32 * 68 * 4),
            (128, 72, 64): ("gemm_skinny", 512, 8 * 64 * 68 * 4), (129, 72, 64): ("gemm_small", 256, 4 * 16384),

@@ -192,6 +192,13 @@ def test_gemm_f32_few_tiles(device, m, n, k, workspace):
         assert (np.isnan(run(x, y).cpu().numpy()) == expected).all()
 
 
+# Above 192 tiles of 128 x 128: aligned ones, whose last row, column and K tiles are partly filled (gemm_f32_mfma), and one that
+# is not aligned (gemm_f32_few, undivided).
+@pytest.mark.parametrize("m,n,k", [(1800, 1804, 20), (1793, 1796, 36), (1801, 1803, 37), (1920, 1792, 16)])
+def test_gemm_f32_many_tiles(device, m, n, k):
+    test_gemm_f32_few_tiles(device, m, n, k, "prepare")
+
+
 # (m, n, k): the kernel and its LDS (a padded f32 tile of each of four waves, or two stages), on both sides of each line of
 # the dispatch.
 F32_KERNELS = {(16, 64, 64): ("gemm_f32_few", 4 * 16 * 68 * 4), (17, 64, 64): ("gemm_f32_few", 4 * 32 * 68 * 4),
