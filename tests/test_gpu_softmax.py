@@ -254,6 +254,28 @@ def test_softmax_workgroup_rows(device, rows, cols, kind):
             assert untouched(d_base, dv)
 
 
+# A wave's rows, a workgroup's (one to four waves' worth and more, aligned and ragged), and rows read again in each pass.
+@pytest.mark.parametrize("cols", [255, 257, 1003, 4104, 9001, 40000, 131072, 140001])
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_softmax_specials_on_every_kernel(device, cols, kind):
+    """NaN, infinities, masks of the type's lowest value and wholly masked rows: NaN where the float64 softmax is NaN (a NaN or
+    +inf in the row, or every element -inf), and its values elsewhere; a row's specials stay in the row."""
+    announce("softmax specials", cols, kind)
+    dtype = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[kind]
+    fwd = {"f32": stable_softmax, "f16": stable_softmax_f16, "bf16": chunked_softmax_bf16}[kind]
+    x = torch.randn(9, cols, generator=torch.Generator(device=device).manual_seed(cols), device=device).to(dtype)
+    lowest = torch.finfo(dtype).min
+    x[1, cols - 1], x[2, 0], x[3, :] = float("nan"), float("inf"), float("-inf")
+    x[4, ::2], x[5, 1:], x[6, :], x[7, :cols - 1] = float("-inf"), lowest, lowest, float("-inf")
+    y, want = intent.jit(fwd, backend="hip").run(x), torch.softmax(x.double(), dim=1)
+    assert bool((y.isnan() == want.isnan()).all()) and bool(y[1:4].isnan().all()) and not bool(y[4:].isnan().any())
+    got, want = (v.nan_to_num(0.0).double().cpu().numpy() for v in (y, want))
+    if kind == "f32":
+        assert_f32_rel(got, want, floor=1e-30)
+    else:
+        assert_16bit(got, want, rel=2.0 ** (-10 if kind == "f16" else -7), abs_=2.0 ** -24)
+
+
 @pytest.mark.parametrize("cols,pad,fwd,bwd", [
     (1024, 0, ("softmax_fwd_pipe", 256), ("softmax_bwd_wave", 128)), (1024, 3, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)),
     (255, 0, ("softmax_fwd_wave", 128), ("softmax_bwd_wave", 128)), (257, 0, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)),
