@@ -4,24 +4,22 @@
 // accumulator = matmul(a, b, acc_dtype=f32); c = cast(accumulator, bf16) (round to
 // nearest even). A [M,K], B [K,N], C [M,N], row-major with row strides lda/ldb/ldc.
 //
-// Design: three MFMA kernels, chosen by the shape (launch_epilogue).
+// Design: three MFMA kernels, chosen by the shape and layout (choose).
 //   * 256 x 256 tiles (gemm_mfma) for many tiles: 8 waves in 2 x 4, each wave 128 x 64 = 4 x 2 tiles of
 //     v_mfma_f32_32x32x16_bf16 (128 accumulator registers per lane, so two waves share
 //     each SIMD); A and B stream into LDS with global_load_lds (five 32 KB stages) and B fragments are read
 //     with transposing LDS reads; the two waves of a SIMD alternate between their MFMA cluster and their
-//     LDS reads (ping-pong), so the matrix pipe is fed while the other wave waits on LDS;
+//     LDS reads (ping-pong), so the matrix pipe is fed while the other wave waits on LDS. The tiles are walked in
+//     groups of 2 tile rows, column by column, in dispatch order: those resident at one time share A row
+//     panels and B column panels, across XCDs through the MALL and within each XCD through its L2;
 //   * 128 x 128 and 64 x 64 tiles (gemm_small) where 256 x 256 tiles would leave CUs idle, and for
 //     operands that the DMA does not take (odd extents, strides or addresses);
 //   * up to 128 rows (gemm_skinny): waves stream B into registers (f16 relu 32 x 14336 x 4096: 221 us in
 //     256 x 256 tiles, 28 there).
-// Tiles that reach past M or N read valid rows and columns in their place and do not store them; past
-// K (a multiple of 8 where the DMA runs) they read zeros.
-//   * the MFMA is issued as D = Bt_frag x A_frag, i.e. the transposed product, so each
-//     lane ends with 4 consecutive output columns of one output row per register
-//     quad and writes them as one 8-byte store;
-//   * 256 x 256 tiles are walked in groups of 2 tile rows, column by column, in dispatch order: the
-//     tiles resident at one time share A row panels and B column panels, across XCDs
-//     through the MALL and within each XCD through its L2.
+// Each issues the MFMA as D = Bt_frag x A_frag, i.e. the transposed product, so that a lane ends with
+// consecutive output columns of one output row and writes 4 of them as one 8-byte store. Tiles that reach past M
+// or N read valid rows and columns in their place and do not store them; past K (a multiple of 8 where the DMA runs)
+// they read zeros.
 #include <stdio.h>
 
 #include <type_traits>
@@ -86,10 +84,12 @@ template <typename E>
 __device__ __forceinline__ uint16_t f32_to_element(float v) { return __builtin_bit_cast(uint16_t, static_cast<E>(v)); }
 
 // Epilogues: quad(i, n, a, b, c, d) receives the f32 accumulators of output row i, columns n .. n+3
-// (n a multiple of 4); one(i, n, a) a single element (the general-shape kernel).
+// (n a multiple of 4); one(i, n, a) a single element (layouts that the DMA does not take). kSums: K may be divided over
+// workgroups, whose sums gemm_splits adds before the epilogue.
 // gemm / bf16_gemm: act(acc) rounded to E.
 template <typename E, int kAct>
 struct CastStore {
+  static constexpr bool kSums = true;
   uint16_t *C;
   int64_t ldc;
   __device__ __forceinline__ void quad(int i, int n, float a, float b, float c, float d) const {
@@ -105,6 +105,7 @@ struct CastStore {
 // division), v = minimum(maximum(v, -128), 127), then the cast to i8, which truncates toward
 // zero. NaN is an illegal cast input; it gives 0 here.
 struct QuantizeStore {
+  static constexpr bool kSums = false;
   const float *bias;
   const uint16_t *residual;   // f16 [M, N]
   int64_t ldr;
@@ -487,7 +488,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_skinny(const uint16_t 
       total.z += v.z;
       total.w += v.w;
     }
-    if (partials != nullptr)
+    if (Epi::kSums && partials != nullptr)
       *reinterpret_cast<float4 *>(partials + (static_cast<int64_t>(blockIdx.y) * M + m0 + row) * N + n0 + col) = total;
     else
       ep.quad(m0 + row, n0 + col, total.x, total.y, total.z, total.w);
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(128 * WN) void gemm_small(const uint16_t *__restric
   if (tile < 0) return;
   const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
 
-  // Slot p = tid + 256 i of a stage's A holds chunk (p % kRowChunks) ^ swz of row p / kRowChunks; of its B,
+  // Slot p = tid + TH i of a stage's A holds chunk (p % kRowChunks) ^ swz of row p / kRowChunks; of its B,
   // chunk (p % (BN / 8)) ^ swz of row p / (BN / 8). Rows past M and columns past N read valid
   // ones instead; their products are not stored.
   const uint16_t *a_src[T::kLoadsA], *b_src[T::kLoadsB];
@@ -713,7 +714,7 @@ __global__ __launch_bounds__(128 * WN) void gemm_small(const uint16_t *__restric
     }
   }
 
-  // acc[mt][nt][4 g + e] is row wm BM / 2 + 32 mt + frag, column wn BN / 2 + 32 nt + 8 g + 4 half + e.
+  // acc[mt][nt][4 g + e] is row wm BM / 2 + 32 mt + frag, column wn BN / WN + 32 nt + 8 g + 4 half + e.
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int i = m0 + wm * (BM / 2) + mt * 32 + frag;
@@ -724,7 +725,7 @@ __global__ __launch_bounds__(128 * WN) void gemm_small(const uint16_t *__restric
       for (int g = 0; g < 4; ++g) {
         const int n = n0 + wn * (BN / WN) + nt * 32 + 8 * g + 4 * half;
         const f32x16_t &v = acc[mt][nt];
-        if (partials != nullptr) {
+        if (Epi::kSums && partials != nullptr) {
           const int64_t width = (N + 3) & ~3;
           if (n < N)
             *reinterpret_cast<float4 *>(partials + (static_cast<int64_t>(blockIdx.y) * M + i) * width + n) =
@@ -858,13 +859,13 @@ int small_splits(int64_t m, int64_t n, int64_t k) {
   return splits < 2 ? 1 : static_cast<int>(splits);
 }
 
-template <typename E, typename Epi, bool kQuads>
+template <typename Epi, bool kQuads>
 void launch_splits(const float *partials, const Epi &ep, int m, int n, int splits, hipStream_t s) {
   const int64_t quads = static_cast<int64_t>(m) * ((n + 3) / 4);
   gemm_splits<Epi, kQuads><<<dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, s>>>(partials, ep, m, n, splits);
 }
 
-// `partials`: null, or room for splits_bytes(m, n, k).
+// `partials`: null (always without Epi::kSums), or room for splits_bytes(m, n, k).
 template <typename E, typename Epi>
 int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t m, int64_t n, int64_t k, int64_t lda,
                     int64_t ldb, bool fast, float *partials, hipStream_t s) {
@@ -881,9 +882,10 @@ int launch_epilogue(const uint16_t *A, const uint16_t *B, const Epi &ep, int64_t
   void *args[] = {&A, &B, &epilogue, &M, &N, &K, &lda, &ldb, &tiles_m, &tiles_n, &partials};
   if (hipLaunchKernel(choice.kernel, grid, dim3(choice.threads), args, 0, s) != hipSuccess)
     return launch_status(kFamilyNames[choice.family]);
-  if (splits > 1) {
-    if (fast) launch_splits<E, Epi, true>(partials, ep, M, N, splits, s);
-    else launch_splits<E, Epi, false>(partials, ep, M, N, splits, s);
+  if constexpr (Epi::kSums) {
+    if (splits == 1) return INTENT_HIP_OK;
+    if (fast) launch_splits<Epi, true>(partials, ep, M, N, splits, s);
+    else launch_splits<Epi, false>(partials, ep, M, N, splits, s);
     if (hipPeekAtLastError() != hipSuccess) return launch_status("gemm_splits");
   }
   return INTENT_HIP_OK;
