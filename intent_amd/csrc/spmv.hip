@@ -227,10 +227,11 @@ __device__ __forceinline__ void block_prefix(const Plan &plan, int block, int mi
 // folded by their lane (the loads of the thread's four rows issued together); rows of 5..127 by a
 // 16-lane group (four rows per wave at a time); medium and large rows are written to their lists
 // at the block's list offset (block_prefix), in row order.
+template <bool kFold>
 __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, const int32_t *__restrict__ col,
                                            const float *__restrict__ val, const float *__restrict__ x,
                                            float *__restrict__ y, int32_t rows, int32_t cols, int64_t nnz, Plan plan,
-                                           int block, bool fold) {
+                                           int block) {
   __shared__ int s_wave[2][4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t base = static_cast<int64_t>(block) * kBlockRows;
@@ -244,7 +245,7 @@ __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, cons
     length[k] = r < rows ? e - b : -1;
   }
   // Lane rows: all column and value loads, then all gathers, then the ordered folds.
-  if (fold) {   // a constant
+  if constexpr (kFold) {
     int32_t c[kRowsPerThread][kLaneRow];
     float v[kRowsPerThread][kLaneRow], xs[kRowsPerThread][kLaneRow];
 #pragma unroll
@@ -311,7 +312,7 @@ __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, cons
     first[1] += s_wave[1][0] + s_wave[1][1] + s_wave[1][2] + s_wave[1][3];
     __syncthreads();
   }
-  if (!fold) return;
+  if constexpr (!kFold) return;
   // Rows of 5..127 nonzeros: group g (16 lanes) takes the g-th pending row of the wave.
   const int g = lane >> 4, l16 = lane & 15;
 #pragma unroll
@@ -552,8 +553,12 @@ __global__ __launch_bounds__(256) void spmv_rows(const int32_t *__restrict__ off
     return;
   }
   const int block = static_cast<int>(blockIdx.x) - cut_groups;
-  if (kSmall && block < small_groups) rows_small(off, col, val, x, y, rows, cols, nnz, block);
-  else rows_block(off, col, val, x, y, rows, cols, nnz, plan, block - (kSmall ? small_groups : 0), !kSmall);
+  if constexpr (kSmall) {
+    if (block < small_groups) rows_small(off, col, val, x, y, rows, cols, nnz, block);
+    else rows_block<false>(off, col, val, x, y, rows, cols, nnz, plan, block - small_groups);
+  } else {
+    rows_block<true>(off, col, val, x, y, rows, cols, nnz, plan, block);
+  }
 }
 
 // Pieces of listed rows. Wave w of a workgroup takes the pieces of list rows i = k + K t for
