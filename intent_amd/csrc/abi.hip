@@ -124,8 +124,8 @@ extern "C" int intent_hip_device_info(int device, IntentHipDeviceInfo *out) {
 extern "C" int intent_hip_kernel_resources(int op, int dtype, int64_t rows, int64_t cols,
                                            IntentHipKernelResources *out) {
   switch (op) {
-    case INTENT_HIP_OP_SOFTMAX_FWD: return softmax_fwd_resources(dtype, nullptr, nullptr, cols, cols, cols, out);
-    case INTENT_HIP_OP_SOFTMAX_BWD: return softmax_bwd_resources(dtype, nullptr, nullptr, nullptr, cols, cols, cols, cols, out);
+    case INTENT_HIP_OP_SOFTMAX_FWD: return softmax_fwd_resources(dtype, nullptr, nullptr, rows, cols, cols, cols, out);
+    case INTENT_HIP_OP_SOFTMAX_BWD: return softmax_bwd_resources(dtype, nullptr, nullptr, nullptr, rows, cols, cols, cols, cols, out);
     // 16-bit products: aligned operands of a K that whole steps divide.
     case INTENT_HIP_OP_GEMM_BF16: dtype = INTENT_HIP_BF16; [[fallthrough]];
     case INTENT_HIP_OP_GEMM:
@@ -176,10 +176,10 @@ extern "C" int intent_hip_call_resources(int op, int dtype, const int64_t *facts
   switch (op) {
     case INTENT_HIP_OP_SOFTMAX_FWD:
       if (const int rc = takes(6)) return rc;
-      return softmax_fwd_resources(dtype, address(0), address(1), f[3], f[4], f[5], out);
+      return softmax_fwd_resources(dtype, address(0), address(1), f[2], f[3], f[4], f[5], out);
     case INTENT_HIP_OP_SOFTMAX_BWD:
       if (const int rc = takes(8)) return rc;
-      return softmax_bwd_resources(dtype, address(0), address(1), address(2), f[4], f[5], f[6], f[7], out);
+      return softmax_bwd_resources(dtype, address(0), address(1), address(2), f[3], f[4], f[5], f[6], f[7], out);
     case INTENT_HIP_OP_GEMM_BF16: dtype = INTENT_HIP_BF16; [[fallthrough]];
     case INTENT_HIP_OP_GEMM:
       if (const int rc = takes(10)) return rc;

@@ -33,10 +33,10 @@ int describe_kernel(const void *kernel, const char *name, int block_threads,
 
 // Kernel selection facts exported by each operator file for intent_hip_kernel_resources() and
 // intent_hip_call_resources().
-int softmax_fwd_resources(int dtype, const void *x, const void *y, int64_t cols, int64_t xs, int64_t ys,
+int softmax_fwd_resources(int dtype, const void *x, const void *y, int64_t rows, int64_t cols, int64_t xs, int64_t ys,
                           IntentHipKernelResources *out);
-int softmax_bwd_resources(int dtype, const void *p, const void *dy, const void *dx, int64_t cols, int64_t ps, int64_t dys,
-                          int64_t dxs, IntentHipKernelResources *out);
+int softmax_bwd_resources(int dtype, const void *p, const void *dy, const void *dx, int64_t rows, int64_t cols, int64_t ps,
+                          int64_t dys, int64_t dxs, IntentHipKernelResources *out);
 int gemm_resources(int dtype, int activation, const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k,
                    int64_t lda, int64_t ldb, int64_t ldc, IntentHipKernelResources *out);
 int gemm_f32_resources(const void *a, const void *b, const void *c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,

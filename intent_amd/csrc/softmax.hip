@@ -17,9 +17,10 @@
 // before it computes the current one, so the reads of one row overlap the exponentials of the
 // previous (16384 x 4096 f16: 46.7 against 52 us, bit-identical; one wave per row and launch
 // leaves HBM idle while a whole round of waves computes).
-// Longer rows, and rows whose layout rules out aligned 128-bit access, belong to a workgroup
-// (softmax_*_block), which holds them in registers too, up to 131072 16-bit or 65536 f32 elements (forward;
-// backward half of that); rows beyond are read again in each pass (softmax_*_stream).
+// Longer rows belong to a workgroup (softmax_*_block), which holds them in registers too, up to 131072 16-bit or
+// 65536 f32 elements (forward; backward half of that); rows beyond are read again in each pass
+// (softmax_*_stream). Rows whose layout rules out aligned 128-bit access do too, except where a wave that reads
+// them element by element is faster (fwd_in_wave, bwd_in_wave).
 #include <math.h>
 
 #include <algorithm>
@@ -635,7 +636,7 @@ Variant pick_fwd_block(int64_t cols) {
   const int64_t elements = kRagged ? cols + kChunk<T> - 1 : cols;
 #define INTENT_ROW_KERNEL softmax_fwd_block
 #define INTENT_ROW_NAME "softmax_fwd_block"
-  if constexpr (kRagged) {
+  if constexpr (kRagged && sizeof(T) == 2) {   // shorter f32 rows belong to a wave
     INTENT_BLOCK(64, 1)
     INTENT_BLOCK(64, 2)
     INTENT_BLOCK(64, 4)
@@ -657,9 +658,11 @@ Variant pick_bwd_block(int64_t cols) {
   const int64_t elements = kRagged ? cols + kChunk<T> - 1 : cols;
 #define INTENT_ROW_KERNEL softmax_bwd_block
 #define INTENT_ROW_NAME "softmax_bwd_block"
-  if constexpr (kRagged) {
+  if constexpr (kRagged && sizeof(T) == 2) {   // shorter f32 rows belong to a wave
     INTENT_BLOCK(64, 1)
     INTENT_BLOCK(64, 2)
+  }
+  if constexpr (kRagged) {
     INTENT_BLOCK(64, 4)
     INTENT_BLOCK(64, 8)
   }
@@ -673,27 +676,22 @@ Variant pick_bwd_block(int64_t cols) {
 }
 #undef INTENT_BLOCK
 
+// Most chunks a wave holds: of single elements 1024 16-bit or 4096 f32 columns, of 16 bytes 4096 columns.
 template <typename T, int V>
+constexpr int kMostChunks = V == 1 ? (sizeof(T) == 4 ? 64 : 16) : sizeof(T) == 4 ? 16 : 8;
+
+template <typename T, int V, int CHUNKS = 1>
 Variant pick_fwd(int chunks) {
-  switch (chunks) {
-    case 1: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 1>), "softmax_fwd_wave"};
-    case 2: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 2>), "softmax_fwd_wave"};
-    case 4: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 4>), "softmax_fwd_wave"};
-    default: return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, 8>), "softmax_fwd_wave"};
-  }
+  if constexpr (CHUNKS < kMostChunks<T, V>)
+    if (chunks > CHUNKS) return pick_fwd<T, V, 2 * CHUNKS>(chunks);
+  return {reinterpret_cast<const void *>(&softmax_fwd_wave<T, V, CHUNKS>), "softmax_fwd_wave"};
 }
 
-template <typename T, int V>
+template <typename T, int V, int CHUNKS = 1>
 Variant pick_bwd(int chunks) {
-  switch (chunks) {
-    case 1: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 1>), "softmax_bwd_wave"};
-    case 2: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 2>), "softmax_bwd_wave"};
-    case 4: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 4>), "softmax_bwd_wave"};
-    case 16:
-      if constexpr (V == 4) return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 16>), "softmax_bwd_wave"};
-      [[fallthrough]];
-    default: return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, 8>), "softmax_bwd_wave"};
-  }
+  if constexpr (CHUNKS < kMostChunks<T, V>)
+    if (chunks > CHUNKS) return pick_bwd<T, V, 2 * CHUNKS>(chunks);
+  return {reinterpret_cast<const void *>(&softmax_bwd_wave<T, V, CHUNKS>), "softmax_bwd_wave"};
 }
 
 int round_chunks(int64_t cols, int per_chunk) {
@@ -703,34 +701,70 @@ int round_chunks(int64_t cols, int per_chunk) {
   return chunks;
 }
 
-// Up to 8 chunks a lane a wave holds an aligned row; longer rows belong to a workgroup, and so do ragged
-// ones, except short ones, whose ends are most of them: those stay with one element per lane and chunk
-// (16384 rows: 65 columns f16 4.6 us against 7.4, 129 f16 6.3 against 7.8, 257 f32 9.4 against 10.5; from there
-// on the workgroup leads: 450 f16 9.1 against 11.8, 1001 f16 16.4 against 31.9).
+// Rows that 16-byte access does not fit: in a wave, one element per lane and chunk (whose time follows the power of two
+// that the chunks round up to), or in a workgroup, which reads 16 bytes a lane and selects at the row's ends. While the
+// operands lie in the 256 MB of the MALL a wave's reads cost it less; past that HBM bounds both and whole lines
+// lead. Measured, workgroup over wave time:
+//   * f32 forward: 1.0 to 1.4 up to 2048 columns in the MALL, 0.77 to 0.95 past it (64M elements); from 2049 columns on
+//     0.5 (2^19 elements in all) to 1.0 (2^25);
+//   * f32 backward: 1.1 to 1.4 up to 2048 columns in the MALL, 0.88 to 0.97 past it; from 2049 on 0.6 to 1.07;
+//   * 16-bit forward: 1.1 to 1.4 up to 256 columns, then 1.0 to 1.2 below 2^23 elements and 0.8 to 1.0 from there; backward
+//     1.0 to 1.5 up to 384 columns in the MALL and 0.7 past it, then up to 800 columns 1.0 to 1.3 below 2^22 elements and
+//     0.6 to 1.0 from there, and beyond 0.5 to 1.05;
+//   * a row just past a step of the workgroup's registers leaves half of them idle: in the MALL, 16-bit from 506 to 640 columns
+//     1.0 to 1.6, from 1018 to 1024 0.92 to 1.31 (backward below 2^22 elements), f32 from 4094 to 4096 with 2048 rows or
+//     more 1.05 to 1.19.
 template <typename T>
-constexpr int64_t kShortRow = sizeof(T) == 4 ? 512 : 256;
+bool in_mall(int operands, int64_t rows, int64_t cols) {
+  return operands * static_cast<int64_t>(sizeof(T)) * rows * cols <= int64_t{256} << 20;
+}
 
 template <typename T>
-Variant select_fwd(const void *x, const void *y, int64_t cols, int64_t xs, int64_t ys) {
+bool fwd_in_wave(int64_t rows, int64_t cols) {
+  if (cols > 4096) return false;
+  if constexpr (sizeof(T) == 4)
+    return cols <= 512 || (in_mall<T>(2, rows, cols) && (cols <= 2048 || (cols > 4093 && rows >= 2048)));
+  const bool past_step = (cols > 505 && cols <= 640) || (cols > 1017 && cols <= 1024);
+  const bool few = cols <= 505 && rows * cols < int64_t{1} << 23;
+  return cols <= 256 || few || (past_step && in_mall<T>(2, rows, cols));
+}
+
+template <typename T>
+bool bwd_in_wave(int64_t rows, int64_t cols) {
+  if (cols > 4096) return false;
+  if constexpr (sizeof(T) == 4)
+    return cols <= 512 || (in_mall<T>(3, rows, cols) && (cols <= 2048 || (cols > 4093 && rows >= 2048)));
+  const bool any = cols <= 384 || (cols > 505 && cols <= 640);
+  const bool few = (cols <= 800 || (cols > 1017 && cols <= 1024)) && rows * cols < int64_t{1} << 22;
+  return cols <= 256 || few || (any && in_mall<T>(3, rows, cols));
+}
+
+// Aligned rows belong to a wave up to kMostChunks (f32 4096 x 4096 backward: 29.5 us, 31.7 in a workgroup). The f32 forward of
+// 2049 to 4096 columns does from 10M elements on that lie in the MALL (workgroup over wave time 0.97 to 1.13, 0.65 to 1.0
+// below, 0.76 to 0.85 past it).
+template <typename T>
+Variant select_fwd(const void *x, const void *y, int64_t rows, int64_t cols, int64_t xs, int64_t ys) {
   constexpr int kVec = kChunk<T>;
   const bool vector = cols % kVec == 0 && xs % kVec == 0 && ys % kVec == 0 && aligned(x, 16) && aligned(y, 16);
-  if (!vector) return cols <= kShortRow<T> ? pick_fwd<T, 1>(round_chunks(cols, kWave)) : pick_fwd_block<T, true>(cols);
+  if (!vector)
+    return fwd_in_wave<T>(rows, cols) ? pick_fwd<T, 1>(round_chunks(cols, kWave)) : pick_fwd_block<T, true>(cols);
   const int chunks = round_chunks(cols, kWave * kVec);
-  if (chunks > 8) return pick_fwd_block<T, false>(cols);
+  const bool wave = chunks <= 8 || (chunks <= kMostChunks<T, kVec> && rows * cols >= int64_t{10} << 20 && in_mall<T>(2, rows, cols));
+  if (!wave) return pick_fwd_block<T, false>(cols);
   if constexpr (sizeof(T) == 2) return pick_fwd_pipe<T>(chunks);
   else return pick_fwd<T, kVec>(chunks);
 }
 
 template <typename T>
-Variant select_bwd(const void *p, const void *dy, const void *dx, int64_t cols, int64_t ps, int64_t dys,
+Variant select_bwd(const void *p, const void *dy, const void *dx, int64_t rows, int64_t cols, int64_t ps, int64_t dys,
                    int64_t dxs) {
   constexpr int kVec = kChunk<T>;
   const bool vector = cols % kVec == 0 && ps % kVec == 0 && dys % kVec == 0 && dxs % kVec == 0 &&
                       aligned(p, 16) && aligned(dy, 16) && aligned(dx, 16);
-  if (!vector) return cols <= kShortRow<T> ? pick_bwd<T, 1>(round_chunks(cols, kWave)) : pick_bwd_block<T, true>(cols);
+  if (!vector)
+    return bwd_in_wave<T>(rows, cols) ? pick_bwd<T, 1>(round_chunks(cols, kWave)) : pick_bwd_block<T, true>(cols);
   const int chunks = round_chunks(cols, kWave * kVec);
-  // f32 4096 x 4096: 29.5 us in a wave, 31.7 in a workgroup.
-  return chunks > (sizeof(T) == 4 ? 16 : 8) ? pick_bwd_block<T, false>(cols) : pick_bwd<T, kVec>(chunks);
+  return chunks > kMostChunks<T, kVec> ? pick_bwd_block<T, false>(cols) : pick_bwd<T, kVec>(chunks);
 }
 
 // Input rows may overlap (any non-negative stride, e.g. a broadcast row); output
@@ -757,7 +791,7 @@ int64_t grid_blocks(const Variant &v, int64_t rows) {
 
 template <typename T>
 int launch_fwd(const void *x, void *y, int64_t rows, int64_t cols, int64_t xs, int64_t ys, hipStream_t stream) {
-  const Variant v = select_fwd<T>(x, y, cols, xs, ys);
+  const Variant v = select_fwd<T>(x, y, rows, cols, xs, ys);
   const dim3 grid(static_cast<unsigned>(grid_blocks(v, rows)));
   int icols = static_cast<int>(cols);
   void *args[] = {const_cast<void **>(&x), &y, &rows, &icols, &xs, &ys};
@@ -768,7 +802,7 @@ int launch_fwd(const void *x, void *y, int64_t rows, int64_t cols, int64_t xs, i
 template <typename T>
 int launch_bwd(const void *p, const void *dy, void *dx, int64_t rows, int64_t cols, int64_t ps, int64_t dys,
                int64_t dxs, hipStream_t stream) {
-  const Variant v = select_bwd<T>(p, dy, dx, cols, ps, dys, dxs);
+  const Variant v = select_bwd<T>(p, dy, dx, rows, cols, ps, dys, dxs);
   const dim3 grid(static_cast<unsigned>(grid_blocks(v, rows)));
   int icols = static_cast<int>(cols);
   void *args[] = {const_cast<void **>(&p), const_cast<void **>(&dy), &dx, &rows, &icols, &ps, &dys, &dxs};
@@ -778,25 +812,25 @@ int launch_bwd(const void *p, const void *dy, void *dx, int64_t rows, int64_t co
 
 }  // namespace
 
-int softmax_fwd_resources(int dtype, const void *x, const void *y, int64_t cols, int64_t xs, int64_t ys,
+int softmax_fwd_resources(int dtype, const void *x, const void *y, int64_t rows, int64_t cols, int64_t xs, int64_t ys,
                           IntentHipKernelResources *out) {
   Variant v;
   switch (dtype) {
-    case INTENT_HIP_F32: v = select_fwd<float>(x, y, cols, xs, ys); break;
-    case INTENT_HIP_F16: v = select_fwd<f16_t>(x, y, cols, xs, ys); break;
-    case INTENT_HIP_BF16: v = select_fwd<bf16_t>(x, y, cols, xs, ys); break;
+    case INTENT_HIP_F32: v = select_fwd<float>(x, y, rows, cols, xs, ys); break;
+    case INTENT_HIP_F16: v = select_fwd<f16_t>(x, y, rows, cols, xs, ys); break;
+    case INTENT_HIP_BF16: v = select_fwd<bf16_t>(x, y, rows, cols, xs, ys); break;
     default: return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "unknown dtype code %d", dtype);
   }
   return describe_kernel(v.kernel, v.name, v.block, out);
 }
 
-int softmax_bwd_resources(int dtype, const void *p, const void *dy, const void *dx, int64_t cols, int64_t ps, int64_t dys,
-                          int64_t dxs, IntentHipKernelResources *out) {
+int softmax_bwd_resources(int dtype, const void *p, const void *dy, const void *dx, int64_t rows, int64_t cols, int64_t ps,
+                          int64_t dys, int64_t dxs, IntentHipKernelResources *out) {
   Variant v;
   switch (dtype) {
-    case INTENT_HIP_F32: v = select_bwd<float>(p, dy, dx, cols, ps, dys, dxs); break;
-    case INTENT_HIP_F16: v = select_bwd<f16_t>(p, dy, dx, cols, ps, dys, dxs); break;
-    case INTENT_HIP_BF16: v = select_bwd<bf16_t>(p, dy, dx, cols, ps, dys, dxs); break;
+    case INTENT_HIP_F32: v = select_bwd<float>(p, dy, dx, rows, cols, ps, dys, dxs); break;
+    case INTENT_HIP_F16: v = select_bwd<f16_t>(p, dy, dx, rows, cols, ps, dys, dxs); break;
+    case INTENT_HIP_BF16: v = select_bwd<bf16_t>(p, dy, dx, rows, cols, ps, dys, dxs); break;
     default: return fail(INTENT_HIP_ERR_INVALID_ARGUMENT, "unknown dtype code %d", dtype);
   }
   return describe_kernel(v.kernel, v.name, v.block, out);

@@ -276,21 +276,65 @@ def test_softmax_specials_on_every_kernel(device, cols, kind):
         assert_16bit(got, want, rel=2.0 ** (-10 if kind == "f16" else -7), abs_=2.0 ** -24)
 
 
-@pytest.mark.parametrize("cols,pad,fwd,bwd", [
-    (1024, 0, ("softmax_fwd_pipe", 256), ("softmax_bwd_wave", 128)), (1024, 3, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)),
-    (255, 0, ("softmax_fwd_wave", 128), ("softmax_bwd_wave", 128)), (257, 0, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)),
-    (4104, 0, ("softmax_fwd_block", 256), ("softmax_bwd_block", 256)), (40000, 1, ("softmax_fwd_block", 1024), ("softmax_bwd_block", 1024)),
-    (140000, 0, ("softmax_fwd_stream", 1024), ("softmax_bwd_stream", 1024))])
-def test_softmax_observes_the_kernel_that_ran(device, cols, pad, fwd, bwd):
-    """Rows at a stride that leaves them unaligned are described as the kernel that takes them."""
-    announce("softmax observation", cols, pad)
-    view = lambda: torch.zeros(3, cols + pad, dtype=torch.float16, device=device)[:, :cols]  # noqa: E731
-    x, y, d = view(), view(), view()
-    for kernel, args, out, want in ((stable_softmax_f16, (x,), y, fwd), (softmax_backward_f16, (x, y), d, bwd)):
-        call = intent.jit(kernel, backend="hip").prepare(*args, outputs=(out,))
+WAVE, ROW = ("softmax_{}_wave", 128), lambda threads: ("softmax_{}_block", threads)  # noqa: E731
+
+
+@pytest.mark.parametrize("kind,rows,cols,pad,fwd,bwd", [
+    ("f16", 3, 1024, 0, ("softmax_fwd_pipe", 256), WAVE), ("f16", 3, 800, 1, ROW(256), WAVE), ("f16", 3, 1016, 3, ROW(256), ROW(256)), ("f16", 3, 255, 0, WAVE, WAVE),
+    ("f16", 3, 4104, 0, ROW(256), ROW(256)), ("f16", 3, 40000, 1, ROW(1024), ROW(1024)),
+    ("f16", 3, 140000, 0, ("softmax_fwd_stream", 1024), ("softmax_bwd_stream", 1024)),
+    ("f16", 32639, 257, 0, WAVE, WAVE), ("f16", 32641, 257, 0, ROW(256), WAVE), ("f16", 17000, 505, 0, ROW(256), ROW(256)),
+    ("f16", 17000, 506, 0, WAVE, WAVE), ("f16", 17000, 641, 0, ROW(256), ROW(256)), ("f16", 4100, 1022, 0, WAVE, WAVE),
+    ("f16", 4110, 1022, 0, WAVE, ROW(256)), ("f16", 3, 1025, 0, ROW(256), ROW(256)),
+    ("f16", 90000, 510, 0, WAVE, ROW(256)), ("f16", 132000, 510, 0, ROW(256), ROW(256)),
+    ("f16", 180000, 257, 0, ROW(256), ROW(256)), ("f32", 80000, 512, 1, WAVE, WAVE), ("f32", 16400, 2047, 0, ROW(256), ROW(256)),
+    ("f32", 3, 4000, 0, ROW(256), WAVE), ("f32", 2622, 4000, 0, WAVE, WAVE), ("f32", 8400, 4000, 0, ROW(256), WAVE),
+    ("f32", 10900, 2047, 0, WAVE, WAVE), ("f32", 10940, 2047, 0, WAVE, ROW(256)), ("f32", 3, 2049, 0, ROW(256), ROW(256)),
+    ("f32", 2047, 4095, 0, ROW(512), ROW(512)), ("f32", 2048, 4095, 0, WAVE, WAVE), ("f32", 3, 4096, 0, ROW(256), WAVE),
+    ("f32", 3, 4100, 0, ROW(512), ROW(512))])
+def test_softmax_observes_the_kernel_that_ran(device, kind, rows, cols, pad, fwd, bwd):
+    """Each line of the dispatch from both sides, and rows at a stride that leaves them unaligned."""
+    announce("softmax observation", kind, rows, cols, pad)
+    dtype = torch.float16 if kind == "f16" else torch.float32
+    p, dy, out = (torch.zeros(rows, cols + pad, dtype=dtype, device=device)[:, :cols] for _ in range(3))
+    lib, code, stride = hiplib.library(), getattr(hiplib, kind.upper()), cols + pad
+    at = [v.data_ptr() for v in (p, dy, out)]
+    if kind == "f16":
+        call = intent.jit(stable_softmax_f16, backend="hip").prepare(p, outputs=(out,))
         call.launch()
-        facts = {r.name: r.value for r in call.observation.resources}
-        assert (call.observation.kernel, facts["block_threads"]) == want
+        facts = {r.name: r.value for r in call.observation.resources} | {"kernel": call.observation.kernel}
+    else:
+        facts = lib.call_resources(hiplib.OP_SOFTMAX_FWD, code, at[0], at[2], rows, cols, stride, stride)
+    assert (facts["kernel"], facts["block_threads"]) == (fwd[0].format("fwd"), fwd[1])
+    facts = lib.call_resources(hiplib.OP_SOFTMAX_BWD, code, *at, rows, cols, stride, stride, stride)
+    assert (facts["kernel"], facts["block_threads"]) == (bwd[0].format("bwd"), bwd[1])
+
+
+# Many ragged rows: the sizes at which a workgroup takes rows that a wave takes when there are fewer, and their neighbours.
+@pytest.mark.parametrize("kind,rows,cols", [("f16", 32641, 257), ("f16", 17000, 505), ("f16", 17000, 515), ("f16", 9000, 1001),
+                                            ("bf16", 17000, 450), ("bf16", 9000, 1001), ("f32", 43000, 521), ("f32", 22400, 1001), ("f32", 33600, 1001), ("f32", 2700, 4000), ("f32", 8400, 4000),
+                                            ("f32", 11000, 2045), ("f32", 2500, 4095), ("f32", 5500, 4095)])
+def test_softmax_many_ragged_rows(device, kind, rows, cols):
+    """Forward and backward against float64 on the device, to the roundings of the sums (as above) and of the result."""
+    announce("softmax many ragged rows", kind, rows, cols)
+    dtype = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[kind]
+    lib, code, stream = hiplib.library(), getattr(hiplib, kind.upper()), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=device).manual_seed(cols)
+    x, dy = ((torch.randn(rows, cols, generator=g, device=device) * s).to(dtype) for s in (3, 1))
+    y, dx = torch.full_like(x, 7.0), torch.full_like(x, 7.0)
+    lib.check(lib.fn["softmax_fwd"](code, x.data_ptr(), y.data_ptr(), rows, cols, cols, cols, stream))
+    lib.check(lib.fn["softmax_bwd"](code, y.data_ptr(), dy.data_ptr(), dx.data_ptr(), rows, cols, cols, cols, cols, stream))
+    unit = {"f32": 1e-5, "f16": 2.0 ** -10, "bf16": 2.0 ** -7}[kind]
+    tiny = {"f32": 1e-37, "f16": 2.0 ** -24, "bf16": 1e-37}[kind]
+    for at in range(0, rows, 4096):
+        s = slice(at, at + 4096)
+        want, p, d = torch.softmax(x[s].double(), dim=1), y[s].double(), dy[s].double()
+        assert bool(((p - want).abs() <= unit * want + tiny).all())
+        proj = (p * d).sum(1, keepdim=True)
+        bound = p * 2.0 ** -24 * (160 * (p * d).abs().sum(1, keepdim=True) + 4 * (d - proj).abs())
+        if kind != "f32":
+            bound = bound + unit * (p * (d - proj)).abs() + tiny
+        assert bool(((dx[s].double() - p * (d - proj)).abs() <= bound + 1e-40).all())
 
 
 def test_softmax_longest_row(device):
