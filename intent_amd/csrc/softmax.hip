@@ -466,8 +466,8 @@ __global__ __launch_bounds__(kBlock) void softmax_bwd_wave(const T *p, const T *
   if (row >= rows) return;
   const T *pr = p + row * ps;
   const T *gr = dy + row * dys;
-  if constexpr (std::is_same<T, f16_t>::value && V == 8) {
-    // dy stays in its raw f16 words and is widened where it is used (the FMAs take f16 operands
+  if constexpr (sizeof(T) == 2 && V == 8) {
+    // dy stays in its raw words and is widened where it is used (f16: the FMAs take the operands
     // directly, v_fma_mix_f32): 81 VGPRs instead of 141, five waves per SIMD instead of three.
     // Backward of the 16384 x 4096 step, bit-identical outputs: 62.0 us, against 75.7 with both
     // rows widened at load and 68.0 with both kept raw (77 VGPRs, six waves). Every chunk is
