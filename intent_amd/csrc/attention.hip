@@ -46,6 +46,8 @@
 // workgroup's item names a sequence of rows in [U,H,D] tensors; and a per-key additive bias
 // (flash_attention_bias_fwd, attention.py:800-836), whose 64 floats per tile are DMA'd beside K
 // and V and enter each score as s (scale log2 e) + bias log2 e.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace intent_hip {
@@ -582,31 +584,37 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd(const uint16_t *__r
     }
 }
 
-// Items of the packed sequences, one workgroup: sequence s has ceil(rows / kBQ) query blocks. Under a causal mask, and with
-// up to 64 sequences, block j of every sequence that has one is listed before any block j - 1: the items'
-// walks (j + 1 blocks of keys) only get shorter, so the last workgroups to start are the shortest (8 prompts of up
-// to 2048 rows, HQ32 HK8 D128: 186 -> 180 us with the head order above). Otherwise
-// each sequence's blocks are listed from the last to the first, sequence after sequence. Offsets
+// Items of the packed sequences, one workgroup: sequence s has ceil(rows / kBQ) query blocks. Up to 64 sequences and
+// `longest_first` items (0: never), block j of every sequence that has one is listed before any block j - 1:
+// under a causal mask the items' walks (j + 1 blocks of keys) then only get shorter, so the last workgroups to start are
+// the shortest (longest_first_items). Otherwise each sequence's blocks are listed from the last to the first,
+// sequence after sequence, and the resident workgroups share the keys and values of fewer sequences. Offsets
 // are clamped into [0, total] and the list into its capacity, so no offsets can send a later
-// workgroup out of bounds.
+// workgroup out of bounds. A wave lists the first order, one lane a sequence; how the two compare with more sequences than
+// that was not measured.
 __global__ __launch_bounds__(1024) void attention_varlen_items(const int32_t *__restrict__ cu, int sequences,
                                                                int total, int2 *__restrict__ items,
                                                                int32_t *__restrict__ count, int capacity,
-                                                               int causal) {
+                                                               int longest_first) {
   __shared__ int s_wave[16];
   __shared__ int s_carry;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (causal && sequences <= 64) {   // uniform: the first wave lists them, lane s sequence s
-    if (wave > 0) return;
-    int blocks = 0;
+  int blocks = 0, most = 0, all = 0;
+  if (longest_first > 0 && sequences <= 64) {   // uniform: lane s of every wave holds sequence s
     if (lane < sequences) {
       const int start = min(max(cu[lane], 0), total);
       const int end = min(max(cu[lane + 1], start), total);
       blocks = (end - start + kBQ - 1) / kBQ;
     }
-    int most = blocks;
+    most = all = blocks;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
+    for (int d = 1; d < 64; d <<= 1) {
+      most = max(most, __shfl_xor(most, d));
+      all += __shfl_xor(all, d);
+    }
+  }
+  if (longest_first > 0 && sequences <= 64 && all <= longest_first) {   // the same in every wave; the first lists them
+    if (wave > 0) return;
     int at = 0;
     for (int j = most - 1; j >= 0; --j) {
       const uint64_t has = __ballot(blocks > j);
@@ -952,6 +960,18 @@ extern "C" int intent_hip_attention_bias_fwd(const void *q, const void *k, const
 // ---------------------------------------------------------------- packed sequences
 namespace {
 
+// Most items that attention_varlen_items lists longest walk first. That evens the ends of a few rounds of the chip's 256
+// CUs, but puts blocks of many sequences side by side, and past some rounds the lost sharing of keys and values in the
+// L2s outweighs the ends: the later the more query heads share a key head, and the shorter its rows. Causal, sequence
+// order against longest first in us (items x heads workgroups): HQ8 HK8 D64, 21 prompts of up to 1599 (624) 62.4, 46.0;
+// HQ32 HK8 D128, 8 of up to 2048 (1184) 170, 163; HQ16 HK16 D128, 32 of up to 2048 (2256) 302, 293; HQ32 HK32 D128,
+// 32 of up to 1024 (2848) 240, 253, 60 of up to 900 (4480) 317, 344; the same in D64 160, 152 and 213, 211, 32 of up to
+// 2048 (4512) 353, 360; HQ32 HK16 D128 (2848) 230, 228, (4512) 538, 560; HQ32 HK8 D128 (4480) 308, 304, (4512) 538, 543.
+int longest_first_items(int64_t heads, int64_t head_group, int64_t d) {
+  const int64_t workgroups = (head_group == 1 ? 9 : 8 * head_group) * 256 * (d == 64 ? 2 : 1);
+  return static_cast<int>(std::min<int64_t>(workgroups / heads, INT32_MAX));
+}
+
 int64_t varlen_capacity(int64_t sequences, int64_t total) { return (total + kBQ - 1) / kBQ + sequences; }
 size_t varlen_workspace(int64_t sequences, int64_t total) {
   return 256 + 8 * static_cast<size_t>(varlen_capacity(sequences, total));
@@ -1011,7 +1031,8 @@ extern "C" int intent_hip_attention_varlen_fwd(int dtype, const void *q, const v
   const hipStream_t s = as_stream(stream);
   attention_varlen_items<<<1, 1024, 0, s>>>(cu_seqlens, static_cast<int>(sequences), static_cast<int>(total),
                                             reinterpret_cast<int2 *>(ws + 256), reinterpret_cast<int32_t *>(ws),
-                                            static_cast<int>(capacity), causal ? 1 : 0);
+                                            static_cast<int>(capacity),
+                                            causal ? longest_first_items(q_heads, head_group, d) : 0);
   if (hipPeekAtLastError() != hipSuccess) return launch_status("attention_varlen_items");
   const dim3 grid(static_cast<unsigned>(capacity * q_heads));
   launch_variant<kPacked>(dtype, d, dv, grid, s, static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k),

@@ -148,3 +148,17 @@ def test_varlen_item_order(device, sequences, heads, group):
     k, v = (inputs.normal(g, (total, heads // group, 64), "f16") for _ in range(2))
     o = run_gqa(device, q, k, v, lengths, 0.125, group)
     assert_16bit(o, oracle.attention_varlen_fwd(q, k, v, offsets(lengths), 0.125, True, head_group=group))
+
+
+@pytest.mark.parametrize("sequences", [34, 35, 36])
+def test_varlen_item_order_lines(device, sequences):
+    """64 heads of their own keys at D = 128 list up to 36 items (2304 workgroups) longest walk first: 35, 36 and 37 items, the
+    longest sequence in the middle."""
+    announce("varlen item order lines", sequences)
+    g = np.random.default_rng(sequences)
+    lengths = [int(n) for n in g.integers(1, 12, sequences)]
+    lengths[sequences // 2] = 300
+    total = sum(lengths)
+    q, k, v = (inputs.normal(g, (total, 64, 128), "f16") for _ in range(3))
+    o = run_gqa(device, q, k, v, lengths, 0.088, 1)
+    assert_16bit(o, oracle.attention_varlen_fwd(q, k, v, offsets(lengths), 0.088, True, head_group=1))
