@@ -142,6 +142,7 @@ struct KeySplit {
   float *m, *den, *acc;
   int64_t rows;
   int grouped;
+  int run;   // head_runs: set by the launch, split or not
 };
 
 // Kernel modes: batched [B,H,S,D] tensors, packed sequences, batched with a key bias, or batched
@@ -172,11 +173,9 @@ __device__ __forceinline__ void lane_halves(float v, float &lo, float &hi) {
   hi = b;
 }
 
-// Index i of `count` dealt to the 8 XCDs in runs: workgroup x goes to XCD x % 8, so with `count` a multiple of 8
-// each XCD gets count / 8 consecutive indices, and query heads that share a key head share its L2 (B4 HQ32 HK8 S4096
-// D128 bf16 causal 671 -> 635 us, B4 HQ16 HK4 S1932 164 -> 156). Heads of their own keys share nothing and keep
-// the plain order (B4 H32 S4096 f16 causal: 0.4% slower in runs, level in the plain order, runs of one side 0.1 to 0.4% apart).
-__device__ __forceinline__ int xcd_run(int i, int count) { return count % 8 == 0 ? (i % 8) * (count / 8) + i / 8 : i; }
+// Index i dealt to the 8 XCDs in runs of `run` (0: in order): workgroup x goes to XCD x % 8, so each XCD gets `run`
+// consecutive indices (head_runs).
+__device__ __forceinline__ int xcd_run(int i, int run) { return run > 0 ? (i % 8) * run + i / 8 : i; }
 
 template <typename E, int D, int DV, int kMode>
 __global__ __launch_bounds__(kThreads, 2) void attention_fwd(const uint16_t *__restrict__ Q,
@@ -218,7 +217,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd(const uint16_t *__r
   if constexpr (kVarlen) {
     const int item = static_cast<int>(blockIdx.x) / heads;   // the heads of an item are neighbours
     h = static_cast<int>(blockIdx.x) % heads;
-    if (head_group > 1) h = xcd_run(h, heads);
+    h = xcd_run(h, split.run);
     if (item >= *r.count) return;                            // the grid covers the item capacity
     const int2 work = r.items[item];
     const int start = min(max(r.cu[work.x], 0), r.total);
@@ -237,7 +236,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd(const uint16_t *__r
     part = split.grouped ? x / items : x % split.count;
     const int bh_count = items / q_blocks;
     qb = q_blocks - 1 - item / bh_count;   // heaviest blocks first
-    const int nth = item % bh_count, bh = head_group > 1 ? xcd_run(nth, bh_count) : nth;
+    const int bh = xcd_run(item % bh_count, split.run);
     b = bh / heads;
     h = bh % heads;
     sq = sq_all;
@@ -755,11 +754,27 @@ using namespace intent_hip;
 
 namespace {
 
+// Consecutive (batch, head) pairs that one XCD gets (0: they go round the XCDs), so that query heads that share a key head
+// share its L2: B4 HQ32 HK8 S4096 D128 bf16 causal 671 -> 635 us, B4 HQ16 HK4 S1932 164 -> 156, B8 HQ32 HK8 S1024 f16 117
+// -> 108. Heads of their own keys share nothing and keep the plain order (B4 H32 S4096 f16 causal 0.4% slower in runs).
+// A part of the chip has no reads to save (under 128 workgroups: B1 HQ64 HK8 S128 D64 6.10 in order, 6.25 in runs). With
+// divided keys the splits of a block already meet in one L2: at D128 runs still lead or are within 3% (B1 HQ24 HK8
+// S1024 38.1 -> 36.5, HQ16 HK8 S2048 48.4 -> 46.4, HQ64 HK8 S768 50.4 -> 46.6; HQ32 HK8 S512 23.0 -> 23.7), at D64 from
+// 32 pairs on within 4% (HQ32 HK8 S512 16.7 -> 15.6, S768 22.3 -> 22.1, S600 20.9 -> 21.7), but 16 pairs, HQ16 HK8
+// S2048, 29.4 -> 30.8, unmasked 40.0 -> 43.4, and 24 pairs 60.3 -> 61.3.
+int head_runs(int64_t pairs, int q_blocks, int head_group, int splits, int d) {
+  if (head_group == 1 || pairs % 8 != 0) return 0;
+  if (splits > 1 ? d == 64 && pairs < 32 : pairs * q_blocks < 128) return 0;
+  return static_cast<int>(pairs / 8);
+}
+
 template <typename E, int D, int DV, int kMode>
 void launch_fwd(dim3 grid, hipStream_t s, const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *O,
                 int heads, int head_group, int sq, int sk, const Geometry &g, float scale, int causal, int q_blocks,
                 const Ragged &r, const KeyBias &kb, const RopeRows &rr = RopeRows{},
-                const KeySplit &split = KeySplit{1, nullptr, nullptr, nullptr}) {
+                KeySplit split = KeySplit{1, nullptr, nullptr, nullptr}) {
+  const int64_t pairs = kMode == kPacked ? heads : static_cast<int64_t>(grid.x) / split.count / q_blocks;
+  split.run = head_runs(pairs, kMode == kPacked ? static_cast<int>(grid.x / heads) : q_blocks, head_group, split.count, D);
   attention_fwd<E, D, DV, kMode><<<grid, dim3(kThreads), 0, s>>>(Q, K, V, O, heads, head_group, sq, sk, g, scale,
                                                                  causal, q_blocks, r, kb, rr, split);
 }
