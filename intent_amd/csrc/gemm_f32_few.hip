@@ -19,8 +19,8 @@ namespace {
 //     per row; column tile t is then the columns 4 r + t;
 //   * 16-byte loads need only 4-byte alignment, so every row stride takes this path; groups of 4 that
 //     reach past K, or past N for natural B, are loaded one element at a time, zeros past K.
-// Measured: linear_f32 256 x 1000 x 2048 158 -> 17.5 us (matrix-rate floor 7; the rest is the first loads, the LDS
-// sum and the second launch), 1 x 4096 x 4096 310 -> 20, 2048 x 1024 x 4096 316 -> 157 (110 TFLOP/s).
+// Measured: linear_f32 256 x 1000 x 2048 158 -> 17.6 us (matrix-rate floor 7; the rest is the first loads, the LDS
+// sum and the second launch), 1 x 4096 x 4096 310 -> 15, 2048 x 1024 x 4096 316 -> 144 (119 TFLOP/s).
 constexpr int kFewCols = 64, kFewUnit = 32, kFewWaves = 4;
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
@@ -173,10 +173,15 @@ __global__ __launch_bounds__(256) void gemm_f32_splits(const float *__restrict__
 }
 
 // Rows of a tile. 64 load two thirds of the operand bytes per product that 32 do, but with at most 128 such tiles
-// twice as many of 32 rows still run in one pass and leave fewer K parts to add: measured (32 against 64 rows)
-// 512^3 9.6 / 11.6 us, 1067 x 312 x 1560 20.7 / 33.5, 128 x 4096 x 1024 17.0 / 20.5, 256 x 1000 x 2048 19.2 / 20.0.
-// Past that a second pass costs more (640 x 832 x 1000, 130 tiles: 30.5 / 22.9; 1024^3 33.4 / 25.3), and in a long
-// K the bytes do (48 x 8192 x 2048 29.6 / 29.3, 128 x 4096 x 4096 52.7 / 49.0).
+// twice as many of 32 rows still run in one pass and leave fewer K parts to add; in a long K the bytes count for more.
+// Measured, 32 against 64 rows, a weight / natural B in us:
+//   * K to 1560: 512^3 9.2 / 8.8 against 10.9 / 10.3, 1067 x 312 x 1560 19.7 / 24.0 and 32.3 / 34.0, 128 x 4096 x 1024
+//     15.3 / 13.8 and 18.5 / 17.8;
+//   * K = 2048: 256 x 1000 17.6 / 17.6 and 18.6 / 18.3, 128 x 4096 25.8 / 25.5 and 26.1 / 27.5, 48 x 8192 25.8 / 25.7 and
+//     24.9 / 26.0;
+//   * K = 3072: 256 x 1000 23.0 / 24.6 and 22.6 / 23.4, 128 x 4096 36.7 / 38.3 and 34.4 / 36.3, 48 x 8192 36.5 / 38.0 and
+//     33.4 / 38.1.
+// More tiles pay a second pass: 640 x 832 x 1000 (130 tiles) 28.7 / 30.0 and 21.7 / 23.4, 1024^3 32.2 / 32.9 and 23.7 / 24.7.
 constexpr int64_t kFewTallTiles = 128, kFewTallDepth = 2048;
 int few_rows(int64_t m, int64_t n, int64_t k) {
   if (m <= 16) return 16;
@@ -188,8 +193,11 @@ int64_t few_tiles(int64_t m, int64_t n, int64_t k) {
   return (m + rows - 1) / rows * ((n + kFewCols - 1) / kFewCols);
 }
 
-// Workgroups along K: about one workgroup per CU, at least 128 k each, and only where the second
-// launch returns more than its 3 us (512^3: 9.6 us against 13.2 unsplit; 256 x 1000 x 2048: 19 against 42).
+// Workgroups along K: about one workgroup per CU, at least 128 k each. The second launch costs about 3 us, which the split
+// returns from K = 512 on, or is level there (a weight's product, divided against whole in us: 64 x 512 x 512 7.5 and
+// 9.2, 256 x 512 x 512 8.3 and 9.2, 512^3 9.4 and 9.3, 16 x 512 x 512 7.3 and 7.1; 512 x 512 x 1024 12.1 and 14.7,
+// 16 x 1024 x 1024 7.8 and 11.4, 256 x 1000 x 2048 17.6 and 25.1). Natural B is 0.4 to 1.8 us behind at K = 512 with 16
+// rows or 128 tiles and leads from 640 on.
 int few_splits(int64_t m, int64_t n, int64_t k) {
   if (m < 1 || n < 1 || k < 512) return 1;
   const int64_t tiles = few_tiles(m, n, k);

@@ -197,8 +197,8 @@ def test_softmax_config2_seed0_fwd_bwd(device):
 
 
 # Rows of a workgroup: both sides of every step of threads and chunks (16-bit 8192, 16384, 32768, 65536, 131072
-# elements; f32 half of that), ragged ends, short ragged rows (up to 256 and 512 elements) and their
-# successors, rows longer than any workgroup's registers.
+# elements; f32 half of that), ragged ends, ragged rows that are a wave's in these numbers (up to 1024 16-bit and 2048 f32
+# columns; many of them below), rows longer than any workgroup's registers.
 @pytest.mark.parametrize("rows,cols", [(5, 255), (5, 257), (9, 505), (3, 513), (7, 1017), (3, 2049), (2, 4095), (2, 4104),
                                        (3, 8185), (2, 8192), (2, 8200), (3, 16384), (2, 16392), (2, 32768), (2, 32776),
                                        (1, 65533), (2, 65544), (1, 131065), (1, 131072), (2, 131080), (1, 140001)])
