@@ -55,7 +55,7 @@ int paged_decode_resources(int64_t batch, int64_t kv_heads, int64_t group, int64
 int spmm_resources(int64_t features, IntentHipKernelResources *out);
 
 // f32 products of few output tiles (gemm_f32_few.hip); `workspace` may be null (one workgroup per tile).
-bool gemm_f32_few_applies(int64_t m, int64_t n);
+bool gemm_f32_few_applies(int64_t m, int64_t n, int64_t k);
 size_t gemm_f32_few_bytes(int64_t m, int64_t n, int64_t k);
 int gemm_f32_few_resources(int64_t m, int64_t n, int64_t k, int transpose_b, IntentHipKernelResources *out);
 int launch_gemm_f32_few(const float *a, const float *b, float *c, int M, int N, int K, int64_t lda, int64_t ldb,

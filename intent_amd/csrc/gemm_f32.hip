@@ -18,7 +18,7 @@
 //     halves, 8 rows apart, use different banks); W (linear_f32) is stored like A;
 //   * the MFMA computes the transposed tile (B fragment first), so each lane holds 4
 //     consecutive output columns of one row per register quad and stores them as one float4.
-// Products of up to 192 such tiles, or of up to 64 rows, run gemm_f32_few.hip instead, and so do layouts that are
+// Products of few such tiles, or of up to 64 rows, run gemm_f32_few.hip instead (gemm_f32_few_applies), and so do layouts that are
 // not 16-byte aligned or whose strides are not multiples of 4 (2048 x 4095 x 4095: 816 us here with scalar loads,
 // 620 - 660 there).
 #include "common.hpp"
@@ -174,7 +174,7 @@ bool large(const void *a, const void *b, const void *c, int64_t m, int64_t n, in
            int64_t ldc, int transpose_b) {
   const bool vec = k % 4 == 0 && (transpose_b || n % 4 == 0) && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
                    aligned(a, 16) && aligned(b, 16) && aligned(c, 16);
-  return vec && !gemm_f32_few_applies(m, n);
+  return vec && !gemm_f32_few_applies(m, n, k);
 }
 
 }  // namespace

@@ -215,12 +215,21 @@ const void *few_kernel(int rows, int transpose_b) { return transpose_b ? few_ker
 
 }  // namespace
 
-// The 128 x 128 kernel takes one round of the chip's 256 CUs for up to 256 tiles (k = 4096: 315 us) and
-// runs at 130 TFLOP/s with many; this one at about 108 whatever the tile count, so it leads up to about 192.
-bool gemm_f32_few_applies(int64_t m, int64_t n) { return m <= 64 || ((m + 127) / 128) * ((n + 127) / 128) <= 192; }
+// The 128 x 128 kernel takes one round of the chip's 256 CUs for up to 256 tiles (k = 4096: 315 us) and runs at 130 TFLOP/s
+// with many; this one at about 108 whatever the tile count, in one pass over the chip up to 64 of those tiles, in two up to 128
+// and three up to 192, each with first loads and an LDS sum that a short K does not hide. Measured, the 128 x 128
+// kernel's time over this one's, natural B / a weight: up to 64 tiles 1.0 to 5 at every K; 65 to 128 tiles K = 32 0.7 / 0.7,
+// 64 0.92 / 0.90, 96 1.1 / 1.04, 256 1.5 / 1.4; 129 to 192 tiles K = 64 0.7 / 0.7, 192 0.9 / 0.87, 320 0.98 / 0.92, 384 1.1 /
+// 1.0 (6144 x 512 0.94 / 0.93), 512 1.1 / 1.1. Up to 64 rows, half of a 128 x 128 tile: 64 x 16384 (128 tiles) K = 16 0.93 /
+// 0.94, 32 1.0 / 1.05, 64 1.4 / 1.4; 33 x 30000 (235) K = 32 0.67 / 0.71, 64 0.92 / 0.91, 96 1.1 / 1.1.
+bool gemm_f32_few_applies(int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = (m + 127) / 128 * ((n + 127) / 128);
+  if (m <= 64) return tiles <= 128 || k >= 96;
+  return tiles <= 64 || (tiles <= 128 && k >= 96) || (tiles <= 192 && k >= 384);
+}
 
 size_t gemm_f32_few_bytes(int64_t m, int64_t n, int64_t k) {
-  const int splits = gemm_f32_few_applies(m, n) ? few_splits(m, n, k) : 1;
+  const int splits = gemm_f32_few_applies(m, n, k) ? few_splits(m, n, k) : 1;
   return splits > 1 ? static_cast<size_t>(splits) * m * ((n + 3) / 4 * 4) * sizeof(float) : 0;
 }
 

@@ -192,9 +192,9 @@ def test_gemm_f32_few_tiles(device, m, n, k, workspace):
         assert (np.isnan(run(x, y).cpu().numpy()) == expected).all()
 
 
-# Above 192 tiles of 128 x 128: aligned ones, whose last row, column and K tiles are partly filled (gemm_f32_mfma), and one that
-# is not aligned (gemm_f32_few, undivided).
-@pytest.mark.parametrize("m,n,k", [(1800, 1804, 20), (1793, 1796, 36), (1801, 1803, 37), (1920, 1792, 16)])
+# Above 192 tiles of 128 x 128, and 130 of a short K: aligned ones, whose last row, column and K tiles are partly filled
+# (gemm_f32_mfma), and one that is not aligned (gemm_f32_few, undivided).
+@pytest.mark.parametrize("m,n,k", [(1800, 1804, 20), (1793, 1796, 36), (1801, 1803, 37), (1920, 1792, 16), (1250, 1660, 68)])
 def test_gemm_f32_many_tiles(device, m, n, k):
     test_gemm_f32_few_tiles(device, m, n, k, "prepare")
 
@@ -203,8 +203,13 @@ def test_gemm_f32_many_tiles(device, m, n, k):
 # the dispatch.
 F32_KERNELS = {(16, 64, 64): ("gemm_f32_few", 4 * 16 * 68 * 4), (17, 64, 64): ("gemm_f32_few", 4 * 32 * 68 * 4),
                (33, 64, 2048): ("gemm_f32_few", 4 * 32 * 68 * 4), (33, 64, 2049): ("gemm_f32_few", 4 * 64 * 68 * 4),
-               (129, 8256, 64): ("gemm_f32_few", 4 * 64 * 68 * 4), (1536, 2048, 64): ("gemm_f32_few", 4 * 64 * 68 * 4),
-               (1540, 2048, 64): ("gemm_f32_mfma", None), (1540, 2048, 65): ("gemm_f32_few", 4 * 64 * 68 * 4)}
+               (64, 16384, 16): ("gemm_f32_few", 4 * 64 * 68 * 4), (64, 16388, 92): ("gemm_f32_mfma", None),
+               (64, 16388, 96): ("gemm_f32_few", 4 * 64 * 68 * 4),
+               (1024, 1024, 16): ("gemm_f32_few", 4 * 64 * 68 * 4), (1028, 1024, 92): ("gemm_f32_mfma", None),
+               (1028, 1024, 96): ("gemm_f32_few", 4 * 64 * 68 * 4), (2048, 1024, 96): ("gemm_f32_few", 4 * 64 * 68 * 4),
+               (2052, 1024, 380): ("gemm_f32_mfma", None), (2052, 1024, 384): ("gemm_f32_few", 4 * 64 * 68 * 4),
+               (1536, 2048, 384): ("gemm_f32_few", 4 * 64 * 68 * 4), (1540, 2048, 384): ("gemm_f32_mfma", None),
+               (1540, 2048, 65): ("gemm_f32_few", 4 * 64 * 68 * 4)}
 
 
 @pytest.mark.parametrize("m,n,k", F32_KERNELS)
