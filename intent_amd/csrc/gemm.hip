@@ -84,7 +84,7 @@ template <typename E>
 __device__ __forceinline__ uint16_t f32_to_element(float v) { return __builtin_bit_cast(uint16_t, static_cast<E>(v)); }
 
 // Epilogues: quad(i, n, a, b, c, d) receives the f32 accumulators of output row i, columns n .. n+3
-// (n a multiple of 4); one(i, n, a) a single element (layouts that the DMA does not take). kSums: K may be divided over
+// (n a multiple of 4); some(i, n, count, v) the first `count` (1 or more) of 4 (layouts that the DMA does not take). kSums: K may be divided over
 // workgroups, whose sums gemm_splits adds before the epilogue.
 // gemm / bf16_gemm: act(acc) rounded to E.
 template <typename E, int kAct>
@@ -97,6 +97,18 @@ struct CastStore {
   }
   __device__ __forceinline__ void one(int i, int n, float a) const {
     C[static_cast<int64_t>(i) * ldc + n] = f32_to_element<E>(activate<kAct>(a));
+  }
+  __device__ __forceinline__ void some(int i, int n, int count, const float (&v)[4]) const {
+    if (count >= 4) {   // one 8-byte store at a 2-byte boundary (4000 x 4001 x 8
+                        // 20.7 us, 48.7 with four stores)
+      struct __attribute__((packed, aligned(2))) Quad { uint32_t w[2]; };
+      const uint2 w = __builtin_bit_cast(uint2, pack4<E, kAct>(v[0], v[1], v[2], v[3]));
+      *reinterpret_cast<Quad *>(C + static_cast<int64_t>(i) * ldc + n) = Quad{{w.x, w.y}};
+      return;
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (e < count) one(i, n + e, v[e]);
   }
 };
 
@@ -133,8 +145,18 @@ struct QuantizeStore {
                        (static_cast<uint32_t>(quantize(d, bias[n + 3], r3, scale[n + 3])) << 24);
     *reinterpret_cast<uint32_t *>(out + static_cast<int64_t>(i) * ldo + n) = q;
   }
-  __device__ __forceinline__ void one(int i, int n, float a) const {
-    out[static_cast<int64_t>(i) * ldo + n] = static_cast<int8_t>(quantize(a, bias[n], residual_at(i, n), scale[n]));
+  // Byte stores may alias every load, so the loads of a group come before its stores (4000 x 4001 x 8 69 us, 80 when
+  // each element's loads waited for the store before).
+  __device__ __forceinline__ void some(int i, int n, int count, const float (&v)[4]) const {
+    int32_t q[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int at = n + (e < count ? e : 0);
+      q[e] = quantize(v[e], bias[at], residual_at(i, at), scale[at]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (e < count) out[static_cast<int64_t>(i) * ldo + n + e] = static_cast<int8_t>(q[e]);
   }
 };
 
@@ -523,8 +545,8 @@ __global__ __launch_bounds__(256) void gemm_splits(const float *__restrict__ par
 // bytes of the busiest CU and the latency of its K steps, and the tiles are chosen to reach every CU.
 // The layouts are those of the 256 x 256 kernel, for any BM, BN and BK. kDma false, for operands that are
 // not 16-byte aligned or whose extents or strides are not multiples of 8: the same tiles through registers (two
-// steps ahead), with 16-byte loads at 2-byte boundaries, single elements only where a chunk reaches past K
-// or N, and single-element stores (bf16 2048 x 2049 x 2047: 97 us; 1222 in f32 FMAs).
+// steps ahead), with 16-byte loads and 8-byte stores at 2-byte boundaries, single elements only where a chunk reaches past
+// K or N (bf16 2048 x 2049 x 2047: 84 us; 1222 in f32 FMAs).
 template <int BM, int BN, int BK, int S, int WN>
 struct SmallTile {
   static constexpr int kThreads = 128 * WN;                       // 2 x WN waves
@@ -732,10 +754,8 @@ __global__ __launch_bounds__(128 * WN) void gemm_small(const uint16_t *__restric
                 make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
         } else if (kDma) {
           if (n < N) ep.quad(i, n, v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) ep.one(i, n + e, v[4 * g + e]);
+        } else if (n < N) {
+          ep.some(i, n, N - n, {v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]});
         }
       }
   }
