@@ -99,7 +99,7 @@ struct CastStore {
     C[static_cast<int64_t>(i) * ldc + n] = f32_to_element<E>(activate<kAct>(a));
   }
   __device__ __forceinline__ void some(int i, int n, int count, const float (&v)[4]) const {
-    if (count >= 4) {   // one 8-byte store at a 2-byte boundary (4000 x 4001 x 8
+    if (count >= 4) {   // one 8-byte store at a 2-byte boundary (4000 x 4001 x 8:
                         // 20.7 us, 48.7 with four stores)
       struct __attribute__((packed, aligned(2))) Quad { uint32_t w[2]; };
       const uint2 w = __builtin_bit_cast(uint2, pack4<E, kAct>(v[0], v[1], v[2], v[3]));

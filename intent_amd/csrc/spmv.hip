@@ -349,10 +349,19 @@ __device__ __forceinline__ void rows_block(const int32_t *__restrict__ off, cons
 // Short rows of a small matrix: one 16-lane group per row, 16 rows per workgroup. rows_block folds 1024 rows per
 // workgroup, which leaves most of the chip idle below some 10^5 rows, each wave walking up to 256 rows in steps
 // of four, a chain of loads each (19413 rows of up to 78: 29.7 us, 16.3 this way; 262100 of up to 100: 53.6,
-// 38.0; from 2^18 rows on the larger workgroups lead, their loads being enough to fill the chip). Up to 4 nonzeros: the group's
+// 38.0; from 2^18 rows on the larger workgroups lead, their loads being enough to fill the chip). Rows of up to four
+// nonzeros are one lane's in rows_block, so matrices of mostly such rows lead there much earlier, and the rows
+// per nonzero decide (folds_small). Up to 4 nonzeros: the group's
 // first lanes take one product each, added in order by all of them; 5 to 127 as in rows_block.
 constexpr int kSmallGroups = 256 / kGroup;
 constexpr int64_t kSmallRows = int64_t{1} << 18;
+// Measured, rows_block's time over rows_small's: rows of 0 to 4 (mean 2) 65536 rows 1.10, 100000 0.96, 131072 0.83, 262144 0.57;
+// a tenth of 20 among rows of 1 (mean 2.9) 131072 1.35, 180000 1.12, 262144 0.92; Zipf 167126 (mean 3.8) 1.57; rows of 4
+// 65536 1.10, 100000 0.98, 180000 0.78; of 2 to 8 or 5 262144 1.9 and 2.5, Zipf 224038 (4.7) 1.06; longer rows 1.9 to 6.
+bool folds_small(int64_t rows, int64_t nnz) {
+  if (nnz <= 5 * rows / 2) return rows <= 88 * 1024;
+  return rows <= (nnz <= 4 * rows ? 220 * 1024 : kSmallRows);
+}
 __device__ __forceinline__ void rows_small(const int32_t *__restrict__ off, const int32_t *__restrict__ col,
                                            const float *__restrict__ val, const float *__restrict__ x,
                                            float *__restrict__ y, int32_t rows, int32_t cols, int64_t nnz, int block) {
@@ -530,12 +539,13 @@ __device__ __forceinline__ void cut_block(const int32_t *__restrict__ off, const
 // per block; small matrices fold in the workgroups of rows_small). The cuts are chains of dependent probes, the short rows are bound by the fabric's
 // random line fetches; in one grid the cut chains run beside the short rows instead of after them
 // (config 5: 165 us for both, against 140 + 52 us as two launches).
-template <bool kSmall>   // up to kSmallRows rows: small_groups > 0, several cutting waves per block
+// kSmall: small_groups > 0 workgroups of rows_small fold the short rows. kShared: `shares` cutting waves per block.
+template <bool kSmall, bool kShared>
 __global__ __launch_bounds__(256) void spmv_rows(const int32_t *__restrict__ off, const int32_t *__restrict__ col,
                                                     const float *__restrict__ val, const float *__restrict__ x,
                                                     float *__restrict__ y, int32_t rows, int32_t cols, int64_t nnz,
                                                     Plan plan, int cut_groups, int shares, int small_groups) {
-  const int cut_shares = kSmall ? shares : 1;
+  const int cut_shares = kShared ? shares : 1;
   __shared__ int32_t s_list[4][kBlockRows];
   if (static_cast<int>(blockIdx.x) < cut_groups) {   // workgroup-uniform
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -869,14 +879,15 @@ extern "C" int intent_hip_csr_spmv_f32(const int32_t *row_offsets, const int32_t
   // Waves per block that cut its listed rows: one walks them all beside the short rows of a large matrix (4.2M rows 337
   // us, 352 with four waves); with few blocks that walk is what the launch waits for (27674 rows 54.7 us, 22.2
   // with 16; 100000 rows 80.7, 27.4; 250000 rows 83.6, 50.4 with four and 56.8 with 16).
-  static_assert(kSmallRows == 256 * kBlockRows, "large matrices cut with one wave per block");
   const int cut_shares = plan.blocks <= 128 ? 16 : plan.blocks <= 256 ? 4 : 1;
   const int cut_groups = listed ? (plan.blocks * cut_shares + 3) / 4 : 0;
-  const int small_groups = rows <= kSmallRows ? static_cast<int>((rows + kSmallGroups - 1) / kSmallGroups) : 0;
+  const int small_groups = folds_small(rows, nnz) ? static_cast<int>((rows + kSmallGroups - 1) / kSmallGroups) : 0;
   const int list_blocks = small_groups > 0 && !listed ? 0 : plan.blocks;
   if (list_blocks > 0)
     spmv_count<<<dim3(static_cast<unsigned>(plan.supers)), dim3(256 * kSuperBlocks), 0, s>>>(row_offsets, r32, nnz, plan);
-  const auto rows_kernel = small_groups > 0 ? &spmv_rows<true> : &spmv_rows<false>;
+  const auto rows_kernel = small_groups > 0 ? &spmv_rows<true, true>
+                           : cut_shares > 1 ? &spmv_rows<false, true>
+                                            : &spmv_rows<false, false>;
   rows_kernel<<<dim3(static_cast<unsigned>(list_blocks + cut_groups + small_groups)), dim3(256), 0, s>>>(
       row_offsets, column_indices, values, x, y, r32, c32, nnz, plan, cut_groups, cut_shares, small_groups);
   if (hipPeekAtLastError() != hipSuccess) return launch_status("spmv_rows");

@@ -318,3 +318,27 @@ def test_listed_rows_of_small_matrices(device, rows, cols):
         got = run(device, offsets, columns, values, vec)
         assert (np.abs(got - want) <= bound).all()
     assert (got == want).all()
+
+
+@pytest.mark.parametrize("rows", [70000, 91000, 130000, 262144])
+def test_mostly_short_rows_fold_in_large_blocks(device, rows):
+    """Matrices of 0 to 4 nonzeros a row and a few listed rows, on both sides of the line past which their short rows are one lane's
+    again, while several waves still cut a block's listed rows: bit-identical to the same rows in a matrix of more than 2^18,
+    exact on rows of up to 4 nonzeros and within a float64 sum's bound elsewhere."""
+    announce("spmv mostly short rows", rows)
+    cols = 1200000
+    rng = np.random.default_rng(rows)
+    lengths = rng.integers(0, 5, rows)
+    lengths[rng.integers(0, rows, 25)] = rng.integers(5, 1500, 25)
+    lengths[-1] = 900
+    offsets, columns = inputs.csr_matrix(rng, lengths, cols)
+    assert 2 * int(offsets[-1]) < 5 * rows
+    values, vec = inputs.uniform(rng, int(offsets[-1]), -1, 1), inputs.uniform(rng, cols, -1, 1)
+    got = run(device, offsets, columns, values, vec)
+    more = np.concatenate([offsets, np.full((1 << 18) + 1 - rows, offsets[-1])]).astype(np.int32)
+    assert np.array_equal(got, run(device, more, columns, values, vec)[:rows])
+    products = values.astype(np.float64) * vec[columns]
+    row_of = np.repeat(np.arange(rows), lengths)
+    assert (np.abs(got - np.bincount(row_of, products, rows)) <= 1e-5 * np.bincount(row_of, np.abs(products), rows)).all()
+    short = lengths <= 4
+    assert np.array_equal(got[short], oracle.csr_spmv(offsets, columns, values, vec)[short])
