@@ -639,6 +639,8 @@ Variant pick_fwd_block(int64_t cols) {
   if constexpr (kRagged && sizeof(T) == 2) {   // shorter f32 rows belong to a wave
     INTENT_BLOCK(64, 1)
     INTENT_BLOCK(64, 2)
+  }
+  if constexpr (kRagged) {
     INTENT_BLOCK(64, 4)
     INTENT_BLOCK(64, 8)
   }

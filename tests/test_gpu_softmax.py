@@ -310,6 +310,18 @@ def test_softmax_observes_the_kernel_that_ran(device, kind, rows, cols, pad, fwd
     assert (facts["kernel"], facts["block_threads"]) == (bwd[0].format("bwd"), bwd[1])
 
 
+def test_softmax_ragged_f32_rows_past_the_mall_go_four_to_a_workgroup(device):
+    """Up to 2048 columns a wave holds the row (no shared memory for partial results): one workgroup a row is bound by their
+    launches (91500 x 550: 185 us, 65)."""
+    announce("softmax f32 waves of a workgroup")
+    lib, x = hiplib.library(), torch.zeros(61100, 1101, device=device)
+    for cols, rows in ((550, 61100), (1021, 34000), (1101, 61100)):
+        at = (x.data_ptr(), x.data_ptr(), x.data_ptr())
+        for op, args in ((hiplib.OP_SOFTMAX_FWD, at[:2]), (hiplib.OP_SOFTMAX_BWD, at)):
+            facts = lib.call_resources(op, hiplib.F32, *args, rows, cols, *[1101] * len(args))
+            assert (facts["block_threads"], facts["lds_bytes"]) == (256, 0)
+
+
 # Many ragged rows: the sizes at which a workgroup takes rows that a wave takes when there are fewer, and their neighbours.
 @pytest.mark.parametrize("kind,rows,cols", [("f16", 32641, 257), ("f16", 17000, 505), ("f16", 17000, 515), ("f16", 9000, 1001),
                                             ("bf16", 17000, 450), ("bf16", 9000, 1001), ("f32", 43000, 521), ("f32", 22400, 1001), ("f32", 33600, 1001), ("f32", 2700, 4000), ("f32", 8400, 4000),
