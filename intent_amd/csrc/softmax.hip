@@ -20,7 +20,7 @@
 // Longer rows belong to a workgroup (softmax_*_block), which holds them in registers too, up to 131072 16-bit or
 // 65536 f32 elements (forward; backward half of that); rows beyond are read again in each pass
 // (softmax_*_stream). Rows whose layout rules out aligned 128-bit access do too, except where a wave that reads
-// them element by element is faster (fwd_in_wave, bwd_in_wave).
+// them element by element is faster (in_wave).
 #include <math.h>
 
 #include <algorithm>
@@ -360,17 +360,29 @@ __device__ __forceinline__ float block_reduce(float v, float *parts) {
 template <int THREADS>
 constexpr int kBlockRows = THREADS == kWave ? 4 : 1;
 
+// The row of workgroup `slot`: rows 16 g + 2 x and 16 g + 2 x + 1 on XCD x, where softmax_bwd_wave, of two rows a workgroup,
+// has them. Aligned f32 rows of 2049 to 4096 columns meet both kernels in one step, and what one wrote is then in
+// the L2 that the other reads (forward and backward of 1024 x 3072 10.2 us, 15.7 in plain order; 2048 x 4096 25.6, 29.1). Where
+// both kernels have one row a workgroup the plain order is faster (f16 384 x 16384 11.4 us, 13.7 in this one).
+__device__ __forceinline__ int64_t paired_row(int64_t slot, int64_t rows) {
+  if (slot >= rows / 16 * 16) return slot;
+  const int64_t in = slot % 16;
+  return slot - in + 2 * (in % 8) + in / 8;
+}
+
 template <typename T, int THREADS, int CHUNKS, bool kRagged>
 __global__ __launch_bounds__(THREADS * kBlockRows<THREADS>) void softmax_fwd_block(const T *x, T *y, int64_t rows, int cols, int64_t xs,
                                                              int64_t ys) {
   constexpr int V = kChunk<T>;
   constexpr bool kHold = CHUNKS * V <= 64;
   constexpr int kRows = kBlockRows<THREADS>;
+  constexpr bool kPaired = sizeof(T) == 4 && !kRagged && THREADS == 256;
   __shared__ float maxima[THREADS / kWave], sums[THREADS / kWave];
   const int thread = kRows > 1 ? threadIdx.x % THREADS : threadIdx.x;
   const Span span = span_of(x, rows, cols, xs);
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * kRows + threadIdx.x / THREADS; row < rows;
-       row += static_cast<int64_t>(gridDim.x) * kRows) {
+  for (int64_t slot = static_cast<int64_t>(blockIdx.x) * kRows + threadIdx.x / THREADS; slot < rows;
+       slot += static_cast<int64_t>(gridDim.x) * kRows) {
+    const int64_t row = kPaired ? paired_row(slot, rows) : slot;
     const T *xr = x + row * xs;
     T *yr = y + row * ys;
     const int shift = kRagged ? row_shift(xr) : 0;
@@ -710,35 +722,26 @@ int round_chunks(int64_t cols, int per_chunk) {
 //   * f32 forward: 1.0 to 1.4 up to 2048 columns in the MALL, 0.77 to 0.95 past it (64M elements); from 2049 columns on
 //     0.5 (2^19 elements in all) to 1.0 (2^25);
 //   * f32 backward: 1.1 to 1.4 up to 2048 columns in the MALL, 0.88 to 0.97 past it; from 2049 on 0.6 to 1.07;
-//   * 16-bit forward: 1.1 to 1.4 up to 256 columns, then 1.0 to 1.2 below 2^23 elements and 0.8 to 1.0 from there; backward
-//     1.0 to 1.5 up to 384 columns in the MALL and 0.7 past it, then up to 800 columns 1.0 to 1.3 below 2^22 elements and
-//     0.6 to 1.0 from there, and beyond 0.5 to 1.05;
-//   * a row just past a step of the workgroup's registers leaves half of them idle: in the MALL, 16-bit from 506 to 640 columns
-//     1.0 to 1.6, from 1018 to 1024 0.92 to 1.31 (backward below 2^22 elements), f32 from 4094 to 4096 with 2048 rows or
-//     more 1.05 to 1.19.
+//   * 16 bits, one rule for both directions, by the time of a forward and a backward in turn (where one takes the wave and
+//     the other the workgroup, a step loses up to 5 us below 2^23 elements and a quarter past it): up to 384
+//     columns 0.97 to 1.2 in the MALL, 0.94 to 1.06 past it; to 505 0.96 to 1.1 below 3M elements, 0.83 to 1.0 from there; to
+//     640, just past a step of the workgroup's registers, 0.94 to 1.2 in the MALL; to 1017 0.83 to 1.1; to 1024, the next
+//     step, 1.01 to 1.17 below 6M, 0.86 to 1.04 from there; then 0.7 to 0.97;
+//   * f32 from 4094 to 4096 columns, a step as well, with 2048 rows or more 1.05 to 1.19 in the MALL.
 template <typename T>
 bool in_mall(int operands, int64_t rows, int64_t cols) {
   return operands * static_cast<int64_t>(sizeof(T)) * rows * cols <= int64_t{256} << 20;
 }
 
+// `operands`: how many of the call's arrays lie in the MALL.
 template <typename T>
-bool fwd_in_wave(int64_t rows, int64_t cols) {
+bool in_wave(int operands, int64_t rows, int64_t cols) {
   if (cols > 4096) return false;
   if constexpr (sizeof(T) == 4)
-    return cols <= 512 || (in_mall<T>(2, rows, cols) && (cols <= 2048 || (cols > 4093 && rows >= 2048)));
-  const bool past_step = (cols > 505 && cols <= 640) || (cols > 1017 && cols <= 1024);
-  const bool few = cols <= 505 && rows * cols < int64_t{1} << 23;
-  return cols <= 256 || few || (past_step && in_mall<T>(2, rows, cols));
-}
-
-template <typename T>
-bool bwd_in_wave(int64_t rows, int64_t cols) {
-  if (cols > 4096) return false;
-  if constexpr (sizeof(T) == 4)
-    return cols <= 512 || (in_mall<T>(3, rows, cols) && (cols <= 2048 || (cols > 4093 && rows >= 2048)));
-  const bool any = cols <= 384 || (cols > 505 && cols <= 640);
-  const bool few = (cols <= 800 || (cols > 1017 && cols <= 1024)) && rows * cols < int64_t{1} << 22;
-  return cols <= 256 || few || (any && in_mall<T>(3, rows, cols));
+    return cols <= 512 || (in_mall<T>(operands, rows, cols) && (cols <= 2048 || (cols > 4093 && rows >= 2048)));
+  if (cols <= 256) return true;
+  if (cols <= 384 || (cols > 505 && cols <= 640)) return in_mall<T>(3, rows, cols);
+  return (cols <= 505 && rows * cols < int64_t{3} << 20) || (cols > 1017 && cols <= 1024 && rows * cols < int64_t{6} << 20);
 }
 
 // Aligned rows belong to a wave up to kMostChunks (f32 4096 x 4096 backward: 29.5 us, 31.7 in a workgroup). The f32 forward of
@@ -749,7 +752,7 @@ Variant select_fwd(const void *x, const void *y, int64_t rows, int64_t cols, int
   constexpr int kVec = kChunk<T>;
   const bool vector = cols % kVec == 0 && xs % kVec == 0 && ys % kVec == 0 && aligned(x, 16) && aligned(y, 16);
   if (!vector)
-    return fwd_in_wave<T>(rows, cols) ? pick_fwd<T, 1>(round_chunks(cols, kWave)) : pick_fwd_block<T, true>(cols);
+    return in_wave<T>(2, rows, cols) ? pick_fwd<T, 1>(round_chunks(cols, kWave)) : pick_fwd_block<T, true>(cols);
   const int chunks = round_chunks(cols, kWave * kVec);
   const bool wave = chunks <= 8 || (chunks <= kMostChunks<T, kVec> && rows * cols >= int64_t{10} << 20 && in_mall<T>(2, rows, cols));
   if (!wave) return pick_fwd_block<T, false>(cols);
@@ -764,7 +767,7 @@ Variant select_bwd(const void *p, const void *dy, const void *dx, int64_t rows, 
   const bool vector = cols % kVec == 0 && ps % kVec == 0 && dys % kVec == 0 && dxs % kVec == 0 &&
                       aligned(p, 16) && aligned(dy, 16) && aligned(dx, 16);
   if (!vector)
-    return bwd_in_wave<T>(rows, cols) ? pick_bwd<T, 1>(round_chunks(cols, kWave)) : pick_bwd_block<T, true>(cols);
+    return in_wave<T>(3, rows, cols) ? pick_bwd<T, 1>(round_chunks(cols, kWave)) : pick_bwd_block<T, true>(cols);
   const int chunks = round_chunks(cols, kWave * kVec);
   return chunks > kMostChunks<T, kVec> ? pick_bwd_block<T, false>(cols) : pick_bwd<T, kVec>(chunks);
 }
